@@ -2,10 +2,9 @@
 // the reference calls F.linear for all of them: layers/linear.py:26,45, models/qwen3.py:21,47,
 // layers/embed_head.py:23).
 //
-//  * me_gemm_tiled: any shape, float32 or bfloat16 inputs, float32 accumulation with plain FMAs
-//    (no matrix-core, no reduced precision). Each output element is one thread's sequential sum
-//    over K, so a row's result does not depend on the other rows of the batch. This is the
-//    float32 path and the fallback for bf16 shapes the MFMA kernel refuses.
+//  * me_gemm_tiled: any shape, bfloat16 inputs, float32 accumulation with plain FMAs: the fallback for shapes
+//    the MFMA kernels refuse. Each output element is one thread's sequential sum over K, so a row's result does
+//    not depend on the other rows of the batch. (The float32 path's product: gemm_f32.hip.)
 //  * me_gemm_skinny_bf16: the decode product, up to 64 rows (the caller decides from which row
 //    count the library is faster). Pure weight streaming: each workgroup owns 16 output features, its 4 waves split
 //    K, a wave reads 256 contiguous bytes of each of its 16 weight rows per step (each load takes 64
@@ -62,17 +61,14 @@ gemm_tiled_kernel(const TI* __restrict__ x, int64_t ldx, const TI* __restrict__ 
 }
 
 extern "C" int me_gemm_tiled(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, int64_t ldy,
-                             int in_dtype, int out_dtype, int M, int N, int K, hipStream_t stream) {
+                             int out_dtype, int M, int N, int K, hipStream_t stream) {
   if (M == 0 || N == 0) return 0;
   ME_CHECK(K >= 1 && ldx >= K && ldw >= K && ldy >= N, "gemm: bad leading dimensions");
   dim3 grid((N + GT_TILE - 1) / GT_TILE, (M + GT_TILE - 1) / GT_TILE), block(256);
   ME_CHECK(grid.y <= 65535, "gemm: too many rows (%d) for one launch", M);
-#define LAUNCH(TI, TO) \
-  gemm_tiled_kernel<TI, TO><<<grid, block, 0, stream>>>((const TI*)x, ldx, (const TI*)w, ldw, (TO*)y, ldy, M, N, K)
-  if (in_dtype == ME_F32 && out_dtype == ME_F32) LAUNCH(float, float);
-  else if (in_dtype == ME_BF16 && out_dtype == ME_BF16) LAUNCH(bf16_t, bf16_t);
-  else if (in_dtype == ME_BF16 && out_dtype == ME_F32) LAUNCH(bf16_t, float);
-  else ME_CHECK(false, "gemm: unsupported dtype pair %d -> %d", in_dtype, out_dtype);
+#define LAUNCH(TO) \
+  gemm_tiled_kernel<bf16_t, TO><<<grid, block, 0, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, ldw, (TO*)y, ldy, M, N, K)
+  if (out_dtype == ME_BF16) LAUNCH(bf16_t); else LAUNCH(float);
 #undef LAUNCH
   ME_LAUNCH_CHECK();
   return 0;

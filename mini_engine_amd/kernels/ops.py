@@ -67,7 +67,8 @@ _CORE_PROTOS = {
     "me_store_kv": [P, P, I, L, L, L, P, P, P, I, I, I, P],
     "me_attn_simple": [P, L, P, L, I, P, P, P, I, P, P, P, L, I, I, I, I, F, I, I, F, P, P, P],
     "me_attn_tail": [P, L, P, L, P, I, P, P, P, I, P, P, P, L, I, I, I, I, F, I, I, F, P, P, P],
-    "me_gemm_tiled": [P, L, P, L, P, L, I, I, I, I, I, P],
+    "me_gemm_tiled": [P, L, P, L, P, L, I, I, I, I, P],
+    "me_gemm_f32": [P, L, P, L, P, L, I, I, I, I, I, P],
     "me_gemm_skinny_bf16": [P, L, P, L, P, L, I, P, I, I, I, I, I, I, I, F, F, P, P],
     "me_gemm_rows_bf16": [P, L, P, L, P, L, I, P, I, I, I, I, I, P],
     "me_gemm_skinny_norm_bf16": [P, I, I, P, P, P, F, P, L, P, L, I, I, I, I, I, P],
@@ -430,7 +431,8 @@ class HipBackend:
         On the matrix-core path the cap and the slopes run inside the kernels (library variants of their own), and so do
         the sinks where a launch forms or merges its last sums. Kept keys behind a window are joined by a second kernel
         (`attn_tail`, then with the sinks) to a softmax whose denominators' logarithms the first has left.
-        The float32 path and odd sizes take the exact kernel (`attn_simple`) for all of it.
+        The float32 path takes `attn_f32` (float32 matrix instructions) for head sizes up to 128 in steps of 16 and pages in
+        steps of 4 keys; odd sizes take the exact kernel (`attn_simple`) for all of it.
 
         q: [T, Hq*D] (a strided view is fine). Rows are ordered decode requests first (one token
         each, `num_decodes` of them), then the others; `prefill_cu` int32 [B - num_decodes + 1]
@@ -566,7 +568,7 @@ class HipBackend:
                allow_partials: bool = False, out: torch.Tensor | None = None):
         """x [M, K] . w[N, K]^T (reference layers/linear.py:25-26: F.linear, no bias).
 
-        float32: plain FMA kernel. bfloat16: the skinny MFMA kernel for up to 32 rows (64 for
+        float32: the float32 matrix instructions (f32_tile). bfloat16: the skinny MFMA kernel for up to 32 rows (64 for
         smaller weights or when K is split), the library product (hipBLASLt, library_product) above
         that, for the head over a large vocabulary and for large weights with several rows
         (library_streams_better), the FMA kernel for shapes the MFMA kernel refuses.
@@ -589,15 +591,15 @@ class HipBackend:
         if x.dtype == torch.float32:
             _check(out_dtype == torch.float32, "linear: float32 inputs give float32 outputs")
             y = new()
-            core().call("me_gemm_tiled", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N,
-                        ME_F32, ME_F32, M, N, K, _stream())
+            core().call("me_gemm_f32", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N,
+                        M, N, K, *f32_tile(M, N), _stream())
             return y
         aligned = (K % 8 == 0 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
                    and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
         if not aligned:
             y = new()
             core().call("me_gemm_tiled", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N,
-                        ME_BF16, _code(out_dtype), M, N, K, _stream())
+                        _code(out_dtype), M, N, K, _stream())
             return y
         mid_parts = mid_takes(M, N, K, True) if (allow_partials and out_dtype == x.dtype) else 0
         if mid_parts > 1:
@@ -1286,6 +1288,8 @@ class HipBackend:
 
 # Dispatch rules. Every threshold below was measured on one MI355X at the layer sizes of Qwen3-0.6B, 8B and 32B;
 # the tables behind each constant are kept in the repository's design notes, one line of reason here.
+# microseconds that one round of the float32 product's tiles takes over a K of 1,024: alone, and each of several
+F32_ROUND_US = {(16, 16): (6.9, 5.9), (16, 32): (7.5, 7.1), (32, 32): (9.2, 9.0), (64, 32): (12.0, 13.5), (64, 64): (19.7, 29.5)}
 SKINNY_MAX_M = 32                          # rows up to which the skinny kernel beats the library product
 SKINNY_WIDE_MAX_M = 64                     # ... for weights of up to SKINNY_WIDE_MAX_WEIGHT elements
 SKINNY_WIDE_MAX_WEIGHT = 5 * 1024 * 1024
@@ -1407,6 +1411,16 @@ def prefill_segments(max_context: int, window: int, num_tokens: int, Hq: int, D:
 
 
 SKINNY_WIDE_MIN_WEIGHT = 1 << 22
+
+
+def f32_tile(M: int, N: int) -> tuple:
+    """(rows, features) of the float32 product's tile: the one whose rounds of workgroups over the compute units cost least
+    (F32_ROUND_US; the bits of a result do not depend on it)."""
+    def cost(tile):
+        rounds = -(-(-(-M // tile[0]) * -(-N // tile[1])) // _COMPUTE_UNITS)
+        first, more = F32_ROUND_US[tile]
+        return first if rounds == 1 else rounds * more
+    return min(F32_ROUND_US, key=cost)
 
 
 def skinny_wide(N: int, K: int) -> int:
