@@ -1,6 +1,6 @@
 // Paged causal attention, the exact and slow form: one workgroup per (query token, head),
-// scalar float32 arithmetic throughout. It is the float32 path of the engine and takes any
-// head size, page size and head grouping.
+// scalar float32 arithmetic throughout. It takes any head size, page size and head grouping; the float32 path's
+// usual sizes run on the float32 matrix instructions instead (attn_f32 below).
 //
 // Formulas as in the reference's pure-torch paged path (layers/attention.py:21-40): key j of
 // the request is kept iff j <= position of the query (and j < context length); scores are
@@ -128,6 +128,194 @@ attn_simple_kernel(const T* __restrict__ q, int64_t q_stride, T* __restrict__ ou
     if (tid + dd * AS_THREADS < D) out[t * out_stride + (int64_t)h * D + tid + dd * AS_THREADS] = from_f32<T>(acc[dd] * inv);
 }
 
+// ------------------------------------------------------------------ the same on the float32 matrix instructions
+// Head sizes up to 128 in steps of 16, pages in steps of 4 keys: products on v_mfma_f32_16x16x4_f32 (float32 operands,
+// products and sums), up to 16 tokens of one request and one head to a workgroup. attn_simple reads every key row and value row
+// once per token from a thread of its own; here they are read once per 16 tokens in pieces of 16 bytes, and what bounds a
+// workgroup is its chain of blocks (64 matrix instructions of 32 cycles for 16 keys at head size 128). A prompt of 300 tokens,
+// 16 heads of 128: 279 -> 25 us. Larger heads would need more registers than a wave has and stay with attn_simple, as do
+// odd head sizes and pages.
+//
+// S^T = K Q^T with the keys as the 16-row operand: a lane then holds the scores of keys 4 g .. 4 g + 3 (g: its lane
+// group) for token lane % 16, which is the operand that O^T += V^T P^T wants, with the lanes' keys as its k. Keys go in
+// blocks of 16 counted from position 0, block i to wave i mod 4; every wave keeps a running maximum, sum and result of its
+// own, and the four meet at the end in one order. A block in which a token sees nothing leaves its numbers as they
+// are, so a token's bits do not depend on the others of its tile, i.e. on how the request was cut.
+// Values of keys that a token does not see meet a probability of zero; where such a value is not a finite number it is
+// taken out of the product and joined by hand for the tokens that do see it.
+template <int NS>        // head size / 16
+__global__ void __launch_bounds__(256)
+attn_f32_kernel(const float* __restrict__ q, int64_t q_stride, float* __restrict__ out, int64_t out_stride,
+                const float* __restrict__ k_cache, const float* __restrict__ v_cache, const int32_t* __restrict__ block_tables,
+                int bt_stride, const int32_t* __restrict__ seq_of_token, const int32_t* __restrict__ positions,
+                const int32_t* __restrict__ context_lens, int num_tokens, int Hq, int Hkv, int page, float scale, int window,
+                int keep_first, float softcap, const float* __restrict__ sinks, const float* __restrict__ slopes) {
+  constexpr int D = 16 * NS;
+  __shared__ float merge_acc[4][16][D + 4];
+  __shared__ float merge_m[4][16], merge_l[4][16];
+  // the workgroup's rows: from row blockIdx.z of a tile of 16, if a request's rows in the tile begin there, to the last of them
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tile = blockIdx.x * 16, z = blockIdx.z, r0 = tile + z;
+  if (r0 >= num_tokens) return;
+  const int b = __builtin_amdgcn_readfirstlane(seq_of_token[r0]);
+  if (z > 0 && seq_of_token[r0 - 1] == b) return;
+  const bool mine = col < 16 - z && r0 + col < num_tokens && seq_of_token[min(r0 + col, num_tokens - 1)] == b;
+  const int h = blockIdx.y, kvh = h / (Hq / Hkv);
+  const int row = mine ? r0 + col : r0;
+  const int32_t* bt = block_tables + (int64_t)b * bt_stride;
+
+  // what this lane's token sees, [lo, hi) and [0, kept) as in attn_simple, and the reach of the tile's tokens together
+  const int pos = positions[row];
+  const int hi = min(pos + 1, context_lens[b]);
+  const int lo = window > 0 ? max(0, pos - window + 1) : (window < 0 ? pos - pos % (-window) : 0);
+  const int kept = (window > 0 && keep_first > 0) ? min(min(keep_first, lo), hi) : 0;
+  int hi_most = hi, hi_least = hi, lo_least = lo, lo_most = lo, kept_most = kept;
+#pragma unroll
+  for (int off = 8; off > 0; off >>= 1) {
+    hi_most = max(hi_most, __shfl_xor(hi_most, off, ME_WAVE)); hi_least = min(hi_least, __shfl_xor(hi_least, off, ME_WAVE));
+    lo_most = max(lo_most, __shfl_xor(lo_most, off, ME_WAVE)); lo_least = min(lo_least, __shfl_xor(lo_least, off, ME_WAVE));
+    kept_most = max(kept_most, __shfl_xor(kept_most, off, ME_WAVE));
+  }
+  hi_most = __builtin_amdgcn_readfirstlane(hi_most); hi_least = __builtin_amdgcn_readfirstlane(hi_least);
+  lo_most = __builtin_amdgcn_readfirstlane(lo_most); lo_least = __builtin_amdgcn_readfirstlane(lo_least);
+  kept_most = __builtin_amdgcn_readfirstlane(kept_most);
+
+  f32x4 fq[NS], fk[NS], fv[NS], acc[NS];
+  const float* qr = q + (int64_t)row * q_stride + (int64_t)h * D + 4 * g;
+#pragma unroll
+  for (int i = 0; i < NS; ++i) {
+    const float* at = qr + 16 * i;
+    fq[i] = f32x4{at[0], at[1], at[2], at[3]};
+    acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  float m = -INFINITY, l = 0.f;
+  const float slope = slopes != nullptr ? slopes[h] : 0.f;
+
+  // this wave's next block of 16 keys at or behind kb (a multiple of 16 that is this wave's) in which some token sees a key
+  auto next_block = [&](int kb) {
+    if (kb >= kept_most && kb + 16 <= lo_least) kb += ((lo_least - 16 - kb) / 64 + 1) * 64;
+    return kb;
+  };
+  auto page_of = [&](int j) { return bt[min(j, hi_most - 1) / page]; };      // hi_most > 0 wherever this is asked
+  auto fetch_keys = [&](int kb, int pg) {
+    const int j = kb + col;
+    const float* kr = k_cache + ((int64_t)(pg < 0 ? 0 : pg) * Hkv + kvh) * page * D + (pg < 0 ? 0 : (min(j, hi_most - 1) % page) * D) + 4 * g;
+#pragma unroll
+    for (int i = 0; i < NS; ++i) fk[i] = *reinterpret_cast<const f32x4*>(kr + 16 * i);
+  };
+  int kb = next_block(16 * wave);
+  int pk = 0, pv = 0;
+  if (kb < hi_most) {
+    pk = page_of(kb + col); pv = page_of(kb + 4 * g);
+    fetch_keys(kb, pk);
+  }
+  while (kb < hi_most) {
+    const int kn = next_block(kb + 64);
+    // four keys of a page lie side by side in every dimension's row of values; a group of four that begins behind the last
+    // key any token sees is read from the last such group of the table's reach instead and zeroed below
+    const int j0 = kb + 4 * g;
+    const float* vr = v_cache + ((int64_t)(pv < 0 ? 0 : pv) * Hkv + kvh) * page * D + (j0 < hi_most ? j0 % page : 0);
+#pragma unroll
+    for (int i = 0; i < NS; ++i) fv[i] = *reinterpret_cast<const f32x4*>(vr + (16 * i + col) * page);
+    int pk_next = 0, pv_next = 0;
+    if (kn < hi_most) { pk_next = page_of(kn + col); pv_next = page_of(kn + 4 * g); }
+    f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+    for (int i = 0; i < NS; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (i & 1) s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(fk[i][j], fq[i][j], s1, 0, 0, 0);
+        else s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(fk[i][j], fq[i][j], s0, 0, 0, 0);
+      }
+    if (kn < hi_most) fetch_keys(kn, pk_next);
+    f32x4 p;
+    bool sees[4];
+    float top = m;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int key = j0 + j;
+      sees[j] = (key >= lo || key < kept) && key < hi && pv >= 0;
+      float s = (s0[j] + s1[j]) * scale;
+      if (softcap > 0.f) s = softcap * tanhf(s / softcap);
+      s -= slope * (float)(pos - key);
+      p[j] = sees[j] ? s : -INFINITY;
+      top = fmaxf(top, p[j]);
+    }
+    top = fmaxf(top, __shfl_xor(top, 16, ME_WAVE));
+    top = fmaxf(top, __shfl_xor(top, 32, ME_WAVE));
+    const float alpha = m == -INFINITY ? 0.f : expf(m - top);        // m finite implies top finite
+#pragma unroll
+    for (int j = 0; j < 4; ++j) p[j] = (sees[j] && top > -INFINITY) ? expf(p[j] - top) : 0.f;
+    l = l * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
+    m = top;
+    const bool inside = kb >= lo_least && kb + 16 <= hi_most && __ballot(pv < 0) == 0;
+    if (!inside) {                               // keys that no token sees: whatever lies there is not a value
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const bool in = (j0 + j >= lo_least || j0 + j < kept_most) && j0 + j < hi_most && pv >= 0;
+#pragma unroll
+        for (int i = 0; i < NS; ++i) fv[i][j] = in ? fv[i][j] : 0.f;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NS; ++i) acc[i] *= alpha;
+    if (!inside || kb < lo_most || kb + 16 > hi_least) {             // some token does not see some key
+      float odd = 0.f;                           // becomes a NaN at the first value that is not finite
+#pragma unroll
+      for (int i = 0; i < NS; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) odd = fmaf(fv[i][j], 0.f, odd);
+      if (__ballot(odd != odd) != 0) {
+        for (int from = 0; from < 4; ++from)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float pj = __shfl(p[j], from * 16 + col, ME_WAVE);
+            const int seen = __shfl((int)sees[j], from * 16 + col, ME_WAVE);
+#pragma unroll
+            for (int i = 0; i < NS; ++i)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const float v = __shfl(fv[i][j], from * 16 + 4 * g + e, ME_WAVE);
+                if (seen && !(fabsf(v) < INFINITY)) acc[i][e] += pj * v;
+              }
+          }
+#pragma unroll
+        for (int i = 0; i < NS; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) fv[i][j] = fabsf(fv[i][j]) < INFINITY ? fv[i][j] : 0.f;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < NS; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(fv[i][j], p[j], acc[i], 0, 0, 0);
+    kb = kn; pk = pk_next; pv = pv_next;
+  }
+  l += __shfl_xor(l, 16, ME_WAVE);
+  l += __shfl_xor(l, 32, ME_WAVE);
+  // a lane holds dimensions 16 i + 4 g .. + 3 of token col
+  if (g == 0) { merge_m[wave][col] = m; merge_l[wave][col] = l; }
+#pragma unroll
+  for (int i = 0; i < NS; ++i) *reinterpret_cast<f32x4*>(&merge_acc[wave][col][16 * i + 4 * g]) = acc[i];
+  __syncthreads();
+  for (int e = tid; e < 16 * D; e += 256) {
+    const int c = e / D, d = e % D;
+    if (c >= 16 - z || r0 + c >= num_tokens || seq_of_token[r0 + c] != b) continue;
+    float top = sinks != nullptr ? sinks[h] : -INFINITY;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) top = fmaxf(top, merge_m[w][c]);
+    float sum = sinks != nullptr ? expf(sinks[h] - top) : 0.f, o = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float a = merge_m[w][c] == -INFINITY ? 0.f : expf(merge_m[w][c] - top);
+      sum += a * merge_l[w][c];
+      o += a * merge_acc[w][c][d];
+    }
+    out[(int64_t)(r0 + c) * out_stride + (int64_t)h * D + d] = o * (sum > 0.f ? 1.f / sum : 0.f);
+  }
+}
+
 extern "C" int me_attn_simple(const void* q, int64_t q_stride, void* out, int64_t out_stride, int dtype,
                               const void* k_cache, const void* v_cache, const int32_t* block_tables,
                               int bt_stride, const int32_t* seq_of_token, const int32_t* positions,
@@ -140,7 +328,15 @@ extern "C" int me_attn_simple(const void* q, int64_t q_stride, void* out, int64_
   ME_CHECK(keep_first >= 0 && softcap >= 0.f, "attention: keep_first and softcap must not be negative");
   dim3 grid(num_tokens, Hq), block(AS_THREADS);
   size_t lds = (size_t)(D + AS_THREADS) * sizeof(float);
-  if (dtype == ME_F32)
+  if (dtype == ME_F32 && D % 16 == 0 && D <= 128 && page % 4 == 0 && num_tokens <= 2147483647ll - 16 && Hq <= 65535 &&
+      (uintptr_t)k_cache % 16 == 0 && (uintptr_t)v_cache % 16 == 0) {
+    const dim3 tiles((unsigned)((num_tokens + 15) / 16), Hq, 16);
+#define AS_F32(NS) case NS: attn_f32_kernel<NS><<<tiles, block, 0, stream>>>((const float*)q, q_stride, (float*)out, out_stride,          \
+        (const float*)k_cache, (const float*)v_cache, block_tables, bt_stride, seq_of_token, positions, context_lens, (int)num_tokens, \
+        Hq, Hkv, page, scale, window, keep_first, softcap, sinks, slopes); break
+    switch (D / 16) { AS_F32(1); AS_F32(2); AS_F32(3); AS_F32(4); AS_F32(5); AS_F32(6); AS_F32(7); AS_F32(8); }
+#undef AS_F32
+  } else if (dtype == ME_F32)
     attn_simple_kernel<float><<<grid, block, lds, stream>>>(
         (const float*)q, q_stride, (float*)out, out_stride, (const float*)k_cache, (const float*)v_cache,
         block_tables, bt_stride, seq_of_token, positions, context_lens, Hq, Hkv, D, page, scale, window, keep_first, softcap, sinks, slopes);

@@ -1,0 +1,75 @@
+"""The float32 path's product and attention at the edges of their tiles. Tolerances: a sum of n float32 products of
+standard normals rounds by at most about 2^-24 sqrt(n) of its size per step, so 1e-6 for up to 3,000 terms added in four parts;
+attention's scores pass an exponential, 1e-5 as everywhere."""
+import pytest
+import torch
+
+import kernel_twins as twin
+from mini_engine_amd.kernels import ops
+from test_kernels_gpu import DEV, _attention_case, close, hip
+
+pytestmark = pytest.mark.gpu
+TILES = sorted(ops.F32_ROUND_US)
+
+
+def _product(x, w, tile):
+    y = torch.full((x.shape[0], w.shape[0]), float("nan"), device=DEV)
+    ops.core().call("me_gemm_f32", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), y.stride(0),
+                    x.shape[0], w.shape[0], x.shape[1], *tile, ops._stream())
+    return y
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (3, 17, 5), (16, 16, 16), (17, 130, 36), (33, 250, 130), (65, 64, 128), (70, 100, 1023),
+                                   (600, 70, 260), (5, 2100, 2999)])
+def test_product_tiles(M, N, K):
+    """Every tile gives the same bits, for all rows together and for some alone; rows that are no whole 16-byte pieces, strides
+    that are not K, an odd first address and an odd row length of the output give the same sums too."""
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    wide, ww = (torch.randn(n, K + 12, device=DEV, generator=g) for n in (M, N))
+    x, w = wide[:, 4:4 + K], ww[:, 8:8 + K]
+    ref = x.double() @ w.double().T
+    first = _product(x, w, TILES[0])
+    assert float((first.double() - ref).norm() / ref.norm()) < 1e-6
+    for tile in TILES[1:]:
+        assert torch.equal(_product(x, w, tile), first)
+    assert torch.equal(hip().linear(x, w), first)
+    some = x[M // 3:M // 3 + 2]
+    assert torch.equal(hip().linear(some, w), first[M // 3:M // 3 + 2])
+    odd = torch.empty(M * (K + 1) + 1, device=DEV)[1:].view(M, K + 1)[:, :K]
+    odd.copy_(x)
+    assert torch.equal(hip().linear(odd, w), first)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,page", [(4, 2, 16, 4), (3, 1, 80, 8), (6, 2, 112, 16), (2, 2, 128, 12), (4, 4, 96, 64)])
+@pytest.mark.parametrize("extra", [{}, {"window": 20}, {"window": 37, "keep_first": 5}, {"chunk": 24}, {"softcap": 3.0}])
+def test_attention_tiles(Hq, Hkv, D, page, extra):
+    """Rows of several requests in one tile of 16, requests that begin inside a tile, decoding rows beside prompts; a
+    request's tokens alone give the same bits as beside others."""
+    window = extra.get("window")
+    seqs = [(40, 1), (300, 1), (17, 17), (5, 2), (129, 33), (70, 15), (64, 16)]
+    args = _attention_case(torch.float32, Hq, Hkv, D, page, seqs, seed=D + page, window=window)
+    if "keep_first" in extra:            # the kept keys' pages are held: all of them here
+        args = _attention_case(torch.float32, Hq, Hkv, D, page, seqs, seed=D + page)
+        args = args[:12] + (window,) + args[13:]
+    more = {k: v for k, v in extra.items() if k != "window"}
+    g = torch.Generator(device=DEV).manual_seed(1)
+    sinks, slopes = torch.randn(Hq, device=DEV, generator=g), torch.rand(Hq, device=DEV, generator=g)
+    for kw in (more, dict(more, sinks=sinks, slopes=slopes)):
+        got = hip().paged_attention(*args, **kw)
+        close(got, twin.paged_attention(*args, **kw), 1e-5)
+        q, seq_of, positions = args[0], args[6], args[7]
+        for a, n in ((19, 2), (23, 9), (54, 16)):
+            part = (q[a:a + n],) + args[1:6] + (seq_of[a:a + n].contiguous(), positions[a:a + n].contiguous()) + args[8:]
+            assert torch.equal(hip().paged_attention(*part, **kw), got[a:a + n])
+
+
+def test_attention_keeps_what_is_not_a_number_to_those_who_see_it():
+    """A value that is not finite reaches the tokens that see its key and no others, and leaves their bits alone."""
+    args = _attention_case(torch.float32, 4, 2, 64, 16, [(40, 40), (9, 9)], seed=3)
+    want = hip().paged_attention(*args)
+    bt, v_cache = args[4], args[2]
+    v_cache[int(bt[0, 1]), 1, 7, 5] = float("inf")           # key 21 of the first request, head 1, dimension 7
+    got = hip().paged_attention(*args)
+    hit = torch.zeros_like(got, dtype=torch.bool)
+    hit[21:40, 2 * 64 + 7] = hit[21:40, 3 * 64 + 7] = True   # the two query heads of that key head
+    assert not torch.isfinite(got[hit]).any() and torch.equal(got[~hit], want[~hit])
