@@ -283,9 +283,10 @@ __device__ __forceinline__ float shape_token(const DrArgs& a, int lane, int nr_r
 }
 
 // One wave per (token, head): the shaped values of every token at once, for a recurrence kernel that then only streams
-// them (PRE): pre_q, pre_k, pre_d [T, H, NR] and pre_x [T, H], float32.
+// them (decay_walk_kernel): pre_q, pre_k, pre_d [T, H, NR] and pre_x [T, H], float32. The rows of a (token, head) lie in the
+// order in which that kernel's lanes take them: row n at (n mod row_groups) NR / row_groups + n / row_groups.
 template <typename TX, int NR, int RULE>
-__global__ void __launch_bounds__(64) decay_prepare_kernel(DrArgs a, float* __restrict__ pre_q, float* __restrict__ pre_k,
+__global__ void __launch_bounds__(64) decay_prepare_kernel(DrArgs a, int row_groups, float* __restrict__ pre_q, float* __restrict__ pre_k,
                                                            float* __restrict__ pre_d, float* __restrict__ pre_x) {
   constexpr int PER = (NR + 63) / 64;
   const int64_t t = blockIdx.x;
@@ -310,8 +311,9 @@ __global__ void __launch_bounds__(64) decay_prepare_kernel(DrArgs a, float* __re
   for (int i = 0; i < PER; ++i) {
     const int n = lane + 64 * i;
     if (n < NR) {
-      pre_q[at + n] = q[i]; pre_k[at + n] = k[i];
-      if (RULE != 3) pre_d[at + n] = d[i];
+      const int64_t to = at + n % row_groups * (NR / row_groups) + n / row_groups;
+      pre_q[to] = q[i]; pre_k[to] = k[i];
+      if (RULE != 3) pre_d[to] = d[i];
     }
   }
   if (lane == 0) {
@@ -320,9 +322,8 @@ __global__ void __launch_bounds__(64) decay_prepare_kernel(DrArgs a, float* __re
   }
 }
 
-template <typename TX, int NR, int RG, int RULE, bool PRE>
-__global__ void __launch_bounds__(64) decay_rows_kernel(DrArgs a, const float* __restrict__ pre_q, const float* __restrict__ pre_k,
-                                                        const float* __restrict__ pre_d, const float* __restrict__ pre_x) {
+template <typename TX, int NR, int RG, int RULE>
+__global__ void __launch_bounds__(64) decay_rows_kernel(DrArgs a) {
   constexpr int PC = 64 / RG;            // columns per wave
   constexpr int RL = NR / RG;            // rows per lane
   constexpr int PER = (NR + 63) / 64;    // rows of q, k and the decay that a lane brings to LDS for the wave
@@ -353,11 +354,11 @@ __global__ void __launch_bounds__(64) decay_rows_kernel(DrArgs a, const float* _
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int n = lane + 64 * i;
-    const bool in = !PRE && n < a.N && n < NR;
-    base[i] = RULE == 3 ? (PRE ? 0.f : a.base[h]) : (in ? a.base[h * a.N + n] : 0.f);
+    const bool in = n < a.N && n < NR;
+    base[i] = RULE == 3 ? a.base[h] : (in ? a.base[h * a.N + n] : 0.f);
     bonus[i] = (RULE == 0 && in) ? a.bonus[h * a.N + n] : 0.f;
   }
-  const float rate = (RULE != 0 && !PRE) ? a.rate[h] : 0.f;
+  const float rate = RULE != 0 ? a.rate[h] : 0.f;
   // a batch of tokens on its way (n*) and the batch being worked on (c*): a lane's own column's v and the token's own
   // number (the write strength, or under the bonus rule sum_n q_n bonus_n k_n)
   float nq[DR_TB][PER], nk[DR_TB][PER], nr[DR_TB][PER], nv[DR_TB], nb[DR_TB];
@@ -370,21 +371,14 @@ __global__ void __launch_bounds__(64) decay_rows_kernel(DrArgs a, const float* _
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
           const int n = lane + 64 * i;
-          if (PRE) {
-            const int64_t at = (row * a.H + h) * NR + (n < NR ? n : 0);
-            nq[j][i] = pre_q[at]; nk[j][i] = pre_k[at];
-            nr[j][i] = RULE == 3 ? (i == 0 ? pre_d[row * a.H + h] : 0.f) : pre_d[at];
-          } else {
-            const bool in = n < a.N && n < NR;
-            nq[j][i] = in ? to_f32<TX>(qp[row * a.q_stride + g * a.N + n]) : 0.f;
-            nk[j][i] = in ? to_f32<TX>(kp[row * a.k_stride + g * a.N + n]) : 0.f;
-            if (RULE == 3) nr[j][i] = i == 0 ? to_f32<TX>(rp[row * a.raw_stride + h]) : 0.f;
-            else nr[j][i] = in ? to_f32<TX>(rp[row * a.raw_stride + h * a.N + n]) : 0.f;
-          }
+          const bool in = n < a.N && n < NR;
+          nq[j][i] = in ? to_f32<TX>(qp[row * a.q_stride + g * a.N + n]) : 0.f;
+          nk[j][i] = in ? to_f32<TX>(kp[row * a.k_stride + g * a.N + n]) : 0.f;
+          if (RULE == 3) nr[j][i] = i == 0 ? to_f32<TX>(rp[row * a.raw_stride + h]) : 0.f;
+          else nr[j][i] = in ? to_f32<TX>(rp[row * a.raw_stride + h * a.N + n]) : 0.f;
         }
         nv[j] = to_f32<TX>(vp[row * a.v_stride + h * a.P + pc]);
-        if (PRE) nb[j] = pre_x[row * a.H + h];
-        else nb[j] = (RULE == 1 || RULE == 3) ? to_f32<TX>(bp[row * a.beta_stride + h]) : 0.f;
+        nb[j] = (RULE == 1 || RULE == 3) ? to_f32<TX>(bp[row * a.beta_stride + h]) : 0.f;
       }
     }
   };
@@ -393,8 +387,7 @@ __global__ void __launch_bounds__(64) decay_rows_kernel(DrArgs a, const float* _
 #pragma unroll
     for (int j = 0; j < DR_TB; ++j) {
       if (t0 + j < n_tok) {
-        float x = nb[j];
-        if (!PRE) x = shape_token<PER, RULE>(a, lane, NR, nq[j], nk[j], nr[j], base, bonus, rate, nb[j]);
+        const float x = shape_token<PER, RULE>(a, lane, NR, nq[j], nk[j], nr[j], base, bonus, rate, nb[j]);
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
           const int n = lane + 64 * i;
@@ -466,24 +459,216 @@ __global__ void __launch_bounds__(64) decay_rows_kernel(DrArgs a, const float* _
   }
 }
 
+// The same walk over values that decay_prepare_kernel has shaped: portions of many tokens. What bounds it is the number of
+// instructions of a wave per token (a request's tokens are a chain, and the chip has a wave or less per SIMD), so a batch of
+// eight tokens is one piece of code without a branch: the exchange and the output sum of a token overlap the next token's
+// reads and updates, a lane brings its share of the batch's shared values in 16-byte pieces that go to LDS as they are, and
+// of the four lanes that hold the same finished sums each stores another token's. The sums are those of decay_rows_kernel in the
+// same order. 2,048 tokens: delta rule, 4 heads of 128 x 128, 344 us, bonus rule, 16 heads of 64 x 64, 216 us (with a branch per
+// token, 4-byte loads and a store per token: 1,105 and 909).
+template <typename TX, int NR, int RG, int RULE>
+__global__ void __launch_bounds__(64) decay_walk_kernel(DrArgs a, const float* __restrict__ pre_q, const float* __restrict__ pre_k,
+                                                        const float* __restrict__ pre_d, const float* __restrict__ pre_x) {
+  constexpr int PC = 64 / RG;            // columns per wave
+  constexpr int RL = NR / RG;            // rows per lane
+  constexpr int PIECES = DR_TB * NR / 4; // 16-byte pieces of a batch's q, k or decays
+  constexpr int ROUNDS = (PIECES + 63) / 64;
+  constexpr bool DELTA = RULE == 1 || RULE == 3, ROWS = RULE != 3;
+  __shared__ f32x4 sq[2][PIECES], sk[2][PIECES], sd[ROWS ? 2 : 1][ROWS ? PIECES : 1];
+  __shared__ float sx[2][DR_TB], sh[2][DR_TB];               // the tokens' own numbers; their heads' decays (RULE 3)
+  const int lane = threadIdx.x;
+  const int col_blocks = (a.P + PC - 1) / PC;
+  const int cb = blockIdx.x % col_blocks;
+  const int h = (blockIdx.x / col_blocks) % a.H;
+  const int b = blockIdx.x / (col_blocks * a.H);
+  const int begin = __builtin_amdgcn_readfirstlane(a.cu[b]);
+  const int n_tok = __builtin_amdgcn_readfirstlane(a.cu[b + 1]) - begin;
+  if (n_tok <= 0) return;
+  const int64_t first = begin;
+  const int p = cb * PC + lane / RG;
+  const int rg = lane % RG;
+  const bool live = p < a.P;
+  const int pc = live ? p : a.P - 1;
+  float* srow = a.state + (int64_t)a.slots[b] * a.state_stride + (int64_t)h * a.N * a.P;
+  float S[RL];
+#pragma unroll
+  for (int i = 0; i < RL; ++i) S[i] = (i * RG + rg < a.N) ? srow[(int64_t)(i * RG + rg) * a.P + pc] : 0.f;
+
+  const TX* values = (const TX*)a.v + first * a.v_stride + h * a.P;
+  const int64_t head0 = first * a.H + h;
+  f32x4 nq[ROUNDS], nk[ROUNDS], nd[ROUNDS];
+  float nx = 0.f, nh = 0.f;
+  TX nv[DR_TB];
+  // what a lane adds to a batch's first address, in bytes (the address itself is the same for all lanes)
+  uint32_t piece[ROUNDS];
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    const int e = min(lane + 64 * r, PIECES - 1);
+    piece[r] = (uint32_t)((e / (NR / 4) * a.H * (NR / 4) + e % (NR / 4)) * 16);
+  }
+  const uint32_t own = (uint32_t)((lane & (DR_TB - 1)) * a.H * 4), column = (uint32_t)(pc * sizeof(TX));
+  auto at = [](const void* base, uint32_t bytes) { return reinterpret_cast<const char*>(base) + bytes; };
+  // the next batch on its way; of a batch that is not whole, tokens behind the last are read from the last one and not used
+  auto fetch = [&](int t0) {
+    if (t0 + DR_TB <= n_tok) {
+      const int64_t row = head0 + (int64_t)t0 * a.H;
+#pragma unroll
+      for (int r = 0; r < ROUNDS; ++r) {
+        nq[r] = *reinterpret_cast<const f32x4*>(at(pre_q + row * NR, piece[r]));
+        nk[r] = *reinterpret_cast<const f32x4*>(at(pre_k + row * NR, piece[r]));
+        if (ROWS) nd[r] = *reinterpret_cast<const f32x4*>(at(pre_d + row * NR, piece[r]));
+      }
+      nx = *reinterpret_cast<const float*>(at(pre_x + row, own));
+      if (!ROWS) nh = *reinterpret_cast<const float*>(at(pre_d + row, own));
+      const TX* vt = values + t0 * a.v_stride;
+#pragma unroll
+      for (int j = 0; j < DR_TB; ++j, vt += a.v_stride) nv[j] = *reinterpret_cast<const TX*>(at(vt, column));
+      return;
+    }
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r) {
+      const int e = min(lane + 64 * r, PIECES - 1);
+      const int64_t from = (head0 + (int64_t)min(t0 + e / (NR / 4), n_tok - 1) * a.H) * NR + e % (NR / 4) * 4;
+      nq[r] = *reinterpret_cast<const f32x4*>(pre_q + from);
+      nk[r] = *reinterpret_cast<const f32x4*>(pre_k + from);
+      if (ROWS) nd[r] = *reinterpret_cast<const f32x4*>(pre_d + from);
+    }
+    const int64_t row = head0 + (int64_t)min(t0 + (lane & (DR_TB - 1)), n_tok - 1) * a.H;
+    nx = pre_x[row];
+    if (!ROWS) nh = pre_d[row];
+#pragma unroll
+    for (int j = 0; j < DR_TB; ++j) nv[j] = values[(int64_t)min(t0 + j, n_tok - 1) * a.v_stride + pc];
+  };
+  struct Shared { float q[RL], k[RL], d[RL], x; };
+  auto read = [&](int buf, int j, Shared& o) {
+    const float* aq = reinterpret_cast<const float*>(&sq[buf][0]) + j * NR + rg * RL;
+    const float* ak = reinterpret_cast<const float*>(&sk[buf][0]) + j * NR + rg * RL;
+    const float* ad = reinterpret_cast<const float*>(&sd[ROWS ? buf : 0][0]) + j * NR + rg * RL;
+#pragma unroll
+    for (int i = 0; i < RL; ++i) {
+      o.q[i] = aq[i]; o.k[i] = ak[i];
+      if (ROWS) o.d[i] = ad[i];
+    }
+    if (!ROWS) o.d[0] = sh[buf][j];
+    o.x = RULE == 2 ? 0.f : sx[buf][j];
+  };
+  auto token = [&](const Shared& o, float v) {
+    float y = 0.f;
+    if (RULE == 0) {
+#pragma unroll
+      for (int i = 0; i < RL; ++i) {
+        y = fmaf(o.q[i], S[i], y);
+        S[i] = fmaf(o.d[i], S[i], o.k[i] * v);
+      }
+    } else if (RULE == 2) {
+#pragma unroll
+      for (int i = 0; i < RL; ++i) {
+        S[i] = fmaf(o.d[i], S[i], o.k[i] * v);
+        y = fmaf(o.q[i], S[i], y);
+      }
+    } else {
+      float dot = 0.f;
+#pragma unroll
+      for (int i = 0; i < RL; ++i) {
+        S[i] *= o.d[ROWS ? i : 0];
+        dot = fmaf(S[i], o.k[i], dot);
+      }
+      dot = group_sum<RG>(dot);
+      const float u = o.x * (v - dot);
+#pragma unroll
+      for (int i = 0; i < RL; ++i) {
+        S[i] = fmaf(o.k[i], u, S[i]);
+        y = fmaf(S[i], o.q[i], y);
+      }
+    }
+    y = group_sum<RG>(y);
+    if (RULE == 0) y = fmaf(o.x, v, y);          // the current token's own term: v_p * sum_n q_n bonus_n k_n
+    return y;
+  };
+  float* out = a.y + first * (int64_t)(a.H * a.P) + h * a.P + p;
+  fetch(0);
+  for (int t0 = 0, buf = 0; t0 < n_tok; t0 += DR_TB, buf ^= 1) {
+    // one wave: what its lanes write to LDS, its lanes read behind it without a barrier
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r) {
+      const int e = lane + 64 * r;
+      if (PIECES % 64 == 0 || e < PIECES) {
+        sq[buf][e] = nq[r]; sk[buf][e] = nk[r];
+        if (ROWS) sd[ROWS ? buf : 0][e] = nd[r];
+      }
+    }
+    if (lane < DR_TB) {
+      sx[buf][lane] = nx;
+      if (!ROWS) sh[buf][lane] = nh;
+    }
+    float v[DR_TB];
+#pragma unroll
+    for (int j = 0; j < DR_TB; ++j) v[j] = to_f32<TX>(nv[j]);
+    asm volatile("" ::: "memory");
+    fetch(t0 + DR_TB);
+    asm volatile("" ::: "memory");
+    if (t0 + DR_TB <= n_tok) {
+      float y[DR_TB];
+      Shared o[2];                               // a token's values are read while the one before it is worked on
+      read(buf, 0, o[0]);
+#pragma unroll
+      for (int j = 0; j < DR_TB; ++j) {
+        if (j + 1 < DR_TB) read(buf, j + 1, o[(j + 1) & 1]);
+        y[j] = token(o[j & 1], v[j]);
+      }
+      // the first four lanes of a column hold the same bits (the others have added in another order): lane rg of them stores
+      // the output of token j0 + rg
+      constexpr int ST = RG < 4 ? RG : 4;
+      if (live && rg < ST) {
+#pragma unroll
+        for (int j0 = 0; j0 < DR_TB; j0 += ST) {
+          float mine = y[j0];
+#pragma unroll
+          for (int j = 1; j < ST; ++j) mine = rg == j ? y[j0 + j] : mine;
+          out[(int64_t)(t0 + j0 + rg) * (a.H * a.P)] = mine;
+        }
+      }
+    } else {
+#pragma unroll 1
+      for (int j = 0; t0 + j < n_tok; ++j) {
+        Shared o;
+        read(buf, j, o);
+        float vj = v[0];
+#pragma unroll
+        for (int i = 1; i < DR_TB; ++i) vj = i == j ? v[i] : vj;
+        const float y = token(o, vj);
+        if (live && rg == 0) out[(int64_t)(t0 + j) * (a.H * a.P)] = y;
+      }
+    }
+  }
+  if (live) {
+#pragma unroll
+    for (int i = 0; i < RL; ++i)
+      if (i * RG + rg < a.N) srow[(int64_t)(i * RG + rg) * a.P + p] = S[i];
+  }
+}
+
 template <typename TX, int NR, int RG, bool PRE>
 static void launch_decay_rows(const DrArgs& a, int rule, int num_seqs, int64_t T, float* pre, hipStream_t stream) {
   constexpr int PC = 64 / RG;
   const dim3 grid((unsigned)(num_seqs * a.H * ((a.P + PC - 1) / PC))), block(64);
-  float* pq = pre; float* pk = pre; float* pd = pre; float* px = pre;
-  if (PRE) {
+  if constexpr (PRE) {
     const int64_t each = T * a.H * NR;
-    pk = pre + each; pd = pre + 2 * each; px = pre + 3 * each;
+    float *pq = pre, *pk = pre + each, *pd = pre + 2 * each, *px = pre + 3 * each;
     const dim3 pgrid((unsigned)T, a.H);
-    if (rule == 0) decay_prepare_kernel<TX, NR, 0><<<pgrid, block, 0, stream>>>(a, pq, pk, pd, px);
-    else if (rule == 2) decay_prepare_kernel<TX, NR, 2><<<pgrid, block, 0, stream>>>(a, pq, pk, pd, px);
-    else if (rule == 3) decay_prepare_kernel<TX, NR, 3><<<pgrid, block, 0, stream>>>(a, pq, pk, pd, px);
-    else decay_prepare_kernel<TX, NR, 1><<<pgrid, block, 0, stream>>>(a, pq, pk, pd, px);
+#define DR_RULE(R)                                                                       \
+  do {                                                                                   \
+    decay_prepare_kernel<TX, NR, R><<<pgrid, block, 0, stream>>>(a, RG, pq, pk, pd, px); \
+    decay_walk_kernel<TX, NR, RG, R><<<grid, block, 0, stream>>>(a, pq, pk, pd, px);     \
+  } while (0)
+    if (rule == 0) DR_RULE(0); else if (rule == 1) DR_RULE(1); else if (rule == 2) DR_RULE(2); else DR_RULE(3);
+#undef DR_RULE
+  } else {
+    if (rule == 0) decay_rows_kernel<TX, NR, RG, 0><<<grid, block, 0, stream>>>(a);
+    else if (rule == 1) decay_rows_kernel<TX, NR, RG, 1><<<grid, block, 0, stream>>>(a);
+    else if (rule == 2) decay_rows_kernel<TX, NR, RG, 2><<<grid, block, 0, stream>>>(a);
+    else decay_rows_kernel<TX, NR, RG, 3><<<grid, block, 0, stream>>>(a);
   }
-  if (rule == 0) decay_rows_kernel<TX, NR, RG, 0, PRE><<<grid, block, 0, stream>>>(a, pq, pk, pd, px);
-  else if (rule == 2) decay_rows_kernel<TX, NR, RG, 2, PRE><<<grid, block, 0, stream>>>(a, pq, pk, pd, px);
-  else if (rule == 3) decay_rows_kernel<TX, NR, RG, 3, PRE><<<grid, block, 0, stream>>>(a, pq, pk, pd, px);
-  else decay_rows_kernel<TX, NR, RG, 1, PRE><<<grid, block, 0, stream>>>(a, pq, pk, pd, px);
 }
 
 // row_groups: lanes that share a column: 1 or 4 (4 gives four times the waves with a quarter of the rows each) with the
@@ -502,7 +687,7 @@ extern "C" int me_decay_rows_recurrence(const void* q, int64_t q_stride, const v
   ME_CHECK(pre == nullptr ? (row_groups == 1 || row_groups == 4) : (row_groups == 4 || row_groups == 16),
            "decay_rows_recurrence: 1 or 4 lanes to a column, 4 or 16 over prepared values");
   ME_CHECK(T >= 0 && T <= 2147483647ll && H <= 65535, "decay_rows_recurrence: too many tokens or heads");
-  ME_CHECK((int64_t)num_seqs * H * ((P + 3) / 4) <= 2147483647ll, "decay_rows_recurrence: too many workgroups");
+  ME_CHECK((int64_t)num_seqs * H * ((P + 3) / 4) <= 2147483647ll && H <= 65535 && P <= (1 << 28), "decay_rows_recurrence: too many workgroups");
   DrArgs a;
   a.q = q; a.k = k; a.v = v; a.raw = raw; a.beta = beta;
   a.q_stride = q_stride; a.k_stride = k_stride; a.v_stride = v_stride; a.raw_stride = raw_stride; a.beta_stride = beta_stride;

@@ -1783,8 +1783,8 @@ def decay_row_groups(num_seqs: int, H: int, N: int, P: int, longest: int = 1, to
     own (unit lengths, decays and their exponentials leave the chain), and 16 lanes share a column while the waves all run at
     once (up to 16 a compute unit, and as many as its 160 KB of LDS hold: a wave keeps q, k and, unless a head has one decay,
     the decays of 16 tokens there), else 4: 8 prompts of 2,048 tokens over 8 heads of 128 x 128, 2,048 waves of 16 lanes to a
-    column, take 1,249 us with one decay per head (all at once) and 2,793 with a decay per row (two rounds; 2,156 with 4
-    lanes). Requests of a few tokens in such a step (`tokens`: the step's) end early and are not counted. Short steps shape inside the
+    column, take 681 us with one decay per head (all at once; 933 with 4 lanes) and 1,088 with a decay per row (two rounds;
+    1,057 with 4 lanes); 16 prompts of 512 tokens 459 and 328. Requests of a few tokens in such a step (`tokens`: the step's) end early and are not counted. Short steps shape inside the
     kernel: 4 lanes where a lane could not keep a whole column in registers, or while one lane to a column leaves compute
     units without a wave; else 1."""
     if longest >= DECAY_PREPARE_MIN_TOKENS:

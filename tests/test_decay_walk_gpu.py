@@ -1,0 +1,46 @@
+"""The walk over shaped tokens in batches of eight: a token's results are the same bits wherever it stands in a batch, in a
+whole batch or in one that ends early, and the state row is the same too."""
+import pytest
+import torch
+
+from mini_engine_amd.kernels import ops
+from test_kernels_gpu import DEV, close, hip
+import kernel_twins as twin
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("groups", [4, 16])
+@pytest.mark.parametrize("rule", ["bonus", "delta", "gated", "delta_head"])
+@pytest.mark.parametrize("H,N,P,dtype", [(2, 20, 12, torch.float32), (3, 64, 64, torch.bfloat16), (2, 128, 37, torch.bfloat16), (1, 256, 5, torch.float32)])
+def test_places_in_a_batch(monkeypatch, H, N, P, dtype, rule, groups):
+    monkeypatch.setattr(ops, "decay_row_groups", lambda *a: (groups, True))
+    g = torch.Generator(device=DEV).manual_seed(N + P)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    T, wide = 41, H if rule == "delta_head" else H * N
+    q, k, v, raw, beta = (rnd(T, n + 3)[:, 1:1 + n].to(dtype) for n in (H * N, H * N, H * P, wide, H))
+    kw = dict(base=rnd(wide) - 1)
+    kw.update(dict(bonus=rnd(wide)) if rule == "bonus" else dict(rate=rnd(H).abs() + 0.1))
+    if rule.startswith("delta"):
+        kw.update(unit_eps=1e-6, q_scale=N ** -0.5)
+    start = rnd(2, H * N * P)
+    slot = torch.tensor([1], dtype=torch.int32, device=DEV)
+
+    def run(lo, n, state):
+        more = dict(kw, beta=beta[lo:lo + n]) if rule.startswith("delta") else kw
+        return hip().decay_rows_recurrence(q[lo:lo + n], k[lo:lo + n], v[lo:lo + n], raw[lo:lo + n], state, slot,
+                                           torch.tensor([0, n], dtype=torch.int32, device=DEV), [n], H, H, N, P, rule, **more)
+
+    whole = start.clone()
+    y = run(0, T, whole)
+    cpu = lambda t: t.cpu() if torch.is_tensor(t) else t
+    want = start.cpu().clone()
+    close(y, twin.decay_rows_recurrence(*(t.cpu() for t in (q, k, v, raw)), want, slot.cpu(), torch.tensor([0, T]), [T], H, H, N, P, rule,
+                                        **{n: cpu(t) for n, t in dict(kw, **(dict(beta=beta) if rule.startswith("delta") else {})).items()}), 2e-5)
+    close(whole, want, 2e-5)
+    for cuts in ((1, 40), (3, 38), (8, 33), (9, 8, 24), (7, 1, 33)):
+        state, lo, parts = start.clone(), 0, []
+        for n in cuts:
+            parts.append(run(lo, n, state))
+            lo += n
+        assert torch.equal(torch.cat(parts), y) and torch.equal(state, whole)
