@@ -40,3 +40,30 @@ def test_gated_norm_widths(n, parts, kind, dtype):
     w = torch.rand(n, device=DEV, generator=g) + 0.5
     close(hip().gated_rms_norm(y, gate, w, 1e-5, 1, kind, dtype), twin.gated_rms_norm(y, gate, w, 1e-5, 1, kind, dtype),
           1e-6 if dtype == torch.float32 else 4e-3)
+
+
+@pytest.mark.parametrize("scoring", ["softmax", "sigmoid", "chosen"])
+@pytest.mark.parametrize("T,E,groups,keep,top,group_top", [(1, 1, 1, 1, 1, 1), (17, 2, 1, 1, 2, 1), (64, 32, 4, 2, 4, 1), (33, 63, 7, 3, 5, 2),
+                                                           (64, 64, 8, 2, 8, 3), (40, 64, 64, 9, 9, 1), (50, 65, 5, 2, 6, 2), (5, 128, 4, 1, 3, 2)])
+def test_choices_in_registers_and_through_lds(T, E, groups, keep, top, group_top, scoring):
+    """Up to 64 experts a lane holds one, beyond they lie in LDS: the twin's choice either way, with pairs of experts of equal
+    scores among them (the lower index wins), also inside the kernel that orders the pairs. Logits are sums of whole numbers,
+    so that both sides have the same ones."""
+    if scoring == "chosen" and groups > 1:
+        groups = keep = 1
+    g = torch.Generator(device=DEV).manual_seed(T + E)
+    x = torch.randint(-3, 4, (T, 24), device=DEV, generator=g).float()
+    router = torch.randint(-2, 3, (E, 24), device=DEV, generator=g).float() * 0.125
+    router[1::2] = router[0:E - E % 2:2]
+    rule = ops.RouteRule(scoring, None, group_top=group_top, normalise=scoring != "sigmoid", scale=1.25)
+    ids, weights = hip().moe_route(x, router, top, groups, keep, rule)
+    want_ids, want_w = twin.moe_route(x.cpu(), router.cpu(), top, groups, keep, rule)
+    scores = torch.softmax(x.cpu() @ router.cpu().t(), -1) if scoring == "softmax" else torch.sigmoid(x.cpu() @ router.cpu().t())
+    gap = scores.unique(dim=-1) if T == 1 else None            # different logits whose scores round alike may go either way
+    same = (ids.cpu() == want_ids).all(-1)
+    assert same.float().mean() >= (1.0 if scoring == "chosen" or gap is not None else 0.9)
+    close(weights.cpu()[same], want_w[same], 2e-6)             # a softmax of 32-bit exponentials
+    up, down = torch.randn(E, 8, 24, device=DEV, generator=g), torch.randn(E, 16, 8, device=DEV, generator=g)
+    got = hip().route_and_run_experts(x.to(torch.bfloat16), router, top, groups, keep, up.to(torch.bfloat16), down.to(torch.bfloat16), rule=rule, gated=False)
+    want = twin.routed_experts(x.cpu().to(torch.bfloat16), ids.cpu(), weights.cpu(), up.cpu().to(torch.bfloat16), down.cpu().to(torch.bfloat16), gated=False)
+    close(got.sum(0), want.sum(0), 3e-2)
