@@ -261,8 +261,22 @@ qk_norm_rope_store_tile_kernel(bf16_t* __restrict__ qkv, int64_t row_stride, con
     const int64_t t = t0 + ti;
     const bool is_q = head < Hq;
     bf16_t* row = qkv + t * row_stride + (int64_t)head * D;
+    // everything the head needs is asked for at once: behind each other the loads are four trips to memory (117 tokens of 16 + 8
+    // heads of 128: 8.7 -> 7.1 us, 2,048 tokens 12.7 -> 9.9 us, with the value heads below)
+    const int position = table ? positions[t] : 0, slot = store && !is_q ? slots[t] : 0;
     const bf16x8r a = *reinterpret_cast<const bf16x8r*>(row + 8 * l);
     const bf16x8r b = *reinterpret_cast<const bf16x8r*>(row + half + 8 * l);
+    const float* w = is_q ? q_w : k_w;
+    float4 wv[4], cv[4];
+    if (w) {
+      wv[0] = *reinterpret_cast<const float4*>(w + 8 * l); wv[1] = *reinterpret_cast<const float4*>(w + 8 * l + 4);
+      wv[2] = *reinterpret_cast<const float4*>(w + half + 8 * l); wv[3] = *reinterpret_cast<const float4*>(w + half + 8 * l + 4);
+    }
+    if (table) {
+      const float4* cs = reinterpret_cast<const float4*>(table + ((int64_t)position * half + 8 * l) * 2);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) cv[i] = cs[i];
+    }
     float x1[8], x2[8];
     float ss = 0.f;
 #pragma unroll
@@ -270,7 +284,6 @@ qk_norm_rope_store_tile_kernel(bf16_t* __restrict__ qkv, int64_t row_stride, con
       x1[i] = static_cast<float>(a[i]); x2[i] = static_cast<float>(b[i]);
       ss += x1[i] * x1[i] + x2[i] * x2[i];
     }
-    const float* w = is_q ? q_w : k_w;
     float inv = 1.f;
     if (w) {
 #pragma unroll
@@ -280,17 +293,15 @@ qk_norm_rope_store_tile_kernel(bf16_t* __restrict__ qkv, int64_t row_stride, con
 #pragma unroll
     for (int i = 0; i < 8; ++i) { x1[i] *= inv; x2[i] *= inv; }
     if (w) {
-      const float4 wa = *reinterpret_cast<const float4*>(w + 8 * l), wb = *reinterpret_cast<const float4*>(w + 8 * l + 4);
-      const float4 wc = *reinterpret_cast<const float4*>(w + half + 8 * l), wd = *reinterpret_cast<const float4*>(w + half + 8 * l + 4);
+      const float4 wa = wv[0], wb = wv[1], wc = wv[2], wd = wv[3];
       const float w1[8] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z, wb.w}, w2[8] = {wc.x, wc.y, wc.z, wc.w, wd.x, wd.y, wd.z, wd.w};
 #pragma unroll
       for (int i = 0; i < 8; ++i) { x1[i] *= w1[i]; x2[i] *= w2[i]; }
     }
     if (table) {
-      const float4* cs = reinterpret_cast<const float4*>(table + ((int64_t)positions[t] * half + 8 * l) * 2);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {   // a float4 holds (cos, sin) of two pairs
-        const float4 c = cs[i];
+        const float4 c = cv[i];
         const float a0 = x1[2 * i], b0 = x2[2 * i], a1 = x1[2 * i + 1], b1 = x2[2 * i + 1];
         x1[2 * i] = a0 * c.x - b0 * c.y; x2[2 * i] = b0 * c.x + a0 * c.y;
         x1[2 * i + 1] = a1 * c.z - b1 * c.w; x2[2 * i + 1] = b1 * c.z + a1 * c.w;
@@ -298,7 +309,6 @@ qk_norm_rope_store_tile_kernel(bf16_t* __restrict__ qkv, int64_t row_stride, con
     }
     bf16_t* dst = row;
     if (!is_q && store) {
-      const int slot = slots[t];
       if (slot < 0) return;
       const int64_t pg = slot / page, off = slot - pg * page;
       dst = k_cache + ((pg * Hkv + (head - Hq)) * (int64_t)page + off) * D;
@@ -319,41 +329,54 @@ qk_norm_rope_store_tile_kernel(bf16_t* __restrict__ qkv, int64_t row_stride, con
   // group is that row and the rows behind it whose slots follow on, up to the end of the aligned eight. Every row
   // lies in exactly one group, and a group is written by the workgroup that holds its first row (which reads up to
   // seven rows of the workgroup behind it). Whole groups take the 16-byte way, the others value by value.
+  // The slots that decide (the row before, the workgroup's own eight and seven behind) are one load of a wave, a lane each; the
+  // groups' channels are dealt to the threads together, and a thread asks for a group's rows at once, whole or not.
   const int dvecs = D >> 3;
+  const int64_t near = t0 - 1 + (threadIdx.x & 15);
+  const int near_slot = near >= 0 && near < num_tokens ? slots[near] : -2;
+  __shared__ int group_row[8], group_slot[8], group_len[8];
+  int groups = 0;
   for (int i = 0; i < cnt; ++i) {
-    const int64_t t = t0 + i;
-    const int s0 = slots[t];
+    const int s0 = __builtin_amdgcn_readlane(near_slot, i + 1);
     if (s0 < 0) continue;
     const int lead = s0 & 7;
-    if (lead != 0 && t > 0 && slots[t - 1] == s0 - 1) continue;       // belongs to the group of a row before it
+    if (lead != 0 && __builtin_amdgcn_readlane(near_slot, i) == s0 - 1) continue;       // belongs to the group of a row before it
     int n = 1;
-    while (n < 8 - lead && t + n < num_tokens && slots[t + n] == s0 + n) ++n;
+    while (n < 8 - lead && __builtin_amdgcn_readlane(near_slot, i + 1 + n) == s0 + n) ++n;
+    if (threadIdx.x == 0) { group_row[groups] = i; group_slot[groups] = s0; group_len[groups] = n; }
+    ++groups;
+  }
+  __syncthreads();
+  const int units = Hkv * dvecs;
+  for (int u = threadIdx.x; u < groups * units; u += 256) {
+    const int group = u / units, unit = u - group * units;
+    const int s0 = group_slot[group], n = group_len[group];
     const int64_t pg = s0 / page, off = s0 - pg * page;               // page % 8 == 0: a group lies within one page
-    for (int unit = threadIdx.x; unit < Hkv * dvecs; unit += 256) {
-      const int kvh = unit / dvecs, dv = unit - kvh * dvecs;
-      const bf16_t* src = qkv + t * row_stride + (int64_t)(v_head + kvh) * D + 8 * dv;
-      bf16_t* dst = v_cache + ((pg * Hkv + kvh) * (int64_t)D + 8 * dv) * page + off;
-      if (n == 8) {
-        u32x4r tok[8];
+    const int kvh = unit / dvecs, dv = unit - kvh * dvecs;
+    const bf16_t* src = qkv + (t0 + group_row[group]) * row_stride + (int64_t)(v_head + kvh) * D + 8 * dv;
+    bf16_t* dst = v_cache + ((pg * Hkv + kvh) * (int64_t)D + 8 * dv) * page + off;
+    u32x4r tok[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) tok[j] = *reinterpret_cast<const u32x4r*>(src + j * row_stride);
+    for (int j = 0; j < 8; ++j) tok[j] = *reinterpret_cast<const u32x4r*>(src + min(j, n - 1) * row_stride);
+    if (n == 8) {
 #pragma unroll
-        for (int d = 0; d < 8; ++d) {   // channel d of the 8 tokens: word d/2 of each token, low or high half
-          u32x4r o;
+      for (int d = 0; d < 8; ++d) {   // channel d of the 8 tokens: word d/2 of each token, low or high half
+        u32x4r o;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const uint32_t lo = tok[2 * j][d >> 1], hi = tok[2 * j + 1][d >> 1];
-            o[j] = (d & 1) ? ((lo >> 16) | (hi & 0xffff0000u)) : ((lo & 0xffffu) | (hi << 16));
-          }
-          *reinterpret_cast<u32x4r*>(dst + (int64_t)d * page) = o;
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t lo = tok[2 * j][d >> 1], hi = tok[2 * j + 1][d >> 1];
+          o[j] = (d & 1) ? ((lo >> 16) | (hi & 0xffff0000u)) : ((lo & 0xffffu) | (hi << 16));
         }
-      } else {
-        for (int j = 0; j < n; ++j) {
-          const bf16x8r v = *reinterpret_cast<const bf16x8r*>(src + j * row_stride);
+        *reinterpret_cast<u32x4r*>(dst + (int64_t)d * page) = o;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (j < n) {
+          const bf16x8r v = __builtin_bit_cast(bf16x8r, tok[j]);
 #pragma unroll
           for (int d = 0; d < 8; ++d) dst[(int64_t)d * page + j] = v[d];
         }
-      }
     }
   }
 }
