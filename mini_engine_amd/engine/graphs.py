@@ -448,7 +448,9 @@ class MixedGraphs:
         pad = total - decode_rows - exact.prefill_tokens
         if pad > r.max_positions:
             return None       # the padding request would stand at positions the engine does not have: run as it is
-        cap = min(max(1024, _pow2_at_least(max(exact.decode_ctx, exact.prefill_ctx, pad))), r.max_positions)
+        # contexts up to 512 keys have a cap of their own: under a cap of 1,024 attention is cut in two segments and merged
+        # (a prompt of 117 tokens at the 0.6B sizes 1.57 -> 1.50 ms)
+        cap = min(max(512, _pow2_at_least(max(exact.decode_ctx, exact.prefill_ctx, pad))), r.max_positions)
         return StepLayout(
             decode_rows=decode_rows, prefill_reqs=exact.prefill_reqs + 1, prefill_tokens=total - decode_rows,
             rows=bucket_of(exact.rows) if exact.rows else 0,
