@@ -73,3 +73,37 @@ def test_attention_keeps_what_is_not_a_number_to_those_who_see_it():
     hit = torch.zeros_like(got, dtype=torch.bool)
     hit[21:40, 2 * 64 + 7] = hit[21:40, 3 * 64 + 7] = True   # the two query heads of that key head
     assert not torch.isfinite(got[hit]).any() and torch.equal(got[~hit], want[~hit])
+
+
+@pytest.mark.parametrize("sinks", [False, True])
+@pytest.mark.parametrize("D,Hq,Hkv,page,keep", [(64, 4, 4, 16, 1), (64, 6, 2, 32, 16), (128, 4, 1, 16, 17), (128, 2, 2, 128, 40), (64, 2, 1, 16, 48)])
+def test_kept_keys_by_pieces_are_those_by_words(D, Hq, Hkv, page, keep, sinks):
+    """Kept keys over pages in steps of 16 against the general kernel (a cache at an odd address takes it): the same sums in the
+    same order, so the same numbers. Tokens in front of the window's end, a page that is gone and a head that saw no key."""
+    g = torch.Generator(device=DEV).manual_seed(D + keep)
+    T, B, pages, window = 70, 2, 12, 20
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    q, out = rnd(T, Hq * D + 8).to(torch.bfloat16), rnd(T, Hq * D).to(torch.bfloat16)
+    lse = rnd(T, Hq) + 2
+    lse[3, 0] = -torch.inf
+    n = pages * Hkv * page * D
+    flat = [rnd(n + 4).to(torch.bfloat16) for _ in range(2)]
+    tables = torch.randperm(pages, device=DEV, generator=g).to(torch.int32).view(B, -1).contiguous()
+    tables[1, 0] = -1
+    seq = (torch.arange(T, device=DEV) >= 40).int()
+    positions = torch.cat((torch.arange(40, device=DEV), torch.arange(10, T - 30, device=DEV))).int()
+    contexts = torch.tensor([40, T - 30], dtype=torch.int32, device=DEV)
+    cap = 3.0 if keep == 17 else 0.0
+    sk, slopes = (rnd(Hq) if sinks else None), (rnd(Hq).abs() if keep == 16 else None)
+    both = []
+    for shift in (0, 4):
+        caches = [torch.empty(n + 4, dtype=torch.bfloat16, device=DEV)[shift:shift + n] for _ in range(2)]
+        for c, f in zip(caches, flat):
+            c.copy_(f[:n])
+        o = out.clone()
+        ops.core().call("me_attn_tail", q.data_ptr(), q.stride(0), o.data_ptr(), o.stride(0), lse.data_ptr(), ops._code(q.dtype),
+                        caches[0].data_ptr(), caches[1].data_ptr(), tables.data_ptr(), tables.stride(0), seq.data_ptr(),
+                        positions.data_ptr(), contexts.data_ptr(), T, Hq, Hkv, D, page, D ** -0.5, window, keep, cap,
+                        ops._ptr(sk), ops._ptr(slopes), ops._stream())
+        both.append(o)
+    assert torch.equal(*both)
