@@ -239,6 +239,46 @@ __global__ void causal_conv_kernel(const TX* __restrict__ x, int64_t x_stride, c
   }
 }
 
+// Up to four taps: eight tokens to a thread, whose inputs are asked for together, with those before them. The walk above has
+// one load in flight and a quarter of the waves; its sums keep their order here.
+// (3,123 tokens, 1,024 channels, four taps: 23.7 -> 7.6 us)
+#define CONV_GROUP 8
+template <typename TX, int TAPS>
+__global__ void causal_conv_group_kernel(const TX* __restrict__ x, int64_t x_stride, const float* __restrict__ w,
+                                         const float* __restrict__ bias, const float* __restrict__ state, int64_t state_stride,
+                                         const int32_t* __restrict__ slots, const int32_t* __restrict__ cu,
+                                         TX* __restrict__ out, int C, int groups_per_seq) {
+  const int b = blockIdx.x / groups_per_seq, group = blockIdx.x - b * groups_per_seq;
+  const int64_t first = cu[b];
+  const int n = (int)(cu[b + 1] - first);
+  const int l0 = group * CONV_GROUP;
+  if (l0 >= n) return;
+  const int c = blockIdx.y * blockDim.x + threadIdx.x;
+  if (c >= C) return;
+  TX in[CONV_GROUP + TAPS - 1];
+  float wv[TAPS], seen[CONV_GROUP + TAPS - 1];
+#pragma unroll
+  for (int i = 0; i < CONV_GROUP + TAPS - 1; ++i)        // positions outside the request: its nearest token, not used
+    in[i] = x[(first + max(0, min(l0 - (TAPS - 1) + i, n - 1))) * x_stride + c];
+#pragma unroll
+  for (int j = 0; j < TAPS; ++j) wv[j] = w[(int64_t)c * TAPS + j];
+  const float bc = bias != nullptr ? bias[c] : 0.f;
+#pragma unroll
+  for (int i = 0; i < CONV_GROUP + TAPS - 1; ++i) seen[i] = to_f32<TX>(in[i]);
+  if (group == 0) {                                      // CONV_GROUP >= TAPS - 1: only the first group looks back past the step
+    const float* held = state + (int64_t)slots[b] * state_stride + (int64_t)c * (TAPS - 1);
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) seen[j] = held[j];
+  }
+#pragma unroll
+  for (int l = 0; l < CONV_GROUP; ++l) {
+    float acc = bc + wv[TAPS - 1] * seen[l + TAPS - 1];
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) acc += wv[j] * seen[l + j];
+    if (l0 + l < n) out[(first + l0 + l) * C + c] = from_f32<TX>(silu_f(acc));
+  }
+}
+
 // The state moves on: per (request, channel) the last taps - 1 inputs of (held inputs, this step's inputs).
 template <typename TX>
 __global__ void causal_conv_state_kernel(const TX* __restrict__ x, int64_t x_stride, float* __restrict__ state,
@@ -298,10 +338,20 @@ extern "C" int me_causal_conv(const void* x, int64_t x_stride, int dtype, const 
     ME_LAUNCH_CHECK();
     return 0;
   }
-  const int blocks_per_seq = (max_tokens + CONV_TOKENS - 1) / CONV_TOKENS;
+  const int per_block = taps >= 2 && taps <= 4 ? CONV_GROUP : CONV_TOKENS;
+  const int blocks_per_seq = (max_tokens + per_block - 1) / per_block;
   ME_CHECK(max_tokens >= 1 && (int64_t)num_seqs * blocks_per_seq <= 2147483647ll, "causal_conv: bad token bound %d", max_tokens);
   const dim3 wgrid((unsigned)(num_seqs * blocks_per_seq), (C + block.x - 1) / block.x);
-  if (dtype == ME_F32)
+#define CG(TX, TAPS) causal_conv_group_kernel<TX, TAPS><<<wgrid, block, 0, stream>>>((const TX*)x, x_stride, w, bias, state, \
+                                                                                     state_stride, slots, cu, (TX*)out, C, blocks_per_seq)
+  if (per_block == CONV_GROUP) {
+    if (dtype == ME_F32) {
+      if (taps == 4) CG(float, 4); else if (taps == 3) CG(float, 3); else CG(float, 2);
+    } else {
+      if (taps == 4) CG(bf16_t, 4); else if (taps == 3) CG(bf16_t, 3); else CG(bf16_t, 2);
+    }
+  } else if (dtype == ME_F32)
+#undef CG
     causal_conv_kernel<float><<<wgrid, block, 0, stream>>>((const float*)x, x_stride, w, bias, state, state_stride, slots, cu,
                                                            (float*)out, C, taps, blocks_per_seq);
   else

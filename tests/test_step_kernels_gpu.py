@@ -67,3 +67,71 @@ def test_choices_in_registers_and_through_lds(T, E, groups, keep, top, group_top
     got = hip().route_and_run_experts(x.to(torch.bfloat16), router, top, groups, keep, up.to(torch.bfloat16), down.to(torch.bfloat16), rule=rule, gated=False)
     want = twin.routed_experts(x.cpu().to(torch.bfloat16), ids.cpu(), weights.cpu(), up.cpu().to(torch.bfloat16), down.cpu().to(torch.bfloat16), gated=False)
     close(got.sum(0), want.sum(0), 3e-2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [4, 252, 1020, 1024, 1028, 2056])
+def test_rows_by_fours_are_those_by_ones(n, dtype):
+    """Bias, gate and token mix of rows that begin at any fourth element, against the same rows one element further on, which the
+    general kernels take: each value is formed by the same steps."""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    T, S = 9, 5
+    rows = torch.randn(T, n + 8, device=DEV, generator=g).to(dtype)
+    gate = torch.randn(T, n + 8, device=DEV, generator=g).to(dtype)
+    odd = lambda t: torch.nn.functional.pad(t, (1, 0))[:, 1:]
+    for nb in (0, 4, n):
+        bias = torch.randn(nb, device=DEV, generator=g)
+        for out_dtype in (torch.float32, torch.bfloat16):
+            assert torch.equal(hip().add_bias(rows[:, 4:4 + n], bias, out_dtype), hip().add_bias(odd(rows)[:, 4:4 + n], bias, out_dtype))
+    a, b = rows.clone(), odd(rows)
+    hip().sigmoid_gate_(a[:, 4:4 + n], gate[:, 4:4 + n])
+    hip().sigmoid_gate_(b[:, 4:4 + n], gate[:, 4:4 + n])
+    assert torch.equal(a, b)
+    mu = torch.randn(S, n, device=DEV, generator=g)
+    cu = torch.tensor([0, 1, 6, T], dtype=torch.int32, device=DEV)
+    seq = torch.tensor([0] + [1] * 5 + [2] * 3, dtype=torch.int32, device=DEV)
+    slots = torch.tensor([2, 0, 3], dtype=torch.int32, device=DEV)
+    first = torch.randn(4, n + 3, device=DEV, generator=g)
+    states = [first.clone(), first.clone()]
+    mixes = [hip().token_shift(x[:, 4:4 + n], mu, st[:, 3:], slots, cu, seq) for x, st in zip((rows, odd(rows)), states)]
+    assert torch.equal(*mixes) and torch.equal(*states)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [1023, 1024, 1025, 2048, 2049, 4096, 4097])
+def test_weighted_sum_and_norm_widths(n, dtype):
+    """Rows in registers from 1,024 to 4,096 numbers, through LDS on either side: a term as partial sums with a bias, one with
+    gate rows. Float32 sums of up to 4,097 squares; one rounding to the output type."""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    T = 5
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    terms = [(rnd(3, T, n), 0.7, rnd(n)), (rnd(T, n).to(dtype), -0.3, None, rnd(T, 2).to(dtype)[:, 1]), (rnd(T, n).to(dtype), 1.1, None)]
+    w, stream = rnd(n), rnd(T, n)
+    got = hip().weighted_sum(terms, w, 1e-6, stream, dtype)
+    cpu = [tuple(v.cpu() if torch.is_tensor(v) else v for v in term) for term in terms]
+    want = twin.weighted_sum(cpu, w.cpu(), 1e-6, stream.cpu(), dtype)
+    close(got[0], want[0], 1e-6 if dtype == torch.float32 else 8e-3)
+    close(got[1], want[1], 1e-6)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("taps", [1, 2, 3, 4, 5])
+def test_short_convolution_over_the_ends_of_its_groups(taps, dtype):
+    """Requests of every length around the eight tokens of a thread; portions of a request give what it gives in one piece."""
+    g = torch.Generator(device=DEV).manual_seed(taps)
+    C, q_lens = 70, [1, 2, 3, 7, 8, 9, 16, 17, 33]
+    T, B = sum(q_lens), len(q_lens)
+    x = torch.randn(T, C + 3, device=DEV, generator=g).to(dtype)[:, 2:2 + C]
+    w, b = torch.randn(C, taps, device=DEV, generator=g), torch.randn(C, device=DEV, generator=g)
+    state = torch.randn(B, C * (taps - 1), device=DEV, generator=g)
+    want_state = state.cpu().clone()
+    slots = torch.arange(B, dtype=torch.int32, device=DEV).flip(0).contiguous()
+    cu = torch.tensor([0] + q_lens, device=DEV).cumsum(0).int()
+    before = state.clone()
+    got = hip().causal_conv(x, w, b, state, slots, cu, q_lens)
+    want = twin.causal_conv(x.cpu(), w.cpu(), b.cpu(), want_state, slots.cpu(), cu.cpu(), q_lens)
+    close(got, want, 1e-6 if dtype == torch.float32 else 8e-3)
+    assert torch.equal(state.cpu(), want_state)
+    pieces = [hip().causal_conv(x[T - 33 + lo:T - 33 + hi], w, b, before, slots[-1:], torch.tensor([0, hi - lo], dtype=torch.int32, device=DEV), [hi - lo])
+              for lo, hi in ((0, 1), (1, 12), (12, 33))]
+    close(torch.cat(pieces), got[T - 33:], 1e-6 if dtype == torch.float32 else 8e-3)
