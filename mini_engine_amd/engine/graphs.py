@@ -448,14 +448,18 @@ class MixedGraphs:
         pad = total - decode_rows - exact.prefill_tokens
         if pad > r.max_positions:
             return None       # the padding request would stand at positions the engine does not have: run as it is
-        # contexts up to 512 keys have a cap of their own: under a cap of 1,024 attention is cut in two segments and merged
-        # (a prompt of 117 tokens at the 0.6B sizes 1.57 -> 1.50 ms)
-        cap = min(max(512, _pow2_at_least(max(exact.decode_ctx, exact.prefill_ctx, pad))), r.max_positions)
+        # Contexts up to 512 keys have a cap of their own for the prompts: under a cap of 1,024 their attention is planned in
+        # two segments, of which no prompt's tile reaches the second, and a launch merges nothing (the same sums; a prompt
+        # of 117 tokens at the 0.6B sizes 1.57 -> 1.50 ms). Decoding rows keep the cap of 1,024: it decides into how many
+        # partitions their keys are cut (16 rows: 4 of 256 under 1,024, 4 of 128 under 512), and with that the order of their sums.
+        reach = _pow2_at_least(max(exact.decode_ctx, exact.prefill_ctx, pad))
+        cap, decode_cap = (min(max(least, reach), r.max_positions) for least in (512, 1024))
+        longest = decode_cap if exact.decode_rows else cap
         return StepLayout(
             decode_rows=decode_rows, prefill_reqs=exact.prefill_reqs + 1, prefill_tokens=total - decode_rows,
             rows=bucket_of(exact.rows) if exact.rows else 0,
-            max_blocks=tuple(max(mb, -(-cap // ps)) for mb in exact.max_blocks),
-            decode_ctx=cap if exact.decode_rows else 0, prefill_ctx=cap, even=exact.even)
+            max_blocks=tuple(max(mb, -(-longest // ps)) for mb in exact.max_blocks),
+            decode_ctx=decode_cap if exact.decode_rows else 0, prefill_ctx=cap, even=exact.even)
 
     def lookup(self, exact: StepLayout):
         """The captured (or about to be captured) layout that takes this step, or None: run it eagerly."""

@@ -12,6 +12,7 @@ import helpers
 import plain_qwen3
 from mini_engine_amd.cache.manager import CacheManager
 from mini_engine_amd.engine.runner import ModelRunner, StepEntry
+from mini_engine_amd.kernels import ops
 from mini_engine_amd.weights.loader import load_model
 
 
@@ -296,6 +297,28 @@ def test_fixed_layouts_with_a_longest_context_that_is_no_multiple_of_8(folders, 
     assert runner.graphs.replays == 6
     assert all(c.context().max_decode_context <= limit for c in runner.graphs.captured.values())
     assert helpers.rel_err(d.result("r"), helpers.plain_logits(folder, ids)) <= helpers.TOL_F32
+
+
+@pytest.mark.parametrize("rows", [0, 1, 8, 16, 20, 32, 61])
+@pytest.mark.parametrize("longest", [40, 300, 512, 513, 1500])
+def test_a_padded_layouts_caps_leave_the_order_of_its_sums(folders, plain_backend, rows, longest):
+    """What a padded layout tells attention about short contexts may save launches, not regroup sums: decoding rows are cut into the
+    partitions that a cap of 1,024 gives them, a prompt's tiles into as many segments of the keys that they have."""
+    from mini_engine_amd.engine.packing import StepLayout
+    model = load_model(folders("A"), "cpu", torch.float32, 4096)
+    manager = CacheManager(20, 16, ModelRunner.windows_of(model), enable_prefix_caching=False)
+    runner = ModelRunner(model, manager, torch.float32, "cpu", 4096, use_graphs=True, mixed_graphs_after=0, mixed_graphs_max_tokens=4096)
+    exact = StepLayout(rows, 1, 30, rows + 1, (-(-longest // 16),), longest if rows else 0, longest, False)
+    padded = runner.mixed_graphs.padded(exact)
+    cap = max(1024, 1 << (longest - 1).bit_length())
+    assert all(mb * 16 >= max(padded.decode_ctx, padded.prefill_ctx) >= longest for mb in padded.max_blocks)
+    if rows:
+        assert ops.decode_partitions(padded.decode_rows, 16, 8, padded.decode_ctx) == ops.decode_partitions(padded.decode_rows, 16, 8, cap)
+    keys, most = ops.prefill_segments(padded.prefill_ctx, 0, padded.prefill_tokens, 16)
+    want, _ = ops.prefill_segments(cap, 0, padded.prefill_tokens, 16)
+    segments = lambda size: -(-longest // size) if size and longest > size else 1
+    assert segments(keys) == segments(want) and (segments(keys) == 1 or keys == want)
+    assert most == 1 or padded.prefill_ctx > 512
 
 
 def test_a_padding_request_longer_than_the_longest_context_is_not_made(folders, plain_backend):
