@@ -14,8 +14,11 @@
 #include "common.h"
 #include <hipblaslt/hipblaslt.h>
 #include <dlfcn.h>
+#include <cstdio>
+#include <cstring>
 #include <map>
 #include <mutex>
+#include <string>
 #include <tuple>
 
 namespace {
@@ -33,6 +36,7 @@ struct Api {
   decltype(&hipblasLtMatmulPreferenceDestroy) pref_destroy = nullptr;
   decltype(&hipblasLtMatmulAlgoGetHeuristic) heuristic = nullptr;
   decltype(&hipblasLtMatmul) matmul = nullptr;
+  std::string (*kernel_name)(hipblasLtHandle_t, hipblasLtMatmulAlgo_t&) = nullptr;   // hipblaslt_ext::getKernelNameFromAlgo
   bool looked = false, ok = false;
 };
 
@@ -76,7 +80,55 @@ bool look_up_api() {
              bind(lib, "hipblasLtMatmulPreferenceDestroy", g_api.pref_destroy) &&
              bind(lib, "hipblasLtMatmulAlgoGetHeuristic", g_api.heuristic) &&
              bind(lib, "hipblasLtMatmul", g_api.matmul);
+  bind(lib, "_ZN13hipblaslt_ext21getKernelNameFromAlgoB5cxx11EPvR22_hipblasLtMatmulAlgo_t", g_api.kernel_name);
   return g_api.ok;
+}
+
+std::string name_of(hipblasLtHandle_t handle, hipblasLtMatmulAlgo_t algo) {
+  try {
+    return g_api.kernel_name ? g_api.kernel_name(handle, algo) : std::string();
+  } catch (...) {
+    return std::string();
+  }
+}
+
+// One of the library's kernels is not taken: its hand-scheduled one of 256 x 256 tiles ("Custom_..."), the heuristic's
+// first choice for the largest products, now and then returns wrong values. Products of 5,968 to 8,005 rows over weights
+// of 4096 x 1024 and 6144 x 1024 beside others of 1024 x 2048 and 1024 x 3072, the same operands again and again: 37 of 1.8
+// million launches of it gave other values (mostly in 32 rows by 32 to 256 features, up to four standard deviations of the
+// result off), none of 1.2 million of the kernels below and none of 3.1 million of those of the other two weights.
+bool is_unsound(const std::string& name) { return name.find("Custom") != std::string::npos; }
+
+// In its place: of the kernels that the heuristic names for the shape and that add up K in one piece (no workspace, so the
+// same sums in the same order: their results are bit for bit those of the kernel above where it is right), with feature tiles
+// that divide N (where they do not, an edge costs every tile: 192 x 256 tiles 108 us at 8,000 rows of 4096 x 1024), the one of
+// the least rounds x (tile area + 280 (height + width)) over the compute units, a fifth more with half the depth in K. us of
+// the unsound kernel / the one chosen / the heuristic's next: 8,000 rows of 4096 x 1024 59 / 65 / 72-78, of 6144 x 1024 86 / 95 /
+// 95; 3,123 rows of 4096 x 1024 27.4 / 27.6 / 38.4; 4,096 rows of 4096 x 4096 89 / 106 / 112; 2,048 rows of 24576 x 4096 270 / 314 / 314.
+bool other_choice(hipblasLtHandle_t handle, const Plan& p, hipblasLtMatmulPreference_t pref, int M, int N, int splits,
+                  hipblasLtMatmulHeuristicResult_t& found) {
+  constexpr int MOST = 32;
+  hipblasLtMatmulHeuristicResult_t offers[MOST];
+  int count = 0, device = 0, units = 0;
+  if (g_api.heuristic(handle, p.desc, p.a, p.b, p.c, p.c, pref, MOST, offers, &count) != HIPBLAS_STATUS_SUCCESS ||
+      hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || units < 1)
+    return false;
+  double least = 0.0;
+  for (int i = 0; i < count; ++i) {
+    const std::string name = name_of(handle, offers[i].algo);
+    const size_t at = name.find("_MT");
+    int height = 0, width = 0, depth = 0;
+    if (offers[i].state != HIPBLAS_STATUS_SUCCESS || offers[i].workspaceSize != 0 || is_unsound(name) || at == std::string::npos ||
+        std::sscanf(name.c_str() + at, "_MT%dx%dx%d", &height, &width, &depth) != 3 || height < 1 || width < 1 || N % height != 0)
+      continue;
+    const int64_t tiles = (int64_t)(N / height) * ((M + width - 1) / width) * splits;
+    const double cost = (double)((tiles + units - 1) / units) * (height * width + 280.0 * (height + width)) * (depth < 64 ? 1.2 : 1.0);
+    if (least == 0.0 || cost < least) {
+      least = cost;
+      found = offers[i];
+    }
+  }
+  return least > 0.0;
 }
 
 // Row-major y = x . w^T is, in the library's column-major terms, D[N, M] = op_T(A)[N, K] . B[K, M]
@@ -111,6 +163,7 @@ bool fill_plan(hipblasLtHandle_t handle, Plan& p, int M, int N, int K, int64_t l
   int count = 0;
   ok = ok && g_api.heuristic(handle, p.desc, p.a, p.b, p.c, p.c, pref, 1, &found, &count) == HIPBLAS_STATUS_SUCCESS &&
        count >= 1 && found.state == HIPBLAS_STATUS_SUCCESS && found.workspaceSize <= workspace_bytes;
+  if (ok && is_unsound(name_of(handle, found.algo))) other_choice(handle, p, pref, M, N, splits, found);
   g_api.pref_destroy(pref);
   if (!ok) return false;
   p.algo = found.algo;
@@ -135,6 +188,20 @@ bool make_plan(hipblasLtHandle_t handle, Plan& p, int M, int N, int K, int64_t l
 extern "C" int me_gemm_library_available() {
   std::lock_guard<std::mutex> lock(g_mutex);
   return look_up_api() ? 1 : 0;
+}
+
+// The name of the kernel that a product over contiguous operands runs, at most n - 1 characters and a zero at `out`; empty if
+// none has been asked for or the library names none.
+extern "C" int me_gemm_library_kernel(int out_dtype, size_t workspace_bytes, int M, int N, int K, int splits, char* out, int n) {
+  ME_CHECK(out != nullptr && n >= 1, "gemm_library: no place for a name");
+  out[0] = 0;
+  int device = 0;
+  ME_CHECK(hipGetDevice(&device) == hipSuccess, "gemm_library: no current device");
+  std::lock_guard<std::mutex> lock(g_mutex);
+  const auto plan = g_plans.find(PlanKey{device, M, N, K, K, K, N, out_dtype, workspace_bytes, splits});
+  if (plan == g_plans.end() || !plan->second.ok) return 0;
+  std::snprintf(out, (size_t)n, "%s", name_of(g_handles.at(device), plan->second.algo).c_str());
+  return 0;
 }
 
 // y[M, N] (bfloat16 or float32, row stride ldy) = x[M, K] (bfloat16, row stride ldx) . w[N, K]^T
