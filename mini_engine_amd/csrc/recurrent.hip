@@ -203,7 +203,8 @@ extern "C" int me_head_gate(void* o, const void* g, int64_t g_stride, int dtype,
 // request come from its state row: per channel taps - 1 values, oldest first. One thread per (token, channel).
 #define CONV_MAX_TAPS 16
 
-#define CONV_TOKENS 32       // tokens of one request that a thread walks
+// tokens of one request that a thread walks, or takes at once (which of the two: the caller's rule, conv_tokens_per_thread)
+#define CONV_TOKENS 32
 
 // One thread per (request, block of CONV_TOKENS tokens, channel): it walks its tokens in order with the last taps - 1
 // inputs in registers, so every input is read once and the step's metadata once per workgroup.
@@ -240,7 +241,8 @@ __global__ void causal_conv_kernel(const TX* __restrict__ x, int64_t x_stride, c
 }
 
 // Up to four taps: eight tokens to a thread, whose inputs are asked for together, with those before them. The walk above has
-// one load in flight and a quarter of the waves; its sums keep their order here.
+// one load in flight and a quarter of the waves; its sums keep their order here. The grid has every request's share of the longest
+// one, empty or not, so steps of one long request among many short ones stay with the walk.
 // (3,123 tokens, 1,024 channels, four taps: 23.7 -> 7.6 us)
 #define CONV_GROUP 8
 template <typename TX, int TAPS>
@@ -320,10 +322,11 @@ __global__ void causal_conv_step_kernel(const TX* __restrict__ x, int64_t x_stri
 
 // max_tokens: no request brings more tokens than this.
 extern "C" int me_causal_conv(const void* x, int64_t x_stride, int dtype, const float* w, const float* bias, float* state,
-                              int64_t state_stride, const int32_t* slots, const int32_t* cu, int max_tokens,
+                              int64_t state_stride, const int32_t* slots, const int32_t* cu, int max_tokens, int per_block,
                               void* out, int64_t T, int num_seqs, int C, int taps, hipStream_t stream) {
   if (T == 0 || C == 0) return 0;
   ME_CHECK(taps >= 1 && taps <= CONV_MAX_TAPS, "causal_conv: %d taps outside 1..%d", taps, CONV_MAX_TAPS);
+  ME_CHECK(per_block == CONV_TOKENS || (per_block == CONV_GROUP && taps >= 2 && taps <= 4), "causal_conv: no form of %d tokens to a thread", per_block);
   const dim3 block(C >= 256 ? 256 : 64);
   ME_CHECK(T <= 2147483647ll && num_seqs <= 65535 && (C + block.x - 1) / block.x <= 65535,
            "causal_conv: too many tokens, requests or channels for one launch");
@@ -338,7 +341,6 @@ extern "C" int me_causal_conv(const void* x, int64_t x_stride, int dtype, const 
     ME_LAUNCH_CHECK();
     return 0;
   }
-  const int per_block = taps >= 2 && taps <= 4 ? CONV_GROUP : CONV_TOKENS;
   const int blocks_per_seq = (max_tokens + per_block - 1) / per_block;
   ME_CHECK(max_tokens >= 1 && (int64_t)num_seqs * blocks_per_seq <= 2147483647ll, "causal_conv: bad token bound %d", max_tokens);
   const dim3 wgrid((unsigned)(num_seqs * blocks_per_seq), (C + block.x - 1) / block.x);

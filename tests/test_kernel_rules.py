@@ -253,3 +253,13 @@ def test_partitions_for_wide_heads():
         for ctx in (1, 129, 2048, 5000, 70000):
             part, parts = ops.wide_head_partitions(*ops.decode_partitions(base, 16, 1, ctx), base, ctx)
             assert part * parts >= ctx and part * (parts - 1) < ctx and part % 32 == 0
+
+
+def test_the_short_convolutions_grid_is_not_mostly_empty():
+    """Whatever a step holds, by eights a launch is small or a workgroup in eight has tokens; prompts of like lengths go by eights."""
+    for q_lens, per in (([8192] + [1] * 63, 32), ([32768] + [1] * 255, 32), ([300] + [1] * 20, 8), ([350] * 8, 8), ([3123], 8), ([9] * 32, 8),
+                        ([8192] + [1] * 31, 8), ([65536, 60000, 3], 8), ([1, 17], 8)):
+        T, B, longest = sum(q_lens), len(q_lens), max(q_lens)
+        assert ops.conv_tokens_per_thread(T, B, longest, 4, 1024) == per, q_lens
+        assert per == 32 or B * -(-longest // 8) * 4 <= max(1 << 17, 32 * -(-T // 8))
+    assert ops.conv_tokens_per_thread(350, 1, 350, 5, 64) == ops.conv_tokens_per_thread(350, 1, 350, 1, 64) == 32

@@ -135,3 +135,22 @@ def test_short_convolution_over_the_ends_of_its_groups(taps, dtype):
     pieces = [hip().causal_conv(x[T - 33 + lo:T - 33 + hi], w, b, before, slots[-1:], torch.tensor([0, hi - lo], dtype=torch.int32, device=DEV), [hi - lo])
               for lo, hi in ((0, 1), (1, 12), (12, 33))]
     close(torch.cat(pieces), got[T - 33:], 1e-6 if dtype == torch.float32 else 8e-3)
+
+
+@pytest.mark.parametrize("taps", [2, 4, 5])
+def test_short_convolution_of_one_long_request_among_short_ones(monkeypatch, taps):
+    """Steps whose grid by eights would be large and mostly empty walk their tokens: both forms add in one order, so the same bits."""
+    g = torch.Generator(device=DEV).manual_seed(taps)
+    C, q_lens = 70, [300] + [1] * 20
+    T, B = sum(q_lens), len(q_lens)
+    x = torch.randn(T, C, device=DEV, generator=g).to(torch.bfloat16)
+    w, state = torch.randn(C, taps, device=DEV, generator=g), torch.randn(B, C * (taps - 1), device=DEV, generator=g)
+    slots, cu = torch.arange(B, dtype=torch.int32, device=DEV), torch.tensor([0] + q_lens, device=DEV).cumsum(0).int()
+    monkeypatch.setattr(ops, "conv_tokens_per_thread", lambda *a: 32)
+    states = [state.clone(), state.clone()]
+    walked = hip().causal_conv(x, w, None, states[0], slots, cu, q_lens)
+    if taps <= 4:
+        monkeypatch.setattr(ops, "conv_tokens_per_thread", lambda *a: 8)
+    assert torch.equal(hip().causal_conv(x, w, None, states[1], slots, cu, q_lens), walked) and torch.equal(*states)
+    want = twin.causal_conv(x.cpu(), w.cpu(), None, state.cpu(), slots.cpu(), cu.cpu(), q_lens)
+    close(walked, want, 8e-3)
