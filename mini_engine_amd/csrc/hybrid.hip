@@ -18,6 +18,11 @@ __device__ __forceinline__ typename Four<T>::type four_of(const T* p) { return *
 static bool by_fours(const void* p, int dtype, int64_t stride) {
   return (uintptr_t)p % (dtype == ME_F32 ? 16 : 8) == 0 && stride % 4 == 0;
 }
+// Whether T rows of n go to the kernels that take a row by fours with a column of workgroups each, and their threads: from 128
+// numbers on (16,384 rows of 64: bias 4.5 us with a thread per number and 6.0 by fours, of 128 6.4 and 6.3, of 256 10.1 and
+// 6.9), and while the grid's first side stays below 2^32 threads.
+static int threads_by_fours(int n) { return n / 4 >= 256 ? 256 : 64; }
+static bool rows_by_fours(int64_t T, int n) { return n % 4 == 0 && n >= 128 && n <= 4000000 && T * threads_by_fours(n) < (1ll << 32); }
 
 // ------------------------------------------------------------------ rows + bias
 // out[t, c] = (sum_p x[p, t, c]) + bias[c] for c < nb, without a bias beyond; x: `parts` stacked slices.
@@ -62,9 +67,9 @@ extern "C" int me_add_bias(const void* x, int x_dtype, int parts, int64_t part_s
   ME_CHECK(parts >= 1 && nb >= 0 && nb <= n, "add_bias: bad slice count or bias length");
   const int64_t total = T * n;
   const dim3 grid((unsigned)((total + 255) / 256 < 65535 ? (total + 255) / 256 : 65535)), block(256);
-  const int threads = n / 4 >= 256 ? 256 : 64;
-  const bool fours = n % 4 == 0 && nb % 4 == 0 && (nb == 0 || by_fours(bias, ME_F32, 0)) && by_fours(x, x_dtype, x_stride) &&
-                     (parts == 1 || part_stride % 4 == 0) && by_fours(out, out_dtype, 0) && T <= 2147483647ll && n <= 4000000;
+  const int threads = threads_by_fours(n);
+  const bool fours = rows_by_fours(T, n) && nb % 4 == 0 && (nb == 0 || by_fours(bias, ME_F32, 0)) && by_fours(x, x_dtype, x_stride) &&
+                     (parts == 1 || part_stride % 4 == 0) && by_fours(out, out_dtype, 0);
   const dim3 rows((unsigned)T, (n / 4 + threads - 1) / threads);
 #define AB(TX, TY) do { \
     if (fours) add_bias_fours_kernel<TX, TY><<<rows, threads, 0, stream>>>((const TX*)x, parts, part_stride, x_stride, bias, nb, (TY*)out, n); \
@@ -107,8 +112,8 @@ extern "C" int me_sigmoid_gate(void* o, int64_t o_stride, const void* g, int64_t
   if (T == 0 || n == 0) return 0;
   const int64_t total = T * n;
   const dim3 grid((unsigned)((total + 255) / 256 < 65535 ? (total + 255) / 256 : 65535)), block(256);
-  if (n % 4 == 0 && by_fours(o, dtype, o_stride) && by_fours(g, dtype, g_stride) && T <= 2147483647ll && n <= 4000000) {
-    const int threads = n / 4 >= 256 ? 256 : 64;
+  if (rows_by_fours(T, n) && by_fours(o, dtype, o_stride) && by_fours(g, dtype, g_stride)) {
+    const int threads = threads_by_fours(n);
     const dim3 rows((unsigned)T, (n / 4 + threads - 1) / threads);
     if (dtype == ME_F32) sigmoid_gate_fours_kernel<float><<<rows, threads, 0, stream>>>((float*)o, o_stride, (const float*)g, g_stride, n);
     else sigmoid_gate_fours_kernel<bf16_t><<<rows, threads, 0, stream>>>((bf16_t*)o, o_stride, (const bf16_t*)g, g_stride, n);
@@ -361,8 +366,8 @@ extern "C" int me_token_shift(const void* x, int64_t x_stride, int dtype, const 
   const dim3 block(n >= 256 ? 256 : 64);
   const unsigned gy = (unsigned)((n + block.x - 1) / block.x < 64 ? (n + block.x - 1) / block.x : 64);
   const dim3 grid((unsigned)T, gy);
-  if (n % 4 == 0 && by_fours(x, dtype, x_stride) && by_fours(mu, ME_F32, 0) && by_fours(out, dtype, 0) && n <= 4000000) {
-    const int threads = n / 4 >= 256 ? 256 : 64;
+  if (rows_by_fours(T, n) && by_fours(x, dtype, x_stride) && by_fours(mu, ME_F32, 0) && by_fours(out, dtype, 0)) {
+    const int threads = threads_by_fours(n);
     const dim3 rows((unsigned)T, (n / 4 + threads - 1) / threads);
     if (dtype == ME_F32)
       token_shift_fours_kernel<float><<<rows, threads, 0, stream>>>((const float*)x, x_stride, mu, S, state, state_stride, slots, cu, seq_of_token, (float*)out, T, n);

@@ -154,3 +154,13 @@ def test_short_convolution_of_one_long_request_among_short_ones(monkeypatch, tap
     assert torch.equal(hip().causal_conv(x, w, None, states[1], slots, cu, q_lens), walked) and torch.equal(*states)
     want = twin.causal_conv(x.cpu(), w.cpu(), None, state.cpu(), slots.cpu(), cu.cpu(), q_lens)
     close(walked, want, 8e-3)
+
+
+def test_a_bias_on_more_rows_than_a_grid_has_by_fours():
+    """2^26 + 8 rows of 128 by fours would be 2^32 threads and more: the general kernel takes them (17 GB of results)."""
+    T, n = (1 << 26) + 8, 128
+    row, bias = torch.randn(1, n, device=DEV).to(torch.bfloat16), torch.randn(n, device=DEV)
+    out = hip().add_bias(row.expand(T, n), bias, torch.bfloat16)
+    want = hip().add_bias(row, bias, torch.bfloat16)
+    for part in out.split(1 << 23):
+        assert bool((part == want).all())
