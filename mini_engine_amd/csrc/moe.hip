@@ -26,6 +26,7 @@
 #include "common.h"
 
 #define MOE_MAX_EXPERTS 1024
+#define MOE_LDS_PAIRS 10240      // pairs whose ids moe_sort keeps in LDS when it makes the choice itself (40 KB)
 #define MOE_TM 64
 
 // ------------------------------------------------------------------ router
@@ -391,7 +392,7 @@ __device__ __forceinline__ int count_one(int* counter, int e, int common) {
 // tile_expert / tile_row: expert and first sorted place of every tile of up to `tile_rows` pairs (expert -1: a tile nobody needs).
 // With `logits` (few tokens) the workgroup first makes the choice itself, a wave per token in turn, and writes ids and
 // weights: the launch of `moe_select` is saved. What bounds it is the length of one workgroup's way: up to 64 experts the
-// choice runs in registers with a wave's next token on its way, the ids stay in LDS, and one wave adds up the classes' places by
+// choice runs in registers with a wave's next token on its way, the ids stay in LDS (up to MOE_LDS_PAIRS of them), and one wave adds up the classes' places by
 // exchanges (32 tokens, 32 experts, 4 of 4 groups: 20.5 us with races through LDS and one thread adding up -> 10.4 us).
 __global__ void __launch_bounds__(1024)
 moe_sort_kernel(int32_t* __restrict__ ids, int P, int routed, int E, int max_tiles, int tile_rows, int32_t* __restrict__ order,
@@ -403,7 +404,7 @@ moe_sort_kernel(int32_t* __restrict__ ids, int P, int routed, int E, int max_til
   const int wave = threadIdx.x >> 6, waves = blockDim.x >> 6, lane = threadIdx.x & 63;
   const int32_t* pairs = ids;                        // where the pairs' ids are read
   if (logits && routed <= 64) {
-    int32_t* chosen = reinterpret_cast<int32_t*>(route_lds);
+    int32_t* chosen = P <= MOE_LDS_PAIRS ? reinterpret_cast<int32_t*>(route_lds) : nullptr;
     const int T = P / rule.top, at = min(lane, routed - 1);
     float next = wave < T ? logits[(int64_t)wave * routed + at] : 0.f;
     for (int t = wave; t < T; t += waves) {
@@ -411,7 +412,7 @@ moe_sort_kernel(int32_t* __restrict__ ids, int P, int routed, int E, int max_til
       if (t + waves < T) next = logits[(int64_t)(t + waves) * routed + at];
       select_token64(x, t, routed, rule, ids, weights, chosen);
     }
-    pairs = chosen;
+    if (chosen) pairs = chosen; else __threadfence_block();
   } else if (logits) {
     float* s = reinterpret_cast<float*>(route_lds) + (size_t)wave * (2 * routed + rule.group_count);
     for (int t = wave; t < P / rule.top; t += waves) select_token(logits, t, routed, rule, s, s + routed, s + 2 * routed, ids, weights);
@@ -475,8 +476,8 @@ extern "C" int me_moe_sort(int32_t* ids, int64_t P, int routed, int identity, in
   if (logits) {
     ME_CHECK(weights && route_rule(rule, routed, top, group_count, group_keep, group_top, sigmoid, normalise, scale, correction) && P % top == 0,
              "moe_sort: bad routing sizes");
-    lds = routed <= 64 ? (size_t)P * 4 : (size_t)16 * (2 * routed + group_count) * 4;
-    ME_CHECK(lds <= 40 * 1024, "moe_sort: %d experts or %lld pairs are too many to choose here", routed, (long long)P);
+    lds = routed > 64 ? (size_t)16 * (2 * routed + group_count) * 4 : P <= MOE_LDS_PAIRS ? (size_t)P * 4 : 0;
+    ME_CHECK(lds <= 40 * 1024, "moe_sort: %d experts are too many to choose here", routed);
   }
   moe_sort_kernel<<<dim3(1), dim3(1024), lds, stream>>>(ids, (int)P, routed, E, max_tiles, tile_rows, order, offsets, tile_expert, tile_row,
                                                         logits, weights, rule);

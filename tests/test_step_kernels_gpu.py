@@ -164,3 +164,22 @@ def test_a_bias_on_more_rows_than_a_grid_has_by_fours():
     want = hip().add_bias(row, bias, torch.bfloat16)
     for part in out.split(1 << 23):
         assert bool((part == want).all())
+
+
+def test_the_pairs_kernel_chooses_for_any_number_of_tokens():
+    """More pairs than their ids have room for in LDS: chosen, counted and ordered all the same (a caller of the entry itself)."""
+    T, E, top, rows = 6000, 32, 2, 64
+    g = torch.Generator(device=DEV).manual_seed(4)
+    logits = torch.randn(T, E, device=DEV, generator=g)
+    P = T * top
+    ids, weights = torch.empty(P, dtype=torch.int32, device=DEV), torch.empty(P, device=DEV)
+    most = P // rows + E
+    order, offsets, expert, row = (torch.empty(k, dtype=torch.int32, device=DEV) for k in (P, E + 1, most, most))
+    ops.core().call("me_moe_sort", ids.data_ptr(), P, E, 0, most, rows, order.data_ptr(), offsets.data_ptr(), expert.data_ptr(), row.data_ptr(),
+                    logits.data_ptr(), weights.data_ptr(), top, 1, 1, *ops.RouteRule("chosen").args(), ops._stream())
+    best = logits.topk(top, -1)
+    assert torch.equal(ids.view(T, top).long(), best.indices)
+    close(weights.view(T, top), torch.softmax(best.values.double(), -1), 2e-6)
+    assert torch.equal(order.sort().values.long(), torch.arange(P, device=DEV))
+    assert torch.equal(ids[order.long()].sort().values, ids[order.long()])
+    assert torch.equal(offsets[1:].long(), torch.bincount(ids.long(), minlength=E).cumsum(0))
