@@ -37,18 +37,20 @@ __device__ __forceinline__ float term_value(const void* ptr, int dtype, int part
   return scale ? scale[i] * v : v;
 }
 
-// The same for 4 neighbours (16-byte loads where the term is float32).
+// The same for 4 neighbours (16-byte loads where the term is float32). AHEAD: see scaled_sum_norm_kernel.
+template <bool AHEAD>
 __device__ __forceinline__ void term_value4(const void* ptr, int dtype, int parts, int64_t stride, const float* scale,
                                             int64_t at, int i, float (&out)[4]) {
   float v[4] = {0.f, 0.f, 0.f, 0.f};
   if (dtype == ME_F32) {
     const float* p = (const float*)ptr + at;
-    for (int q0 = 0; q0 < parts; q0 += 4) {        // four parts asked for at once
-      float4 t[4];
+    constexpr int AT_ONCE = AHEAD ? 4 : 1;
+    for (int q0 = 0; q0 < parts; q0 += AT_ONCE) {
+      float4 t[AT_ONCE];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) t[q] = *reinterpret_cast<const float4*>(p + min(q0 + q, parts - 1) * stride);
+      for (int q = 0; q < AT_ONCE; ++q) t[q] = *reinterpret_cast<const float4*>(p + min(q0 + q, parts - 1) * stride);
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
+      for (int q = 0; q < AT_ONCE; ++q)
         if (q0 + q < parts) { v[0] += t[q].x; v[1] += t[q].y; v[2] += t[q].z; v[3] += t[q].w; }
     }
   } else {
@@ -67,7 +69,11 @@ __device__ __forceinline__ void term_value4(const void* ptr, int dtype, int part
 // One workgroup per row; the row stays in LDS between the sum and the norms. The terms are walked by a loop that the
 // compiler unrolls, so that their pointers stay in scalar registers. VEC: rows in whole groups of 4 with every operand
 // 16-byte aligned: a thread takes 4 neighbours at a time.
-template <typename TY, bool VEC>
+// AHEAD: launches of few rows, which are the way of their loads: four partial sums and the norms' weights (up to 4 numbers a
+// thread; wider rows ask behind the sum) are asked for with the row, 32 rows of 1,024 with four partial sums 8.8 -> 5.6 us.
+// Many rows fill the chip, and what the loads ahead cost in registers they pay with time (3,123 rows of 1,024 with one
+// float32 term 12.2 us and 12.8 with the loads ahead, of 2,048 21.6 and 22.5).
+template <typename TY, bool VEC, bool AHEAD>
 __global__ void __launch_bounds__(1024)
 scaled_sum_norm_kernel(const void* __restrict__ stream_in, int stream_dtype, SumTerms terms, float mult,
                        float* __restrict__ stream_out, const float* __restrict__ w1, const float* __restrict__ w2,
@@ -76,9 +82,7 @@ scaled_sum_norm_kernel(const void* __restrict__ stream_in, int stream_dtype, Sum
   extern __shared__ __align__(16) float row[];
   const int64_t t = blockIdx.x;
   float ss = 0.f;
-  // the norms' weights are asked for with the row (4 numbers a thread; wider rows ask behind the sum): the launch of a few
-  // rows is the way of its loads, 32 rows of 1,024 with four partial sums 8.8 -> 5.6 us
-  const bool near = w1 && n <= 4 * (int)blockDim.x;
+  const bool near = AHEAD && w1 && n <= 4 * (int)blockDim.x;
   float a1[4], a2[4];
   if (near) {
 #pragma unroll
@@ -103,7 +107,7 @@ scaled_sum_norm_kernel(const void* __restrict__ stream_in, int stream_dtype, Sum
       float add[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int k = 0; k < PS_MAX_TERMS; ++k)
-        if (k < terms.count) term_value4(terms.ptr[k], terms.dtype[k], terms.parts[k], terms.part_stride[k], terms.scale[k], at, i, add);
+        if (k < terms.count) term_value4<AHEAD>(terms.ptr[k], terms.dtype[k], terms.parts[k], terms.part_stride[k], terms.scale[k], at, i, add);
       float s[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -186,11 +190,14 @@ extern "C" int me_scaled_sum_norm(const void* stream_in, int stream_dtype, int c
   int threads = T >= 512 ? 256 : 1024;
   while (threads > 64 && threads * per / 2 >= n) threads >>= 1;
   const size_t lds = (size_t)n * sizeof(float);
-#define PS_LAUNCH(TY, V)                                                                                                   \
-  scaled_sum_norm_kernel<TY, V><<<dim3((unsigned)T), dim3(threads), lds, stream>>>(stream_in, stream_dtype, terms, mult, stream_out, \
-                                                                                w1, w2, (TY*)y1, (TY*)y2, n, eps)
-  if (out_dtype == ME_F32) { if (vec) PS_LAUNCH(float, true); else PS_LAUNCH(float, false); }
-  else { if (vec) PS_LAUNCH(bf16_t, true); else PS_LAUNCH(bf16_t, false); }
+#define PS_LAUNCH(TY, V, A)                                                                                                \
+  scaled_sum_norm_kernel<TY, V, A><<<dim3((unsigned)T), dim3(threads), lds, stream>>>(stream_in, stream_dtype, terms, mult, stream_out, \
+                                                                                   w1, w2, (TY*)y1, (TY*)y2, n, eps)
+#define PS_PICK(TY) do { \
+    if (T >= 512) { if (vec) PS_LAUNCH(TY, true, false); else PS_LAUNCH(TY, false, false); } \
+    else if (vec) PS_LAUNCH(TY, true, true); else PS_LAUNCH(TY, false, true); } while (0)
+  if (out_dtype == ME_F32) PS_PICK(float); else PS_PICK(bf16_t);
+#undef PS_PICK
 #undef PS_LAUNCH
   ME_LAUNCH_CHECK();
   return 0;

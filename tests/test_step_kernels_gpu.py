@@ -183,3 +183,21 @@ def test_the_pairs_kernel_chooses_for_any_number_of_tokens():
     assert torch.equal(order.sort().values.long(), torch.arange(P, device=DEV))
     assert torch.equal(ids[order.long()].sort().values, ids[order.long()])
     assert torch.equal(offsets[1:].long(), torch.bincount(ids.long(), minlength=E).cumsum(0))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,parts", [(1024, 1), (1024, 5), (2056, 3), (1001, 4), (8200, 2)])
+def test_sums_and_norms_of_few_and_of_many_rows_are_the_same(n, parts, dtype):
+    """From 512 rows on a row's loads go one after the other and fewer threads share a row: the sums are the same bits as in a
+    launch of few rows, the norms add their squares in another order (and round once to the output type)."""
+    g = torch.Generator(device=DEV).manual_seed(n + parts)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    T = 512
+    stream, sums, rows = rnd(T, n), rnd(parts, T, n), rnd(T, n).to(dtype)
+    w1, w2, s1 = rnd(n), rnd(n), rnd(n)
+    many = hip().scaled_sum_norm(stream, [(sums, s1), (rows, None)], 0.45, w1, w2, 1e-5, dtype)
+    few = hip().scaled_sum_norm(stream[500:], [(sums[:, 500:].contiguous(), s1), (rows[500:], None)], 0.45, w1, w2, 1e-5, dtype)
+    assert torch.equal(many[0][500:], few[0])
+    for a, b in zip(many[1:], few[1:]):
+        close(a[500:], b, 1e-6 if dtype == torch.float32 else 8e-3)
+    close(many[0], stream + 0.45 * (s1 * sums.sum(0) + rows.float()), 1e-6)
