@@ -144,7 +144,7 @@ attn_simple_kernel(const T* __restrict__ q, int64_t q_stride, T* __restrict__ ou
 // Values of keys that a token does not see meet a probability of zero; where such a value is not a finite number it is
 // taken out of the product and joined by hand for the tokens that do see it.
 template <int NS>        // head size / 16
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 2)       // two waves to a SIMD asked for: without it head size 96 took 276 registers and scratch, now 151
 attn_f32_kernel(const float* __restrict__ q, int64_t q_stride, float* __restrict__ out, int64_t out_stride,
                 const float* __restrict__ k_cache, const float* __restrict__ v_cache, const int32_t* __restrict__ block_tables,
                 int bt_stride, const int32_t* __restrict__ seq_of_token, const int32_t* __restrict__ positions,
@@ -267,6 +267,7 @@ attn_f32_kernel(const float* __restrict__ q, int64_t q_stride, float* __restrict
 #pragma unroll
         for (int j = 0; j < 4; ++j) odd = fmaf(fv[i][j], 0.f, odd);
       if (__ballot(odd != odd) != 0) {
+#pragma unroll 1                                 // (a rare way: unrolled, it costs head sizes up to 48 a wave or two per SIMD)
         for (int from = 0; from < 4; ++from)
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
