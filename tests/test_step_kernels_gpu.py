@@ -42,6 +42,21 @@ def test_gated_norm_widths(n, parts, kind, dtype):
           1e-6 if dtype == torch.float32 else 4e-3)
 
 
+def _clear_choices(logits, scoring, groups, group_top):
+    """The tokens whose choice 32 bits cannot turn: scores of different logits, and of groups of them, lie 1e-5 of the larger
+    apart or more (equal ones are equal on both sides, and the lower index wins)."""
+    scores = {"softmax": torch.softmax(logits, -1), "sigmoid": torch.sigmoid(logits), "chosen": logits}[scoring]
+    per = scores.shape[1] // groups
+    totals = scores.view(-1, groups, per).topk(min(group_top, per), -1).values.sum(-1)
+
+    def apart(values):
+        v = values.sort(-1).values
+        gap, size = v[:, 1:] - v[:, :-1], v.abs()[:, 1:].maximum(v.abs()[:, :-1])
+        return ((gap <= 1e-12 * size) | (gap > 1e-5 * size)).all(-1)
+
+    return apart(scores) & apart(totals)
+
+
 @pytest.mark.parametrize("scoring", ["softmax", "sigmoid", "chosen"])
 @pytest.mark.parametrize("T,E,groups,keep,top,group_top", [(1, 1, 1, 1, 1, 1), (17, 2, 1, 1, 2, 1), (64, 32, 4, 2, 4, 1), (33, 63, 7, 3, 5, 2),
                                                            (64, 64, 8, 2, 8, 3), (40, 64, 64, 9, 9, 1), (50, 65, 5, 2, 6, 2), (5, 128, 4, 1, 3, 2)])
@@ -58,11 +73,10 @@ def test_choices_in_registers_and_through_lds(T, E, groups, keep, top, group_top
     rule = ops.RouteRule(scoring, None, group_top=group_top, normalise=scoring != "sigmoid", scale=1.25)
     ids, weights = hip().moe_route(x, router, top, groups, keep, rule)
     want_ids, want_w = twin.moe_route(x.cpu(), router.cpu(), top, groups, keep, rule)
-    scores = torch.softmax(x.cpu() @ router.cpu().t(), -1) if scoring == "softmax" else torch.sigmoid(x.cpu() @ router.cpu().t())
-    gap = scores.unique(dim=-1) if T == 1 else None            # different logits whose scores round alike may go either way
-    same = (ids.cpu() == want_ids).all(-1)
-    assert same.float().mean() >= (1.0 if scoring == "chosen" or gap is not None else 0.9)
-    close(weights.cpu()[same], want_w[same], 2e-6)             # a softmax of 32-bit exponentials
+    clear = _clear_choices(x.cpu().double() @ router.cpu().double().t(), scoring, groups, group_top)
+    assert clear.float().mean() > 0.9
+    assert torch.equal(ids.cpu()[clear], want_ids[clear])
+    close(weights.cpu()[clear], want_w[clear], 2e-6)           # a softmax of 32-bit exponentials
     up, down = torch.randn(E, 8, 24, device=DEV, generator=g), torch.randn(E, 16, 8, device=DEV, generator=g)
     got = hip().route_and_run_experts(x.to(torch.bfloat16), router, top, groups, keep, up.to(torch.bfloat16), down.to(torch.bfloat16), rule=rule, gated=False)
     want = twin.routed_experts(x.cpu().to(torch.bfloat16), ids.cpu(), weights.cpu(), up.cpu().to(torch.bfloat16), down.cpu().to(torch.bfloat16), gated=False)
@@ -156,14 +170,27 @@ def test_short_convolution_of_one_long_request_among_short_ones(monkeypatch, tap
     close(walked, want, 8e-3)
 
 
-def test_a_bias_on_more_rows_than_a_grid_has_by_fours():
-    """2^26 + 8 rows of 128 by fours would be 2^32 threads and more: the general kernel takes them (17 GB of results)."""
-    T, n = (1 << 26) + 8, 128
-    row, bias = torch.randn(1, n, device=DEV).to(torch.bfloat16), torch.randn(n, device=DEV)
-    out = hip().add_bias(row.expand(T, n), bias, torch.bfloat16)
-    want = hip().add_bias(row, bias, torch.bfloat16)
-    for part in out.split(1 << 23):
-        assert bool((part == want).all())
+@pytest.mark.parametrize("scoring", ["softmax", "sigmoid", "chosen"])
+@pytest.mark.parametrize("E,groups,keep,top,group_top", [(8, 1, 1, 3, 1), (32, 4, 2, 4, 2), (63, 7, 7, 8, 1), (64, 8, 3, 8, 3), (64, 64, 20, 20, 1), (48, 1, 1, 48, 1)])
+def test_the_choice_in_registers_is_that_through_lds(E, groups, keep, top, group_top, scoring):
+    """Whole groups of further experts with a bias of minus infinity take the same tokens to the form beyond 64 experts: the same
+    ids and the same weights, bit for bit, ties and corrections included."""
+    g = torch.Generator(device=DEV).manual_seed(E + top)
+    T, n, per = 77, 40, E // groups
+    x = torch.randn(T, n, device=DEV, generator=g)
+    router = torch.randn(E, n, device=DEV, generator=g) * 0.3
+    router[1::3] = router[0::3][:router[1::3].shape[0]]        # equal scores
+    more = per * -(-(65 - E) // per)
+    wide = torch.cat((router, torch.zeros(more, n, device=DEV)))
+    bias = torch.cat((torch.zeros(E, device=DEV), torch.full((more,), -torch.inf, device=DEV)))
+    for correction in (None, torch.rand(E, device=DEV, generator=g)):
+        if scoring == "chosen" and correction is not None:
+            continue
+        far = None if correction is None else torch.cat((correction, torch.full((more,), -9.0, device=DEV)))
+        rule = lambda c, b: ops.RouteRule(scoring, c, group_top=group_top, normalise=True, scale=1.5, bias=b)
+        narrow = hip().moe_route(x, router, top, groups, keep, rule(correction, None))
+        there = hip().moe_route(x, wide, top, groups + more // per, keep, rule(far, bias))
+        assert torch.equal(narrow[0], there[0]) and torch.equal(narrow[1], there[1])
 
 
 def test_the_pairs_kernel_chooses_for_any_number_of_tokens():
@@ -183,6 +210,16 @@ def test_the_pairs_kernel_chooses_for_any_number_of_tokens():
     assert torch.equal(order.sort().values.long(), torch.arange(P, device=DEV))
     assert torch.equal(ids[order.long()].sort().values, ids[order.long()])
     assert torch.equal(offsets[1:].long(), torch.bincount(ids.long(), minlength=E).cumsum(0))
+
+
+def test_a_bias_on_more_rows_than_a_grid_has_by_fours():
+    """2^26 + 8 rows of 128 by fours would be 2^32 threads and more: the general kernel takes them (17 GB of results)."""
+    T, n = (1 << 26) + 8, 128
+    row, bias = torch.randn(1, n, device=DEV).to(torch.bfloat16), torch.randn(n, device=DEV)
+    out = hip().add_bias(row.expand(T, n), bias, torch.bfloat16)
+    want = hip().add_bias(row, bias, torch.bfloat16)
+    for part in out.split(1 << 23):
+        assert bool((part == want).all())
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
