@@ -1800,11 +1800,14 @@ def decay_row_groups(num_seqs: int, H: int, N: int, P: int, longest: int = 1, to
     """(lanes that share a column of the state in `decay_rows_recurrence`, whether a first kernel shapes the tokens' values).
     A request is a chain: the fewer rows a lane walks per token, the shorter the chain's step, at the price of more waves
     and an exchange between lanes. Steps of long requests: the values of all tokens are shaped at once by a kernel of its
-    own (unit lengths, decays and their exponentials leave the chain), and 16 lanes share a column while the waves all run at
-    once (up to 16 a compute unit, and as many as its 160 KB of LDS hold: a wave keeps q, k and, unless a head has one decay,
-    the decays of 16 tokens there), else 4: 8 prompts of 2,048 tokens over 8 heads of 128 x 128, 2,048 waves of 16 lanes to a
-    column, take 681 us with one decay per head (all at once; 933 with 4 lanes) and 1,088 with a decay per row (two rounds;
-    1,057 with 4 lanes); 16 prompts of 512 tokens 459 and 328. Requests of a few tokens in such a step (`tokens`: the step's) end early and are not counted. Short steps shape inside the
+    own (unit lengths, decays and their exponentials leave the chain), and 16 lanes share a column while that is at most as many
+    waves as a unit's 160 KB of LDS hold, 16 at most (a wave keeps q, k and, unless a head has one decay, the decays of 16
+    tokens there), else 4: 8 prompts of 2,048 tokens over 8 heads of 128 x 128, 2,048 waves of 16 lanes to a column, take 681 us
+    with one decay per head (933 with 4 lanes) and 1,088 with a decay per row (two rounds; 1,057 with 4 lanes); 16 prompts
+    of 512 tokens 459 and 328. A wave of 65 to 128 rows needs 171 registers, so 8 run on a unit where its LDS would hold 9: with
+    one decay per head the ninth's share is a second round, which still pays (9 prompts of 512 tokens 231 us, 241 with 4 lanes; of
+    2,048 882 and 941), a larger one does not (12 prompts of 512 251 and 245, of 2,048 1,023 and 984). Requests of a few tokens in
+    such a step (`tokens`: the step's) end early and are not counted. Short steps shape inside the
     kernel: 4 lanes where a lane could not keep a whole column in registers, or while one lane to a column leaves compute
     units without a wave; else 1."""
     if longest >= DECAY_PREPARE_MIN_TOKENS:
