@@ -188,7 +188,7 @@ __global__ void weighted_sum_norm_kernel(WsArgs a, const float* __restrict__ w, 
 
 // Rows of 1,024 to 4,096: a thread holds its values (the same ones, so the row's sum keeps its order) in registers and asks for a
 // term's, the stream's and the weights' all at once; the general kernel goes to memory for one value at a time.
-// (3,123 rows of 1,024, two terms: 20.8 -> 13.1 us)
+// (3,123 rows of 1,024, two terms: 20.8 -> 13.1 us; which launches it takes: rows_in_registers)
 template <typename TY, int NV>
 __global__ void __launch_bounds__(256)
 weighted_sum_norm_regs_kernel(WsArgs a, const float* __restrict__ w, float eps, const float* __restrict__ stream_in,
@@ -253,6 +253,20 @@ weighted_sum_norm_regs_kernel(WsArgs a, const float* __restrict__ w, float eps, 
   }
 }
 
+// Up to how many rows the form in registers takes a launch whose float32 terms have `sums` partial sums together. Its 65, 128
+// and 238 registers leave a compute unit 7, 4 and 2 workgroups where the general kernel has 8: as long as the launch is a round or
+// two of them that costs nothing, and reads of bfloat16 rows, one trip a term, are ahead at any number; but every partial sum is
+// a trip of its own that few waves wait out. us, general kernel / registers: rows of 2,560, one float32 term and one of bfloat16 at
+// 1,024 rows 21 / 18, at 2,048 26 / 33, with three partial sums at 512 rows 20 / 13, at 1,024 28 / 31, at 8,192 169 / 346; of
+// 2,048, one term at 16,384 rows 196 / 148, nine partial sums at 1,024 rows 35 / 29, at 2,048 39 / 54; of 1,024, three at 8,192 rows
+// 51 / 42, nine at 2,048 22 / 28.
+static int64_t rows_in_registers(int n, int64_t sums, int64_t any) {
+  if (sums == 0) return any;
+  if (n <= 1024) return sums <= 4 ? any : 1024;
+  if (n <= 2048) return sums == 1 ? any : 1024;
+  return sums == 1 ? 1024 : 512;
+}
+
 extern "C" int me_weighted_sum(int count, const void** terms, const int* dtypes, const int* parts, const int64_t* part_strides,
                                const float* scales, const float** biases, float* out, const float* w, float eps,
                                const float* stream_in, float* stream_out, void* rounded, int rounded_dtype, int64_t T, int n,
@@ -261,8 +275,10 @@ extern "C" int me_weighted_sum(int count, const void** terms, const int* dtypes,
   ME_CHECK(count >= 1 && count <= WS_MAX_TERMS, "weighted_sum: 1..%d terms", WS_MAX_TERMS);
   WsArgs a;
   a.count = count; a.n = n;
+  int64_t sums = 0;
   for (int i = 0; i < count; ++i) {
     ME_CHECK(parts[i] >= 1 && (dtypes[i] == ME_F32 || parts[i] == 1), "weighted_sum: partial sums are float32");
+    if (dtypes[i] == ME_F32) sums += parts[i];
     a.term[i] = terms[i]; a.dtype[i] = dtypes[i]; a.parts[i] = parts[i]; a.part_stride[i] = part_strides[i];
     a.scale[i] = scales[i]; a.bias[i] = biases[i];
     a.gate[i] = gates ? gates[i] : nullptr; a.gate_dtype[i] = gates ? gate_dtypes[i] : ME_F32; a.gate_stride[i] = gates ? gate_strides[i] : 0;
@@ -279,7 +295,7 @@ extern "C" int me_weighted_sum(int count, const void** terms, const int* dtypes,
     if (n <= 1024) weighted_sum_norm_regs_kernel<TY, 4><<<grid, block, 0, stream>>>(a, w, eps, stream_in, stream_out, (TY*)rounded); \
     else if (n <= 2048) weighted_sum_norm_regs_kernel<TY, 8><<<grid, block, 0, stream>>>(a, w, eps, stream_in, stream_out, (TY*)rounded); \
     else weighted_sum_norm_regs_kernel<TY, 16><<<grid, block, 0, stream>>>(a, w, eps, stream_in, stream_out, (TY*)rounded); } while (0)
-    if (n >= 1024 && n <= 4096) {
+    if (n >= 1024 && n <= 4096 && T <= rows_in_registers(n, sums, T)) {
       if (rounded == nullptr || rounded_dtype == ME_F32) WS(float);
       else WS(bf16_t);
     } else if (rounded == nullptr || rounded_dtype == ME_F32)

@@ -128,6 +128,21 @@ def test_weighted_sum_and_norm_widths(n, dtype):
     close(got[1], want[1], 1e-6)
 
 
+@pytest.mark.parametrize("n,parts", [(1024, 4), (1024, 5), (1030, 1), (2048, 2), (2049, 1), (3000, 3), (4096, 1)])
+def test_weighted_sums_of_few_and_of_many_rows_are_the_same_bits(n, parts):
+    """Launches of 512 or 1,024 rows and more whose terms are partial sums go through LDS, fewer rows through registers: the
+    same steps and sums in the same order."""
+    g = torch.Generator(device=DEV).manual_seed(n + parts)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    w, bias = rnd(n), rnd(n)
+    for T in (512, 513, 1024, 1025):
+        sums, rows, gate, stream = rnd(parts, T, n), rnd(T, n).to(torch.bfloat16), rnd(T, 1), rnd(T, n)
+        at = lambda lo: [(sums[:, lo:].contiguous(), 0.7, bias), (rows[lo:], -0.3, None, gate[lo:, 0])]
+        many = hip().weighted_sum(at(0), w, 1e-6, stream, torch.bfloat16)
+        few = hip().weighted_sum(at(T - 9), w, 1e-6, stream[T - 9:], torch.bfloat16)
+        assert torch.equal(many[0][T - 9:], few[0]) and torch.equal(many[1][T - 9:], few[1])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("taps", [1, 2, 3, 4, 5])
 def test_short_convolution_over_the_ends_of_its_groups(taps, dtype):
