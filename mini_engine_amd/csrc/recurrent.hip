@@ -732,10 +732,8 @@ __global__ void recurrence_carry_kernel(RecArgs a) {
 }
 
 // A step of single tokens (token b is request b's): the state streams through once. One workgroup of four waves per
-// (request, head, 64 columns); each wave takes a quarter of the N rows, eight rows' loads in flight at a time, and
-// the four partial outputs meet in LDS. Nothing of the state stays in registers, so many waves fit a SIMD, which is
-// what a kernel that only waits for memory needs.
-// HB: rows that a wave asks for at once, the first of them before it meets the others: a quarter of 128 rows is one trip to
+// (request, head, 64 columns); each wave takes a quarter of the N rows, and the four partial outputs meet in LDS.
+// HB: rows that a wave asks for at once and holds until they are written back, the first of them before it meets the others: a quarter of 128 rows is one trip to
 // memory instead of four behind each other (8 requests, 16 heads of 128 x 128, 16.8 MB read and written: 10.4 -> 8.1 us).
 template <typename TX, int HB>
 __global__ void __launch_bounds__(256) recurrence_step_kernel(RecArgs a) {
@@ -1172,7 +1170,13 @@ extern "C" int me_gated_rms_norm(const float* y, int parts, int64_t part_stride,
     }
   }
   const dim3 grid((unsigned)T), block(n >= 1024 ? 256 : (n > 256 ? 128 : 64));
-  if (groups == 1 && n >= 1024 && n <= 8192) {
+  // Rows of several partial sums: each sum is a trip to memory of its own, and a compute unit has 5 workgroups of the form in
+  // registers over 2,049 to 4,096 numbers and 2 beyond (98 and 194 registers) where the general kernel has 8, so launches of more than
+  // a round or two of them go there. Three sums, us, general / registers: 2,560 numbers at 1,024 rows 19 / 16, at 2,048 22 / 30, at
+  // 8,192 116 / 138; 5,120 at 512 rows 30 / 21, at 1,024 35 / 40, at 8,192 258 / 406; 6,144 at 4,096 rows 175 / 236; 8,192 numbers, no
+  // thread idle, 297 / 268; of one sum 8,192 rows of 5,120 158 / 92.
+  const bool long_way = parts > 1 && ((n > 2048 && n <= 4096 && T > 1024) || (n > 4096 && n <= 7168 && T > 512));
+  if (groups == 1 && n >= 1024 && n <= 8192 && !long_way) {
 #define GR(TX, K)                                                                                                                       \
   do {                                                                                                                                  \
     if (n <= 1024) gated_rms_norm_regs_kernel<TX, K, 4><<<grid, block, 0, stream>>>(y, parts, part_stride, (const TX*)gate, gate_stride, w, (TX*)out, n, eps);      \

@@ -42,6 +42,17 @@ def test_gated_norm_widths(n, parts, kind, dtype):
           1e-6 if dtype == torch.float32 else 4e-3)
 
 
+@pytest.mark.parametrize("kind", ["silu_before", "sigmoid_behind", "silu_behind"])
+@pytest.mark.parametrize("n,few,many", [(2049, 1024, 1025), (4096, 1024, 1025), (4097, 512, 513), (7168, 512, 513)])
+def test_gated_norms_of_few_and_of_many_rows_are_the_same_bits(n, few, many, kind):
+    """Rows of several partial sums go through LDS from a number of rows on: the same steps and sums in the same order."""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    y, gate = torch.randn(3, many, n, device=DEV, generator=g), torch.randn(many, n, device=DEV, generator=g).to(torch.bfloat16)
+    w = torch.rand(n, device=DEV, generator=g) + 0.5
+    out = hip().gated_rms_norm(y, gate, w, 1e-5, 1, kind, torch.bfloat16)
+    assert torch.equal(out[:few], hip().gated_rms_norm(y[:, :few].contiguous(), gate[:few], w, 1e-5, 1, kind, torch.bfloat16))
+
+
 def _clear_choices(logits, scoring, groups, group_top):
     """The tokens whose choice 32 bits cannot turn: scores of different logits, and of groups of them, lie 1e-5 of the larger
     apart or more (equal ones are equal on both sides, and the lower index wins)."""
