@@ -20,9 +20,9 @@
 #define GT_TILE 64
 #define GT_BK 16
 
-template <typename TI, typename TO>
+template <typename TO>
 __global__ void __launch_bounds__(256)
-gemm_tiled_kernel(const TI* __restrict__ x, int64_t ldx, const TI* __restrict__ w, int64_t ldw,
+gemm_tiled_kernel(const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ w, int64_t ldw,
                   TO* __restrict__ y, int64_t ldy, int M, int N, int K) {
   __shared__ float xs[GT_BK][GT_TILE + 1];
   __shared__ float ws[GT_BK][GT_TILE + 1];
@@ -35,8 +35,8 @@ gemm_tiled_kernel(const TI* __restrict__ x, int64_t ldx, const TI* __restrict__ 
     for (int e = tid; e < GT_TILE * GT_BK; e += 256) {
       const int r = e / GT_BK, kk = e % GT_BK;
       const int k = k0 + kk;
-      xs[kk][r] = (m0 + r < M && k < K) ? to_f32<TI>(x[(int64_t)(m0 + r) * ldx + k]) : 0.f;
-      ws[kk][r] = (n0 + r < N && k < K) ? to_f32<TI>(w[(int64_t)(n0 + r) * ldw + k]) : 0.f;
+      xs[kk][r] = (m0 + r < M && k < K) ? to_f32<bf16_t>(x[(int64_t)(m0 + r) * ldx + k]) : 0.f;
+      ws[kk][r] = (n0 + r < N && k < K) ? to_f32<bf16_t>(w[(int64_t)(n0 + r) * ldw + k]) : 0.f;
     }
     __syncthreads();
 #pragma unroll
@@ -67,7 +67,7 @@ extern "C" int me_gemm_tiled(const void* x, int64_t ldx, const void* w, int64_t 
   dim3 grid((N + GT_TILE - 1) / GT_TILE, (M + GT_TILE - 1) / GT_TILE), block(256);
   ME_CHECK(grid.y <= 65535, "gemm: too many rows (%d) for one launch", M);
 #define LAUNCH(TO) \
-  gemm_tiled_kernel<bf16_t, TO><<<grid, block, 0, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, ldw, (TO*)y, ldy, M, N, K)
+  gemm_tiled_kernel<TO><<<grid, block, 0, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, ldw, (TO*)y, ldy, M, N, K)
   if (out_dtype == ME_BF16) LAUNCH(bf16_t); else LAUNCH(float);
 #undef LAUNCH
   ME_LAUNCH_CHECK();

@@ -14,8 +14,9 @@
 // Measured (us; in brackets a kernel of 64 x 64 tiles through LDS with plain multiply-adds, the 32-bit product before): 300
 // rows of 4096 x 1024 42 (194), 1024 x 2048 24 (380), 6144 x 1024 58 (200), 1024 x 3072 36 (560), 151936 x 1024 1,258 (2,400;
 // 74 TFLOP/s, about half of the 157 that the matrix pipes could do at 2.4 GHz: a full chip of them does not keep that clock;
-// 80 workgroups alone reach 82 % of it). One row of 4096 x 1024: 6.9. Error against 64 bits over 1,024-3,072 terms 3-5e-7
-// of the result's norm, less than one chain of multiply-adds (four shorter chains).
+// 80 workgroups alone reach 82 % of it). Few and many rows: one row of 4096 x 1024 7.3 (125), of 4096 x 12288 34 (1,694), 64 rows
+// of it 93 (2,008), 4,096 rows 4,990 (8,480; 83 TFLOP/s). Error against 64 bits over 1,024-3,072 terms 3-5e-7 of the result's
+// norm, less than one chain of multiply-adds (four shorter chains).
 #include "common.h"
 
 // Keeps a step's loads where they are issued (else they sink to their use in the next round of the ring).

@@ -410,8 +410,9 @@ extern "C" int me_qk_norm_rope_store(void* qkv, int dtype, int64_t num_tokens, i
                    reinterpret_cast<uintptr_t>(qkv) % 16 == 0 && reinterpret_cast<uintptr_t>(k_cache) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(q_w) % 16 == 0 && reinterpret_cast<uintptr_t>(k_w) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(table) % 16 == 0;
-  // many tokens of bfloat16: 8 tokens per workgroup group. From 128 tokens on: below that the steps are
-  // decode steps, whose slots are scattered, and the form above is faster for those (64 tokens: 6.4 against 7.6 us).
+  // many tokens of bfloat16: 8 tokens per workgroup group. From 128 tokens on: below that a workgroup per token is faster, be
+  // the slots scattered (decode steps) or in a row (16 + 8 heads of 128, us, a workgroup per token / per 8 tokens: 64 tokens
+  // scattered 6.3 / 9.7, in a row 3.1 / 4.3; 120 tokens 7.4 / 10.2, 3.4 / 4.5).
   const int lph16 = D / 16;
   const bool tile = vec && dtype == ME_BF16 && num_tokens >= 128 && D % 16 == 0 && lph16 >= 1 && lph16 <= 64 &&
                     (lph16 & (lph16 - 1)) == 0 && (!store || (page % 8 == 0 && reinterpret_cast<uintptr_t>(v_cache) % 16 == 0));

