@@ -70,9 +70,9 @@ __device__ __forceinline__ void term_value4(const void* ptr, int dtype, int part
 // compiler unrolls, so that their pointers stay in scalar registers. VEC: rows in whole groups of 4 with every operand
 // 16-byte aligned: a thread takes 4 neighbours at a time.
 // AHEAD: launches of few rows, which are the way of their loads: four partial sums and the norms' weights (up to 4 numbers a
-// thread; wider rows ask behind the sum) are asked for with the row, 32 rows of 1,024 with four partial sums 8.8 -> 5.6 us.
-// Many rows fill the chip, and what the loads ahead cost in registers they pay with time (3,123 rows of 1,024 with one
-// float32 term 12.2 us and 12.8 with the loads ahead, of 2,048 21.6 and 22.5).
+// thread; wider rows ask behind the sum) are asked for with the row, the stream's values in front of the terms, 32 rows of 1,024
+// with four partial sums 8.8 -> 5.6 us (one sum costs 0.1-0.2 us by it). Many rows fill the chip: there the loads ahead pay where a
+// value has three partial sums or more or where the launch comes from memory and not from the memory-side cache (asks_ahead).
 template <typename TY, bool VEC, bool AHEAD>
 __global__ void __launch_bounds__(1024)
 scaled_sum_norm_kernel(const void* __restrict__ stream_in, int stream_dtype, SumTerms terms, float mult,
@@ -96,18 +96,22 @@ scaled_sum_norm_kernel(const void* __restrict__ stream_in, int stream_dtype, Sum
     for (int i = threadIdx.x * 4; i < n; i += blockDim.x * 4) {
       const int64_t at = t * n + i;
       float base[4];
-      if (stream_dtype == ME_F32) {
-        const float4 b = *reinterpret_cast<const float4*>((const float*)stream_in + at);
-        base[0] = b.x; base[1] = b.y; base[2] = b.z; base[3] = b.w;
-      } else {
-        const bf16x4 b = *reinterpret_cast<const bf16x4*>((const bf16_t*)stream_in + at);
+      auto own = [&] {
+        if (stream_dtype == ME_F32) {
+          const float4 b = *reinterpret_cast<const float4*>((const float*)stream_in + at);
+          base[0] = b.x; base[1] = b.y; base[2] = b.z; base[3] = b.w;
+        } else {
+          const bf16x4 b = *reinterpret_cast<const bf16x4*>((const bf16_t*)stream_in + at);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) base[j] = static_cast<float>(b[j]);
-      }
+          for (int j = 0; j < 4; ++j) base[j] = static_cast<float>(b[j]);
+        }
+      };
+      if (AHEAD) own();
       float add[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int k = 0; k < PS_MAX_TERMS; ++k)
         if (k < terms.count) term_value4<AHEAD>(terms.ptr[k], terms.dtype[k], terms.parts[k], terms.part_stride[k], terms.scale[k], at, i, add);
+      if (!AHEAD) own();
       float s[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -154,6 +158,19 @@ scaled_sum_norm_kernel(const void* __restrict__ stream_in, int stream_dtype, Sum
   }
 }
 
+// Whether a launch of T rows takes the form with the loads ahead. bytes: the stream in and out and a norm, to which the terms'
+// come; numbers: of one term. us, without / with the loads ahead: 1,024 rows of 1,024 with one float32 sum 6.0 / 6.4, with eight
+// 10.8 / 9.5; 3,123 rows of 2,048 with one 21.6 / 22.5; 2,048 rows of 4,096 with four 41 / 38; 8,192 rows of 4,096 (256 MB of
+// cache passed) with one 109 / 103, with bfloat16 rows alone 104 / 94, with two sums 133 / 120.
+static bool asks_ahead(const SumTerms& terms, int64_t T, int64_t bytes, int64_t numbers) {
+  int most = 0;
+  for (int k = 0; k < terms.count; ++k) {
+    if (terms.dtype[k] == ME_F32 && terms.parts[k] > most) most = terms.parts[k];
+    bytes += numbers * terms.parts[k] * (terms.dtype[k] == ME_F32 ? 4 : 2);
+  }
+  return T < 512 || most >= 3 || bytes > (256ll << 20);
+}
+
 // terms: `count` entries of (pointer, dtype, parts, part stride in elements, scale pointer or null).
 extern "C" int me_scaled_sum_norm(const void* stream_in, int stream_dtype, int count, const void* const* term_ptr,
                                   const int* term_dtype, const int* term_parts, const int64_t* term_stride,
@@ -190,11 +207,12 @@ extern "C" int me_scaled_sum_norm(const void* stream_in, int stream_dtype, int c
   int threads = T >= 512 ? 256 : 1024;
   while (threads > 64 && threads * per / 2 >= n) threads >>= 1;
   const size_t lds = (size_t)n * sizeof(float);
+  const bool ahead = asks_ahead(terms, T, T * n * (out_dtype == ME_F32 ? 12 : 10), T * n);
 #define PS_LAUNCH(TY, V, A)                                                                                                \
   scaled_sum_norm_kernel<TY, V, A><<<dim3((unsigned)T), dim3(threads), lds, stream>>>(stream_in, stream_dtype, terms, mult, stream_out, \
                                                                                    w1, w2, (TY*)y1, (TY*)y2, n, eps)
 #define PS_PICK(TY) do { \
-    if (T >= 512) { if (vec) PS_LAUNCH(TY, true, false); else PS_LAUNCH(TY, false, false); } \
+    if (!ahead) { if (vec) PS_LAUNCH(TY, true, false); else PS_LAUNCH(TY, false, false); } \
     else if (vec) PS_LAUNCH(TY, true, true); else PS_LAUNCH(TY, false, true); } while (0)
   if (out_dtype == ME_F32) PS_PICK(float); else PS_PICK(bf16_t);
 #undef PS_PICK
