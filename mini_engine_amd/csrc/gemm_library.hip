@@ -182,6 +182,30 @@ bool make_plan(hipblasLtHandle_t handle, Plan& p, int M, int N, int K, int64_t l
   return false;
 }
 
+// The device's handle, made on first use; null if no hipBLASLt is loaded or it gives none. Under g_mutex.
+hipblasLtHandle_t handle_of(int device) {
+  if (!look_up_api()) return nullptr;
+  auto h = g_handles.find(device);
+  if (h == g_handles.end()) {
+    hipblasLtHandle_t made = nullptr;
+    if (g_api.create(&made) != HIPBLAS_STATUS_SUCCESS) return nullptr;
+    h = g_handles.emplace(device, made).first;
+  }
+  return h->second;
+}
+
+// The plan of a key, made on first use (std::map keeps its address). Under g_mutex.
+const Plan& plan_of(hipblasLtHandle_t handle, const PlanKey& key) {
+  auto it = g_plans.find(key);
+  if (it == g_plans.end()) {
+    const auto& [device, M, N, K, ldx, ldw, ldy, out_dtype, workspace_bytes, splits] = key;
+    Plan made;
+    made.ok = make_plan(handle, made, M, N, K / splits, ldx, ldw, ldy, out_dtype, workspace_bytes, splits);
+    it = g_plans.emplace(key, made).first;
+  }
+  return it->second;
+}
+
 }  // namespace
 
 // 1 if the process holds a hipBLASLt that this file can call, else 0.
@@ -190,17 +214,20 @@ extern "C" int me_gemm_library_available() {
   return look_up_api() ? 1 : 0;
 }
 
-// The name of the kernel that a product over contiguous operands runs, at most n - 1 characters and a zero at `out`; empty if
-// none has been asked for or the library names none.
+// The name of the kernel that a product over contiguous operands runs through `me_gemm_library_bf16`, at most n - 1 characters
+// and a zero at `out`; empty if the library has none for the shape or does not name it.
 extern "C" int me_gemm_library_kernel(int out_dtype, size_t workspace_bytes, int M, int N, int K, int splits, char* out, int n) {
   ME_CHECK(out != nullptr && n >= 1, "gemm_library: no place for a name");
   out[0] = 0;
+  ME_CHECK(M >= 1 && N >= 1 && K >= 1 && splits >= 1 && K % splits == 0, "gemm_library: empty product %d x %d x %d", M, N, K);
+  ME_CHECK(out_dtype == ME_BF16 || out_dtype == ME_F32, "gemm_library: unknown output dtype %d", out_dtype);
   int device = 0;
   ME_CHECK(hipGetDevice(&device) == hipSuccess, "gemm_library: no current device");
   std::lock_guard<std::mutex> lock(g_mutex);
-  const auto plan = g_plans.find(PlanKey{device, M, N, K, K, K, N, out_dtype, workspace_bytes, splits});
-  if (plan == g_plans.end() || !plan->second.ok) return 0;
-  std::snprintf(out, (size_t)n, "%s", name_of(g_handles.at(device), plan->second.algo).c_str());
+  hipblasLtHandle_t handle = handle_of(device);
+  if (handle == nullptr) return 0;
+  const Plan& plan = plan_of(handle, PlanKey{device, M, N, K, K, K, N, out_dtype, workspace_bytes, splits});
+  if (plan.ok) std::snprintf(out, (size_t)n, "%s", name_of(handle, plan.algo).c_str());
   return 0;
 }
 
@@ -221,7 +248,6 @@ extern "C" int me_gemm_library_bf16(const void* x, int64_t ldx, const void* w, i
   ME_CHECK(x != nullptr && w != nullptr && y != nullptr, "gemm_library: null operand");
   ME_CHECK(splits >= 1 && K % splits == 0 && (splits == 1 || ((K / splits) % 8 == 0 && out_dtype == ME_F32)),
            "gemm_library: %d splits of K=%d need equal slices of a multiple of 8 and float32 partial sums", splits, K);
-  const int Ks = K / splits;
   int device = 0;
   ME_CHECK(hipGetDevice(&device) == hipSuccess, "gemm_library: no current device");
   const Plan* plan = nullptr;
@@ -232,28 +258,16 @@ extern "C" int me_gemm_library_bf16(const void* x, int64_t ldx, const void* w, i
       me_set_error("gemm_library: no hipBLASLt is loaded in this process");
       return -3;
     }
-    auto h = g_handles.find(device);
-    if (h == g_handles.end()) {
-      hipblasLtHandle_t made = nullptr;
-      if (g_api.create(&made) != HIPBLAS_STATUS_SUCCESS) {
-        me_set_error("gemm_library: hipblasLtCreate failed");
-        return -3;
-      }
-      h = g_handles.emplace(device, made).first;
+    handle = handle_of(device);
+    if (handle == nullptr) {
+      me_set_error("gemm_library: hipblasLtCreate failed");
+      return -3;
     }
-    handle = h->second;
-    const PlanKey key{device, M, N, K, ldx, ldw, ldy, out_dtype, workspace_bytes, splits};
-    auto it = g_plans.find(key);
-    if (it == g_plans.end()) {
-      Plan made;
-      made.ok = make_plan(handle, made, M, N, Ks, ldx, ldw, ldy, out_dtype, workspace == nullptr ? 0 : workspace_bytes, splits);
-      it = g_plans.emplace(key, made).first;
-    }
-    if (!it->second.ok) {
+    plan = &plan_of(handle, PlanKey{device, M, N, K, ldx, ldw, ldy, out_dtype, workspace == nullptr ? 0 : workspace_bytes, splits});
+    if (!plan->ok) {
       me_set_error("gemm_library: hipBLASLt offers no algorithm for %d x %d x %d", M, N, K);
       return -3;
     }
-    plan = &it->second;  // std::map keeps the address
   }
   const float one = 1.f, zero = 0.f;
   const hipblasStatus_t status = g_api.matmul(handle, plan->desc, &one, w, plan->a, x, plan->b, &zero, y, plan->c, y,

@@ -74,6 +74,7 @@ _CORE_PROTOS = {
     "me_gemm_rows_bf16": [P, L, P, L, P, L, I, P, I, I, I, I, I, P],
     "me_gemm_skinny_norm_bf16": [P, I, I, P, P, P, F, P, L, P, L, I, I, I, I, I, P],
     "me_gemm_mid_bf16": [P, L, P, L, P, L, I, I, I, I, I, I, F, F, P, P],
+    "me_gemm_tile_bf16": [P, L, P, L, P, L, I, I, I, I, I, I, F, F, P, I, I, P],
     "me_gemm_library_bf16": [P, L, P, L, P, L, I, P, ctypes.c_size_t, I, I, I, I, P],
     "me_add_rms_norm": [P, I, I, L, P, P, P, P, L, I, F, P],
     "me_add_rms_norm_partials": [P, I, L, P, P, P, P, L, I, F, P],
@@ -246,6 +247,17 @@ def library_product(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, sp
     if out is not None:
         out.copy_(y)
         return out
+    return y
+
+
+def _tile_product(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, slices: int = 1, gated: int = 0, form: tuple = (0.0, 1.0),
+                  bias: torch.Tensor | None = None) -> torch.Tensor:
+    """x [M, K] . w[N, K]^T by csrc/gemm_tile.hip into y: [M, N], float32 partial sums [slices, M, N], or with `gated` (1: formed
+    from the unrounded sums, 2: from the sums rounded to bfloat16) [M, N / 2]."""
+    M, K = x.shape
+    N = w.shape[0]
+    core().call("me_gemm_tile_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), y.shape[-1], _code(y.dtype), slices,
+                M, N, K, gated, *form, _ptr(bias), *tile_choice(M, N, K, slices)[0], _stream())
     return y
 
 
@@ -605,11 +617,15 @@ class HipBackend:
         mid_parts = mid_takes(M, N, K, True) if (allow_partials and out_dtype == x.dtype) else 0
         if mid_parts > 1:
             parts = torch.empty((mid_parts, M, N), dtype=torch.float32, device=x.device)
+            if mid_crowded(M, N, mid_parts) and tile_fits(x, w, mid_parts):
+                return _tile_product(x, w, parts, mid_parts)
             core().call("me_gemm_mid_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), parts.data_ptr(), N,
                         ME_F32, mid_parts, M, N, K, 0, 0.0, 1.0, None, _stream())
             return parts
         splits = library_splits(M, N, K) if (allow_partials and out_dtype == x.dtype) else 1
         if splits > 1:
+            if M <= TILE_SLICES_MAX_M and tile_fits(x, w, splits):
+                return _tile_product(x, w, torch.empty((splits, M, N), dtype=torch.float32, device=x.device), splits)
             parts = library_product(x, w, torch.float32, splits)
             if parts is not None:
                 return parts
@@ -632,20 +648,22 @@ class HipBackend:
             core().call("me_gemm_skinny_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N,
                         _code(out_dtype), None, 1, M, N, K, 0, 0, skinny_wide(N, K), 0.0, 1.0, None, _stream())
             return y
-        if mid_takes(M, N, K, False) == 1:
+        if mid_takes(M, N, K, False) == 1 and not (mid_crowded(M, N, 1) and tile_fits(x, w)):
             y = new()
             core().call("me_gemm_mid_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N,
                         _code(out_dtype), 1, M, N, K, 0, 0.0, 1.0, None, _stream())
             return y
-        # many rows, or the head over a large vocabulary: the library product (float32 accumulation; the
-        # float32 output form keeps the logits unrounded)
+        if tile_takes(M, N, K) and tile_fits(x, w):
+            return _tile_product(x, w, new())
+        # what is left of the many rows, or the head over a large vocabulary: the library product (float32 accumulation;
+        # the float32 output form keeps the logits unrounded)
         return library_product(x, w, out_dtype, out=out)
 
     def gated_linear(self, x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, clamp: tuple | None = None) -> torch.Tensor:
         """silu(x . w[:I]^T) * (x . w[I:]^T) for a packed gate/up weight w [2 I, K] (gate rows first), as one
         launch: the product's workgroups pair each gate feature with its up feature when they merge their waves,
-        from the unrounded sums (the separate kernels round the product to bfloat16 first). For the row counts
-        `gated_linear_fuses` admits. `bias` (float32 [2 I]) joins the sums first; `clamp` (limit, alpha): the form of
+        from the unrounded sums (the separate kernels round the product to bfloat16 first; so does the kernel for many
+        rows, `gated_linear_tiles`). For the row counts `gated_linear_fuses` admits. `bias` (float32 [2 I]) joins the sums first; `clamp` (limit, alpha): the form of
         `glu_clamped` in place of silu(gate) * up. Returns [M, I]. (reference layers/linear.py:29-45, layers/activation.py:5-7.)"""
         _check(gated_linear_fuses(x, w), "gated_linear: bfloat16, few rows, see gated_linear_fuses")
         M, K = x.shape
@@ -654,6 +672,10 @@ class HipBackend:
         _check(bias is None or (bias.dtype == torch.float32 and bias.shape == (N,) and bias.is_contiguous()), "gated_linear: bias float32 [2 I]")
         _check(clamp is None or clamp[0] > 0, "gated_linear: the limit must be positive")
         form = (0.0, 1.0) if clamp is None else (float(clamp[0]), float(clamp[1]))
+        if M > GATED_EPILOGUE_MAX_M and gated_linear_tiles(M, w) and tile_fits(x, w):
+            # the gates as those forms that had these rows before this kernel make them: rounded where the gating was a kernel
+            # of its own behind the product
+            return _tile_product(x, w, y, gated=1 if mid_takes(M, N, K, False) == 1 else 2, form=form, bias=bias)
         if M > GATED_EPILOGUE_MAX_M:        # a few hundred rows over a small weight: the gating in that kernel's epilogue
             core().call("me_gemm_mid_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N // 2,
                         ME_BF16, 1, M, N, K, 1, *form, _ptr(bias), _stream())
@@ -1605,6 +1627,74 @@ def mid_takes(M: int, N: int, K: int, partials: bool) -> int:
     return 1 if M <= 256 else 0
 
 
+# Tile of csrc/gemm_tile.hip -> (us of a launch, us of a workgroup, us of a step of 64 of K for a workgroup that has its compute
+# unit to itself, and for each of several that share one, workgroups that fit a compute unit), fitted to 6,300 times: 22 weights
+# of the layer sizes of 0.6B to 32B, 40 to 8,192 rows, one result and 2, 4 and 8 slices of K.
+TILE_COST = {(256, 256): (0.0, 10.6, 1.02, 1.02, 1), (256, 192): (0.0, 9.5, 0.91, 0.91, 1), (192, 256): (0.0, 9.0, 0.89, 0.89, 1),
+             (128, 256): (0.0, 6.2, 0.75, 0.75, 1), (256, 128): (0.0, 6.6, 0.70, 0.70, 1), (128, 192): (0.0, 5.6, 0.74, 0.61, 2),
+             (128, 128): (0.0, 4.0, 0.48, 0.44, 2), (64, 128): (0.5, 2.4, 0.37, 0.30, 3), (128, 64): (1.5, 1.6, 0.35, 0.31, 3),
+             (64, 64): (2.1, 0.8, 0.29, 0.20, 5)}
+TILE_MIN_ROWS = 33
+TILE_SURE_K = 2048
+TILE_MIN_TFLOPS = 1000
+TILE_SLICES_MAX_M = 256
+
+
+@lru_cache(maxsize=4096)      # asked once per product of a step: ten tiles each time
+def tile_choice(M: int, N: int, K: int, slices: int = 1) -> tuple:
+    """((rows, features) of the tile that csrc/gemm_tile.hip takes for M rows against a weight [N, K] in `slices` slices of
+    K, the us that `TILE_COST` expects of it): the tile whose busiest compute unit is done first. Over the products that
+    the costs were fitted to it is 0.7 % behind the fastest tile on average with one result (11 % at worst), 2 % with slices."""
+    def cost(tile):
+        launch, each, alone, shared, fit = TILE_COST[tile]
+        busiest = -(-(-(-M // tile[0]) * -(-N // tile[1])) * slices // _COMPUTE_UNITS)
+        return launch + each * busiest + -(-(K // 64) // slices) * max(alone * -(-busiest // fit), shared * busiest)
+    best = min(TILE_COST, key=cost)
+    return best, cost(best)
+
+
+def tile_takes(M: int, N: int, K: int) -> bool:
+    """Whether the product of M rows against a bfloat16 weight [N, K] that neither the kernels for few rows nor slices of K
+    take goes to csrc/gemm_tile.hip rather than to the library. Over a K of up to 2,048: always (137 products of 65 to 8,192
+    rows: 0.91 to 1.5 times as fast, 1.13 on average; 512 rows of 4096 x 1024 11.3 -> 8.9 us, 2,048 rows of 1024 x 1024
+    11.7 -> 8.8). Over a longer K where the tiles fill the compute units, which is where `tile_choice` expects 1,000
+    TFLOP/s or more (2,048 rows of 24576 x 4096 362 -> 290 us, 3,123 of it 692 -> 514, 2,048 of 6144 x 4096 90 -> 78); where
+    they do not, the library's smaller tiles are ahead (300 rows of 2560 x 4096 17.8 / 19.1, 1,280 of 4096 x 4096 46 / 51)."""
+    if M < TILE_MIN_ROWS or N >= LIBRARY_MIN_N and M < 128:
+        return False
+    return K <= TILE_SURE_K or 2e-6 * M * N * K / tile_choice(M, N, K)[1] >= TILE_MIN_TFLOPS
+
+
+def tile_fits(x: torch.Tensor, w: torch.Tensor, slices: int = 1) -> bool:
+    """Whether csrc/gemm_tile.hip can compute x . w^T in that many slices of K: K in two steps of 64 or more for each, whole
+    16-byte pieces in every row, 32-bit offsets."""
+    K, steps = x.shape[1], x.shape[1] // 64
+    return (K % 64 == 0 and w.shape[0] % 8 == 0 and (slices - 1) * -(-steps // slices) <= steps - 2
+            and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and x.shape[0] * x.stride(0) < 1 << 31 and w.shape[0] * w.stride(0) < 1 << 31)
+
+
+def mid_crowded(M: int, N: int, slices: int) -> bool:
+    """Whether the kernel of csrc/gemm_mid.hip would have more workgroups than compute units: it runs one to a unit (96 KB of
+    LDS), so that the rest wait for a second round, where the tiles of csrc/gemm_tile.hip share a unit. 200 rows of
+    6144 x 1024 12.1 / 8.7 us, 512 rows of 1024 x 3072 in four slices 10.6 / 8.5; up to 256 workgroups the former is ahead by
+    a microsecond (its steps are 128 of K)."""
+    return -(-M // 64) * -(-N // 64) * slices > _COMPUTE_UNITS
+
+
+def gated_linear_tiles(rows: int, w: torch.Tensor) -> bool:
+    """Whether `rows` rows against the packed gate/up weight w [2 I, K] go through csrc/gemm_tile.hip with the gating in its
+    epilogue: from 33 rows on, where no kernel for few rows has the product. Against the library's product and a gating kernel
+    behind it (78 products of 40 to 8,192 rows over the gate/up weights of 0.6B to 32B) 0.97 to 2 times as fast, 1.28 on
+    average: 512 rows of 6144 x 1024 17.7 -> 10.6 us, 2,048 rows of 24576 x 4096 390 -> 281."""
+    if not FUSE_GATE_INTO_GATE_UP or rows < TILE_MIN_ROWS or w.dtype != torch.bfloat16 or w.dim() != 2 or w.stride(1) != 1:
+        return False
+    N, K = w.shape
+    if N % 16 or K % 64 or K < 128 or skinny_takes(rows, N, K):
+        return False
+    return mid_takes(rows, N, K, False) != 1 or mid_crowded(rows, N, 1)
+
+
 def prefill_waves(max_context: int, num_tokens: int, num_seqs: int, Hq: int, Hkv: int, col_tiles: int, max_segs: int) -> int:
     """Waves per SIMD (2 or 3) of the prefill attention kernel whose loads write LDS themselves (head size 128).
 
@@ -1850,7 +1940,8 @@ def gated_linear_rows(rows: int, w: torch.Tensor) -> bool:
 def gated_linear_fuses(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether `gated_linear` takes rows x [M, K] and the packed gate/up weight w [2 I, K]."""
     return (x.dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and x.stride(1) == 1
-            and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and gated_linear_rows(x.shape[0], w))
+            and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
+            and (gated_linear_rows(x.shape[0], w) or (gated_linear_tiles(x.shape[0], w) and tile_fits(x, w))))
 
 
 def norm_linear_fuses(x: torch.Tensor, w: torch.Tensor) -> bool:

@@ -46,9 +46,8 @@ class SwiGLU(FeedForward):
             y = self.down.forward(self.gate_up.forward(x, gated=True, bias=self.gate_up_bias), allow_partials=True)
             return Biased(y, self.down_bias) if self.defer_bias else ops.add_bias(y, self.down_bias, self.down.weight.dtype)
         rows = x.rows() if isinstance(x, PendingNorm) else x.shape[0]
-        if ops.gated_linear_rows(rows, self.gate_up.weight):
-            # few rows (or a few hundred over a small weight): the gating in the gate/up product's epilogue (every gate formed
-            # once), a plain down product
+        if ops.gated_linear_rows(rows, self.gate_up.weight) or ops.gated_linear_tiles(rows, self.gate_up.weight):
+            # the gating in the gate/up product's epilogue (every gate formed once), a plain down product
             return self.down.forward(self.gate_up.forward(x, gated=True), allow_partials=True)
         gu = self.gate_up.forward(x)
         return ops.silu_mul_linear(gu, self.down.weight, allow_partials=True)

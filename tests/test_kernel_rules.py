@@ -263,3 +263,26 @@ def test_the_short_convolutions_grid_is_not_mostly_empty():
         assert ops.conv_tokens_per_thread(T, B, longest, 4, 1024) == per, q_lens
         assert per == 32 or B * -(-longest // 8) * 4 <= max(1 << 17, 32 * -(-T // 8))
     assert ops.conv_tokens_per_thread(350, 1, 350, 5, 64) == ops.conv_tokens_per_thread(350, 1, 350, 1, 64) == 32
+
+
+def test_tiles_for_many_rows_fit_the_kernel_and_leave_what_it_cannot_take():
+    """Whatever sizes come: the tile is one of the kernel's, and K, strides or features that the kernel refuses stay where they
+    were; few rows and the head over a vocabulary for few rows stay too."""
+    import random
+    rng = random.Random(11)
+    for _ in range(3000):
+        M, N, K = rng.randint(1, 9000), 8 * rng.randint(1, 4000), 8 * rng.randint(1, 800)
+        slices = rng.choice([1, 1, 2, 4, 8])
+        x, w = torch.empty(M, K, dtype=torch.bfloat16, device="meta"), torch.empty(N, K, dtype=torch.bfloat16, device="meta")
+        steps = K // 64
+        assert ops.tile_fits(x, w, slices) == (K % 64 == 0 and steps - (slices - 1) * -(-steps // slices) >= 2)
+        if K >= 64:
+            assert ops.tile_choice(M, N, K, slices)[0] in ops.TILE_COST
+        if ops.tile_takes(M, N, max(K, 64)):
+            assert M > 32 and (N < ops.LIBRARY_MIN_N or M >= 128)
+    assert ops.tile_choice(2048, 24576, 4096)[0] == (256, 256) and ops.tile_choice(512, 1024, 2048, 4)[0] in ((64, 64), (64, 128), (128, 64))
+    assert ops.tile_takes(2048, 24576, 4096) and not ops.tile_takes(300, 2560, 4096) and ops.tile_takes(2048, 1024, 1024)
+    w = torch.empty(6144, 1024, dtype=torch.bfloat16)
+    assert all(ops.gated_linear_tiles(m, w) for m in (200, 257, 2048)) and not any(ops.gated_linear_tiles(m, w) for m in (8, 16, 32, 64, 128))
+    assert not ops.gated_linear_tiles(2048, w.float()) and not ops.gated_linear_tiles(2048, torch.empty(6136, 1024, dtype=torch.bfloat16))
+    assert not ops.tile_fits(torch.empty(64, 136, dtype=torch.bfloat16)[:, 4:132], torch.empty(64, 128, dtype=torch.bfloat16))    # not 16-byte aligned

@@ -1,0 +1,100 @@
+"""The product of many rows whose tiles go through LDS in quarters of a step (csrc/gemm_tile.hip): every tile at the edges of
+its rows, features and steps of K, against float64."""
+import pytest
+import torch
+
+from mini_engine_amd.kernels import ops
+from test_kernels_gpu import DEV, close, hip, twin
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(M, N, K, pad=0):
+    g = torch.Generator(device=DEV).manual_seed(M * 7 + N + K)
+    x = torch.randn(M, K + pad, device=DEV, generator=g).bfloat16()[:, :K]
+    w = (torch.randn(N, K + pad, device=DEV, generator=g) * 0.05).bfloat16()[:, :K]
+    return x, w
+
+
+def _launch(x, w, y, slices, tile, gated=0, bias=None, limit=0.0, alpha=1.0):
+    M, K = x.shape
+    ops.core().call("me_gemm_tile_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), y.shape[-1], ops._code(y.dtype),
+                    slices, M, w.shape[0], K, gated, limit, alpha, ops._ptr(bias), *tile, ops._stream())
+
+
+@pytest.mark.parametrize("tile", list(ops.TILE_COST), ids=lambda t: f"{t[0]}x{t[1]}")
+def test_every_tile_at_its_edges(tile):
+    """One row, one more and one fewer than a tile; features that end inside a tile; two steps of K (no step in between), three
+    and many, rows of a longer stride; one result in both types, slices of K with a shorter last one, the gating."""
+    rows, features = tile
+    for M, N, K, pad in ((1, 8, 128, 0), (rows - 1, features, 192, 8), (rows + 1, features + 8, 256, 0), (2 * rows + 3, 2 * features - 16, 1088, 64),
+                         (9 * rows + 5, features + 64, 320, 0)):
+        x, w = _operands(M, N, K, pad)
+        ref = x.double() @ w.double().t()
+        y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+        _launch(x, w, y, 1, tile)
+        close(y, ref, 4e-3)                      # one rounding to bfloat16: 2^-9 of a value at most
+        y = torch.full((M, N), float("nan"), dtype=torch.float32, device=DEV)
+        _launch(x, w, y, 1, tile)
+        close(y, ref, 2e-5)
+        for slices in (2, 3, 8):
+            steps = K // 64
+            if (slices - 1) * -(-steps // slices) <= steps - 2:
+                y = torch.full((slices, M, N), float("nan"), dtype=torch.float32, device=DEV)
+                _launch(x, w, y, slices, tile)
+                close(y.sum(0), ref, 2e-5)
+        if N % 16 == 0:
+            y = torch.full((M, N // 2), float("nan"), dtype=torch.bfloat16, device=DEV)
+            _launch(x, w, y, 1, tile, 2)
+            two = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+            _launch(x, w, two, 1, tile)
+            assert torch.equal(y, hip().silu_and_mul(two))                     # rounded sums: the two kernels' bits
+            _launch(x, w, y, 1, tile, 2, None, 1.5, 1.702)
+            assert torch.equal(y, hip().glu_clamped(two, 1.5, 1.702))
+            _launch(x, w, y, 1, tile, 1)
+            close(y, torch.nn.functional.silu(ref[:, :N // 2]) * ref[:, N // 2:], 6e-3)
+            bias = torch.randn(N, device=DEV)
+            _launch(x, w, y, 1, tile, 1, bias)
+            b = ref + bias.double()
+            close(y, torch.nn.functional.silu(b[:, :N // 2]) * b[:, N // 2:], 6e-3)
+            _launch(x, w, y, 1, tile, 1, None, 1.5, 1.702)
+            gate, up = ref[:, :N // 2].clamp(max=1.5), ref[:, N // 2:].clamp(-1.5, 1.5)
+            close(y, gate * torch.sigmoid(1.702 * gate) * (up + 1), 6e-3)
+
+
+def test_a_row_of_infinities_and_not_a_numbers_stays_in_its_row():
+    x, w = _operands(300, 520, 256)
+    want = hip().linear(x, w)
+    x[7, 3], x[299, 0] = float("inf"), float("nan")
+    got = hip().linear(x, w)
+    keep = [i for i in range(300) if i not in (7, 299)]
+    assert torch.equal(got[keep], want[keep]) and bool(torch.isnan(got[299]).all()) and not bool(torch.isfinite(got[7]).any())
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 1024, 1024), (513, 1024, 3072), (257, 6144, 1024), (200, 6144, 1024), (1100, 4096, 2048), (2048, 6144, 4096)])
+def test_what_the_rules_send_there(M, N, K):
+    """`linear` and `gated_linear` through the dispatch, replayed from a graph with other rows between the replays."""
+    x, w = _operands(M, N, K)
+    assert ops.tile_fits(x, w)
+    for _ in range(2):
+        close(hip().linear(x, w), x.double() @ w.double().t(), 4e-3)
+    if ops.gated_linear_fuses(x, w):
+        # sums rounded before the gating: 2^-9 each of gate (times up to 1 + gate in its silu), up and result
+        close(hip().gated_linear(x, w), twin.gated_linear(x, w, compute_dtype=torch.float64), 1.5e-2)
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+        y = hip().linear(x, w)
+    for _ in range(3):
+        x.copy_(torch.randn(M, K, device=DEV))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, hip().linear(x, w))
+
+
+def test_what_the_kernel_refuses():
+    x, w = _operands(70, 64, 128)
+    y = torch.empty(70, 64, dtype=torch.bfloat16, device=DEV)
+    for args in ((x[:, :96], w[:, :96], y, 1, (64, 64)), (x, w, y, 1, (64, 96)), (x, w, y.float(), 2, (64, 64)), (x, w[:60], y[:, :60], 1, (64, 64))):
+        with pytest.raises(ops.KernelError):
+            _launch(*args)
