@@ -5,6 +5,7 @@
 // besides the projections is formed here in float32: decays and their exponentials, softplus, write strengths, unit
 // lengths.
 #include "common.h"
+#include <type_traits>
 
 __device__ __forceinline__ float hy_sigmoid(float v) { return 1.0f / (1.0f + expf(-v)); }
 __device__ __forceinline__ float hy_softplus(float v) { return v > 20.f ? v : log1pf(expf(v)); }
@@ -659,23 +660,32 @@ __global__ void __launch_bounds__(64) decay_rows_kernel(DrArgs a) {
 }
 
 // The same walk over values that decay_prepare_kernel has shaped: portions of many tokens. What bounds it is the number of
-// instructions of a wave per token (a request's tokens are a chain, and the chip has a wave or less per SIMD), so a batch of
-// eight tokens is one piece of code without a branch: the exchange and the output sum of a token overlap the next token's
-// reads and updates, a lane brings its share of the batch's shared values in 16-byte pieces that go to LDS as they are, and
-// of the four lanes that hold the same finished sums each stores another token's. The sums are those of decay_rows_kernel in the
-// same order. 2,048 tokens: delta rule, 4 heads of 128 x 128, 344 us, bonus rule, 16 heads of 64 x 64, 216 us (with a branch per
-// token, 4-byte loads and a store per token: 1,105 and 909).
-template <typename TX, int NR, int RG, int RULE>
-__global__ void __launch_bounds__(64) decay_walk_kernel(DrArgs a, const float* __restrict__ pre_q, const float* __restrict__ pre_k,
-                                                        const float* __restrict__ pre_d, const float* __restrict__ pre_x) {
+// instructions of a wave per token (a request's tokens are a chain, the chip has few waves per SIMD, and a lone wave of a SIMD
+// issues one instruction in eight cycles or so), so a batch of eight tokens is one piece of code without a branch: the exchange
+// and the output sum of a token overlap the next token's reads and updates, and shared values are brought in 16-byte pieces that
+// go to LDS as they are. With W = 4 four waves hold the same columns: each of them carries the state through every token,
+// but forms, exchanges and stores the outputs of every fourth only, and brings a quarter of the shared values; batches
+// are twice as long, for eight tokens take less time than the next eight need to come from memory (the bound of the rules with
+// short chains: about 105 ns a token whatever their instructions), and tokens are read from LDS two or three ahead. The sums are
+// those of decay_rows_kernel in the same order. With the kernel that shapes the values, 2,048 tokens beside 1,075, one wave /
+// four: delta rule, 4 heads of 128 x 128, 344 / 265 us, bonus rule, 16 heads of 64 x 64, 230 / 143 us.
+template <typename TX, int NR, int RG, int RULE, int W>
+__global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const float* __restrict__ pre_q, const float* __restrict__ pre_k,
+                                                            const float* __restrict__ pre_d, const float* __restrict__ pre_x) {
+  constexpr int TB = W == 4 ? 16 : DR_TB;       // tokens of a batch: with more of them on their way than a trip to memory takes
+  constexpr int AHEAD = NR <= 64 ? 3 : NR <= 128 ? 2 : 1;    // tokens whose shared values are read from LDS ahead
   constexpr int PC = 64 / RG;            // columns per wave
   constexpr int RL = NR / RG;            // rows per lane
-  constexpr int PIECES = DR_TB * NR / 4; // 16-byte pieces of a batch's q, k or decays
-  constexpr int ROUNDS = (PIECES + 63) / 64;
-  constexpr bool DELTA = RULE == 1 || RULE == 3, ROWS = RULE != 3;
+  constexpr int PIECES = TB * NR / 4; // 16-byte pieces of a batch's q, k or decays
+  constexpr int ROUNDS = (PIECES + 64 * W - 1) / (64 * W);
+  constexpr int VALUES = TB * PC, VROUNDS = (VALUES + 64 * W - 1) / (64 * W);
+  constexpr bool ROWS = RULE != 3;
+  constexpr bool SHARED_V = NR <= 128;   // the columns' values go through LDS too; with 256 rows a lane asks for its own
   __shared__ f32x4 sq[2][PIECES], sk[2][PIECES], sd[ROWS ? 2 : 1][ROWS ? PIECES : 1];
-  __shared__ float sx[2][DR_TB], sh[2][DR_TB];               // the tokens' own numbers; their heads' decays (RULE 3)
-  const int lane = threadIdx.x;
+  __shared__ __align__(16) float sv[2][SHARED_V ? VALUES : 1];              // [column][token]
+  __shared__ float sx[2][TB], sh[2][TB];               // the tokens' own numbers; their heads' decays (RULE 3)
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col_blocks = (a.P + PC - 1) / PC;
   const int cb = blockIdx.x % col_blocks;
   const int h = (blockIdx.x / col_blocks) % a.H;
@@ -697,19 +707,36 @@ __global__ void __launch_bounds__(64) decay_walk_kernel(DrArgs a, const float* _
   const int64_t head0 = first * a.H + h;
   f32x4 nq[ROUNDS], nk[ROUNDS], nd[ROUNDS];
   float nx = 0.f, nh = 0.f;
-  TX nv[DR_TB];
+  TX nv[SHARED_V ? VROUNDS : TB];
   // what a lane adds to a batch's first address, in bytes (the address itself is the same for all lanes)
   uint32_t piece[ROUNDS];
+  int column[VROUNDS];                                       // of a value that a thread brings, and its place in sv
+  int place[VROUNDS];
 #pragma unroll
   for (int r = 0; r < ROUNDS; ++r) {
-    const int e = min(lane + 64 * r, PIECES - 1);
+    const int e = min(tid + 64 * W * r, PIECES - 1);
     piece[r] = (uint32_t)((e / (NR / 4) * a.H * (NR / 4) + e % (NR / 4)) * 16);
   }
-  const uint32_t own = (uint32_t)((lane & (DR_TB - 1)) * a.H * 4), column = (uint32_t)(pc * sizeof(TX));
+#pragma unroll
+  for (int r = 0; r < VROUNDS; ++r) {
+    const int e = min(tid + 64 * W * r, VALUES - 1);
+    column[r] = min(cb * PC + e % PC, a.P - 1);
+    place[r] = e % PC * TB + e / PC;
+  }
+  const int my_token = tid & (TB - 1);
+  const uint32_t own = (uint32_t)(my_token * a.H * 4);
   auto at = [](const void* base, uint32_t bytes) { return reinterpret_cast<const char*>(base) + bytes; };
   // the next batch on its way; of a batch that is not whole, tokens behind the last are read from the last one and not used
   auto fetch = [&](int t0) {
-    if (t0 + DR_TB <= n_tok) {
+    if (t0 >= n_tok) return;
+    if (!SHARED_V) {
+#pragma unroll
+      for (int j = 0; j < TB; ++j) nv[j] = values[(int64_t)min(t0 + j, n_tok - 1) * a.v_stride + pc];
+    } else
+#pragma unroll
+    for (int r = 0; r < VROUNDS; ++r)
+      nv[r] = values[(int64_t)min(t0 + min(tid + 64 * W * r, VALUES - 1) / PC, n_tok - 1) * a.v_stride + column[r]];
+    if (t0 + TB <= n_tok) {
       const int64_t row = head0 + (int64_t)t0 * a.H;
 #pragma unroll
       for (int r = 0; r < ROUNDS; ++r) {
@@ -719,51 +746,48 @@ __global__ void __launch_bounds__(64) decay_walk_kernel(DrArgs a, const float* _
       }
       nx = *reinterpret_cast<const float*>(at(pre_x + row, own));
       if (!ROWS) nh = *reinterpret_cast<const float*>(at(pre_d + row, own));
-      const TX* vt = values + t0 * a.v_stride;
-#pragma unroll
-      for (int j = 0; j < DR_TB; ++j, vt += a.v_stride) nv[j] = *reinterpret_cast<const TX*>(at(vt, column));
       return;
     }
 #pragma unroll
     for (int r = 0; r < ROUNDS; ++r) {
-      const int e = min(lane + 64 * r, PIECES - 1);
+      const int e = min(tid + 64 * W * r, PIECES - 1);
       const int64_t from = (head0 + (int64_t)min(t0 + e / (NR / 4), n_tok - 1) * a.H) * NR + e % (NR / 4) * 4;
       nq[r] = *reinterpret_cast<const f32x4*>(pre_q + from);
       nk[r] = *reinterpret_cast<const f32x4*>(pre_k + from);
       if (ROWS) nd[r] = *reinterpret_cast<const f32x4*>(pre_d + from);
     }
-    const int64_t row = head0 + (int64_t)min(t0 + (lane & (DR_TB - 1)), n_tok - 1) * a.H;
+    const int64_t row = head0 + (int64_t)min(t0 + my_token, n_tok - 1) * a.H;
     nx = pre_x[row];
     if (!ROWS) nh = pre_d[row];
-#pragma unroll
-    for (int j = 0; j < DR_TB; ++j) nv[j] = values[(int64_t)min(t0 + j, n_tok - 1) * a.v_stride + pc];
   };
   struct Shared { float q[RL], k[RL], d[RL], x; };
-  auto read = [&](int buf, int j, Shared& o) {
+  auto read = [&](int buf, int j, Shared& o, bool reads_out) {
     const float* aq = reinterpret_cast<const float*>(&sq[buf][0]) + j * NR + rg * RL;
     const float* ak = reinterpret_cast<const float*>(&sk[buf][0]) + j * NR + rg * RL;
     const float* ad = reinterpret_cast<const float*>(&sd[ROWS ? buf : 0][0]) + j * NR + rg * RL;
 #pragma unroll
     for (int i = 0; i < RL; ++i) {
-      o.q[i] = aq[i]; o.k[i] = ak[i];
+      if (reads_out) o.q[i] = aq[i];
+      o.k[i] = ak[i];
       if (ROWS) o.d[i] = ad[i];
     }
     if (!ROWS) o.d[0] = sh[buf][j];
-    o.x = RULE == 2 ? 0.f : sx[buf][j];
+    o.x = RULE == 2 || (RULE == 0 && !reads_out) ? 0.f : sx[buf][j];
   };
-  auto token = [&](const Shared& o, float v) {
+  // the state behind a token and, where this wave is to give it, the token's output
+  auto token = [&](const Shared& o, float v, bool reads_out) {
     float y = 0.f;
     if (RULE == 0) {
 #pragma unroll
       for (int i = 0; i < RL; ++i) {
-        y = fmaf(o.q[i], S[i], y);
+        if (reads_out) y = fmaf(o.q[i], S[i], y);
         S[i] = fmaf(o.d[i], S[i], o.k[i] * v);
       }
     } else if (RULE == 2) {
 #pragma unroll
       for (int i = 0; i < RL; ++i) {
         S[i] = fmaf(o.d[i], S[i], o.k[i] * v);
-        y = fmaf(o.q[i], S[i], y);
+        if (reads_out) y = fmaf(o.q[i], S[i], y);
       }
     } else {
       float dot = 0.f;
@@ -777,76 +801,109 @@ __global__ void __launch_bounds__(64) decay_walk_kernel(DrArgs a, const float* _
 #pragma unroll
       for (int i = 0; i < RL; ++i) {
         S[i] = fmaf(o.k[i], u, S[i]);
-        y = fmaf(S[i], o.q[i], y);
+        if (reads_out) y = fmaf(S[i], o.q[i], y);
       }
     }
+    if (!reads_out) return 0.f;
     y = group_sum<RG>(y);
     if (RULE == 0) y = fmaf(o.x, v, y);          // the current token's own term: v_p * sum_n q_n bonus_n k_n
     return y;
   };
   float* out = a.y + first * (int64_t)(a.H * a.P) + h * a.P + p;
-  fetch(0);
-  for (int t0 = 0, buf = 0; t0 < n_tok; t0 += DR_TB, buf ^= 1) {
-    // one wave: what its lanes write to LDS, its lanes read behind it without a barrier
+  int t0 = 0, buf = 0;
+  // the batch that has come goes to LDS, the next one is asked for, and the columns' values of the batch are read
+  auto next_batch = [&](float (&v)[TB]) {
 #pragma unroll
     for (int r = 0; r < ROUNDS; ++r) {
-      const int e = lane + 64 * r;
-      if (PIECES % 64 == 0 || e < PIECES) {
+      const int e = tid + 64 * W * r;
+      if (PIECES % (64 * W) == 0 || e < PIECES) {
         sq[buf][e] = nq[r]; sk[buf][e] = nk[r];
         if (ROWS) sd[ROWS ? buf : 0][e] = nd[r];
       }
     }
-    if (lane < DR_TB) {
-      sx[buf][lane] = nx;
-      if (!ROWS) sh[buf][lane] = nh;
+    if (!SHARED_V) {
+#pragma unroll
+      for (int j = 0; j < TB; ++j) v[j] = to_f32<TX>(nv[j]);
+    } else
+#pragma unroll
+    for (int r = 0; r < VROUNDS; ++r)
+      if (VALUES % (64 * W) == 0 || tid + 64 * W * r < VALUES) sv[buf][place[r]] = to_f32<TX>(nv[r]);
+    if (tid < TB) {
+      sx[buf][tid] = nx;
+      if (!ROWS) sh[buf][tid] = nh;
     }
-    float v[DR_TB];
-#pragma unroll
-    for (int j = 0; j < DR_TB; ++j) v[j] = to_f32<TX>(nv[j]);
     asm volatile("" ::: "memory");
-    fetch(t0 + DR_TB);
-    asm volatile("" ::: "memory");
-    if (t0 + DR_TB <= n_tok) {
-      float y[DR_TB];
-      Shared o[2];                               // a token's values are read while the one before it is worked on
-      read(buf, 0, o[0]);
+    fetch(t0 + TB);
+    // the batch is in LDS; the other buffer, which the next batch will take, has been read by all (one wave needs no
+    // barrier: what its lanes write to LDS, its lanes read behind it)
+    if (W > 1) __syncthreads(); else asm volatile("" ::: "memory");
+    if (SHARED_V) {
 #pragma unroll
-      for (int j = 0; j < DR_TB; ++j) {
-        if (j + 1 < DR_TB) read(buf, j + 1, o[(j + 1) & 1]);
-        y[j] = token(o[j & 1], v[j]);
+      for (int j = 0; j < TB; ++j) v[j] = sv[buf][lane / RG * TB + j];
+    }
+  };
+  auto walk = [&](auto which) {                  // a wave's whole batches: it gives the outputs of tokens which, which + W, ... of each
+    constexpr int ME = decltype(which)::value, MINE = TB / W;
+    for (; t0 + TB <= n_tok; t0 += TB, buf ^= 1) {
+      float v[TB], y[MINE];
+      next_batch(v);
+      Shared o[AHEAD + 1];                       // a token's values are read while those before it are worked on
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) read(buf, j, o[j], j % W == ME);
+#pragma unroll
+      for (int j = 0; j < TB; ++j) {
+        if (j + AHEAD < TB) read(buf, j + AHEAD, o[(j + AHEAD) % (AHEAD + 1)], (j + AHEAD) % W == ME);
+        const float yj = token(o[j % (AHEAD + 1)], v[j], j % W == ME);
+        if (j % W == ME) y[j / W] = yj;
       }
       // the first four lanes of a column hold the same bits (the others have added in another order): lane rg of them stores
-      // the output of token j0 + rg
-      constexpr int ST = RG < 4 ? RG : 4;
+      // the wave's output i0 + rg
+      constexpr int ST = RG < 4 ? (RG < MINE ? RG : MINE) : (MINE < 4 ? MINE : 4);
       if (live && rg < ST) {
 #pragma unroll
-        for (int j0 = 0; j0 < DR_TB; j0 += ST) {
-          float mine = y[j0];
+        for (int i0 = 0; i0 < MINE; i0 += ST) {
+          float mine = y[i0];
 #pragma unroll
-          for (int j = 1; j < ST; ++j) mine = rg == j ? y[j0 + j] : mine;
-          out[(int64_t)(t0 + j0 + rg) * (a.H * a.P)] = mine;
+          for (int i = 1; i < ST; ++i) mine = rg == i ? y[i0 + i] : mine;
+          out[(int64_t)(t0 + ME + W * (i0 + rg)) * (a.H * a.P)] = mine;
         }
       }
-    } else {
+    }
+  };
+  static_assert(W == 1 || W == 4, "each wave's walk is code of its own");
+  fetch(0);
+  if (W == 1 || wave == 0) walk(std::integral_constant<int, 0>{});
+  else if (wave == 1) walk(std::integral_constant<int, 1 % W>{});
+  else if (wave == 2) walk(std::integral_constant<int, 2 % W>{});
+  else walk(std::integral_constant<int, 3 % W>{});
+  if (t0 < n_tok) {                              // a last batch that is not whole
+    float v[TB];
+    next_batch(v);
+    if (wave == 0) {                             // its outputs and the state behind it are the first wave's
 #pragma unroll 1
       for (int j = 0; t0 + j < n_tok; ++j) {
         Shared o;
-        read(buf, j, o);
+        read(buf, j, o, true);
         float vj = v[0];
 #pragma unroll
-        for (int i = 1; i < DR_TB; ++i) vj = i == j ? v[i] : vj;
-        const float y = token(o, vj);
+        for (int i = 1; i < TB; ++i) vj = i == j ? v[i] : vj;
+        const float y = token(o, vj, true);
         if (live && rg == 0) out[(int64_t)(t0 + j) * (a.H * a.P)] = y;
       }
     }
   }
-  if (live) {
+  if (live && wave == 0) {
 #pragma unroll
     for (int i = 0; i < RL; ++i)
       if (i * RG + rg < a.N) srow[(int64_t)(i * RG + rg) * a.P + p] = S[i];
   }
 }
 
+// Workgroups up to which four waves share the walk of a column group: beyond, the waves of one SIMD share its instructions, and
+// the state carried four times costs more than it saves. us, one wave / four: 128 rows, 384 workgroups 202 / 172, 512 147 / 154;
+// 64 rows, 768 workgroups 167 / 142 (delta rule) and 138 / 95 (bonus), 1,024 142 / 177 and 119 / 118. With 256 rows the batches'
+// LDS leaves no room for longer ones, and without them four waves gain nothing (624 / 650).
+template <int NR> constexpr unsigned dr_shared_max() { return NR <= 64 ? 768 : NR <= 128 ? 384 : 0; }
 template <typename TX, int NR, int RG, bool PRE>
 static void launch_decay_rows(const DrArgs& a, int rule, int num_seqs, int64_t T, float* pre, hipStream_t stream) {
   constexpr int PC = 64 / RG;
@@ -858,7 +915,10 @@ static void launch_decay_rows(const DrArgs& a, int rule, int num_seqs, int64_t T
 #define DR_RULE(R)                                                                       \
   do {                                                                                   \
     decay_prepare_kernel<TX, NR, R><<<pgrid, block, 0, stream>>>(a, RG, pq, pk, pd, px); \
-    decay_walk_kernel<TX, NR, RG, R><<<grid, block, 0, stream>>>(a, pq, pk, pd, px);     \
+    constexpr bool SHARES = RG == 16 && dr_shared_max<NR>() > 0;                         \
+    if (SHARES && grid.x <= dr_shared_max<NR>())                                         \
+      decay_walk_kernel<TX, NR, RG, R, SHARES ? 4 : 1><<<grid, 256, 0, stream>>>(a, pq, pk, pd, px); \
+    else decay_walk_kernel<TX, NR, RG, R, 1><<<grid, block, 0, stream>>>(a, pq, pk, pd, px); \
   } while (0)
     if (rule == 0) DR_RULE(0); else if (rule == 1) DR_RULE(1); else if (rule == 2) DR_RULE(2); else DR_RULE(3);
 #undef DR_RULE

@@ -44,3 +44,40 @@ def test_places_in_a_batch(monkeypatch, H, N, P, dtype, rule, groups):
             parts.append(run(lo, n, state))
             lo += n
         assert torch.equal(torch.cat(parts), y) and torch.equal(state, whole)
+
+
+@pytest.mark.parametrize("rule", ["bonus", "delta", "gated", "delta_head"])
+@pytest.mark.parametrize("H,N,P,count", [(2, 64, 64, 3), (12, 64, 64, 4), (13, 64, 64, 4), (3, 128, 128, 4), (4, 128, 132, 3), (2, 20, 30, 2), (1, 256, 7, 3)])
+def test_waves_that_share_a_walk(H, N, P, count, rule):
+    """Several requests at once, at the numbers of workgroups up to which four waves share a column group's walk and just
+    beyond: batches of 16 and of 8 that end early, a request without tokens, the same bits as each request alone."""
+    g = torch.Generator(device=DEV).manual_seed(N + P + H)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    lens = [33, 0, 16, 47][:count]
+    T, wide = sum(lens), H if rule == "delta_head" else H * N
+    q, k, v, raw, beta = (rnd(T, n).to(torch.bfloat16) for n in (H * N, H * N, H * P, wide, H))
+    kw = dict(base=rnd(wide) - 1)
+    kw.update(dict(bonus=rnd(wide)) if rule == "bonus" else dict(rate=rnd(H).abs() + 0.1))
+    if rule.startswith("delta"):
+        kw.update(unit_eps=1e-6, q_scale=N ** -0.5)
+    start = rnd(count, H * N * P)
+
+    def run(lo, hi, which, lens, state):
+        more = dict(kw, beta=beta[lo:hi]) if rule.startswith("delta") else kw
+        cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+        return hip().decay_rows_recurrence(q[lo:hi], k[lo:hi], v[lo:hi], raw[lo:hi], state, torch.tensor(which, dtype=torch.int32, device=DEV), cu,
+                                           lens, H, H, N, P, rule, **more)
+
+    together = start.clone()
+    y = run(0, T, list(range(count)), lens, together)
+    cpu = lambda t: t.cpu() if torch.is_tensor(t) else t
+    want = start.cpu().clone()
+    close(y, twin.decay_rows_recurrence(*(t.cpu() for t in (q, k, v, raw)), want, torch.arange(count), torch.tensor([0] + lens).cumsum(0), lens, H, H, N, P, rule,
+                                        **{n: cpu(t) for n, t in dict(kw, **(dict(beta=beta) if rule.startswith("delta") else {})).items()}), 2e-5)
+    close(together, want, 2e-5)
+    lo = 0
+    for i, n in enumerate(lens):
+        if n:
+            state = start.clone()
+            assert torch.equal(run(lo, lo + n, [i], [n], state), y[lo:lo + n]) and torch.equal(state[i], together[i])
+        lo += n
