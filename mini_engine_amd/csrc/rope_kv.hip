@@ -233,7 +233,7 @@ qk_norm_rope_store_vec_kernel(T* __restrict__ qkv, int64_t row_stride, const flo
 
 // ------------------------------------------------------------------ many tokens: 8 tokens per workgroup
 // The same arithmetic for steps with many tokens (prefill). Grid (groups of 8 consecutive tokens,
-// q/k workgroups + one value workgroup). q and k heads: LPH = D/16 lanes share a head, a lane reads 8 values of each
+// q/k workgroups + value workgroups of v_heads heads each). q and k heads: LPH = D/16 lanes share a head, a lane reads 8 values of each
 // half (16 bytes), their 8 (cos, sin), and writes both back. Value heads: a thread takes 8 channels
 // of a head, reads them for 8 tokens, transposes the 8x8 block in registers and writes one
 // 16-byte piece per channel into the transposed page (for 8 tokens whose slots are consecutive places of
@@ -247,7 +247,7 @@ qk_norm_rope_store_tile_kernel(bf16_t* __restrict__ qkv, int64_t row_stride, con
                                const float* __restrict__ k_w, float eps, const float* __restrict__ table,
                                const int32_t* __restrict__ positions, const int32_t* __restrict__ slots,
                                bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache, int Hq, int Hkv, int D,
-                               int page, int store, int v_head, int64_t num_tokens, int qk_groups) {
+                               int page, int store, int v_head, int64_t num_tokens, int qk_groups, int v_heads) {
   const int64_t t0 = (int64_t)blockIdx.x * 8;
   const int cnt = (int)min((int64_t)8, num_tokens - t0);
   const int half = D >> 1;
@@ -320,7 +320,7 @@ qk_norm_rope_store_tile_kernel(bf16_t* __restrict__ qkv, int64_t row_stride, con
     *reinterpret_cast<bf16x8r*>(dst + half + 8 * l) = o2;
     return;
   }
-  // ---- value heads: the last workgroup of the 8 tokens
+  // ---- value heads: the last workgroups of the 8 tokens, v_heads heads each
   // The values go into the transposed page [channel][place]. Eight tokens whose slots are the eight places of an
   // aligned group (consecutive, the first a multiple of 8) are written as one 16-byte piece per channel. Which rows
   // of the batch form such a group has nothing to do with where the workgroups' rows begin (decode rows stand in
@@ -347,12 +347,13 @@ qk_norm_rope_store_tile_kernel(bf16_t* __restrict__ qkv, int64_t row_stride, con
     ++groups;
   }
   __syncthreads();
-  const int units = Hkv * dvecs;
+  const int first_head = ((int)blockIdx.y - qk_groups) * v_heads;
+  const int units = min(v_heads, Hkv - first_head) * dvecs;
   for (int u = threadIdx.x; u < groups * units; u += 256) {
     const int group = u / units, unit = u - group * units;
     const int s0 = group_slot[group], n = group_len[group];
     const int64_t pg = s0 / page, off = s0 - pg * page;               // page % 8 == 0: a group lies within one page
-    const int kvh = unit / dvecs, dv = unit - kvh * dvecs;
+    const int in_group = unit / dvecs, dv = unit - in_group * dvecs, kvh = first_head + in_group;
     const bf16_t* src = qkv + (t0 + group_row[group]) * row_stride + (int64_t)(v_head + kvh) * D + 8 * dv;
     bf16_t* dst = v_cache + ((pg * Hkv + kvh) * (int64_t)D + 8 * dv) * page + off;
     u32x4r tok[8];
@@ -419,11 +420,16 @@ extern "C" int me_qk_norm_rope_store(void* qkv, int dtype, int64_t num_tokens, i
   if (tile) {
     const int per_group = 256 / lph16;
     const int qk_groups = (8 * (Hq + Hkv) + per_group - 1) / per_group;
-    dim3 grid((unsigned)((num_tokens + 7) / 8), qk_groups + (store ? 1 : 0)), block(256);
+    // The value heads of eight tokens go to four workgroups. Rows whose slots stand alone (decoding requests beside a prompt) are
+    // written in pieces of 2 bytes, a line each, 8,192 of them for eight rows of 8 heads of 128; a workgroup that had all of
+    // them was what its launch waited for (us, one workgroup / four, 8.3 being the least that this way of timing shows: 489
+    // tokens beside 23 such rows 10.5 / 8.3, 1,500 beside 8 12.5 / 8.7, 2,000 beside 60 14.8 / 12.3, 4,096 alone 17.6 / 17.0).
+    const int v_heads = Hkv > 4 ? (Hkv + 3) / 4 : 1;
+    dim3 grid((unsigned)((num_tokens + 7) / 8), qk_groups + (store ? (Hkv + v_heads - 1) / v_heads : 0)), block(256);
 #define LAUNCH_TILE(L)                                                                                     \
   qk_norm_rope_store_tile_kernel<L><<<grid, block, 0, stream>>>((bf16_t*)qkv, row_stride, q_w, k_w, eps, table, \
                                                                 positions, slots, (bf16_t*)k_cache,       \
-                                                                (bf16_t*)v_cache, Hq, Hkv, D, page, store, v_head, num_tokens, qk_groups)
+                                                                (bf16_t*)v_cache, Hq, Hkv, D, page, store, v_head, num_tokens, qk_groups, v_heads)
     switch (lph16) {
       case 1: LAUNCH_TILE(1); break; case 2: LAUNCH_TILE(2); break; case 4: LAUNCH_TILE(4); break;
       case 8: LAUNCH_TILE(8); break; case 16: LAUNCH_TILE(16); break; case 32: LAUNCH_TILE(32); break;

@@ -878,3 +878,28 @@ def test_kernels_refuse_what_they_cannot_do():
         hip().qk_norm_rope_store(torch.zeros(1, 3 * 600, device=DEV), None, None, 0.0, None,
                                  torch.zeros(1, device=DEV, dtype=torch.int32), torch.zeros(1, device=DEV, dtype=torch.int32),
                                  torch.zeros(1, 1, 4, 600, device=DEV), torch.zeros(1, 1, 600, 4, device=DEV), 1, 1, 600, 4, True)
+
+
+@pytest.mark.parametrize("Hkv", [1, 3, 4, 5, 8])
+def test_cache_write_of_lone_rows_beside_whole_groups_by_any_number_of_heads(Hkv):
+    """Decoding rows (slots that stand alone) in front of a prompt's rows, whole groups of eight and a last one that is cut: the
+    value heads are dealt to workgroups by heads, also where their number does not come out even."""
+    Hq, D, page, dec, toks = 2 * Hkv, 64, 16, 11, 133
+    g = torch.Generator(device=DEV).manual_seed(Hkv)
+    T, pages = dec + toks, dec + toks // page + 2
+    qkv = torch.randn(T, (Hq + 2 * Hkv) * D, device=DEV, generator=g).bfloat16()
+    w, table = torch.rand(D, device=DEV, generator=g) + 0.5, torch.randn(512, D // 2, 2, device=DEV, generator=g)
+    positions = torch.cat((torch.arange(dec) * 7, torch.arange(toks) + 3)).int().to(DEV)
+    slots = torch.cat((torch.arange(dec) * page + 5, dec * page + 3 + torch.arange(toks))).int().to(DEV)
+    got = [t.clone() for t in (qkv, torch.zeros(pages, Hkv, page, D, device=DEV).bfloat16(), torch.zeros(pages, Hkv, D, page, device=DEV).bfloat16())]
+    hip().qk_norm_rope_store(got[0], w, w, 1e-6, table, positions, slots, got[1], got[2], Hq, Hkv, D, page)
+    values = qkv[:, (Hq + Hkv) * D:].view(T, Hkv, D)
+    want = torch.zeros_like(got[2])
+    for t, s in enumerate(slots.tolist()):
+        want[s // page, :, :, s % page] = values[t]
+    assert torch.equal(got[2], want)
+    one = [qkv.clone(), torch.zeros_like(got[1]), torch.zeros_like(got[2])]          # a workgroup per token: the same bits
+    for lo in range(0, T, 100):
+        hip().qk_norm_rope_store(one[0][lo:lo + 100], w, w, 1e-6, table, positions[lo:lo + 100].contiguous(), slots[lo:lo + 100].contiguous(),
+                                 one[1], one[2], Hq, Hkv, D, page)
+    assert all(torch.equal(a, b) for a, b in zip(got, one))
