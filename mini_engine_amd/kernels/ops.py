@@ -257,7 +257,7 @@ def _tile_product(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, slices: int
     M, K = x.shape
     N = w.shape[0]
     core().call("me_gemm_tile_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), y.shape[-1], _code(y.dtype), slices,
-                M, N, K, gated, *form, _ptr(bias), *tile_choice(M, N, K, slices)[0], _stream())
+                M, N, K, gated, *form, _ptr(bias), *tile_choice(M, N, K, slices, gated > 0)[0], _stream())
     return y
 
 
@@ -1634,6 +1634,11 @@ TILE_COST = {(256, 256): (0.0, 10.6, 1.02, 1.02, 1), (256, 192): (0.0, 9.5, 0.91
              (128, 256): (0.0, 6.2, 0.75, 0.75, 1), (256, 128): (0.0, 6.6, 0.70, 0.70, 1), (128, 192): (0.0, 5.6, 0.74, 0.61, 2),
              (128, 128): (0.0, 4.0, 0.48, 0.44, 2), (64, 128): (0.5, 2.4, 0.37, 0.30, 3), (128, 64): (1.5, 1.6, 0.35, 0.31, 3),
              (64, 64): (2.1, 0.8, 0.29, 0.20, 5)}
+# ... and what is added to a workgroup's us to choose a tile for the gating: its exponentials and divisions cost the wide tiles 5-7 us
+# a workgroup (a compute unit has one of them, and two waves to a SIMD), while workgroups that share a unit hide them.
+# Fitted to 900 times over five gate/up weights, 40 to 6,000 rows.
+TILE_GATING = {(256, 256): -0.8, (256, 192): 0.9, (192, 256): 1.0, (128, 256): 1.2, (256, 128): -0.4, (128, 192): -0.1,
+               (128, 128): -1.5, (64, 128): -1.3, (128, 64): -1.3, (64, 64): -1.4}
 TILE_MIN_ROWS = 33
 TILE_SURE_K = 2048
 TILE_MIN_TFLOPS = 1000
@@ -1641,12 +1646,16 @@ TILE_SLICES_MAX_M = 256
 
 
 @lru_cache(maxsize=4096)      # asked once per product of a step: ten tiles each time
-def tile_choice(M: int, N: int, K: int, slices: int = 1) -> tuple:
+def tile_choice(M: int, N: int, K: int, slices: int = 1, gated: bool = False) -> tuple:
     """((rows, features) of the tile that csrc/gemm_tile.hip takes for M rows against a weight [N, K] in `slices` slices of
     K, the us that `TILE_COST` expects of it): the tile whose busiest compute unit is done first. Over the products that
-    the costs were fitted to it is 0.7 % behind the fastest tile on average with one result (11 % at worst), 2 % with slices."""
+    the costs were fitted to it is 0.7 % behind the fastest tile on average with one result (11 % at worst), 2 % with slices, 0.8 %
+    with the gating (2.8 %, 19 % at worst, without `TILE_GATING`: 512 rows of 6144 x 1024 13.8 -> 11.6 us, 256 of 19456 x 2560
+    49.6 -> 43.2)."""
     def cost(tile):
         launch, each, alone, shared, fit = TILE_COST[tile]
+        if gated:
+            each += TILE_GATING[tile]
         busiest = -(-(-(-M // tile[0]) * -(-N // tile[1])) * slices // _COMPUTE_UNITS)
         return launch + each * busiest + -(-(K // 64) // slices) * max(alone * -(-busiest // fit), shared * busiest)
     best = min(TILE_COST, key=cost)
