@@ -486,13 +486,20 @@ struct RecArgs {
 // HPB heads and PPB blocks of 64 columns per wave; CL = HPB * PPB columns per lane. KEYS: the waves of the first column
 // block also keep the summed keys of their NT rows, one row per lane; a batch's products with q meet in LDS, where eight
 // lanes add up a token's (HPB 1 only).
+// What bounds it: one or two waves to a SIMD, which issue an instruction every 8-9 cycles and wait for whatever they read too
+// late. Hence a batch is asked for as it lies in memory and converted a batch later, four tokens are one piece without a branch,
+// and rows of k and q come from LDS two pieces of eight rows ahead. us, converted at the fetch and read where used / this: 16
+// heads of 128 x 128, one request of 60 tokens 84 / 39, of 350 138 / 86, of 2,048 190 / 166, 16 of 700 855 / 692; 32 heads of
+// 128 x 64 with step sizes 81 / 36, 131 / 80, 177 / 149, 785 / 600; 301 requests, one of 300 tokens and the rest of one, 776 / 760.
+// Only the 48-row form loses where no request has more than three tokens (4 heads of 48 x 100, eight requests 14.6 / 18.5; one
+// of 60 tokens 74 / 56); a branch behind a piece's first token does not bring it back.
 template <typename TX, int NT, int PASS, int HPB, int PPB, bool KEYS>
 __global__ void __launch_bounds__(64) recurrence_kernel(RecArgs a) {
   static_assert(!KEYS || HPB == 1, "summed keys: one head per wave");
   constexpr int CL = HPB * PPB;
   constexpr int KR = REC_TB * NT / 64;               // k (and q) values a lane carries to LDS per batch of tokens
   using Cell = std::conditional_t<PASS == 1, float, float2>;       // the first pass of spans reads no q
-  __shared__ Cell skq[REC_TB][NT];
+  __shared__ __align__(16) Cell skq[REC_TB][NT];
   __shared__ float sa[HPB][REC_TB], sb[HPB][REC_TB];
   __shared__ float nd[KEYS && PASS != 1 ? REC_TB : 1][KEYS && PASS != 1 ? NT : 1];
   const bool keys = KEYS && blockIdx.y == 0;
@@ -524,52 +531,39 @@ __global__ void __launch_bounds__(64) recurrence_kernel(RecArgs a) {
   const TX* kp = (const TX*)a.k + (int64_t)g * a.N + n0;
   const bool silu = a.silu != 0;
 
-  // what a lane fetches for a batch of tokens
-  float kreg[KR], qreg[KR], vreg[CL][REC_TB], areg = 1.f, breg = 0.f;
+  // what a lane asks for for a batch of tokens, as it lies in memory: conversions and selects come when the batch is taken
+  // (on what has just been asked for they would wait for it)
+  TX kraw[KR], qraw[KR], vraw[CL][REC_TB], draw = (TX)0.f;
+  float araw = 1.f, braw = 0.f;
   // every load is unconditional, from an address clamped into the span and the slice; what lies outside becomes zero
   // afterwards (a load behind a branch would make the wave wait for each one before it asks for the next)
   const int n_last = a.N - 1 - n0;
+  const int my_sub = lane < HPB * REC_TB ? lane : 0, my_head = h0 + my_sub / REC_TB, my_tt = my_sub % REC_TB;
   auto fetch = [&](int64_t tb) {
     const int nt = (int)(t1 - tb < REC_TB ? t1 - tb : REC_TB);
 #pragma unroll
     for (int r = 0; r < KR; ++r) {
       const int i = lane + r * 64, tt = i / NT, nn = i - tt * NT;
-      const bool have = tt < nt && nn <= n_last;
       const int64_t at = tb + (tt < nt ? tt : nt - 1);
       const int col = nn <= n_last ? nn : n_last;
-      const float kk = to_f32<TX>(kp[at * a.k_stride + col]);
-      kreg[r] = have ? kk : 0.f;
-      if (PASS != 1) {
-        const float qq = to_f32<TX>(qp[at * a.q_stride + col]);
-        qreg[r] = have ? qq : 0.f;
-      }
+      kraw[r] = kp[at * a.k_stride + col];
+      if (PASS != 1) qraw[r] = qp[at * a.q_stride + col];
     }
 #pragma unroll
     for (int j = 0; j < CL; ++j)
 #pragma unroll
-      for (int tt = 0; tt < REC_TB; ++tt) {
-        const float x = to_f32<TX>(((const TX*)a.v)[(tb + (tt < nt ? tt : nt - 1)) * a.v_stride + (int64_t)head[j] * a.P + p[j]]);
-        vreg[j][tt] = (tt < nt && on[j]) ? x : 0.f;
-      }
-    {
-      const int sub = lane < HPB * REC_TB ? lane : 0;
-      const int hh = h0 + sub / REC_TB, tt = sub % REC_TB;
-      const int64_t at = tb + (tt < nt ? tt : nt - 1);
-      if (a.dt) {
-        const float z = to_f32<TX>(((const TX*)a.dt)[at * a.dt_stride + hh]) + a.dt_bias[hh];
-        const float step = z > 20.f ? z : log1pf(expf(z));
-        areg = expf(-a.rate[hh] * step);
-        breg = step;
-      } else if (a.coef_a) {
-        areg = a.coef_a[at * a.H + hh];
-        breg = a.coef_b[at * a.H + hh];
-      } else {
-        areg = a.decay[hh];
-        breg = 1.f;
-      }
-      if (tt >= nt) { areg = 1.f; breg = 0.f; }
+      for (int tt = 0; tt < REC_TB; ++tt)
+        vraw[j][tt] = ((const TX*)a.v)[(tb + (tt < nt ? tt : nt - 1)) * a.v_stride + (int64_t)head[j] * a.P + p[j]];
+    const int64_t at = tb + (my_tt < nt ? my_tt : nt - 1);
+    if (a.dt) {
+      draw = ((const TX*)a.dt)[at * a.dt_stride + my_head];
+    } else if (a.coef_a) {
+      araw = a.coef_a[at * a.H + my_head];
+      braw = a.coef_b[at * a.H + my_head];
     }
   };
+  const float my_bias = a.dt ? a.dt_bias[my_head] : 0.f, my_rate = a.dt ? a.rate[my_head] : 0.f;
+  const float my_decay = a.dt || a.coef_a ? 1.f : a.decay[my_head];
 
   fetch(t0);
   float S[CL][NT];
@@ -614,54 +608,105 @@ __global__ void __launch_bounds__(64) recurrence_kernel(RecArgs a) {
 #pragma unroll
     for (int r = 0; r < KR; ++r) {
       const int i = lane + r * 64, tt = i / NT, nn = i - tt * NT;
-      float kk = kreg[r], qq = PASS != 1 ? qreg[r] : 0.f;
+      const bool have = tt < nt && nn <= n_last;
+      float kk = have ? to_f32<TX>(kraw[r]) : 0.f, qq = PASS != 1 && have ? to_f32<TX>(qraw[r]) : 0.f;
       if (silu) { kk = silu_f(kk); qq = silu_f(qq); }
       if constexpr (PASS == 1) skq[tt][nn] = kk;
       else skq[tt][nn] = make_float2(kk, qq);
     }
+    float areg = my_decay, breg = 1.f;
+    if (a.dt) {
+      const float z = to_f32<TX>(draw) + my_bias;
+      const float step = z > 20.f ? z : log1pf(expf(z));
+      areg = expf(-my_rate * step);
+      breg = step;
+    } else if (a.coef_a) {
+      areg = araw;
+      breg = braw;
+    }
+    if (my_tt >= nt) { areg = 1.f; breg = 0.f; }      // tokens beyond the span leave the state as it is
     if (lane < HPB * REC_TB) { sa[lane / REC_TB][lane % REC_TB] = areg; sb[lane / REC_TB][lane % REC_TB] = breg; }
 #pragma unroll
     for (int j = 0; j < CL; ++j)
 #pragma unroll
-      for (int tt = 0; tt < REC_TB; ++tt) vv[j][tt] = silu ? silu_f(vreg[j][tt]) : vreg[j][tt];
+      for (int tt = 0; tt < REC_TB; ++tt) {
+        const float x = tt < nt && on[j] ? to_f32<TX>(vraw[j][tt]) : 0.f;
+        vv[j][tt] = silu ? silu_f(x) : x;
+      }
+    asm volatile("" ::: "memory");
     if (tb + REC_TB < t1) fetch(tb + REC_TB);         // the next batch travels while this one is computed
     __syncthreads();
+    // Four tokens are one piece of code without a branch, and their rows of k and q are read from LDS in pieces of eight rows,
+    // two pieces ahead: read where they are used, every pair of rows waited for LDS (1.4 us a token of 32 rows).
+    constexpr int PART = 4, CH = 8, PER = NT / CH, AHEAD = 2, CELLS = (int)sizeof(Cell) * CH / 16;
+    static_assert(NT % CH == 0 && REC_TB % PART == 0, "whole pieces");
 #pragma unroll
-    for (int tt = 0; tt < REC_TB; ++tt) {
-      if (tt >= nt) break;
-      float da[CL], bv[CL], acc[CL];
+    for (int part = 0; part < REC_TB; part += PART) {
+      if (part >= nt) break;
+      f32x4 ring[AHEAD + 1][CELLS];
+      auto read = [&](int c) {
+        const f32x4* from = reinterpret_cast<const f32x4*>(&skq[part + c / PER][c % PER * CH]);
 #pragma unroll
-      for (int j = 0; j < CL; ++j) {
-        const int hj = HPB == 2 ? j : 0;
-        da[j] = sa[hj][tt];
-        bv[j] = sb[hj][tt] * vv[j][tt];
-        acc[j] = 0.f;
-      }
+        for (int e = 0; e < CELLS; ++e) ring[c % (AHEAD + 1)][e] = from[e];
+      };
+      float out[CL][PART];
 #pragma unroll
-      for (int i = 0; i < NT; ++i) {
-        if constexpr (PASS == 1) {
-          const float kk = skq[tt][i];
+      for (int c = 0; c < AHEAD; ++c) read(c);
 #pragma unroll
-          for (int j = 0; j < CL; ++j) S[j][i] = da[j] * S[j][i] + kk * bv[j];
-        } else {
-          const float2 kq = skq[tt][i];
+      for (int u = 0; u < PART; ++u) {
+        const int tt = part + u;
+        float da[CL], bv[CL], acc[CL];
 #pragma unroll
-          for (int j = 0; j < CL; ++j) {
-            S[j][i] = da[j] * S[j][i] + kq.x * bv[j];
-            acc[j] += S[j][i] * kq.y;
+        for (int j = 0; j < CL; ++j) {
+          const int hj = HPB == 2 ? j : 0;
+          da[j] = sa[hj][tt];
+          bv[j] = sb[hj][tt] * vv[j][tt];
+          acc[j] = 0.f;
+        }
+#pragma unroll
+        for (int piece = 0; piece < PER; ++piece) {
+          const int c = u * PER + piece;
+          asm volatile("" ::: "memory");
+          if (c + AHEAD < PART * PER) read(c + AHEAD);
+          asm volatile("" ::: "memory");
+#pragma unroll
+          for (int r = 0; r < CH; ++r) {
+            const int i = piece * CH + r;
+            if constexpr (PASS == 1) {
+              const float kk = ring[c % (AHEAD + 1)][r / 4][r % 4];
+#pragma unroll
+              for (int j = 0; j < CL; ++j) S[j][i] = da[j] * S[j][i] + kk * bv[j];
+            } else {
+              const float kx = ring[c % (AHEAD + 1)][r / 2][2 * (r % 2)], ky = ring[c % (AHEAD + 1)][r / 2][2 * (r % 2) + 1];
+#pragma unroll
+              for (int j = 0; j < CL; ++j) {
+                S[j][i] = da[j] * S[j][i] + kx * bv[j];
+                acc[j] += S[j][i] * ky;
+              }
+            }
           }
+          __builtin_amdgcn_sched_barrier(0);          // else all pieces are read first, and their registers leave one wave to a SIMD
+        }
+        if (PASS == 1) {
+#pragma unroll
+          for (int j = 0; j < HPB; ++j) total_decay[j] *= sa[j][tt];
+        }
+#pragma unroll
+        for (int j = 0; j < CL; ++j) {
+          if (PASS != 1) asm volatile("" : "+v"(acc[j]));      // else the sum is formed where it is stored, and all of q stays until then
+          out[j][u] = acc[j];
         }
       }
-      if (PASS == 1) {
-#pragma unroll
-        for (int j = 0; j < HPB; ++j) total_decay[j] *= sa[j][tt];
-      } else {
+      if (PASS != 1) {
 #pragma unroll
         for (int j = 0; j < CL; ++j)
-          if (on[j]) {
-            if (slice == 0) acc[j] += skip[j] * vv[j][tt];
-            a.y[slice * a.y_slice_stride + (tb + tt) * ((int64_t)a.H * a.P) + (int64_t)head[j] * a.P + p[j]] = acc[j];
-          }
+          if (on[j])
+#pragma unroll
+            for (int u = 0; u < PART; ++u)
+              if (part + u < nt) {
+                if (slice == 0) out[j][u] += skip[j] * vv[j][part + u];
+                a.y[slice * a.y_slice_stride + (tb + part + u) * ((int64_t)a.H * a.P) + (int64_t)head[j] * a.P + p[j]] = out[j][u];
+              }
       }
     }
     if (KEYS && keys) {

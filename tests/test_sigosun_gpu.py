@@ -166,6 +166,37 @@ def test_linear_recurrence(monkeypatch, dtype, H, G, N, P, selective, columns):
     assert torch.equal(st5[3], full[3]) and torch.equal(st5[:, :3], full[:, :3])
 
 
+@pytest.mark.parametrize("columns", [1, 2])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,N,P", [(2, 16, 20), (2, 32, 64), (2, 48, 100), (2, 64, 65), (2, 128, 128)])
+def test_recurrence_in_pieces_of_four_tokens(monkeypatch, dtype, H, N, P, columns):
+    """Requests that end at, before and behind the kernel's pieces of four and batches of eight tokens, and one that is cut
+    into spans, against the token-by-token twin (2e-5: the inputs are exact in both, up to 133 float32 sums in another order);
+    a request of NaNs between them stays alone, as does the state of a slot that no request names."""
+    monkeypatch.setattr(ops, "RECURRENCE_COLUMNS", columns)
+    torch.manual_seed(N + P)
+    q_lens = [1, 2, 3, 4, 5, 6, 7, 8, 9, 11, 12, 13, 16, 133]
+    cu, seq, slots = _steps_meta(q_lens, [14, 0, 4, 1, 3, 2, 9, 8, 7, 6, 13, 11, 12, 10])
+    T, bad = sum(q_lens), 4
+    rows = torch.randn(T, 2 * H * N + H * P, device=DEV).to(dtype)
+    rows[int(cu[bad]):int(cu[bad + 1])] = float("nan")
+    q, k, v = rows[:, :H * N], rows[:, H * N:2 * H * N], rows[:, 2 * H * N:]
+    kw = dict(decay=torch.tensor([0.9, 0.99], device=DEV), skip=torch.randn(H, device=DEV))
+    full = torch.randn(15, H * N * P, device=DEV)
+    st_h, st_c = full.clone(), full.cpu().clone()
+    y = hip().linear_recurrence(q, k, v, st_h, slots, cu, q_lens, H, H, N, P, **kw)
+    y = (y.sum(0) if y.dim() == 3 else y).cpu()
+    want = twin.linear_recurrence(q.cpu(), k.cpu(), v.cpu(), st_c, slots.cpu(), cu.cpu(), q_lens, H, H, N, P, **{n: t.cpu() for n, t in kw.items()})
+    of_bad = torch.arange(int(cu[bad]), int(cu[bad + 1]))
+    assert bool(y[of_bad].isnan().all()) and bool(st_h[3].isnan().all())
+    good = torch.ones(T, dtype=torch.bool)
+    good[of_bad] = False
+    close(y[good], want[good], 2e-5)
+    others = [s for s in range(15) if s != 3]
+    close(st_h[others], st_c[others], 2e-5)
+    assert torch.equal(st_h[5], full[5])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("kind,groups,parts", [("silu_before", 1, 1), ("silu_before", 4, 2), ("sigmoid_behind", 1, 3)])
 def test_gated_rms_norm(dtype, kind, groups, parts):
