@@ -12,8 +12,8 @@
 // as B: a lane then holds 4 consecutive features of one token. K may be split over workgroups (grid z): float32
 // partial sums [S, M, N] for a consumer that adds them. Workgroups that share weight rows run on the same XCD.
 // An iteration is a chain of wait, barrier, LDS reads and 8 products (about 500 cycles for 128 cycles of matrix
-// work), so the kernel takes 7 us whatever the row count up to 256 and loses to the library's larger tiles
-// beyond; the caller (ops.mid_takes) knows where it is ahead. Where K is a multiple of 128 an iteration walks 128 of
+// work), so the kernel takes 7 us whatever the row count up to 256 and loses to larger tiles (csrc/gemm_tile.hip, the
+// library) beyond; the callers (ops.mid_takes, ops.mid_crowded) know where it is ahead. Where K is a multiple of 128 an iteration walks 128 of
 // K instead (BK = 128: rows of 256 bytes, 16 pieces, piece c of row R at position c ^ (R & 15); 96 KB of LDS for
 // the three stages): half as many iterations, each with 16 products behind the same wait and barrier.
 #include "common.h"

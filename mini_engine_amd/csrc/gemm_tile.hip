@@ -17,9 +17,11 @@
 // What bounds it: the matrix pipes at the clock that a full chip keeps for tiles of 256 x 256 (8,192 x 8,192 x 8,192: 1,554
 // TFLOP/s, the library's kernel 1,307); the reads of LDS for the others, whose waves have fewer products for an operand read
 // (256 x 128: 176 KB of LDS traffic a step at 128 bytes a cycle is 0.6 us, which is what a step takes; 128 x 128 96 KB, 0.33
-// of 0.44 us). us, the library / this: 2,048 rows of 24576 x 4096 362 / 290 (with the gating 281, and no kernel of 28 us
-// behind it), of 6144 x 4096 90 / 78, of 4096 x 4096 57 / 56, of 4096 x 12288 168 / 158, of 6144 x 1024 26.2 / 24.8 (with the
-// gating 23.4), of 1024 x 2048 15.3 / 13.3; 512 rows of 4096 x 1024 11.2 / 8.6, of 6144 x 1024 with the gating 13.3 + 4.4 / 10.6.
+// of 0.44 us). us, the library / this: 2,048 rows of 24576 x 4096 362 / 290 (with the gating 362 + 28 of a kernel behind
+// it / 307), of 6144 x 4096 90 / 78, of 4096 x 4096 57 / 56, of 4096 x 12288 168 / 158, of 6144 x 1024 26.2 / 24.8 (with the
+// gating 30.5), of 1024 x 2048 15.3 / 13.3; 512 rows of 4096 x 1024 11.2 / 8.6, of 6144 x 1024 with the gating 13.3 + 4.4 / 11.6.
+// Sums that are rounded before the gating, with the library's exponential, cost a tile 1-3 us more than unrounded ones would
+// (281 and 23.4): the bits stay those of the product and the gating kernel.
 //
 // Outputs in bfloat16 are written 16 bytes a lane, 64 contiguous bytes of a row by four lanes: within a wave's half of the
 // features the weight rows are laid into LDS so that two matrix results of a lane are 8 consecutive features (8-byte stores

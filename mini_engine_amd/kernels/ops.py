@@ -582,14 +582,16 @@ class HipBackend:
         """x [M, K] . w[N, K]^T (reference layers/linear.py:25-26: F.linear, no bias).
 
         float32: the float32 matrix instructions (f32_tile). bfloat16: the skinny MFMA kernel for up to 32 rows (64 for
-        smaller weights or when K is split), the library product (hipBLASLt, library_product) above
-        that, for the head over a large vocabulary and for large weights with several rows
+        smaller weights or when K is split), the tiled kernel up to 256 rows over small weights (mid_takes), the kernel of
+        large tiles for more rows (tile_takes, mid_crowded), the library product (hipBLASLt, library_product) for what is
+        left of them, for the head over a large vocabulary and for large weights with several rows
         (library_streams_better), the FMA kernel for shapes the MFMA kernel refuses.
         With allow_partials the result may be float32 partial sums [S, M, N] over slices of K for a
         consumer that adds them: from the skinny kernel when the output features are few
         (choose_ksplit), from the rows kernel for 17-32 rows over large weights (rows_takes), from the tiled
-        kernel for 33 to a few hundred rows over weights up to 27 M elements (mid_slices), from the
-        library as a strided batch for 33-1,024 rows over larger weights (library_splits).
+        kernel for 33 to a few hundred rows over weights up to 27 M elements (mid_slices; large tiles where mid_crowded),
+        from large tiles up to 256 rows and from the library as a strided batch up to 1,024 over larger weights
+        (library_splits).
         `out` (not with allow_partials): a contiguous [M, N] tensor of the output dtype to write into."""
         _check(x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1], f"linear: {tuple(x.shape)} x {tuple(w.shape)}^T")
         _check(x.dtype == w.dtype, f"linear: activation {x.dtype} and weight {w.dtype} differ")
@@ -663,8 +665,9 @@ class HipBackend:
         """silu(x . w[:I]^T) * (x . w[I:]^T) for a packed gate/up weight w [2 I, K] (gate rows first), as one
         launch: the product's workgroups pair each gate feature with its up feature when they merge their waves,
         from the unrounded sums (the separate kernels round the product to bfloat16 first; so does the kernel for many
-        rows, `gated_linear_tiles`). For the row counts `gated_linear_fuses` admits. `bias` (float32 [2 I]) joins the sums first; `clamp` (limit, alpha): the form of
-        `glu_clamped` in place of silu(gate) * up. Returns [M, I]. (reference layers/linear.py:29-45, layers/activation.py:5-7.)"""
+        rows, `gated_linear_tiles`). For the row counts `gated_linear_fuses` admits. `bias` (float32 [2 I]) joins the sums
+        first; `clamp` (limit, alpha): the form of `glu_clamped` in place of silu(gate) * up. Returns [M, I].
+        (reference layers/linear.py:29-45, layers/activation.py:5-7.)"""
         _check(gated_linear_fuses(x, w), "gated_linear: bfloat16, few rows, see gated_linear_fuses")
         M, K = x.shape
         N = w.shape[0]
@@ -1694,8 +1697,7 @@ def mid_crowded(M: int, N: int, slices: int) -> bool:
 def gated_linear_tiles(rows: int, w: torch.Tensor) -> bool:
     """Whether `rows` rows against the packed gate/up weight w [2 I, K] go through csrc/gemm_tile.hip with the gating in its
     epilogue: from 33 rows on, where no kernel for few rows has the product. Against the library's product and a gating kernel
-    behind it (78 products of 40 to 8,192 rows over the gate/up weights of 0.6B to 32B) 0.97 to 2 times as fast, 1.28 on
-    average: 512 rows of 6144 x 1024 17.7 -> 10.6 us, 2,048 rows of 24576 x 4096 390 -> 281."""
+    behind it: 512 rows of 6144 x 1024 17.7 -> 11.6 us, 2,048 rows of 24576 x 4096 390 -> 307."""
     if not FUSE_GATE_INTO_GATE_UP or rows < TILE_MIN_ROWS or w.dtype != torch.bfloat16 or w.dim() != 2 or w.stride(1) != 1:
         return False
     N, K = w.shape
