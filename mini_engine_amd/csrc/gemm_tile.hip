@@ -39,8 +39,8 @@ __device__ __forceinline__ void tile_dma16(const bf16_t* gbase, uint32_t voff, u
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(base) : "memory");
 }
 template <int N> __device__ __forceinline__ void tile_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-// Nothing crosses it in either direction, matrix instructions included: a quarter's reads are waited for in front of its
-// products, so a wave that has passed the barrier behind them has its operands in registers.
+__device__ __forceinline__ void tile_wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+// Nothing crosses it in either direction, matrix instructions included.
 __device__ __forceinline__ void tile_barrier() {
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("s_barrier" ::: "memory");
@@ -178,11 +178,15 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __rest
         for (int j = 0; j < MH; ++j)
           acc[hw * NH + i][hx * MH + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[hw][i][s], fx[j][s], acc[hw * NH + i][hx * MH + j], 0, 0, 0);
     __builtin_amdgcn_s_setprio(0);
+    tile_wait_lds();
     tile_barrier();
   };
   // Why no wait is missing. A region is read in one quarter q by both halves of the waves; the half that runs late reads it
   // half a quarter after, and has it in registers before the barrier behind its products, which the other half passes at the
-  // end of its reads of quarter q + 1. The request that overwrites the region is made in quarter q + 2. What quarter q reads
+  // end of its reads of quarter q + 1. The request that overwrites the region is made in quarter q + 2. That holds for the operands
+  // of the quarter's own products and for those read a quarter ahead (features' first half, in quarter 3 and in front of the first
+  // step) because every barrier but the one between a quarter's reads and its products comes behind a wait for all reads of LDS;
+  // those read ahead have had the quarter's products to arrive. What quarter q reads
   // has been waited for by the wave that asked for it in quarter q - 1 before a barrier that every reader has passed.
   auto step = [&](int k, auto kind) {                                 // kind 0: two steps or more follow, 1: one, 2: none
     constexpr int KIND = decltype(kind)::value;
@@ -214,6 +218,7 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __rest
   wait(TILE_INT(REGION_W1), TILE_INT(5));
   tile_barrier();
   read_w(0, 0, fw[0]);
+  tile_wait_lds();
   if (PING && late) tile_barrier();
   int k = 0;
   for (; k < steps - 2; ++k) step(k, TILE_INT(0));

@@ -9,7 +9,8 @@ import pytest
 
 from mini_engine_amd.kernels import build
 
-READELF = shutil.which("llvm-readelf", path=os.pathsep.join(("/opt/rocm/llvm/bin", os.environ.get("PATH", ""))))
+_TOOLS = os.pathsep.join(("/opt/rocm/llvm/bin", os.environ.get("PATH", "")))
+READELF, OBJDUMP = (shutil.which(tool, path=_TOOLS) for tool in ("llvm-readelf", "llvm-objdump"))
 
 
 def _code_objects(blob: bytes):
@@ -49,3 +50,59 @@ def test_float32_attention_keeps_to_its_registers(tmp_path):
     assert sorted(seen) == list(range(16, 129, 16))
     for head, (scratch, registers) in seen.items():
         assert scratch == 0 and registers <= 256, (head, scratch, registers)
+
+
+def _reads_on_their_way(code: list) -> dict:
+    """The most LDS reads that can be on their way at each instruction, over all paths. `code`: (address, name, operands, the
+    address a branch goes to or None)."""
+    place = {address: i for i, (address, *_) in enumerate(code)}
+    most, todo = {0: 0}, [0]
+    while todo:
+        i = todo.pop()
+        _, name, operands, target = code[i]
+        n = most[i]
+        if name.startswith("ds_read"):
+            n = min(n + 1, 99)
+        elif name == "s_waitcnt":
+            m = re.search(r"lgkmcnt\((\d+)\)", operands)
+            n = min(n, int(m.group(1))) if m else n
+        after = [] if name == "s_endpgm" else [i + 1]
+        if target is not None:
+            after = [place[target]] + (after if name.startswith("s_cbranch") else [])
+        for j in after:
+            if j < len(code) and most.get(j, -1) < n:
+                most[j] = n
+                todo.append(j)
+    return most
+
+
+@pytest.mark.skipif(OBJDUMP is None, reason="no llvm-objdump")
+def test_tile_products_read_lds_before_others_may_write_it(tmp_path):
+    """Every barrier of the tile product's kernels but the one in front of a quarter's products, which raises the wave's priority
+    behind itself, has no LDS read on its way: what is read a quarter ahead is in registers before another wave can ask for
+    the load that writes over it."""
+    library = os.path.join(build.PKG_LIB, "libme_core.so")
+    if not os.path.exists(library):
+        pytest.skip("the core library is not built")
+    kernels = barriers = 0
+    for i, blob in enumerate(_code_objects(open(library, "rb").read())):
+        if b"gemm_tile_kernel" not in blob:
+            continue
+        path = tmp_path / f"{i}.elf"
+        path.write_bytes(blob)
+        text = subprocess.run([OBJDUMP, "-d", str(path)], capture_output=True, text=True, check=True).stdout
+        for part in re.split(r"^([0-9a-f]+) <(\S*gemm_tile_kernel\S*)>:$", text, flags=re.M)[1:][2::3]:
+            kernels += 1
+            code = []
+            for line in part.splitlines():
+                if m := re.match(r"\s+(\w+)(.*?)\s*// ([0-9A-F]+):.*?(?:<\S+?\+0x([0-9a-f]+)>)?$", line):
+                    code.append((int(m.group(3), 16), m.group(1), m.group(2), m.group(4)))
+            code = [(a, name, ops, code[0][0] + int(to, 16) if to and name.startswith(("s_branch", "s_cbranch")) else None) for a, name, ops, to in code]
+            most = _reads_on_their_way(code)
+            names = [name for _, name, _, _ in code]
+            for j in [j for j, name in enumerate(names) if name == "s_barrier"]:
+                if names[j + 1] == "s_setprio" and int(code[j + 1][2]) == 1:
+                    continue
+                barriers += 1
+                assert most[j] == 0, (kernels, hex(code[j][0]), most[j])
+    assert kernels == 30 and barriers >= kernels * 12        # 12 quarters in the code of a kernel
