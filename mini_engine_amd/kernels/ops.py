@@ -626,7 +626,7 @@ class HipBackend:
             return parts
         splits = library_splits(M, N, K) if (allow_partials and out_dtype == x.dtype) else 1
         if splits > 1:
-            if M <= TILE_SLICES_MAX_M and tile_fits(x, w, splits):
+            if M <= TILE_SLICES_MAX_M and K <= TILE_SLICES_MAX_K and tile_fits(x, w, splits):
                 return _tile_product(x, w, torch.empty((splits, M, N), dtype=torch.float32, device=x.device), splits)
             parts = library_product(x, w, torch.float32, splits)
             if parts is not None:
@@ -650,12 +650,13 @@ class HipBackend:
             core().call("me_gemm_skinny_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N,
                         _code(out_dtype), None, 1, M, N, K, 0, 0, skinny_wide(N, K), 0.0, 1.0, None, _stream())
             return y
-        if mid_takes(M, N, K, False) == 1 and not (mid_crowded(M, N, 1) and tile_fits(x, w)):
+        mid = mid_takes(M, N, K, False) == 1
+        if mid and not (mid_crowded(M, N, 1) and tile_fits(x, w)):
             y = new()
             core().call("me_gemm_mid_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N,
                         _code(out_dtype), 1, M, N, K, 0, 0.0, 1.0, None, _stream())
             return y
-        if tile_takes(M, N, K) and tile_fits(x, w):
+        if (mid or tile_takes(M, N, K)) and tile_fits(x, w):
             return _tile_product(x, w, new())
         # what is left of the many rows, or the head over a large vocabulary: the library product (float32 accumulation;
         # the float32 output form keeps the logits unrounded)
@@ -1634,7 +1635,7 @@ def mid_takes(M: int, N: int, K: int, partials: bool) -> int:
 # unit to itself, and for each of several that share one, workgroups that fit a compute unit), fitted to 6,300 times: 22 weights
 # of the layer sizes of 0.6B to 32B, 40 to 8,192 rows, one result and 2, 4 and 8 slices of K.
 TILE_COST = {(256, 256): (0.0, 10.6, 1.02, 1.02, 1), (256, 192): (0.0, 9.5, 0.91, 0.91, 1), (192, 256): (0.0, 9.0, 0.89, 0.89, 1),
-             (128, 256): (0.0, 6.2, 0.75, 0.75, 1), (256, 128): (0.0, 6.6, 0.70, 0.70, 1), (128, 192): (0.0, 5.6, 0.74, 0.61, 2),
+             (128, 256): (0.0, 6.2, 0.75, 0.75, 1), (256, 128): (0.0, 6.6, 0.70, 0.70, 1), (128, 192): (0.0, 5.6, 0.82, 0.61, 2),
              (128, 128): (0.0, 4.0, 0.48, 0.44, 2), (64, 128): (0.5, 2.4, 0.37, 0.30, 3), (128, 64): (1.5, 1.6, 0.35, 0.31, 3),
              (64, 64): (2.1, 0.8, 0.29, 0.20, 5)}
 # ... and what is added to a workgroup's us to choose a tile for the gating: its exponentials and divisions cost the wide tiles 5-7 us
@@ -1643,9 +1644,12 @@ TILE_COST = {(256, 256): (0.0, 10.6, 1.02, 1.02, 1), (256, 192): (0.0, 9.5, 0.91
 TILE_GATING = {(256, 256): -0.8, (256, 192): 0.9, (192, 256): 1.0, (128, 256): 1.2, (256, 128): -0.4, (128, 192): -0.1,
                (128, 128): -1.5, (64, 128): -1.3, (128, 64): -1.3, (64, 64): -1.4}
 TILE_MIN_ROWS = 33
-TILE_SURE_K = 2048
-TILE_MIN_TFLOPS = 1000
-TILE_SLICES_MAX_M = 256
+TILE_SURE_K = 1024
+TILE_LEVEL_K = 2048
+TILE_LEVEL_FILL = 0.8
+TILE_USED_ROWS = 0.86
+TILE_SLICES_MAX_M = 256          # library / own tiles, us: 40-256 rows of 44 weights and row counts 1.2 on average, from 300 rows on 1.0
+TILE_SLICES_MAX_K = 16384        # ... (2560 x 4096 at 200 rows 17.4 / 13.9, at 512 17.8 / 20.0); 5120 x 25600 at 160 rows 64 / 74
 
 
 @lru_cache(maxsize=4096)      # asked once per product of a step: ten tiles each time
@@ -1667,14 +1671,25 @@ def tile_choice(M: int, N: int, K: int, slices: int = 1, gated: bool = False) ->
 
 def tile_takes(M: int, N: int, K: int) -> bool:
     """Whether the product of M rows against a bfloat16 weight [N, K] that neither the kernels for few rows nor slices of K
-    take goes to csrc/gemm_tile.hip rather than to the library. Over a K of up to 2,048: always (137 products of 65 to 8,192
-    rows: 0.91 to 1.5 times as fast, 1.13 on average; 512 rows of 4096 x 1024 11.3 -> 8.9 us, 2,048 rows of 1024 x 1024
-    11.7 -> 8.8). Over a longer K where the tiles fill the compute units, which is where `tile_choice` expects 1,000
-    TFLOP/s or more (2,048 rows of 24576 x 4096 362 -> 290 us, 3,123 of it 692 -> 514, 2,048 of 6144 x 4096 90 -> 78); where
-    they do not, the library's smaller tiles are ahead (300 rows of 2560 x 4096 17.8 / 19.1, 1,280 of 4096 x 4096 46 / 51)."""
+    take goes to csrc/gemm_tile.hip rather than to the library. Timed beside each other over 26 weights of the layer sizes of 0.6B to
+    32B, 33 to 8,192 rows (library / this, us):
+    tiles of 256 x 256 are ahead in each of 114 products (1.07-2.7 times: 2,048 rows of 24576 x 4096 348 / 305, 4,096 of 4096 x 1024
+    36.6 / 32.4); the other tiles have fewer products for an operand read, and the library has more shapes of them;
+    over a K of up to 1,024, where the library's launches take 11 us at least, they are ahead by 1.17 on average (512 rows of 4096 x 1024
+    10.9 / 9.0; of 108 products 9 are behind by 3 to 10 %, 800 of 6144 x 1024 15.8 / 17.6);
+    up to 2,048 level or ahead where the tiles fill their rounds over the compute units to four fifths (2,048 rows of 4096 x 2048
+    34.2 / 33.0), mostly behind where they do not (1,280 of it 25.0 / 28.3; but 200 of 12288 x 2048 26.9 / 22.2) and with those of
+    192 x 256 (800 of 12288 x 2048 39.5 / 43.9); over a longer K behind by 3 to 70 % in half of the products (1,536 of 4096 x 12288
+    140 / 155) and ahead by more in a sixth."""
     if M < TILE_MIN_ROWS or N >= LIBRARY_MIN_N and M < 128:
         return False
-    return K <= TILE_SURE_K or 2e-6 * M * N * K / tile_choice(M, N, K)[1] >= TILE_MIN_TFLOPS
+    if K <= TILE_SURE_K:
+        return True
+    rows, features = tile = tile_choice(M, N, K)[0]
+    if tile == (256, 256):
+        return True
+    rounds = -(-(-(-M // rows) * -(-N // features)) // _COMPUTE_UNITS)
+    return K <= TILE_LEVEL_K and tile != (192, 256) and M * N >= TILE_LEVEL_FILL * rounds * _COMPUTE_UNITS * rows * features
 
 
 def tile_fits(x: torch.Tensor, w: torch.Tensor, slices: int = 1) -> bool:
@@ -1696,14 +1711,28 @@ def mid_crowded(M: int, N: int, slices: int) -> bool:
 
 def gated_linear_tiles(rows: int, w: torch.Tensor) -> bool:
     """Whether `rows` rows against the packed gate/up weight w [2 I, K] go through csrc/gemm_tile.hip with the gating in its
-    epilogue: from 33 rows on, where no kernel for few rows has the product. Against the library's product and a gating kernel
-    behind it: 512 rows of 6144 x 1024 17.7 -> 11.6 us, 2,048 rows of 24576 x 4096 390 -> 307."""
+    epilogue, where no kernel for few rows has the product. Against the library's product and a gating kernel behind it (us, both /
+    this): over a K of up to 2,048 ahead in 65 of 66 products, 1.19 on average (512 rows of 6144 x 1024 19.5 / 11.8, 2,048 of it
+    37 / 32; 800 of 12288 x 2048 47.6 / 48.6), over a longer K with tiles of 256 x 256 in 71 of 71 (2,048 rows of 24576 x 4096 385 / 318) and
+    with smaller ones by 1.05 on average. Behind are tiles of 192 x 256 over a K of 4,096 or more in two rounds or more where their
+    rows are not used, for the library has tiles of 160 rows (24576 x 4096 at 800 rows 151 / 171, 880 177 / 169, 960 171 / 170; 51200 x 5120 at
+    800 rows 378 / 411, 860 410 / 413; in one round a prompt of 300 tokens through 36 layers of 24576 x 4096 takes 7.78 / 7.72 ms,
+    of 800 13.9 / 14.3), and up to 64 rows of a K beyond 4,096, which the library reads faster (50 rows of 51200 x 5120 102 / 108)."""
     if not FUSE_GATE_INTO_GATE_UP or rows < TILE_MIN_ROWS or w.dtype != torch.bfloat16 or w.dim() != 2 or w.stride(1) != 1:
         return False
     N, K = w.shape
     if N % 16 or K % 64 or K < 128 or skinny_takes(rows, N, K):
         return False
-    return mid_takes(rows, N, K, False) != 1 or mid_crowded(rows, N, 1)
+    if mid_takes(rows, N, K, False) == 1:
+        return mid_crowded(rows, N, 1)
+    if K < 4096:
+        return True
+    if K > 4096 and rows <= 64:
+        return False
+    if tile_choice(rows, N, K, 1, True)[0] != (192, 256):
+        return True
+    tiles = -(-rows // 192)
+    return tiles * -(-N // 256) <= _COMPUTE_UNITS or rows >= TILE_USED_ROWS * 192 * tiles
 
 
 def prefill_waves(max_context: int, num_tokens: int, num_seqs: int, Hq: int, Hkv: int, col_tiles: int, max_segs: int) -> int:
