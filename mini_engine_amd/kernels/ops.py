@@ -651,12 +651,13 @@ class HipBackend:
                         _code(out_dtype), None, 1, M, N, K, 0, 0, skinny_wide(N, K), 0.0, 1.0, None, _stream())
             return y
         mid = mid_takes(M, N, K, False) == 1
-        if mid and not (mid_crowded(M, N, 1) and tile_fits(x, w)):
+        tiles = tile_fits(x, w) and (out is None or out.data_ptr() % 16 == 0)      # an `out` may begin anywhere
+        if mid and not (mid_crowded(M, N, 1) and tiles):
             y = new()
             core().call("me_gemm_mid_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N,
                         _code(out_dtype), 1, M, N, K, 0, 0.0, 1.0, None, _stream())
             return y
-        if (mid or tile_takes(M, N, K)) and tile_fits(x, w):
+        if (mid or tile_takes(M, N, K)) and tiles:
             return _tile_product(x, w, new())
         # what is left of the many rows, or the head over a large vocabulary: the library product (float32 accumulation;
         # the float32 output form keeps the logits unrounded)

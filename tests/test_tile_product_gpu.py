@@ -92,6 +92,19 @@ def test_what_the_rules_send_there(M, N, K):
         assert torch.equal(y, hip().linear(x, w))
 
 
+@pytest.mark.parametrize("M,N,K", [(300, 1024, 1024), (257, 6144, 1024), (2048, 1024, 2048)])
+def test_an_out_that_begins_anywhere(M, N, K):
+    """`linear` writes into any contiguous `out`, also one that is not aligned to the 16 bytes that the kernel's stores want."""
+    x, w = _operands(M, N, K)
+    want = hip().linear(x, w)
+    for shift in (1, 4, 8):
+        room = torch.full((M * N + 16,), 7.0, dtype=torch.bfloat16, device=DEV)
+        y = hip().linear(x, w, out=room[shift:shift + M * N].view(M, N))
+        close(y, x.double() @ w.double().t(), 4e-3)
+        assert y.data_ptr() == room.data_ptr() + 2 * shift and bool((room[:shift] == 7).all()) and bool((room[shift + M * N:] == 7).all())
+        assert shift % 8 or torch.equal(y, want)
+
+
 def test_what_the_kernel_refuses():
     x, w = _operands(70, 64, 128)
     y = torch.empty(70, 64, dtype=torch.bfloat16, device=DEV)
