@@ -681,11 +681,15 @@ __global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const floa
   constexpr int VALUES = TB * PC, VROUNDS = (VALUES + 64 * W - 1) / (64 * W);
   constexpr bool ROWS = RULE != 3;
   constexpr bool SHARED_V = NR <= 128;   // the columns' values go through LDS too; with 256 rows a lane asks for its own
+  // A lane that holds 64 rows has no registers left over: the last batch shares the code around the others and the loads of a
+  // batch's values their addresses (63 registers spilled otherwise, 32 so: 16 prompts of 512 tokens over 4 heads of 256 x 64, bonus rule
+  // 463 -> 415 us, delta rule 529 -> 512); elsewhere a wave is level or slower with it (16 lanes to a column, delta rule 167 / 190).
+  constexpr bool TIGHT = NR / RG > 32;
   __shared__ f32x4 sq[2][PIECES], sk[2][PIECES], sd[ROWS ? 2 : 1][ROWS ? PIECES : 1];
   __shared__ __align__(16) float sv[2][SHARED_V ? VALUES : 1];              // [column][token]
   __shared__ float sx[2][TB], sh[2][TB];               // the tokens' own numbers; their heads' decays (RULE 3)
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x, lane = W == 1 ? tid : tid & 63;
+  const int wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col_blocks = (a.P + PC - 1) / PC;
   const int cb = blockIdx.x % col_blocks;
   const int h = (blockIdx.x / col_blocks) % a.H;
@@ -728,14 +732,15 @@ __global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const floa
   auto at = [](const void* base, uint32_t bytes) { return reinterpret_cast<const char*>(base) + bytes; };
   // the next batch on its way; of a batch that is not whole, tokens behind the last are read from the last one and not used
   auto fetch = [&](int t0) {
-    if (t0 >= n_tok) return;
-    if (!SHARED_V) {
+    if (!TIGHT && t0 >= n_tok) return;
+    if (SHARED_V) {
+#pragma unroll
+      for (int r = 0; r < VROUNDS; ++r)
+        nv[r] = values[(int64_t)min(t0 + min(tid + 64 * W * r, VALUES - 1) / PC, n_tok - 1) * a.v_stride + column[r]];
+    } else if (!TIGHT) {
 #pragma unroll
       for (int j = 0; j < TB; ++j) nv[j] = values[(int64_t)min(t0 + j, n_tok - 1) * a.v_stride + pc];
-    } else
-#pragma unroll
-    for (int r = 0; r < VROUNDS; ++r)
-      nv[r] = values[(int64_t)min(t0 + min(tid + 64 * W * r, VALUES - 1) / PC, n_tok - 1) * a.v_stride + column[r]];
+    }
     if (t0 + TB <= n_tok) {
       const int64_t row = head0 + (int64_t)t0 * a.H;
 #pragma unroll
@@ -746,6 +751,11 @@ __global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const floa
       }
       nx = *reinterpret_cast<const float*>(at(pre_x + row, own));
       if (!ROWS) nh = *reinterpret_cast<const float*>(at(pre_d + row, own));
+      if (TIGHT) {
+        const TX* vt = values + t0 * a.v_stride;
+#pragma unroll
+        for (int j = 0; j < TB; ++j, vt += a.v_stride) nv[j] = *reinterpret_cast<const TX*>(at(vt, (uint32_t)(pc * sizeof(TX))));
+      }
       return;
     }
 #pragma unroll
@@ -759,6 +769,10 @@ __global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const floa
     const int64_t row = head0 + (int64_t)min(t0 + my_token, n_tok - 1) * a.H;
     nx = pre_x[row];
     if (!ROWS) nh = pre_d[row];
+    if (TIGHT) {
+#pragma unroll
+      for (int j = 0; j < TB; ++j) nv[j] = values[(int64_t)min(t0 + j, n_tok - 1) * a.v_stride + pc];
+    }
   };
   struct Shared { float q[RL], k[RL], d[RL], x; };
   auto read = [&](int buf, int j, Shared& o, bool reads_out) {
@@ -842,11 +856,25 @@ __global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const floa
       for (int j = 0; j < TB; ++j) v[j] = sv[buf][lane / RG * TB + j];
     }
   };
+// a last batch that is not whole (no lambda: the choice of a value would become an address, and v memory)
+#define DR_LAST_BATCH                                             \
+  _Pragma("unroll 1") for (int j = 0; t0 + j < n_tok; ++j) {      \
+    Shared o;                                                     \
+    read(buf, j, o, true);                                        \
+    float vj = v[0];                                              \
+    _Pragma("unroll") for (int i = 1; i < TB; ++i) vj = i == j ? v[i] : vj; \
+    const float y = token(o, vj, true);                           \
+    if (live && rg == 0) out[(int64_t)(t0 + j) * (a.H * a.P)] = y; \
+  }
   auto walk = [&](auto which) {                  // a wave's whole batches: it gives the outputs of tokens which, which + W, ... of each
     constexpr int ME = decltype(which)::value, MINE = TB / W;
-    for (; t0 + TB <= n_tok; t0 += TB, buf ^= 1) {
+    for (; t0 + (TIGHT ? 1 : TB) <= n_tok; t0 += TB, buf ^= 1) {
       float v[TB], y[MINE];
       next_batch(v);
+      if (TIGHT && t0 + TB > n_tok) {
+        DR_LAST_BATCH
+        continue;
+      }
       Shared o[AHEAD + 1];                       // a token's values are read while those before it are worked on
 #pragma unroll
       for (int j = 0; j < AHEAD; ++j) read(buf, j, o[j], j % W == ME);
@@ -876,22 +904,12 @@ __global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const floa
   else if (wave == 1) walk(std::integral_constant<int, 1 % W>{});
   else if (wave == 2) walk(std::integral_constant<int, 2 % W>{});
   else walk(std::integral_constant<int, 3 % W>{});
-  if (t0 < n_tok) {                              // a last batch that is not whole
+  if (!TIGHT && t0 < n_tok) {
     float v[TB];
     next_batch(v);
-    if (wave == 0) {                             // its outputs and the state behind it are the first wave's
-#pragma unroll 1
-      for (int j = 0; t0 + j < n_tok; ++j) {
-        Shared o;
-        read(buf, j, o, true);
-        float vj = v[0];
-#pragma unroll
-        for (int i = 1; i < TB; ++i) vj = i == j ? v[i] : vj;
-        const float y = token(o, vj, true);
-        if (live && rg == 0) out[(int64_t)(t0 + j) * (a.H * a.P)] = y;
-      }
-    }
+    if (wave == 0) DR_LAST_BATCH                 // its outputs and the state behind it are the first wave's
   }
+#undef DR_LAST_BATCH
   if (live && wave == 0) {
 #pragma unroll
     for (int i = 0; i < RL; ++i)

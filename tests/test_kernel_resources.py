@@ -52,6 +52,38 @@ def test_float32_attention_keeps_to_its_registers(tmp_path):
         assert scratch == 0 and registers <= 256, (head, scratch, registers)
 
 
+def _needs(tmp_path, kernel_name: str, *fields) -> dict:
+    """Of each built kernel whose name holds `kernel_name`: the numbers of its metadata."""
+    library = os.path.join(build.PKG_LIB, "libme_core.so")
+    if not os.path.exists(library):
+        pytest.skip("the core library is not built")
+    found = {}
+    for i, code in enumerate(_code_objects(open(library, "rb").read())):
+        if kernel_name.encode() not in code:
+            continue
+        path = tmp_path / f"{i}.elf"
+        path.write_bytes(code)
+        notes = subprocess.run([READELF, "--notes", str(path)], capture_output=True, text=True, check=True).stdout
+        for kernel in notes.split("- .agpr_count:")[1:]:
+            name = re.search(r"\.name:\s+(\S+)", kernel).group(1)
+            if kernel_name in name:
+                found[name] = tuple(int(re.search(rf"\.{field}:\s+(\d+)", kernel).group(1)) for field in fields)
+    return found
+
+
+@pytest.mark.skipif(READELF is None, reason="no llvm-readelf")
+def test_the_decay_walk_keeps_to_its_registers(tmp_path):
+    """Only the form whose lanes hold 64 rows spills, and no more than the rows that its registers cannot hold beside a batch (40);
+    of waves of up to 128 rows with 16 lanes to a column two run on a SIMD, of up to 64 three."""
+    seen = {}
+    for name, needs in _needs(tmp_path, "decay_walk_kernel", "vgpr_spill_count", "vgpr_count").items():
+        rows, lanes, rule, waves = (int(n) for n in re.findall(r"Li(\d+)E", name))
+        seen[name] = (rows, lanes)
+        assert needs[0] <= (40 if rows // lanes > 32 else 0), (name, needs)
+        assert lanes != 16 or rows > 128 or needs[1] <= (256 if rows > 64 else 168), (name, needs)
+    assert set(seen.values()) == {(rows, lanes) for rows in (32, 64, 128, 256) for lanes in (4, 16)}
+
+
 def _reads_on_their_way(code: list) -> dict:
     """The most LDS reads that can be on their way at each instruction, over all paths. `code`: (address, name, operands, the
     address a branch goes to or None)."""
