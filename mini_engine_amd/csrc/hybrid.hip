@@ -918,10 +918,12 @@ __global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const floa
 }
 
 // Workgroups up to which four waves share the walk of a column group: beyond, the waves of one SIMD share its instructions, and
-// the state carried four times costs more than it saves. us, one wave / four: 128 rows, 384 workgroups 202 / 172, 512 147 / 154;
-// 64 rows, 768 workgroups 167 / 142 (delta rule) and 138 / 95 (bonus), 1,024 142 / 177 and 119 / 118. With 256 rows the batches'
-// LDS leaves no room for longer ones, and without them four waves gain nothing (624 / 650).
-template <int NR> constexpr unsigned dr_shared_max() { return NR <= 64 ? 768 : NR <= 128 ? 384 : 0; }
+// the state carried four times costs more than it saves. us, one wave / four, requests of 1,100 tokens, bonus and delta rule: 128 rows, 256
+// workgroups 159 / 131 and 185 / 158, 320 (two on some compute units) 182 / 198 and 205 / 216, 512 187 / 211 and 213 / 234; 64 rows, 512
+// workgroups 122 / 98 and 154 / 150, 768 143 / 126 and 178 / 184, 832 156 / 170 and 188 / 257. Of 128 rows the delta rules keep it up to
+// 384: between a layer's other launches three prompts of 1,100 tokens over 4 heads take 195 / 188 us. With 256 rows the
+// batches' LDS leaves no room for longer ones, and without them four waves gain nothing (624 / 650).
+template <int NR, int RULE> constexpr unsigned dr_shared_max() { return NR <= 64 ? 768 : NR <= 128 ? (RULE == 1 || RULE == 3 ? 384 : 256) : 0; }
 template <typename TX, int NR, int RG, bool PRE>
 static void launch_decay_rows(const DrArgs& a, int rule, int num_seqs, int64_t T, float* pre, hipStream_t stream) {
   constexpr int PC = 64 / RG;
@@ -933,8 +935,8 @@ static void launch_decay_rows(const DrArgs& a, int rule, int num_seqs, int64_t T
 #define DR_RULE(R)                                                                       \
   do {                                                                                   \
     decay_prepare_kernel<TX, NR, R><<<pgrid, block, 0, stream>>>(a, RG, pq, pk, pd, px); \
-    constexpr bool SHARES = RG == 16 && dr_shared_max<NR>() > 0;                         \
-    if (SHARES && grid.x <= dr_shared_max<NR>())                                         \
+    constexpr bool SHARES = RG == 16 && dr_shared_max<NR, R>() > 0;                      \
+    if (SHARES && grid.x <= dr_shared_max<NR, R>())                                      \
       decay_walk_kernel<TX, NR, RG, R, SHARES ? 4 : 1><<<grid, 256, 0, stream>>>(a, pq, pk, pd, px); \
     else decay_walk_kernel<TX, NR, RG, R, 1><<<grid, block, 0, stream>>>(a, pq, pk, pd, px); \
   } while (0)

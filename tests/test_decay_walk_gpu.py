@@ -47,7 +47,7 @@ def test_places_in_a_batch(monkeypatch, H, N, P, dtype, rule, groups):
 
 
 @pytest.mark.parametrize("rule", ["bonus", "delta", "gated", "delta_head"])
-@pytest.mark.parametrize("H,N,P,count", [(2, 64, 64, 3), (12, 64, 64, 4), (13, 64, 64, 4), (3, 128, 128, 4), (4, 128, 132, 3), (2, 20, 30, 2), (1, 256, 7, 3)])
+@pytest.mark.parametrize("H,N,P,count", [(2, 64, 64, 3), (12, 64, 64, 4), (13, 64, 64, 4), (3, 128, 128, 4), (2, 128, 128, 4), (2, 128, 132, 4), (4, 128, 132, 3), (2, 20, 30, 2), (1, 256, 7, 3)])
 def test_waves_that_share_a_walk(H, N, P, count, rule):
     """Several requests at once, at the numbers of workgroups up to which four waves share a column group's walk and just
     beyond: batches of 16 and of 8 that end early, a request without tokens, the same bits as each request alone."""
