@@ -1933,9 +1933,12 @@ def decay_row_groups(num_seqs: int, H: int, N: int, P: int, longest: int = 1, to
     """(lanes that share a column of the state in `decay_rows_recurrence`, whether a first kernel shapes the tokens' values).
     A request is a chain: the fewer rows a lane walks per token, the shorter the chain's step, at the price of more waves
     and an exchange between lanes. Steps of long requests: the values of all tokens are shaped at once by a kernel of its
-    own (unit lengths, decays and their exponentials leave the chain), and 16 lanes share a column while that is at most as many
-    waves as a unit's 160 KB of LDS hold, 16 at most (a wave keeps q, k and, unless a head has one decay, the decays of 16
-    tokens there), else 4: 8 prompts of 2,048 tokens over 8 heads of 128 x 128, 2,048 waves of 16 lanes to a column, take 681 us
+    own (unit lengths, decays and their exponentials leave the chain), and 16 lanes share a column up to a number of waves to a
+    compute unit, else 4. Up to 64 rows it is the number from which 4 lanes are ahead, 9 and with one decay per head 11: 16
+    heads of 64 x 64, prompts of 512 tokens, 16 lanes / 4, bonus, delta rule and the latter with one decay: 8 of them 120 / 129, 146 / 158
+    and 131 / 148 us, 10 152 / 139, 174 / 172 and 145 / 173, 12 185 / 142, 210 / 192 and 180 / 181, 13 209 / 159, 248 / 204 and 189 / 188. Beyond 64
+    rows as many as a unit's 160 KB of LDS hold (a wave keeps q, k and, unless a head has one decay, the decays of 16 tokens
+    there): 8 prompts of 2,048 tokens over 8 heads of 128 x 128, 2,048 waves of 16 lanes to a column, take 681 us
     with one decay per head (933 with 4 lanes) and 1,088 with a decay per row (two rounds; 1,057 with 4 lanes); 16 prompts
     of 512 tokens 459 and 328. A wave of 65 to 128 rows needs 171 registers, so 8 run on a unit where its LDS would hold 9: with
     one decay per head the ninth's share is a second round, which still pays (9 prompts of 512 tokens 231 us, 241 with 4 lanes; of
@@ -1946,7 +1949,7 @@ def decay_row_groups(num_seqs: int, H: int, N: int, P: int, longest: int = 1, to
     if longest >= DECAY_PREPARE_MIN_TOKENS:
         chains = num_seqs if tokens is None else min(num_seqs, -(-tokens // longest))
         rows = 32 if N <= 32 else 64 if N <= 64 else 128 if N <= 128 else 256
-        per_unit = min(16, 160 * 1024 // ((2 if one_decay else 3) * 16 * rows * 4 + 64))
+        per_unit = min(11 if one_decay else 9, 160 * 1024 // ((2 if one_decay else 3) * 16 * rows * 4 + 64))
         return (16 if chains * H * -(-P // 4) <= per_unit * _COMPUTE_UNITS else 4), True
     if N > 64:
         return 4, False

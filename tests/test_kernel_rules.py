@@ -304,3 +304,10 @@ def test_many_rows_go_where_they_were_timed_to_be_faster():
     for M, N, K, both, own in GATED_PRODUCTS:
         w = torch.empty(N, K, dtype=torch.bfloat16, device="meta")
         assert ops.gated_linear_tiles(M, w) == (own < both), (M, N, K)
+
+
+def test_lanes_to_a_column_of_up_to_64_rows_go_by_what_was_timed():
+    """16 heads of 64 x 64, prompts of 512 tokens: 16 lanes up to 9 waves to a compute unit (11 with one decay per head), 4 beyond."""
+    lanes = lambda prompts, one: ops.decay_row_groups(prompts, 16, 64, 64, 512, 512 * prompts, one)
+    assert [lanes(n, False) for n in (3, 8, 9, 10, 12, 13)] == [(16, True)] * 3 + [(4, True)] * 3
+    assert [lanes(n, True) for n in (8, 10, 11, 12, 16)] == [(16, True)] * 3 + [(4, True)] * 2
