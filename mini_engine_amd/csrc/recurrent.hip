@@ -491,9 +491,11 @@ struct RecArgs {
 // and rows of k and q come from LDS two pieces of eight rows ahead. us, converted at the fetch and read where used / this: 16
 // heads of 128 x 128, one request of 60 tokens 84 / 39, of 350 138 / 86, of 2,048 190 / 166, 16 of 700 855 / 692; 32 heads of
 // 128 x 64 with step sizes 81 / 36, 131 / 80, 177 / 149, 785 / 600; 301 requests, one of 300 tokens and the rest of one, 776 / 760.
-// Only the 48-row form loses where no request has more than three tokens (4 heads of 48 x 100, eight requests 14.6 / 18.5; one
-// of 60 tokens 74 / 56); a branch behind a piece's first token does not bring it back.
-template <typename TX, int NT, int PASS, int HPB, int PPB, bool KEYS>
+// PART 1: a piece is one token, whose rows are read where they are used: 80 registers fewer (64 rows: 209 -> 139), so three waves to
+// a SIMD instead of two, and a smaller code. For short requests, whose pieces of four would be mostly empty, and for many of
+// them (`ops.recurrence_one_by_one`; us, pieces of four / of one: 64 requests of 2 tokens, 16 heads of 128 x 128 51 / 38, 300 requests of a
+// token and one of two, 4 heads of 48 x 100 52 / 28, 256 requests of three, 8 heads of 64 x 64 32 / 23).
+template <typename TX, int NT, int PASS, int HPB, int PPB, bool KEYS, int PART>
 __global__ void __launch_bounds__(64) recurrence_kernel(RecArgs a) {
   static_assert(!KEYS || HPB == 1, "summed keys: one head per wave");
   constexpr int CL = HPB * PPB;
@@ -636,9 +638,9 @@ __global__ void __launch_bounds__(64) recurrence_kernel(RecArgs a) {
     asm volatile("" ::: "memory");
     if (tb + REC_TB < t1) fetch(tb + REC_TB);         // the next batch travels while this one is computed
     __syncthreads();
-    // Four tokens are one piece of code without a branch, and their rows of k and q are read from LDS in pieces of eight rows,
+    // PART tokens are one piece of code without a branch, and of four their rows of k and q are read from LDS in pieces of eight rows,
     // two pieces ahead: read where they are used, every pair of rows waited for LDS (1.4 us a token of 32 rows).
-    constexpr int PART = 4, CH = 8, PER = NT / CH, AHEAD = 2, CELLS = (int)sizeof(Cell) * CH / 16;
+    constexpr int CH = 8, PER = NT / CH, AHEAD = PART == 1 ? 0 : 2, CELLS = (int)sizeof(Cell) * CH / 16;
     static_assert(NT % CH == 0 && REC_TB % PART == 0, "whole pieces");
 #pragma unroll
     for (int part = 0; part < REC_TB; part += PART) {
@@ -865,22 +867,24 @@ __global__ void __launch_bounds__(256) recurrence_step_kernel(RecArgs a) {
 }
 
 template <typename TX, int NT, int HPB, int PPB, bool KEYS>
-static int launch_recurrence(RecArgs& a, int num_seqs, int spans, hipStream_t stream) {
+static int launch_recurrence(RecArgs& a, int num_seqs, int spans, int one_by_one, hipStream_t stream) {
   const int slices = (a.N + NT - 1) / NT;
   const dim3 block(64);
   const unsigned pblocks = (a.P + 64 * PPB - 1) / (64 * PPB);
   if (spans <= 1) {
-    recurrence_kernel<TX, NT, 0, HPB, PPB, KEYS><<<dim3(num_seqs * (a.H / HPB), pblocks, slices), block, 0, stream>>>(a);
+    const dim3 grid(num_seqs * (a.H / HPB), pblocks, slices);
+    if (one_by_one) recurrence_kernel<TX, NT, 0, HPB, PPB, KEYS, 1><<<grid, block, 0, stream>>>(a);
+    else recurrence_kernel<TX, NT, 0, HPB, PPB, KEYS, 4><<<grid, block, 0, stream>>>(a);
     ME_LAUNCH_CHECK();
     return 0;
   }
   const dim3 grid(num_seqs * (a.H / HPB), pblocks, slices * spans);
-  recurrence_kernel<TX, NT, 1, HPB, PPB, KEYS><<<grid, block, 0, stream>>>(a);
+  recurrence_kernel<TX, NT, 1, HPB, PPB, KEYS, 4><<<grid, block, 0, stream>>>(a);
   ME_LAUNCH_CHECK();
   const int64_t per_req = (int64_t)a.H * a.N * a.P + (KEYS ? (int64_t)a.H * a.N : 0);
   recurrence_carry_kernel<<<dim3((unsigned)((per_req + 255) / 256), num_seqs), dim3(256), 0, stream>>>(a);
   ME_LAUNCH_CHECK();
-  recurrence_kernel<TX, NT, 2, HPB, PPB, KEYS><<<grid, block, 0, stream>>>(a);
+  recurrence_kernel<TX, NT, 2, HPB, PPB, KEYS, 4><<<grid, block, 0, stream>>>(a);
   ME_LAUNCH_CHECK();
   return 0;
 }
@@ -888,14 +892,14 @@ static int launch_recurrence(RecArgs& a, int num_seqs, int spans, hipStream_t st
 // spans <= 1: every request's tokens in one pass. Otherwise the tokens are cut into spans of `span` tokens that run
 // side by side (at most `spans` per request), and scratch holds spans * H * N * P + spans * H floats per request.
 // keys: the summed keys beside the states, in the same state rows (see RecArgs); scratch then holds spans * H * N more.
-// columns: 1, or 2: a lane keeps two columns of the state (two blocks of 64 columns of one head where P > 64, else
+// one_by_one: a single pass (spans <= 1) takes the form for short requests. columns: 1, or 2: a lane keeps two columns of the state (two blocks of 64 columns of one head where P > 64, else
 // the same columns of two neighbouring heads of one group, which needs an even number of heads per group).
 extern "C" int me_linear_recurrence(const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
                                     int64_t v_stride, int dtype, const void* dt, int64_t dt_stride, const float* decay,
                                     const float* dt_bias, const float* rate, const float* skip, float* state,
                                     int64_t state_stride, const int32_t* slots, const int32_t* cu, float* y,
                                     int64_t y_slice_stride, int num_seqs, int H, int G, int N, int P, int rows_per_wave,
-                                    int columns, int silu, int span, int spans, float* scratch, const float* coef_a,
+                                    int columns, int silu, int span, int spans, int one_by_one, float* scratch, const float* coef_a,
                                     const float* coef_b, float* keys, float* key_dot, int64_t dot_slice_stride, const void* gate_i,
                                     const void* gate_f, int64_t gate_stride, const float* bias_i, const float* bias_f, float cap,
                                     float* gate_m, int64_t gate_m_stride, hipStream_t stream) {
@@ -942,10 +946,10 @@ extern "C" int me_linear_recurrence(const void* q, int64_t q_stride, const void*
   ME_CHECK((int64_t)slices * a.max_spans <= 65535, "recurrence: too many slices and spans for one launch");
 #define REC_NT(TX, NT)                                                                               \
   do {                                                                                               \
-    if (keys) return launch_recurrence<TX, NT, 1, 1, true>(a, num_seqs, spans, stream);              \
-    if (columns == 1) return launch_recurrence<TX, NT, 1, 1, false>(a, num_seqs, spans, stream);     \
-    if (two_heads) return launch_recurrence<TX, NT, 2, 1, false>(a, num_seqs, spans, stream);        \
-    return launch_recurrence<TX, NT, 1, 2, false>(a, num_seqs, spans, stream);                       \
+    if (keys) return launch_recurrence<TX, NT, 1, 1, true>(a, num_seqs, spans, one_by_one, stream);              \
+    if (columns == 1) return launch_recurrence<TX, NT, 1, 1, false>(a, num_seqs, spans, one_by_one, stream);     \
+    if (two_heads) return launch_recurrence<TX, NT, 2, 1, false>(a, num_seqs, spans, one_by_one, stream);        \
+    return launch_recurrence<TX, NT, 1, 2, false>(a, num_seqs, spans, one_by_one, stream);                       \
   } while (0)
 #define REC(TX)                                                                              \
   switch (rows_per_wave) {                                                                   \

@@ -81,7 +81,7 @@ _CORE_PROTOS = {
     "me_activation": [P, L, P, I, I, L, I, P],
     "me_head_gate": [P, P, L, I, L, I, I, P],
     "me_causal_conv": [P, L, I, P, P, P, L, P, P, I, I, P, L, I, I, I, P],
-    "me_linear_recurrence": [P, L, P, L, P, L, I, P, L, P, P, P, P, P, L, P, P, P, L, I, I, I, I, I, I, I, I, I, I, P,
+    "me_linear_recurrence": [P, L, P, L, P, L, I, P, L, P, P, P, P, P, L, P, P, P, L, I, I, I, I, I, I, I, I, I, I, I, P,
                              P, P, P, P, L, P, P, L, P, P, F, P, L, P],
     "me_soft_gates": [P, P, L, I, P, P, F, P, L, P, P, P, P, P, I, I, P],
     "me_memory_readout": [P, I, L, P, P, F, P, L, I, P, P, L, I, I, F, P, P, L, P, P, F, P, L, P, P],
@@ -848,7 +848,7 @@ class HipBackend:
             core().call("me_linear_recurrence", q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
                         _code(dtype), _ptr(dt), 0 if dt is None else dt.stride(0), _ptr(decay), _ptr(dt_bias), _ptr(rate), _ptr(skip),
                         state.data_ptr(), state.stride(0), state_slots.data_ptr(), cu_seqlens.data_ptr(), y.data_ptr(), T * H * P,
-                        B, H, G, N, P, 0, 1, int(silu), 0, 1, None,
+                        B, H, G, N, P, 0, 1, int(silu), 0, 1, 0, None,
                         *(none if gates is None else (None, None, key_state.data_ptr(), dot.data_ptr(), T * H)),
                         *(no_gates if gates is None else gates.args()), _stream())
             return y if gates is None else MemoryReads(y, dot, None, gates)
@@ -867,7 +867,7 @@ class HipBackend:
         core().call("me_linear_recurrence", q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
                     _code(dtype), _ptr(dt), 0 if dt is None else dt.stride(0), _ptr(decay), _ptr(dt_bias), _ptr(rate), _ptr(skip),
                     state.data_ptr(), state.stride(0), state_slots.data_ptr(), cu_seqlens.data_ptr(), y.data_ptr(), T * H * P,
-                    B, H, G, N, P, per_wave, columns, int(silu), span, spans, _ptr(scratch),
+                    B, H, G, N, P, per_wave, columns, int(silu), span, spans, recurrence_one_by_one(q_lens, H * -(-P // 64) * slices // columns, per_wave), _ptr(scratch),
                     *(none if gates is None else (factors[0].data_ptr(), factors[1].data_ptr(), key_state.data_ptr(), dot.data_ptr(), T * H)),
                     *no_gates, _stream())
         return y if gates is None else MemoryReads(y, dot, factors[2], gates)
@@ -1879,6 +1879,18 @@ RECURRENCE_STEP_MAX_ROWS = 4096     # state rows up to which the single-token ke
 RECURRENCE_COLUMNS = int(_os.environ.get("ME_RECURRENCE_COLUMNS", "0"))     # 1 or 2 force the columns per lane (for timing one against the other)
 RECURRENCE_MIN_SPAN = 64
 RECURRENCE_WAVES = 4096        # waves that keep the 256 compute units busy: 16 a unit, 4 a SIMD
+
+
+def recurrence_one_by_one(q_lens, waves_per_request: int, rows_per_wave: int) -> int:
+    """Whether a step's requests go through the recurrence's kernel token by token (1) or in pieces of four tokens (0). Pieces of
+    one need fewer registers, so that more waves run at once, and compute nothing for tokens that are not there; pieces of four
+    hide the reads of LDS. us, of four / of one: up to 8 tokens level or ahead (64 requests of 2 tokens, 16 heads of 128 x 128 51 / 38,
+    of 4 51 / 40, 8 requests of 8 tokens 12.9 / 13.6), of 12 behind (8 requests 15.7 / 17.1); waves of 48 rows, whose code is
+    the largest for its work, up to 32 (8 requests of 24 tokens, 4 heads of 48 x 100 28 / 26); from as many waves on as keep the
+    chip busy up to 64 (300 requests of one token beside one of 16, 16 heads of 128 x 128 317 / 270,
+    beside one of 64 342 / 303; 2,400 waves of 8 heads of 64 x 64 62 / 68)."""
+    longest = max(q_lens, default=0)
+    return int(longest <= 8 or (rows_per_wave == 48 and longest <= 32) or (longest <= 64 and len(q_lens) * waves_per_request >= RECURRENCE_WAVES))
 
 
 def recurrence_spans(q_lens: list, waves_per_request: int, most_spans: int = 8191) -> tuple:

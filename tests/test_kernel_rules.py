@@ -311,3 +311,11 @@ def test_lanes_to_a_column_of_up_to_64_rows_go_by_what_was_timed():
     lanes = lambda prompts, one: ops.decay_row_groups(prompts, 16, 64, 64, 512, 512 * prompts, one)
     assert [lanes(n, False) for n in (3, 8, 9, 10, 12, 13)] == [(16, True)] * 3 + [(4, True)] * 3
     assert [lanes(n, True) for n in (8, 10, 11, 12, 16)] == [(16, True)] * 3 + [(4, True)] * 2
+
+
+def test_short_requests_pass_the_recurrence_token_by_token():
+    """What was timed: up to 8 tokens, waves of 48 rows up to 32, and up to 64 where the requests fill the chip."""
+    one = ops.recurrence_one_by_one
+    assert one([1] * 7 + [2], 64, 64) and one([8] * 8, 64, 64) and not one([12] * 8, 64, 64) and not one([60], 64, 64)
+    assert one([24] * 8, 8, 48) and not one([60], 8, 48)
+    assert one([1] * 300 + [16], 64, 64) and one([1] * 300 + [64], 64, 64) and not one([1] * 300 + [64], 8, 64) and not one([1] * 300 + [300], 64, 64)

@@ -197,6 +197,34 @@ def test_recurrence_in_pieces_of_four_tokens(monkeypatch, dtype, H, N, P, column
     assert torch.equal(st_h[5], full[5])
 
 
+@pytest.mark.parametrize("columns", [1, 2])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,N,P", [(2, 16, 20), (2, 32, 64), (2, 48, 100), (2, 64, 65), (2, 128, 128)])
+def test_recurrence_token_by_token(monkeypatch, dtype, H, N, P, columns):
+    """The form for short requests: around its batches of eight tokens, against the token-by-token twin (2e-5: the inputs are exact in
+    both, up to 70 float32 sums in another order), and the bits of the form that takes tokens in fours."""
+    monkeypatch.setattr(ops, "RECURRENCE_COLUMNS", columns)
+    torch.manual_seed(N + P)
+    q_lens = [1, 2, 3, 4, 5, 6, 7, 8, 9, 16, 17, 70]
+    cu, seq, slots = _steps_meta(q_lens, [12, 0, 4, 1, 3, 2, 9, 8, 7, 6, 11, 10])
+    T = sum(q_lens)
+    q, k, v = torch.randn(T, 2 * H * N + H * P, device=DEV).to(dtype).split((H * N, H * N, H * P), 1)
+    kw = dict(dt=torch.randn(T, H, device=DEV).to(dtype), dt_bias=torch.randn(H, device=DEV), rate=torch.rand(H, device=DEV), skip=torch.randn(H, device=DEV), silu=True)
+    full = torch.randn(13, H * N * P, device=DEV)
+    got = []
+    for one_by_one in (1, 0):
+        monkeypatch.setattr(ops, "recurrence_one_by_one", lambda *a: one_by_one)
+        state = full.clone()
+        got.append((hip().linear_recurrence(q, k, v, state, slots, cu, q_lens, H, H, N, P, **kw), state))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    st_c = full.cpu().clone()
+    want = twin.linear_recurrence(q.cpu(), k.cpu(), v.cpu(), st_c, slots.cpu(), cu.cpu(), q_lens, H, H, N, P,
+                                  **{n: t.cpu() if torch.is_tensor(t) else t for n, t in kw.items()})
+    y = got[0][0]
+    close((y.sum(0) if y.dim() == 3 else y).cpu(), want, 2e-5)
+    close(got[0][1], st_c, 2e-5)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("kind,groups,parts", [("silu_before", 1, 1), ("silu_before", 4, 2), ("sigmoid_behind", 1, 3)])
 def test_gated_rms_norm(dtype, kind, groups, parts):
