@@ -535,6 +535,9 @@ __global__ void __launch_bounds__(64) recurrence_kernel(RecArgs a) {
 
   // what a lane asks for for a batch of tokens, as it lies in memory: conversions and selects come when the batch is taken
   // (on what has just been asked for they would wait for it)
+  // a float32 step size goes to araw, and factors to braw first: what the two branches of `fetch` store last would otherwise
+  // become one store to either variable, which puts both into memory
+  constexpr bool F32 = std::is_same_v<TX, float>;
   TX kraw[KR], qraw[KR], vraw[CL][REC_TB], draw = (TX)0.f;
   float araw = 1.f, braw = 0.f;
   // every load is unconditional, from an address clamped into the span and the slice; what lies outside becomes zero
@@ -558,10 +561,11 @@ __global__ void __launch_bounds__(64) recurrence_kernel(RecArgs a) {
         vraw[j][tt] = ((const TX*)a.v)[(tb + (tt < nt ? tt : nt - 1)) * a.v_stride + (int64_t)head[j] * a.P + p[j]];
     const int64_t at = tb + (my_tt < nt ? my_tt : nt - 1);
     if (a.dt) {
-      draw = ((const TX*)a.dt)[at * a.dt_stride + my_head];
+      const TX given = ((const TX*)a.dt)[at * a.dt_stride + my_head];
+      if constexpr (F32) araw = given; else draw = given;
     } else if (a.coef_a) {
-      araw = a.coef_a[at * a.H + my_head];
       braw = a.coef_b[at * a.H + my_head];
+      araw = a.coef_a[at * a.H + my_head];
     }
   };
   const float my_bias = a.dt ? a.dt_bias[my_head] : 0.f, my_rate = a.dt ? a.rate[my_head] : 0.f;
@@ -618,7 +622,7 @@ __global__ void __launch_bounds__(64) recurrence_kernel(RecArgs a) {
     }
     float areg = my_decay, breg = 1.f;
     if (a.dt) {
-      const float z = to_f32<TX>(draw) + my_bias;
+      const float z = (F32 ? araw : to_f32<TX>(draw)) + my_bias;
       const float step = z > 20.f ? z : log1pf(expf(z));
       areg = expf(-my_rate * step);
       breg = step;
