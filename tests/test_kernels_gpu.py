@@ -785,8 +785,8 @@ def test_library_product_is_called_directly(M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [(33, 4096, 12288), (256, 4096, 4096), (200, 2560, 9728), (300, 4096, 12288), (700, 5120, 8192), (200, 1368, 12288 + 64)])
 def test_linear_library_slices_of_k(M, N, K):
-    """o and down at 33 to 1,024 rows over large weights (where the tiled kernel's slices are not ahead): the library
-    runs slices of K as one strided batch and the consumer adds the float32 partial sums."""
+    """o and down at 33 to 1,024 rows over large weights (where the tiled kernel's slices are not ahead): the library, or up to 256
+    rows the kernel of large tiles, runs slices of K and the consumer adds the float32 partial sums."""
     from mini_engine_amd.kernels import ops
     splits = ops.library_splits(M, N, K)
     assert ops.mid_takes(M, N, K, True) == 0

@@ -54,6 +54,8 @@ def test_every_tile_at_its_edges(tile):
             _launch(x, w, y, 1, tile, 1)
             close(y, torch.nn.functional.silu(ref[:, :N // 2]) * ref[:, N // 2:], 6e-3)
             bias = torch.randn(N, device=DEV)
+            _launch(x, w, y, 1, tile, 2, bias)
+            assert torch.equal(y, hip().silu_and_mul(two, bias=bias))
             _launch(x, w, y, 1, tile, 1, bias)
             b = ref + bias.double()
             close(y, torch.nn.functional.silu(b[:, :N // 2]) * b[:, N // 2:], 6e-3)
@@ -71,6 +73,76 @@ def test_a_row_of_infinities_and_not_a_numbers_stays_in_its_row():
     assert torch.equal(got[keep], want[keep]) and bool(torch.isnan(got[299]).all()) and not bool(torch.isfinite(got[7]).any())
 
 
+class _Recorded:
+    """A library that notes the names of the entry points asked of it."""
+
+    def __init__(self, lib, names):
+        self._lib, self._names = lib, names
+        self.fns = {name: self._noting(name, fn) for name, fn in lib.fns.items()}
+
+    def _noting(self, name, fn):
+        def run(*args):
+            self._names.append(name)
+            return fn(*args)
+        return run
+
+    def call(self, name, *args):
+        self._names.append(name)
+        return self._lib.call(name, *args)
+
+    def __getattr__(self, name):
+        return getattr(self._lib, name)
+
+
+def _products(monkeypatch, run) -> tuple:
+    """The result of `run`, and the products and gating kernels that it launched."""
+    names, lib = [], ops.core()
+    with monkeypatch.context() as m:
+        m.setattr(ops, "core", lambda: _Recorded(lib, names))
+        y = run()
+    return y, [n[3:] for n in names]
+
+
+TILE, MID, LIBRARY, GATE = "gemm_tile_bf16", "gemm_mid_bf16", "gemm_library_bf16", "gate_mul"
+
+
+@pytest.mark.parametrize("M,N,K,route", [(300, 1024, 1024, TILE), (513, 1024, 3072, LIBRARY), (257, 6144, 1024, TILE), (200, 6144, 1024, TILE), (128, 6144, 1024, MID),
+                                         (1100, 4096, 2048, LIBRARY), (2048, 4096, 2048, TILE), (2048, 6144, 4096, LIBRARY), (2048, 24576, 4096, TILE), (300, 1028, 1024, LIBRARY)])
+def test_each_product_runs_where_the_rules_send_it(monkeypatch, M, N, K, route):
+    x, w = _operands(M, N, K)
+    y, ran = _products(monkeypatch, lambda: hip().linear(x, w))
+    assert ran == [route]
+    close(y, x.double() @ w.double().t(), 4e-3)
+
+
+@pytest.mark.parametrize("M,N,K,slices,route", [(512, 1024, 3072, 4, TILE), (64, 1024, 3072, 8, MID), (33, 4096, 12288, 8, TILE), (256, 4096, 4096, 8, TILE), (300, 4096, 12288, 4, LIBRARY),
+                                                (700, 5120, 8192, 2, LIBRARY), (200, 4100, 4096, 8, LIBRARY), (160, 5120, 25600, 8, LIBRARY)])
+def test_each_product_in_slices_runs_where_the_rules_send_it(monkeypatch, M, N, K, slices, route):
+    """Slices of K as float32 partial sums: crowded slices of the tiled kernel and few rows of the library's go to the tiles; what
+    the tiles cannot take (4,100 features) or are slower for (a K beyond 16,384) stays."""
+    x, w = _operands(M, N, K)
+    y, ran = _products(monkeypatch, lambda: hip().linear(x, w, None, allow_partials=True))
+    assert ran == [route] and y.shape == (slices, M, N) and y.dtype == torch.float32
+    close(y.sum(0), x.double() @ w.double().t(), 2e-5)
+
+
+@pytest.mark.parametrize("M,N,K,route", [(200, 6144, 1024, [TILE]), (512, 6144, 1024, [TILE]), (128, 6144, 1024, [MID]), (2048, 6144, 4096, [TILE]), (800, 24576, 4096, [LIBRARY, GATE]),
+                                         (300, 2048, 200, [LIBRARY, GATE])])
+@pytest.mark.parametrize("biased", [False, True])
+def test_each_gated_product_runs_where_the_rules_send_it(monkeypatch, M, N, K, route, biased):
+    """A packed gate/up map as the feed-forward calls it: one launch, or the product and the gating kernel."""
+    from mini_engine_amd.parts.linear import Linear
+    x, w = _operands(M, N, K)
+    part = Linear(K, N)
+    part.set_param("weight", w)
+    bias = torch.randn(N, device=DEV) if biased else None
+    y, ran = _products(monkeypatch, lambda: part.forward(x, gated=True, bias=bias))
+    assert ran == route
+    sums = x.double() @ w.double().t()
+    sums = sums + bias.double() if biased else sums
+    close(y, torch.nn.functional.silu(sums[:, :N // 2]) * sums[:, N // 2:], 1.5e-2)
+
+
 @pytest.mark.parametrize("M,N,K", [(300, 1024, 1024), (513, 1024, 3072), (257, 6144, 1024), (200, 6144, 1024), (1100, 4096, 2048), (2048, 6144, 4096)])
 def test_what_the_rules_send_there(M, N, K):
     """`linear` and `gated_linear` through the dispatch, replayed from a graph with other rows between the replays."""
@@ -78,9 +150,9 @@ def test_what_the_rules_send_there(M, N, K):
     assert ops.tile_fits(x, w)
     for _ in range(2):
         close(hip().linear(x, w), x.double() @ w.double().t(), 4e-3)
-    if ops.gated_linear_fuses(x, w):
-        # sums rounded before the gating: 2^-9 each of gate (times up to 1 + gate in its silu), up and result
-        close(hip().gated_linear(x, w), twin.gated_linear(x, w, compute_dtype=torch.float64), 1.5e-2)
+    assert ops.gated_linear_fuses(x, w)
+    # sums rounded before the gating: 2^-9 each of gate (times up to 1 + gate in its silu), up and result
+    close(hip().gated_linear(x, w), twin.gated_linear(x, w, compute_dtype=torch.float64), 1.5e-2)
     graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
