@@ -178,18 +178,19 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __rest
         for (int j = 0; j < MH; ++j)
           acc[hw * NH + i][hx * MH + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[hw][i][s], fx[j][s], acc[hw * NH + i][hx * MH + j], 0, 0, 0);
     __builtin_amdgcn_s_setprio(0);
-    tile_wait_lds();
     tile_barrier();
   };
   // Why no wait is missing. A region is read in one quarter q by both halves of the waves; the half that runs late reads it
   // half a quarter after, and has it in registers before the barrier behind its products, which the other half passes at the
-  // end of its reads of quarter q + 1. The request that overwrites the region is made in quarter q + 2. That holds for the operands
-  // of the quarter's own products and for those read a quarter ahead (features' first half, in quarter 3 and in front of the first
-  // step) because every barrier but the one between a quarter's reads and its products comes behind a wait for all reads of LDS;
-  // those read ahead have had the quarter's products to arrive. What quarter q reads
-  // has been waited for by the wave that asked for it in quarter q - 1 before a barrier that every reader has passed.
+  // end of its reads of quarter q + 1. The request that overwrites the region is made in quarter q + 2. The features' first half, read
+  // in quarter 3 (and in front of the first step) for the quarter behind, is waited for at the beginning of that quarter: a late wave
+  // has it before the barrier in front of its products, which an early wave passes in front of its quarter 1, where the request is made.
+  // It has had a quarter's products to arrive by then. (Four waves are never apart: there the products of quarter 0 wait in time.)
+  // What quarter q reads has been waited for by the wave that asked for it in quarter q - 1 before a barrier that every reader has
+  // passed.
   auto step = [&](int k, auto kind) {                                 // kind 0: two steps or more follow, 1: one, 2: none
     constexpr int KIND = decltype(kind)::value;
+    if (PING) tile_wait_lds();
     read_x(k, 0);
     if constexpr (KIND < 2) { ask(k + 1, TILE_INT(REGION_X1)); wait(TILE_INT(REGION_X1), TILE_INT(5)); } else wait(TILE_INT(REGION_X1), TILE_INT(1));
     multiply(0, 0);
@@ -218,7 +219,6 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __rest
   wait(TILE_INT(REGION_W1), TILE_INT(5));
   tile_barrier();
   read_w(0, 0, fw[0]);
-  tile_wait_lds();
   if (PING && late) tile_barrier();
   int k = 0;
   for (; k < steps - 2; ++k) step(k, TILE_INT(0));

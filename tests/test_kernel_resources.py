@@ -97,35 +97,40 @@ def test_the_recurrence_for_short_requests_leaves_room_for_three_waves(tmp_path)
     assert seen == {16, 32, 48, 64}
 
 
-def _reads_on_their_way(code: list) -> dict:
-    """The most LDS reads that can be on their way at each instruction, over all paths. `code`: (address, name, operands, the
-    address a branch goes to or None)."""
+def _late_reads(code: list) -> dict:
+    """The most LDS reads that can be on their way at each barrier although another barrier lies between, over all paths. `code`:
+    (address, name, operands, the address a branch goes to or None); reads come back in the order in which they were asked for."""
     place = {address: i for i, (address, *_) in enumerate(code)}
-    most, todo = {0: 0}, [0]
+    most, todo, late = {0: (0, 0)}, [0], {}                     # reads from before the last barrier, reads since
     while todo:
         i = todo.pop()
         _, name, operands, target = code[i]
-        n = most[i]
+        old, new = most[i]
         if name.startswith("ds_read"):
-            n = min(n + 1, 99)
-        elif name == "s_waitcnt":
-            m = re.search(r"lgkmcnt\((\d+)\)", operands)
-            n = min(n, int(m.group(1))) if m else n
+            new = min(new + 1, 99)
+        elif name == "s_waitcnt" and (m := re.search(r"lgkmcnt\((\d+)\)", operands)):
+            new = min(new, int(m.group(1)))
+            old = min(old, int(m.group(1)) - new)
+        elif name == "s_barrier":
+            late[i] = max(late.get(i, 0), old)
+            old, new = min(old + new, 99), 0
         after = [] if name == "s_endpgm" else [i + 1]
         if target is not None:
             after = [place[target]] + (after if name.startswith("s_cbranch") else [])
         for j in after:
-            if j < len(code) and most.get(j, -1) < n:
-                most[j] = n
+            was = most.get(j, (-1, -1))
+            now = (max(was[0], old), max(was[1], new))
+            if j < len(code) and now != was:
+                most[j] = now
                 todo.append(j)
-    return most
+    return late
 
 
 @pytest.mark.skipif(OBJDUMP is None, reason="no llvm-objdump")
 def test_tile_products_read_lds_before_others_may_write_it(tmp_path):
-    """Every barrier of the tile product's kernels but the one in front of a quarter's products, which raises the wave's priority
-    behind itself, has no LDS read on its way: what is read a quarter ahead is in registers before another wave can ask for
-    the load that writes over it."""
+    """What a wave of the tile product's kernels reads a quarter ahead is in registers before another wave can ask for the load that
+    writes over it: with eight waves, of which half run later than the others, before the next barrier in front of a quarter's products
+    (one that raises the wave's priority behind itself), with four before the next barrier."""
     library = os.path.join(build.PKG_LIB, "libme_core.so")
     if not os.path.exists(library):
         pytest.skip("the core library is not built")
@@ -136,18 +141,17 @@ def test_tile_products_read_lds_before_others_may_write_it(tmp_path):
         path = tmp_path / f"{i}.elf"
         path.write_bytes(blob)
         text = subprocess.run([OBJDUMP, "-d", str(path)], capture_output=True, text=True, check=True).stdout
-        for part in re.split(r"^([0-9a-f]+) <(\S*gemm_tile_kernel\S*)>:$", text, flags=re.M)[1:][2::3]:
+        pieces = re.split(r"^[0-9a-f]+ <(\S*gemm_tile_kernel\S*)>:$", text, flags=re.M)[1:]
+        for name, part in zip(pieces[::2], pieces[1::2]):
             kernels += 1
             code = []
             for line in part.splitlines():
                 if m := re.match(r"\s+(\w+)(.*?)\s*// ([0-9A-F]+):.*?(?:<\S+?\+0x([0-9a-f]+)>)?$", line):
                     code.append((int(m.group(3), 16), m.group(1), m.group(2), m.group(4)))
             code = [(a, name, ops, code[0][0] + int(to, 16) if to and name.startswith(("s_branch", "s_cbranch")) else None) for a, name, ops, to in code]
-            most = _reads_on_their_way(code)
-            names = [name for _, name, _, _ in code]
-            for j in [j for j, name in enumerate(names) if name == "s_barrier"]:
-                if names[j + 1] == "s_setprio" and int(code[j + 1][2]) == 1:
-                    continue
-                barriers += 1
-                assert most[j] == 0, (kernels, hex(code[j][0]), most[j])
+            waves = int(re.search(r"ILi(\d+)ELi(\d+)E", name).group(1)) * int(re.search(r"ILi(\d+)ELi(\d+)E", name).group(2))
+            for j, late in _late_reads(code).items():
+                if waves == 4 or (code[j + 1][1] == "s_setprio" and int(code[j + 1][2]) == 1):
+                    barriers += 1
+                    assert late == 0, (name, hex(code[j][0]), late)
     assert kernels == 30 and barriers >= kernels * 12        # 12 quarters in the code of a kernel
