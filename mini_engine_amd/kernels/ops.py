@@ -1646,8 +1646,7 @@ TILE_GATING = {(256, 256): -0.8, (256, 192): 0.9, (192, 256): 1.0, (128, 256): 1
                (128, 128): -1.5, (64, 128): -1.3, (128, 64): -1.3, (64, 64): -1.4}
 TILE_MIN_ROWS = 33
 TILE_SURE_K = 1024
-TILE_LEVEL_K = 2048
-TILE_LEVEL_FILL = 0.8
+TILE_FILL = 0.8
 TILE_USED_ROWS = 0.86
 TILE_SLICES_MAX_M = 256          # library / own tiles, us: 40-256 rows of 44 weights and row counts 1.2 on average, from 300 rows on 1.0
 TILE_SLICES_MAX_K = 16384        # ... (2560 x 4096 at 200 rows 17.4 / 13.9, at 512 17.8 / 20.0); 5120 x 25600 at 160 rows 64 / 74
@@ -1673,24 +1672,27 @@ def tile_choice(M: int, N: int, K: int, slices: int = 1, gated: bool = False) ->
 def tile_takes(M: int, N: int, K: int) -> bool:
     """Whether the product of M rows against a bfloat16 weight [N, K] that neither the kernels for few rows nor slices of K
     take goes to csrc/gemm_tile.hip rather than to the library. Timed beside each other over 26 weights of the layer sizes of 0.6B to
-    32B, 33 to 8,192 rows (library / this, us):
-    tiles of 256 x 256 are ahead in each of 114 products (1.07-2.7 times: 2,048 rows of 24576 x 4096 348 / 305, 4,096 of 4096 x 1024
+    32B, 33 to 8,192 rows, repeated and in a replayed chain with other kernels and weights that come from memory (library / this, us):
+    tiles of 256 x 256 are ahead in each of 114 products (1.07-2.8 times: 2,048 rows of 24576 x 4096 348 / 305, 4,096 of 4096 x 1024
     36.6 / 32.4); the other tiles have fewer products for an operand read, and the library has more shapes of them;
-    over a K of up to 1,024, where the library's launches take 11 us at least, they are ahead by 1.17 on average (512 rows of 4096 x 1024
-    10.9 / 9.0; of 108 products 9 are behind by 3 to 10 %, 800 of 6144 x 1024 15.8 / 17.6);
-    up to 2,048 level or ahead where the tiles fill their rounds over the compute units to four fifths (2,048 rows of 4096 x 2048
-    34.2 / 33.0), mostly behind where they do not (1,280 of it 25.0 / 28.3; but 200 of 12288 x 2048 26.9 / 22.2) and with those of
-    192 x 256 (800 of 12288 x 2048 39.5 / 43.9); over a longer K behind by 3 to 70 % in half of the products (1,536 of 4096 x 12288
-    140 / 155) and ahead by more in a sixth."""
+    those of 256 x 128 and 256 x 192 are level or ahead where they fill their rounds over the compute units to four fifths
+    (2,048 rows of 4096 x 12288 176 / 169, of 4096 x 2048 34.2 / 33.0; in a prompt of 2,048 tokens 118 / 114 on average) and behind where they
+    do not (1,536 rows of 4096 x 12288 140 / 155, 1,280 of 4096 x 2048 25.0 / 28.3);
+    over a K of up to 2,048 those of 128 x 128 are level (900 rows of 4096 x 2048 25.4 / 23.2, 3,123 of 1024 x 2048 22.2 / 23.2) and ahead
+    between many other kernels (the latter in a prompt of two requests 25.0 / 20.5);
+    over a K of up to 1,024, where the library's launches take 11 us at least, all are ahead by 1.04 to 1.17 on average (512 rows of
+    4096 x 1024 10.9 / 9.0; the worst of 108 products 800 rows of 6144 x 1024 15.8 / 17.6).
+    The others are behind: 192 x 256 (800 rows of 12288 x 2048 39.5 / 43.9, 1,800 of 5120 x 25600 375 / 415), the small ones over a
+    K beyond 1,024 (64 x 64 0.88 and 128 x 64 0.93 times as fast on average; 700 rows of 1024 x 2048 in a prompt 13.1 / 15.6)."""
     if M < TILE_MIN_ROWS or N >= LIBRARY_MIN_N and M < 128:
         return False
     if K <= TILE_SURE_K:
         return True
     rows, features = tile = tile_choice(M, N, K)[0]
-    if tile == (256, 256):
+    if tile == (256, 256) or tile == (128, 128) and K <= 2 * TILE_SURE_K:
         return True
     rounds = -(-(-(-M // rows) * -(-N // features)) // _COMPUTE_UNITS)
-    return K <= TILE_LEVEL_K and tile != (192, 256) and M * N >= TILE_LEVEL_FILL * rounds * _COMPUTE_UNITS * rows * features
+    return tile in ((256, 128), (256, 192)) and M * N >= TILE_FILL * rounds * _COMPUTE_UNITS * rows * features
 
 
 def tile_fits(x: torch.Tensor, w: torch.Tensor, slices: int = 1) -> bool:

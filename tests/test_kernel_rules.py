@@ -291,7 +291,8 @@ def test_tiles_for_many_rows_fit_the_kernel_and_leave_what_it_cannot_take():
 # rows, features, K: us of the library's product and of the own tile that `tile_choice` takes, timed in turn on one MI355X
 PRODUCTS = [(2048, 24576, 4096, 348, 305), (4096, 4096, 1024, 36.6, 32.4), (512, 4096, 1024, 10.9, 9.0), (1800, 5120, 25600, 375, 415), (1800, 10240, 5120, 168, 183),
             (4096, 5120, 8192, 270, 291), (800, 24576, 4096, 139, 166), (1536, 4096, 12288, 140, 155), (1280, 4096, 2048, 25.0, 28.3), (800, 12288, 2048, 39.5, 43.9),
-            (40, 12288, 2048, 16.1, 17.8), (2048, 4096, 2048, 34.2, 33.0), (2048, 1024, 2048, 15.9, 14.9), (2048, 1024, 1024, 11.3, 9.1), (6000, 4096, 4096, 157, 164)]
+            (40, 12288, 2048, 16.1, 17.8), (200, 12288, 2048, 26.9, 22.2), (2048, 4096, 2048, 34.2, 33.0), (2048, 4096, 12288, 176, 169), (2048, 4096, 4096, 60.9, 60.4),
+            (2048, 1024, 1024, 11.3, 9.1), (6000, 4096, 4096, 157, 164), (900, 4096, 2048, 25.4, 23.2), (700, 1024, 2048, 13.1, 15.6), (3123, 1024, 2048, 25.0, 20.5)]
 # the library's product with the gating kernel behind it, and the tile with the gating in its epilogue
 GATED_PRODUCTS = [(512, 6144, 1024, 19.5, 11.8), (2048, 6144, 1024, 37.4, 31.9), (350, 24576, 4096, 84.4, 82.7),
                   (780, 24576, 4096, 149.2, 166.7), (800, 24576, 4096, 151.3, 171.2), (880, 24576, 4096, 177.2, 169.2), (512, 24576, 4096, 97.8, 92.9), (2048, 24576, 4096, 384.6, 318.4),

@@ -107,7 +107,7 @@ TILE, MID, LIBRARY, GATE = "gemm_tile_bf16", "gemm_mid_bf16", "gemm_library_bf16
 
 
 @pytest.mark.parametrize("M,N,K,route", [(300, 1024, 1024, TILE), (513, 1024, 3072, LIBRARY), (257, 6144, 1024, TILE), (200, 6144, 1024, TILE), (128, 6144, 1024, MID),
-                                         (1100, 4096, 2048, LIBRARY), (2048, 4096, 2048, TILE), (2048, 6144, 4096, LIBRARY), (2048, 24576, 4096, TILE), (300, 1028, 1024, LIBRARY)])
+                                         (1100, 4096, 2048, LIBRARY), (2048, 4096, 2048, TILE), (2048, 6144, 4096, TILE), (1536, 4096, 4096, LIBRARY), (2048, 24576, 4096, TILE), (300, 1028, 1024, LIBRARY)])
 def test_each_product_runs_where_the_rules_send_it(monkeypatch, M, N, K, route):
     x, w = _operands(M, N, K)
     y, ran = _products(monkeypatch, lambda: hip().linear(x, w))
