@@ -17,9 +17,9 @@
 // What bounds it: the matrix pipes at the clock that a full chip keeps for tiles of 256 x 256 (8,192 x 8,192 x 8,192: 1,554
 // TFLOP/s, the library's kernel 1,307); the reads of LDS for the others, whose waves have fewer products for an operand read
 // (256 x 128: 176 KB of LDS traffic a step at 128 bytes a cycle is 0.6 us, which is what a step takes; 128 x 128 96 KB, 0.33
-// of 0.44 us). us, the library / this: 2,048 rows of 24576 x 4096 362 / 290 (with the gating 362 + 28 of a kernel behind
-// it / 307), of 6144 x 4096 90 / 78, of 4096 x 4096 57 / 56, of 4096 x 12288 168 / 158, of 6144 x 1024 26.2 / 24.8 (with the
-// gating 30.5), of 1024 x 2048 15.3 / 13.3; 512 rows of 4096 x 1024 11.2 / 8.6, of 6144 x 1024 with the gating 13.3 + 4.4 / 11.6.
+// of 0.44 us). us, the library / this: 2,048 rows of 24576 x 4096 348 / 303 (with the gating 385 with a kernel
+// behind it / 310), of 6144 x 4096 83 / 81, of 4096 x 4096 61 / 58, of 4096 x 12288 176 / 163, of 6144 x 1024 28.6 / 27.6 (with
+// the gating 37.4 / 30.0), of 4096 x 1024 22.2 / 19.1; 512 rows of 4096 x 1024 10.9 / 9.0, of 6144 x 1024 with the gating 19.5 / 11.8.
 // Sums that are rounded before the gating, with the library's exponential, cost a tile 1-3 us more than unrounded ones would
 // (281 and 23.4): the bits stay those of the product and the gating kernel.
 //
