@@ -12,6 +12,7 @@ v1/v2 decode dispatcher), and the eager torch ops named in each docstring.
 from __future__ import annotations
 
 import ctypes
+import math
 from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p
 from functools import lru_cache
 
@@ -581,7 +582,7 @@ class HipBackend:
                allow_partials: bool = False, out: torch.Tensor | None = None):
         """x [M, K] . w[N, K]^T (reference layers/linear.py:25-26: F.linear, no bias).
 
-        float32: the float32 matrix instructions (f32_tile). bfloat16: the skinny MFMA kernel for up to 32 rows (64 for
+        float32: three bfloat16 parts of every operand (f32_tile). bfloat16: the skinny MFMA kernel for up to 32 rows (64 for
         smaller weights or when K is split), the tiled kernel up to 256 rows over small weights (mid_takes), the kernel of
         large tiles for more rows (tile_takes, mid_crowded), the library product (hipBLASLt, library_product) for what is
         left of them, for the head over a large vocabulary and for large weights with several rows
@@ -1316,8 +1317,10 @@ class HipBackend:
 
 # Dispatch rules. Every threshold below was measured on one MI355X at the layer sizes of Qwen3-0.6B, 8B and 32B;
 # the tables behind each constant are kept in the repository's design notes, one line of reason here.
-# microseconds that one round of the float32 product's tiles takes over a K of 1,024: alone, and each of several
-F32_ROUND_US = {(16, 16): (6.9, 5.9), (16, 32): (7.5, 7.1), (32, 32): (9.2, 9.0), (64, 32): (12.0, 13.5), (64, 64): (19.7, 29.5)}
+# what one round of the float32 product's tiles costs over a K of 1,024 (us, fitted: see f32_tile): alone, and each of several; a
+# tile that was never the best one alone, or never in several rounds, is not taken there
+F32_ROUND_US = {(16, 16): (4.7, 15.3), (16, 32): (8.2, math.inf), (32, 32): (11.3, math.inf), (64, 32): (math.inf, 8.3),
+                (32, 64): (13.7, 8.8), (64, 64): (14.7, 15.7), (64, 128): (math.inf, 27.4)}
 SKINNY_MAX_M = 32                          # rows up to which the skinny kernel beats the library product
 SKINNY_WIDE_MAX_M = 64                     # ... for weights of up to SKINNY_WIDE_MAX_WEIGHT elements
 SKINNY_WIDE_MAX_WEIGHT = 5 * 1024 * 1024
@@ -1443,14 +1446,14 @@ SKINNY_WIDE_MIN_WEIGHT = 1 << 22
 
 def f32_tile(M: int, N: int) -> tuple:
     """(rows, features) of the float32 product's tile: the one whose rounds of workgroups over the compute units cost least
-    (F32_ROUND_US; the bits of a result do not depend on it). Of 195 products of 1 to 3,000 rows, 384 to 24,576 features and 80 to
-    12,288 terms it picks one within 10 % of the best tile for 179; the worst are few features in part of a round (300 rows of 384
-    features of 3,072 terms 38 us, 26 with 32 x 32)."""
+    (F32_ROUND_US; the bits of a result do not depend on it), of those that are not half empty. Of 414 products of 1 to 2,048 rows,
+    384 to 151,936 features and 512 to 6,144 terms it picks one within 10 % of the best tile for 401, 1.3 % behind it on average; the
+    worst are few features in part of a round (300 rows of 384 features of 3,072 terms 17.3 us, 14.9 with 16 x 16)."""
     def cost(tile):
         rounds = -(-(-(-M // tile[0]) * -(-N // tile[1])) // _COMPUTE_UNITS)
         first, more = F32_ROUND_US[tile]
         return first if rounds == 1 else rounds * more
-    return min(F32_ROUND_US, key=cost)
+    return min((t for t in F32_ROUND_US if t[0] == 16 or t[0] < 2 * M), key=cost)
 
 
 def skinny_wide(N: int, K: int) -> int:

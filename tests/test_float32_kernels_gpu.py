@@ -40,6 +40,40 @@ def test_product_tiles(M, N, K):
     assert torch.equal(hip().linear(odd, w), first)
 
 
+@pytest.mark.parametrize("M,N,K", [(2, 40, 32), (19, 33, 100), (50, 150, 516), (130, 64, 300)])
+def test_product_by_parts(M, N, K):
+    """Values are split into three parts exactly: weights that came as bfloat16, weights with all bits, and both in one launch,
+    block by block along K, give every tile the same bits; against 64 bits the error is that of float32 sums. Infinities and what is
+    not a number come out as plain float32 sums give them, and leave the other outputs their bits."""
+    g = torch.Generator(device=DEV).manual_seed(M * K)
+    x = torch.randn(M, K, device=DEV, generator=g) * torch.exp(4 * torch.randn(M, K, device=DEV, generator=g))
+    full = torch.randn(N, K, device=DEV, generator=g)
+    mixed = full.to(torch.bfloat16).float()
+    mixed[N // 2:, K // 3:] = full[N // 2:, K // 3:]
+    for w in (full, full.to(torch.bfloat16).float(), mixed):
+        first = _product(x, w, TILES[0])
+        assert all(torch.equal(_product(x, w, tile), first) for tile in TILES[1:])
+        # of the sum of the products' sizes: 2^-24 for each sum that is rounded, twice for each of a chain's matrix instructions (its
+        # own 32 terms, then with what was there; six for a block of 32, a chain has every fourth block) and two where chains
+        # meet, and 3 x 2^-24 of a product for the three products of parts that are not formed
+        bound = 2.0 ** -24 * (12 * -(-K // 128) + 2 + 3) * (x.double().abs() @ w.double().abs().T)
+        assert bool(((first.double() - x.double() @ w.double().T).abs() <= bound).all())
+    odd = x.clone()
+    odd[0, 3], odd[M - 1, K - 1] = float("inf"), float("nan")
+    w = full.clone()
+    w[N - 1, 1], w[N // 2, 0] = -float("inf"), 3.4e38          # rounds up to an infinity in bfloat16
+    for tile in TILES:
+        got = _product(odd, w, tile)
+        assert torch.isnan(got[M - 1]).all()
+        assert torch.equal(got[0, : N // 2], torch.sign(w[: N // 2, 3]) * float("inf"))
+        rows = slice(1, M - 1)
+        assert torch.equal(got[rows, N - 1], -torch.sign(x[rows, 1]) * float("inf"))
+        assert torch.equal(got[rows, : N // 2], _product(x, full, tile)[rows, : N // 2])
+        want = odd[rows].double() @ w[N // 2].double()
+        inside = want.abs() < 3e38
+        assert torch.allclose(got[rows, N // 2].double()[inside], want[inside], rtol=1e-5)
+
+
 @pytest.mark.parametrize("Hq,Hkv,D,page", [(4, 2, 16, 4), (3, 1, 80, 8), (6, 2, 112, 16), (2, 2, 128, 12), (4, 4, 96, 64)])
 @pytest.mark.parametrize("extra", [{}, {"window": 20}, {"window": 37, "keep_first": 5}, {"chunk": 24}, {"softcap": 3.0}])
 def test_attention_tiles(Hq, Hkv, D, page, extra):
