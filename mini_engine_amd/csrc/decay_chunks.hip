@@ -16,12 +16,6 @@
 #include "decay.h"
 #include <type_traits>
 
-#define DC_TOKENS 16
-
-// Chunk i of request b has place cu[b] / 16 + b + i (whole division): the places of two requests never meet, there are at most T / 16 +
-// B, and neither the host nor a scan over the requests is needed to give them out.
-__device__ __forceinline__ int64_t chunk_place(const int32_t* cu, int b) { return cu[b] / DC_TOKENS + b; }
-
 // Floats that a chunk of one head takes: c q [tokens, rows], what it writes (K^) [rows, tokens], c_16, A; delta rules: c k, T; and v.
 __host__ __device__ constexpr int chunk_fixed(int rows, bool delta) { return (delta ? 49 : 33) * rows + (delta ? 512 : 256); }
 __host__ __device__ constexpr int64_t chunk_floats(int rows, bool delta, int col_blocks) { return chunk_fixed(rows, delta) + (int64_t)256 * col_blocks; }
@@ -41,15 +35,7 @@ decay_chunk_kernel(DrArgs a, int num_seqs, int col_blocks, float* __restrict__ c
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t place = blockIdx.x;
   const int h = blockIdx.y, g = h / (a.H / a.G);
-  // the request: the last one whose first place is not behind this one
-  int b = -1;
-  for (int b0 = 0; b0 < num_seqs; b0 += 64) {
-    const bool in = b0 + lane < num_seqs && chunk_place(a.cu, min(b0 + lane, num_seqs - 1)) <= place;
-    const int count = __popcll(__ballot(in));
-    b += count;
-    if (count < 64) break;
-  }
-  b = __builtin_amdgcn_readfirstlane(b);
+  const int b = chunk_request(a.cu, num_seqs, place, lane);
   if (b < 0) return;
   const int begin = a.cu[b], at = (int)(place - chunk_place(a.cu, b)) * C, n_tok = min(C, a.cu[b + 1] - begin - at);
   if (n_tok <= 0) return;
@@ -289,28 +275,6 @@ decay_chunk_walk_kernel(DrArgs a, const float* __restrict__ chunks, int groups, 
     o.v = at(from + FIXED + cb * 256, lane16);
     asm volatile("" ::: "memory");
   };
-  // acc += M X for a 16 x 16 matrix M of this chunk (a lane has four of its numbers) that is zero above its diagonal
-  auto lower = [&](const f32x4& M, const f32x4& X, f32x4 acc) {
-    // a zero times what is not a number would reach the tokens in front of it: then row by row, later tokens taken out
-    float odd = 0.f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) odd = fmaf(X[e], 0.f, odd);
-    if (__builtin_expect(__ballot(odd != 0.f) != 0, 0)) {
-      f32x4 r = acc;
-#pragma unroll 1
-      for (int i = 0; i < C; ++i) {
-        f32x4 one = acc;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) one = __builtin_amdgcn_mfma_f32_16x16x4f32(M[e], 4 * g + e <= i ? X[e] : 0.f, one, 0, 0, 0);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = 4 * g + e == i ? one[e] : r[e];
-      }
-      return r;
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(M[e], X[e], acc, 0, 0, 0);
-    return acc;
-  };
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   // this wave's rows of M^T S, [tokens, columns]
   auto read_state = [&](const f32x4* M) {
@@ -351,7 +315,7 @@ decay_chunk_walk_kernel(DrArgs a, const float* __restrict__ chunks, int groups, 
           __syncthreads();                                   // the other buffer's sums have been read by all when this is passed again
           u -= sum_of(part_u[d & 1]);
           read = read_state(c.q);
-          u = lower(c.T, u, zero);
+          u = chunk_lower(c.T, u, zero, g);
         } else {
           read = read_state(c.q);
         }
@@ -373,7 +337,7 @@ decay_chunk_walk_kernel(DrArgs a, const float* __restrict__ chunks, int groups, 
 #pragma unroll
     for (int d = ME; d < 4; d += WAVES) {
       if (WHOLE || i0 + d < count) {
-        const f32x4 y = lower(A[d / WAVES], U[d / WAVES], sum_of(sums[d]));
+        const f32x4 y = chunk_lower(A[d / WAVES], U[d / WAVES], sum_of(sums[d]), g);
         float* to = out + (int64_t)(C * (i0 + d)) * (a.H * a.P);
 #pragma unroll
         for (int e = 0; e < 4; ++e)

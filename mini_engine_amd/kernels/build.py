@@ -29,7 +29,7 @@ HIPCC_FLAGS = [
     "-Wno-unused-command-line-argument", "-Wno-unknown-attributes",
 ]
 CORE_SOURCES = ["elementwise.hip", "rope_kv.hip", "attention_simple.hip",
-                "gemm.hip", "gemm_f32.hip", "gemm_mid.hip", "gemm_tile.hip", "gemm_library.hip", "sampling.hip", "recurrent.hip", "parallel.hip", "moe.hip", "hybrid.hip", "decay_chunks.hip", "latent.hip",
+                "gemm.hip", "gemm_f32.hip", "gemm_mid.hip", "gemm_tile.hip", "gemm_library.hip", "sampling.hip", "recurrent.hip", "parallel.hip", "moe.hip", "hybrid.hip", "decay_chunks.hip", "linear_chunks.hip", "latent.hip",
                 "streams.hip"]
 ATTN_SOURCE = "attention_mfma.hip"
 HEADERS = ["common.h", "errors.inc", "sampling.h", "decay.h"]

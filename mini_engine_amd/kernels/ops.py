@@ -104,6 +104,7 @@ _CORE_PROTOS = {
     "me_token_shift": [P, L, I, P, I, P, L, P, P, P, P, L, I, P],
     "me_decay_rows_recurrence": [P, L, P, L, P, L, P, L, P, L, I, P, P, P, P, L, P, P, P, I, I, I, I, I, I, I, F, F, I, L, P, P],
     "me_decay_rows_chunks": [P, L, P, L, P, L, P, L, P, L, P, P, P, P, L, P, P, P, I, I, I, I, I, I, I, F, F, L, P, L, P],
+    "me_linear_chunks": [P, L, P, L, P, L, P, L, P, P, P, P, P, L, P, P, P, I, I, I, I, I, I, L, P, L, P],
     "me_sample": [P, L, P, P, P, P, I, I, P],
     "me_sample_static": [P, L, P, P, P, I, I, P],
 }
@@ -820,7 +821,7 @@ class HipBackend:
         on too. With gates the summed keys are kept beside the states, n_t = a_t n_(t-1) + b_t k_t (`key_state`: a float32 view [slots,
         H * N] of the same state rows), and the result is a `MemoryReads` for `memory_readout`. `silu`: q, k and v pass silu
         on their way in. `q_lens`: the requests' token counts on the host: long ones are cut into spans that run side
-        by side (`recurrence_spans`). Returns float32 [T, H * P], or partial sums [S, T, H * P] over slices of N
+        by side (`recurrence_spans`), or taken sixteen tokens at a time (`linear_chunks_take`). Returns float32 [T, H * P], or partial sums [S, T, H * P] over slices of N
         for a consumer that adds them."""
         T, B = v.shape[0], state_slots.numel()
         dtype = v.dtype
@@ -854,6 +855,16 @@ class HipBackend:
                         *(none if gates is None else (None, None, key_state.data_ptr(), dot.data_ptr(), T * H)),
                         *(no_gates if gates is None else gates.args()), _stream())
             return y if gates is None else MemoryReads(y, dot, None, gates)
+        if gates is None and linear_chunks_take(dtype, H, N, P, q_lens):
+            NR = 32 if N <= 32 else 64 if N <= 64 else 128
+            room = (T // 16 + B) * (G * (32 * NR + 256) + H * (304 + 256 * -(-P // 16)))
+            chunks = _scratch(room, v.device, "recurrence")
+            y = torch.empty((T, H * P), dtype=torch.float32, device=v.device)
+            core().call("me_linear_chunks", q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), _ptr(dt),
+                        0 if dt is None else dt.stride(0), _ptr(decay), _ptr(dt_bias), _ptr(rate), _ptr(skip), state.data_ptr(), state.stride(0),
+                        state_slots.data_ptr(), cu_seqlens.data_ptr(), y.data_ptr(), B, H, G, N, P, int(silu), T, chunks.data_ptr(), chunks.numel(),
+                        _stream())
+            return y
         per_wave = recurrence_rows_per_wave(N)
         slices = -(-N // per_wave)
         columns = recurrence_columns(q_lens, H, G, P, slices) if gates is None else 1
@@ -1955,6 +1966,28 @@ def expert_tile_rows(T: int, top: int, E: int) -> int:
 
 
 DECAY_PREPARE_MIN_TOKENS = 9      # requests of this many tokens or more: the tokens' values are shaped by a kernel of its own
+
+
+LINEAR_CHUNKS_MIN_TOKENS = 16            # ... of the longest request while (request, head, 64 columns) triples are up to LINEAR_CHUNKS_FEW,
+LINEAR_CHUNKS_FEW = 256
+LINEAR_CHUNKS_MIN_TOKENS_MORE = 64       # ... with more of them and fewer than LINEAR_CHUNKS_MANY requests,
+LINEAR_CHUNKS_MANY = 64
+LINEAR_CHUNKS_MIN_TOKENS_MANY = 128      # ... and with that many
+
+
+def linear_chunks_take(dtype, H: int, N: int, P: int, q_lens) -> bool:
+    """Whether `linear_recurrence` takes sixteen tokens of a request at a time (csrc/linear_chunks.hip): bfloat16 rows, as many state
+    rows as four waves hold, and requests long enough. A chunk costs the same whether it has sixteen tokens or one, so what counts is how
+    long the longest request, the other form's chain, is beside all of them. us, pieces of four tokens / chunks: one request, 16
+    heads of 128 x 128, of 16 tokens 15.2 / 10.2, of 64 38 / 12, of 350 82 / 27, of 2,048 168 / 98; 8 of 16 tokens 17.3 / 17.1 (32 heads 25 / 28),
+    of 64 47 / 27, of up to 350 161 / 51; 64 requests of 16 65 / 82, of 60 154 / 133, 8 heads of 64 x 64, of 40 30 / 32; one of 64 among 300 of one
+    token 278 / 362, one of 300 among 200 535 / 242; 16 of 700 685 / 320."""
+    if dtype != torch.bfloat16 or N > 128:
+        return False
+    longest, count = max(q_lens), len(q_lens)
+    if count * H * -(-P // 64) <= LINEAR_CHUNKS_FEW:
+        return longest >= LINEAR_CHUNKS_MIN_TOKENS
+    return longest >= (LINEAR_CHUNKS_MIN_TOKENS_MORE if count < LINEAR_CHUNKS_MANY else LINEAR_CHUNKS_MIN_TOKENS_MANY)
 
 
 DECAY_CHUNKS_MIN_TOKENS = 128
