@@ -4,8 +4,11 @@
 // projection's rows, an elementwise sigmoid gate). Everything that the recurrence reads
 // besides the projections is formed here in float32: decays and their exponentials, softplus, write strengths, unit
 // lengths.
-#include "decay.h"
+#include "common.h"
 #include <type_traits>
+
+__device__ __forceinline__ float hy_sigmoid(float v) { return 1.0f / (1.0f + expf(-v)); }
+__device__ __forceinline__ float hy_softplus(float v) { return v > 20.f ? v : log1pf(expf(v)); }
 
 // Four adjacent values at an address of four elements' alignment, and the test for it.
 template <typename T> struct Four;
@@ -417,7 +420,67 @@ extern "C" int me_token_shift(const void* x, int64_t x_stride, int dtype, const 
 // their way while the current eight are worked on, so a wave waits for memory once per eight tokens. The products
 // and sums of the walk are written as explicit fused multiply-adds: a token's result then does not depend on its place
 // among the eight (the compiler is free to fuse each unrolled copy otherwise).
+struct DrArgs {
+  const void* q; const void* k; const void* v; const void* raw; const void* beta;
+  int64_t q_stride, k_stride, v_stride, raw_stride, beta_stride;
+  const float* base; const float* rate; const float* bonus;
+  float* state; int64_t state_stride;
+  const int32_t* slots; const int32_t* cu;
+  float* y;
+  int H, G, N, P;
+  int unit; float unit_eps, q_scale;
+};
+
 #define DR_TB 8          // tokens whose shared values are formed at once and wait in LDS
+
+// Sum over the RG neighbouring lanes that share a state column (RG 1, 4 or 16, aligned groups), left in all of them: lane
+// exchanges inside a row of 16 lanes (quad permutations, then rotations of the row), no trip through LDS.
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+template <int RG>
+__device__ __forceinline__ float group_sum(float v) {
+  if (RG >= 2) v += dpp_f<0xB1>(v);      // quad_perm [1, 0, 3, 2]
+  if (RG >= 4) v += dpp_f<0x4E>(v);      // quad_perm [2, 3, 0, 1]
+  if (RG >= 8) v += dpp_f<0x124>(v);     // row_ror 4
+  if (RG >= 16) v += dpp_f<0x128>(v);    // row_ror 8
+  return v;
+}
+
+// What a token's q, k, raw decay and write strength become before the recurrence reads them, for one wave that holds
+// rows lane, lane + 64, ... of one head: q and k at unit length and scaled, the decay, and the token's own number
+// (sigmoid(beta), or sum_n q_n bonus_n k_n under the bonus rule), which every lane gets.
+// (RULE 3: every lane holds the head's one raw decay and its base in d[0], base[0] and gets the decay there.)
+template <int PER, int RULE>
+__device__ __forceinline__ float shape_token(const DrArgs& a, int lane, int nr_rows, float (&q)[PER], float (&k)[PER], float (&d)[PER],
+                                             const float (&base)[PER], const float (&bonus)[PER], float rate, float beta) {
+  float qs = a.q_scale, ks = 1.0f;
+  if (a.unit) {
+    float q2 = 0.f, k2 = 0.f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) { q2 += q[i] * q[i]; k2 += k[i] * k[i]; }
+    qs = a.q_scale / sqrtf(wave_sum(q2) + a.unit_eps);
+    ks = 1.0f / sqrtf(wave_sum(k2) + a.unit_eps);
+  }
+  float own = 0.f;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int n = lane + 64 * i;
+    q[i] *= qs;
+    k[i] *= ks;
+    if (RULE == 3) continue;
+    float dv;
+    if (RULE == 0) dv = expf(-expf(d[i] + base[i]));
+    else if (RULE == 2) dv = expf(-rate * hy_softplus(-(d[i] + base[i])));
+    else dv = expf(-rate * hy_softplus(d[i] + base[i]));
+    d[i] = (n < a.N && n < nr_rows) ? dv : 1.0f;
+    own += q[i] * bonus[i] * k[i];
+  }
+  if (RULE == 3) d[0] = expf(-rate * hy_softplus(d[0] + base[0]));
+  if (RULE == 2) return 0.f;
+  return (RULE == 1 || RULE == 3) ? hy_sigmoid(beta) : wave_sum(own);
+}
 
 // One wave per (token, head): the shaped values of every token at once, for a recurrence kernel that then only streams
 // them (decay_walk_kernel): pre_q, pre_k, pre_d [T, H, NR] and pre_x [T, H], float32. The rows of a (token, head) lie in the

@@ -4,12 +4,12 @@
 //   S <- c_16 S + sum_j k_j ((a_{j+1} ... a_16) b_j v_j)^T
 // as products on the float32 matrix instructions. The decays are numbers per token here, so q, k and q . k are the same for all heads of
 // a group. A first kernel lays out q, k and their products per chunk and group, decays and v per chunk and head; a second walks a
-// request's chunks as decay_chunk_walk_kernel does. Every product of decays is formed as such (an exponential of a sum, or a power of a
+// request's chunks. Every product of decays is formed as such (an exponential of a sum, or a power of a
 // fixed decay), none by a division. us, four tokens at a time in spans side by side (recurrent.hip) / so, both kernels: 8 requests of up to
 // 350 tokens, 16 heads of 128 x 128, fixed decays, 161 / 51, 32 heads of 128 x 64 over shared keys with step sizes 146 / 46; one of 2,048
 // tokens 168 / 98, 153 / 91; 16 of 700 685 / 320, 591 / 224. Error against 64 bits (700 tokens, relative to the norm of y): fixed decays of
 // 0.97 to 0.9999 1.1e-6 / 1.7e-7, step sizes 1.3e-7 / 1.0e-7.
-#include "decay.h"
+#include "chunks.h"
 #include <type_traits>
 
 struct LinArgs {
@@ -132,16 +132,21 @@ linear_chunk_kernel(LinArgs a, float* __restrict__ group_chunks, float* __restri
   if (i == 2) out[288 + j] = over(-1, C - 1);
 }
 
-// As decay_chunk_walk_kernel: one workgroup per request, head and 16 columns, the state's rows shared by its waves, outputs after four
-// chunks. What bounds it: 16 matrix instructions of 32 cycles a chunk and wave with 128 rows, a chain of eight of them when the chip
-// is not full.
+// One workgroup per request, head and 16 columns; its waves share the state's rows, RT tiles of 16 each. A lane holds rows 4 g .. 4 g + 3
+// (g: its lane group) of a column of each tile, which is what a matrix instruction leaves in it and what the next one wants as its
+// operand, so neither the state nor what is added to it ever moves between lanes; products are formed in instructions of four k each. Only
+// outputs need the sum over all rows: they come after four chunks, a quarter a wave (in every chunk, one wave's output made all
+// wait: 64 rows 0.57 -> 0.35 us a chunk). Operands are asked for two chunks ahead (four: no faster, and short requests half as slow
+// again for their registers). What bounds it: 16 matrix instructions of 32 cycles a chunk and wave with 128 rows where the chip is full, else
+// the chain through them, 0.65 us a chunk.
 template <typename TX, int NR, int WAVES>
-__global__ void __launch_bounds__(64 * WAVES, 2)
+__global__ void __launch_bounds__(64 * WAVES, 2)       // up to 256 registers, of which matrix instructions then use the ordinary ones: no copies
 linear_chunk_walk_kernel(LinArgs a, const float* __restrict__ group_chunks, const float* __restrict__ head_chunks, int groups) {
   constexpr int C = DC_TOKENS, RT = NR / (16 * WAVES);
   __shared__ f32x4 part_y[2][4][WAVES][64];
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // the column blocks of one request and head, which read the same operands, run on one XCD
   const int slot = blockIdx.x >> 3, group = slot / a.col_blocks * 8 + (blockIdx.x & 7), cb = slot % a.col_blocks;
   if (group >= groups) return;
   const int b = group / a.H, h = group % a.H;
@@ -187,6 +192,9 @@ linear_chunk_walk_kernel(LinArgs a, const float* __restrict__ group_chunks, cons
     asm volatile("" ::: "memory");
   };
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  // Code of each wave's own, and for whole chunks no branch around a load or a store: the wait for a chunk's operands then counts
+  // what was asked for behind them; behind a branch it would be for everything. (A lane behind the last column has that column's
+  // numbers and stores them again.)
   Chunk o[2];
   fetch(0, o[0]);
   fetch(1, o[1]);

@@ -29,10 +29,10 @@ HIPCC_FLAGS = [
     "-Wno-unused-command-line-argument", "-Wno-unknown-attributes",
 ]
 CORE_SOURCES = ["elementwise.hip", "rope_kv.hip", "attention_simple.hip",
-                "gemm.hip", "gemm_f32.hip", "gemm_mid.hip", "gemm_tile.hip", "gemm_library.hip", "sampling.hip", "recurrent.hip", "parallel.hip", "moe.hip", "hybrid.hip", "decay_chunks.hip", "linear_chunks.hip", "latent.hip",
+                "gemm.hip", "gemm_f32.hip", "gemm_mid.hip", "gemm_tile.hip", "gemm_library.hip", "sampling.hip", "recurrent.hip", "parallel.hip", "moe.hip", "hybrid.hip", "linear_chunks.hip", "latent.hip",
                 "streams.hip"]
 ATTN_SOURCE = "attention_mfma.hip"
-HEADERS = ["common.h", "errors.inc", "sampling.h", "decay.h"]
+HEADERS = ["common.h", "errors.inc", "sampling.h", "chunks.h"]
 # Head sizes that build_all() compiles ahead of use; any other multiple of 16 up to 512 is compiled when a model first needs it.
 DEFAULT_HEAD_DIMS = (16, 32, 48, 64, 80, 128, 256)
 CAPPED_HEAD_DIMS = (32, 64, 128)          # ... of the variant with a cap on the scores

@@ -103,7 +103,6 @@ _CORE_PROTOS = {
     "me_heads_linear": [P, L, L, P, P, L, L, I, L, I, I, I, P],
     "me_token_shift": [P, L, I, P, I, P, L, P, P, P, P, L, I, P],
     "me_decay_rows_recurrence": [P, L, P, L, P, L, P, L, P, L, I, P, P, P, P, L, P, P, P, I, I, I, I, I, I, I, F, F, I, L, P, P],
-    "me_decay_rows_chunks": [P, L, P, L, P, L, P, L, P, L, P, P, P, P, L, P, P, P, I, I, I, I, I, I, I, F, F, L, P, L, P],
     "me_linear_chunks": [P, L, P, L, P, L, P, L, P, P, P, P, P, L, P, P, P, I, I, I, I, I, I, L, P, L, P],
     "me_sample": [P, L, P, P, P, P, I, I, P],
     "me_sample_static": [P, L, P, P, P, I, I, P],
@@ -1149,18 +1148,8 @@ class HipBackend:
         _check(_is_i32(state_slots) and _is_i32(cu_seqlens, B + 1) and len(q_lens) == B and sum(q_lens) == T, "decay_rows_recurrence: metadata")
         _check(1 <= N <= 256 and H % G == 0, "decay_rows_recurrence: up to 256 state rows, heads a multiple of the groups")
         y = torch.empty((T, H * P), dtype=torch.float32, device=v.device)
-        NR = 32 if N <= 32 else 64 if N <= 64 else 128 if N <= 128 else 256
-        if decay_chunks_take(dtype, N, max(q_lens)):
-            delta = rule.startswith("delta")
-            room = (T // 16 + B) * H * ((49 * NR + 512 if delta else 33 * NR + 256) + 256 * -(-P // 16))
-            chunks = _scratch(room, v.device, "decay_rows")
-            core().call("me_decay_rows_chunks", q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
-                        raw.data_ptr(), raw.stride(0), _ptr(beta), 0 if beta is None else beta.stride(0),
-                        base.data_ptr(), _ptr(rate), _ptr(bonus), state.data_ptr(), state.stride(0), state_slots.data_ptr(),
-                        cu_seqlens.data_ptr(), y.data_ptr(), B, H, G, N, P, DECAY_RULES[rule], int(unit_eps is not None),
-                        float(unit_eps or 0.0), float(q_scale), T, chunks.data_ptr(), chunks.numel(), _stream())
-            return y
         groups, prepared = decay_row_groups(B, H, N, P, max(q_lens), T, per_head)
+        NR = 32 if N <= 32 else 64 if N <= 64 else 128 if N <= 128 else 256
         pre = _scratch(3 * T * H * NR + T * H, v.device, "decay_rows") if prepared else None
         core().call("me_decay_rows_recurrence", q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
                     raw.data_ptr(), raw.stride(0), _ptr(beta), 0 if beta is None else beta.stride(0), _code(dtype),
@@ -1988,18 +1977,6 @@ def linear_chunks_take(dtype, H: int, N: int, P: int, q_lens) -> bool:
     if count * H * -(-P // 64) <= LINEAR_CHUNKS_FEW:
         return longest >= LINEAR_CHUNKS_MIN_TOKENS
     return longest >= (LINEAR_CHUNKS_MIN_TOKENS_MORE if count < LINEAR_CHUNKS_MANY else LINEAR_CHUNKS_MIN_TOKENS_MANY)
-
-
-DECAY_CHUNKS_MIN_TOKENS = 128
-
-
-def decay_chunks_take(dtype, N: int, longest: int) -> bool:
-    """Whether `decay_rows_recurrence` takes sixteen tokens of a request at a time (csrc/decay_chunks.hip): bfloat16 rows (a token's
-    bits then depend on its place in the step, which the 32-bit path promises they do not), as many state rows as four waves hold,
-    and requests so long that the kernel that prepares the chunks pays: one of 100 tokens, delta rule, 4 heads of 128 x 128, token by token /
-    by chunks 25 / 26 us, bonus rule, 16 heads of 64 x 64 19 / 20, of 2,048 tokens 260 / 142 and 140 / 74; 64 requests of 96 tokens
-    486 / 330, 100 of them 337 / 270, so a step of many could have it earlier, which is left for the bits that a request has alone."""
-    return dtype == torch.bfloat16 and N <= 128 and longest >= DECAY_CHUNKS_MIN_TOKENS
 
 
 def decay_row_groups(num_seqs: int, H: int, N: int, P: int, longest: int = 1, tokens: int | None = None, one_decay: bool = False) -> tuple:
