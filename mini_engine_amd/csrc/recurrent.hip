@@ -782,7 +782,32 @@ __global__ void recurrence_carry_kernel(RecArgs a) {
   }
 }
 
-// A step of single tokens (token b is request b's): the state streams through once. One workgroup of four waves per
+// A token's a and b (RecArgs).
+template <typename TX>
+__device__ __forceinline__ void step_factors(const RecArgs& a, int b, int h, float& da, float& db) {
+  if (a.dt) {
+    const float z = to_f32<TX>(((const TX*)a.dt)[(int64_t)b * a.dt_stride + h]) + a.dt_bias[h];
+    const float step = z > 20.f ? z : log1pf(expf(z));
+    da = expf(-a.rate[h] * step);
+    db = step;
+  } else if (a.gates.i) {
+    float gi, gf;
+    read_gates<TX>(a.gates, b, h, gi, gf);
+    const float before = a.gates.m[(int64_t)a.slots[b] * a.gates.m_stride + h];     // moved on by whoever reads the outputs
+    const float now = fmaxf(gf + before, gi);
+    da = expf(gf + before - now);
+    db = expf(gi - now);
+  } else if (a.coef_a) {
+    da = a.coef_a[(int64_t)b * a.H + h];
+    db = a.coef_b[(int64_t)b * a.H + h];
+  } else {
+    da = a.decay[h];
+    db = 1.f;
+  }
+}
+
+// A step of single tokens (token b is request b's): the state streams through once, past the caches, which do not hold it until the
+// next step (64 requests, 16 heads of 128 x 128: 31.4 -> 24.7 us, 5.4 TB/s). One workgroup of four waves per
 // (request, head, 64 columns); each wave takes a quarter of the N rows, and the four partial outputs meet in LDS.
 // HB: rows that a wave asks for at once and holds until they are written back, the first of them before it meets the others: a quarter of 128 rows is one trip to
 // memory instead of four behind each other (8 requests, 16 heads of 128 x 128, 16.8 MB read and written: 10.4 -> 8.1 us).
@@ -804,7 +829,7 @@ __global__ void __launch_bounds__(256) recurrence_step_kernel(RecArgs a) {
   const int r0 = wave * per, r1 = r0 + per < a.N ? r0 + per : a.N;
   float held[HB];
 #pragma unroll
-  for (int i = 0; i < HB; ++i) held[i] = row[(int64_t)max(min(r0 + i, r1 - 1), 0) * a.P];
+  for (int i = 0; i < HB; ++i) held[i] = __builtin_nontemporal_load(&row[(int64_t)max(min(r0 + i, r1 - 1), 0) * a.P]);
   for (int i = threadIdx.x; i < a.N; i += 256) {
     float kk = to_f32<TX>(((const TX*)a.k)[(int64_t)b * a.k_stride + (int64_t)g * a.N + i]);
     float qq = to_f32<TX>(((const TX*)a.q)[(int64_t)b * a.q_stride + (int64_t)g * a.N + i]);
@@ -814,25 +839,7 @@ __global__ void __launch_bounds__(256) recurrence_step_kernel(RecArgs a) {
   float vv = to_f32<TX>(((const TX*)a.v)[(int64_t)b * a.v_stride + (int64_t)h * a.P + pc]);
   if (silu) vv = silu_f(vv);
   float da, db;
-  if (a.dt) {
-    const float z = to_f32<TX>(((const TX*)a.dt)[(int64_t)b * a.dt_stride + h]) + a.dt_bias[h];
-    const float step = z > 20.f ? z : log1pf(expf(z));
-    da = expf(-a.rate[h] * step);
-    db = step;
-  } else if (a.gates.i) {
-    float gi, gf;
-    read_gates<TX>(a.gates, b, h, gi, gf);
-    const float before = a.gates.m[(int64_t)a.slots[b] * a.gates.m_stride + h];     // moved on by whoever reads the outputs
-    const float now = fmaxf(gf + before, gi);
-    da = expf(gf + before - now);
-    db = expf(gi - now);
-  } else if (a.coef_a) {
-    da = a.coef_a[(int64_t)b * a.H + h];
-    db = a.coef_b[(int64_t)b * a.H + h];
-  } else {
-    da = a.decay[h];
-    db = 1.f;
-  }
+  step_factors<TX>(a, b, h, da, db);
   const float bv = db * vv;
   __syncthreads();
   float acc = 0.f;
@@ -840,13 +847,13 @@ __global__ void __launch_bounds__(256) recurrence_step_kernel(RecArgs a) {
 #pragma unroll
     for (int i = 0; i < HB; ++i)
       if (r + i < r1) {
-        const float next = da * held[i] + sk[r + i] * bv;
-        acc += next * sq[r + i];
-        if (on) row[(int64_t)(r + i) * a.P] = next;
+        const float next = fmaf(sk[r + i], bv, da * held[i]);
+        acc = fmaf(next, sq[r + i], acc);
+        if (on) __builtin_nontemporal_store(next, &row[(int64_t)(r + i) * a.P]);
       }
     if (r + HB < r1) {
 #pragma unroll
-      for (int i = 0; i < HB; ++i) held[i] = row[(int64_t)min(r + HB + i, r1 - 1) * a.P];
+      for (int i = 0; i < HB; ++i) held[i] = __builtin_nontemporal_load(&row[(int64_t)min(r + HB + i, r1 - 1) * a.P]);
     }
   }
   part[wave * 64 + lane] = acc;
@@ -867,6 +874,78 @@ __global__ void __launch_bounds__(256) recurrence_step_kernel(RecArgs a) {
     }
     dot = block_sum(dot, scratch);
     if (threadIdx.x == 0) a.key_dot[(int64_t)b * a.H + h] = dot;
+  }
+}
+
+// The same step for few requests, whose state a workgroup to a compute unit would draw alone: 32 columns to a workgroup, so twice as
+// many, and four columns of a row to a lane, so a quarter of the loads and stores. The rows of a quarter lie with eight
+// lanes then, and what they become goes through LDS to the lane that adds up a column in the order of the other form: the same
+// bits. us, other form with cached accesses / without / this, 16 heads of 128 x 128: one request 5.3 / 5.3 / 3.8, 8 of them 7.7 / 6.6 /
+// 5.5, 24 13.9 / 9.8 / 10.1, 64 31.4 / 24.7 / 27.6; 32 heads of 128 x 64 with step sizes, 8 requests 8.0 / 6.7 / 5.6.
+// N <= NR; columns, state rows and their places in whole steps of four.
+template <typename TX, int NR>
+__global__ void __launch_bounds__(256) recurrence_step_few_kernel(RecArgs a) {
+  constexpr int COLS = 32, PITCH = COLS + 4, RPL = NR / 32;      // rows of a quarter that a lane has
+  __shared__ float sk[NR], sq[NR], part[4][COLS];
+  __shared__ __align__(16) float made[NR][PITCH];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int b = blockIdx.x / a.H, h = blockIdx.x - b * a.H;
+  const int g = h / (a.H / a.G);
+  const int four = (lane & 7) * 4, r_in = lane >> 3;
+  const int p = blockIdx.y * COLS + four;
+  const bool on = p < a.P;
+  const int pc = on ? p : 0;
+  const bool silu = a.silu != 0;
+  float* row = a.state + (int64_t)a.slots[b] * a.state_stride + (int64_t)h * a.N * a.P + pc;
+  const int per = (a.N + 3) / 4, r0 = wave * per, r1 = min(r0 + per, a.N);
+  f32x4 held[RPL];
+#pragma unroll
+  for (int i = 0; i < RPL; ++i)
+    held[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(row + (int64_t)max(min(r0 + i * 8 + r_in, r1 - 1), 0) * a.P));
+  for (int i = threadIdx.x; i < a.N; i += 256) {
+    float kk = to_f32<TX>(((const TX*)a.k)[(int64_t)b * a.k_stride + (int64_t)g * a.N + i]);
+    float qq = to_f32<TX>(((const TX*)a.q)[(int64_t)b * a.q_stride + (int64_t)g * a.N + i]);
+    if (silu) { kk = silu_f(kk); qq = silu_f(qq); }
+    sk[i] = kk; sq[i] = qq;
+  }
+  const TX* values = (const TX*)a.v + (int64_t)b * a.v_stride + (int64_t)h * a.P;
+  float da, db;
+  step_factors<TX>(a, b, h, da, db);
+  f32x4 bv;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float vv = to_f32<TX>(values[pc + e]);
+    bv[e] = db * (silu ? silu_f(vv) : vv);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < RPL; ++i) {
+    const int r = r0 + i * 8 + r_in;
+    if (r < r1) {
+      f32x4 next;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) next[e] = fmaf(sk[r], bv[e], da * held[i][e]);
+      if (on) __builtin_nontemporal_store(next, reinterpret_cast<f32x4*>(row + (int64_t)r * a.P));
+      *reinterpret_cast<f32x4*>(&made[r][four]) = next;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 4 * COLS) {
+    const int quarter = threadIdx.x / COLS, c = threadIdx.x % COLS, q0 = quarter * per, q1 = min(q0 + per, a.N);
+    float acc = 0.f;
+#pragma unroll 8
+    for (int r = q0; r < q1; ++r) acc = fmaf(made[r][c], sq[r], acc);
+    part[quarter][c] = acc;
+  }
+  __syncthreads();
+  const int c = threadIdx.x, out = blockIdx.y * COLS + c;
+  if (c < COLS && out < a.P) {
+    float y = part[0][c] + part[1][c] + part[2][c] + part[3][c];
+    if (a.skip) {
+      const float vv = to_f32<TX>(values[out]);
+      y += a.skip[h] * (silu ? silu_f(vv) : vv);
+    }
+    a.y[(int64_t)b * a.H * a.P + (int64_t)h * a.P + out] = y;
   }
 }
 
@@ -934,7 +1013,22 @@ extern "C" int me_linear_recurrence(const void* q, int64_t q_stride, const void*
   a.gates.cap = cap; a.gates.m = gate_m; a.gates.m_stride = gate_m_stride;
   if (rows_per_wave == 0) {                // a step of single tokens: one pass over the state, one output
     ME_CHECK((int64_t)(2 * N + 256) * 4 <= 64 * 1024 && (P + 63) / 64 <= 65535, "recurrence: a state of %d rows does not fit the step kernel", N);
+    // up to two workgroups of the form for many requests to a compute unit (16 heads of 128 x 128: 12 requests 7.6 us, for few 6.4; 16
+    // 8.0 and 7.6; 20 8.9 and 8.9; 24 9.8 and 10.1)
     const dim3 grid(num_seqs * H, (P + 63) / 64);
+    if (keys == nullptr && N > 16 && N <= 128 && P % 4 == 0 && state_stride % 4 == 0 && (uintptr_t)state % 16 == 0 &&
+        (int64_t)grid.x * grid.y <= 512) {
+      const dim3 few(grid.x, (P + 31) / 32);
+#define REC_FEW(NR)                                                                                    \
+  do {                                                                                                 \
+    if (dtype == ME_F32) recurrence_step_few_kernel<float, NR><<<few, dim3(256), 0, stream>>>(a);      \
+    else recurrence_step_few_kernel<bf16_t, NR><<<few, dim3(256), 0, stream>>>(a);                     \
+  } while (0)
+      if (N <= 32) REC_FEW(32); else if (N <= 64) REC_FEW(64); else REC_FEW(128);
+#undef REC_FEW
+      ME_LAUNCH_CHECK();
+      return 0;
+    }
     const size_t lds = (size_t)(2 * N + 256) * sizeof(float);
 #define REC_STEP(HB)                                                                                   \
   do {                                                                                                 \

@@ -30,6 +30,32 @@ def test_a_state_of_any_height_moves_on_by_one_token(N, P, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,H,G,N,P,selective", [(3, 2, 1, 17, 4, False), (1, 3, 3, 31, 36, True), (2, 2, 2, 32, 32, False), (5, 4, 2, 33, 100, True),
+                                                 (3, 2, 2, 63, 28, False), (2, 2, 1, 64, 64, True), (2, 3, 1, 65, 132, False), (4, 2, 2, 127, 68, True),
+                                                 (8, 4, 4, 128, 128, False), (256, 2, 1, 20, 8, True), (257, 2, 1, 20, 8, True)])
+def test_both_forms_of_the_step_give_the_same_bits(B, H, G, N, P, selective, dtype):
+    """Up to 512 workgroups' worth of requests and heads four columns go to a lane, unless the states lie at places that are no whole steps
+    of four numbers: one step from the same states at such places and at others; states that are not in the step stay."""
+    g = torch.Generator(device=DEV).manual_seed(N + P)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    q, k, v = (rnd(B, w + 5)[:, 2:2 + w].to(dtype) for w in (G * N, G * N, H * P))
+    kw = (dict(dt=rnd(B, H).to(dtype), dt_bias=rnd(H) - 2, rate=rnd(H).abs() + 0.2, skip=rnd(H)) if selective else
+          dict(decay=torch.tensor([0.9, 0.99, 1.0, -0.5], device=DEV)[:H].contiguous(), silu=True))
+    start, got = rnd(B + 2, H * N * P), []
+    for at in (4, 3):
+        state = torch.zeros(B + 2, 8 + H * N * P + -H * N * P % 4, device=DEV)
+        state[:, at:at + H * N * P] = start
+        slots = torch.arange(B, device=DEV).flip(0).int() + 1
+        y = hip().linear_recurrence(q, k, v, state[:, at:at + H * N * P], slots, torch.arange(B + 1, device=DEV).int(), [1] * B, H, G, N, P, **kw)
+        rest = state.clone()
+        rest[:, at:at + H * N * P] = 0
+        assert not rest.any()
+        got.append((y, state[:, at:at + H * N * P].clone()))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    assert torch.equal(got[0][1][0], start[0]) and torch.equal(got[0][1][-1], start[-1]) and not torch.equal(got[0][1][1], start[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("kind", ["silu_before", "sigmoid_behind", "silu_behind"])
 @pytest.mark.parametrize("n,parts", [(1023, 1), (1024, 1), (1025, 2), (2048, 1), (2049, 1), (4097, 3), (8192, 1), (8200, 1)])
 def test_gated_norm_widths(n, parts, kind, dtype):
