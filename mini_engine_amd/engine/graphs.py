@@ -351,6 +351,9 @@ SMALL_STEP_FLOPS = 1.0e14
 # Up to this many times the host-bound size a step is still worth replaying when its layout repeats exactly (the host's
 # launches leave gaps between kernels of a few microseconds each): a 2,048-token prompt at the 0.6B sizes 5.40 -> 5.08 ms.
 EXACT_LAYOUT_FACTOR = 6
+# Twice as far for a model with mixers side by side of which one walks: they run beside each other in captured steps only
+# (`SideBySide`), which pays whatever bounds the step launched one by one.
+BRANCHES_LAYOUT_FACTOR = 12
 
 
 def host_bound_tokens(model) -> int:
@@ -402,7 +405,7 @@ class MixedGraphs:
     over the padded step.
 
     Steps beyond `max_tokens` and up to `max_exact_tokens` (six times as many: up to there the host's launches
-    still leave gaps between the GPU's kernels) take a layout with the step's own token and request counts and
+    still leave gaps between the GPU's kernels; more where a capture holds branches) take a layout with the step's own token and request counts and
     only the context cap and the rows of logits rounded, if nobody decodes in them: prompts of one length alone, or
     a long prompt's portions under a fixed budget, come up again and again exactly so, and nothing is lost to
     padding when they do not."""
@@ -415,7 +418,8 @@ class MixedGraphs:
         self.capture_after = capture_after
         self.max_graphs = max_graphs
         self.max_tokens = host_bound_tokens(runner.model) if max_tokens is None else max_tokens
-        self.max_exact_tokens = EXACT_LAYOUT_FACTOR * self.max_tokens
+        branches = max_tokens is None and any(getattr(part, "captures_branches", False) for part in runner.model.parts())
+        self.max_exact_tokens = (BRANCHES_LAYOUT_FACTOR if branches else EXACT_LAYOUT_FACTOR) * self.max_tokens
         self.captured: dict = {}
         self.sightings: dict = {}
         self.pool = runner.graph_pool() if capture else None

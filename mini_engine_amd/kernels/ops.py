@@ -190,6 +190,14 @@ class second_workspace:
     def __init__(self, slot: int = 1):
         self.slot = slot
 
+    @staticmethod
+    def made(device, slot: int = 1) -> bool:
+        """Whether products can be captured on a second stream: its workspace is there, or is allocated now. None can be in a capture, and
+        without one torch's own route to the library would make a handle for the stream, which a capture refuses."""
+        if _library_workspaces.get(slot) is None and library_is_direct() and not torch.cuda.is_current_stream_capturing():
+            _library_workspaces[slot] = torch.empty(LIBRARY_WORKSPACE_BYTES, dtype=torch.uint8, device=device)
+        return _library_workspaces.get(slot) is not None
+
     def __enter__(self):
         global _workspace_slot
         self.before, _workspace_slot = _workspace_slot, self.slot

@@ -241,6 +241,37 @@ def test_cuts_through_captured_steps(tavevik_folders, case, dtype):
     case(Env(tavevik_folders, dtype, graphs=True), "pair")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["float32", "bfloat16"])
+def test_prompts_of_captured_steps_run_both_mixers_beside_each_other(tavevik_folders, dtype, monkeypatch):
+    """Captured, a step of any number of tokens has the right mixers on a second stream: prompts of 90 tokens alone and in pairs, the
+    same steps many times with other eager work between them, give the bits of a model whose mixers run one behind the other."""
+    from mini_engine_amd.parts import hybrid
+    branches = []
+
+    class Counted(hybrid.side_branch):
+        def __init__(self, device, slot=1):
+            branches.append(torch.cuda.is_current_stream_capturing())
+            super().__init__(device, slot)
+
+    monkeypatch.setattr(hybrid, "side_branch", Counted)
+    drivers, counts = [], []
+    for beside in (True, False):
+        runner, manager, _ = Env(tavevik_folders, dtype, graphs=True).runner("pair", 200, 4)
+        for part in runner.model.parts():
+            if isinstance(part, hybrid.SideBySide):
+                assert part.captures_branches
+                part.captures_branches = beside
+        drivers.append(helpers.Driver(runner, manager))
+    for i in range(6):
+        ids = {f"{r}{i}": helpers.random_ids(90, C.CONFIGS["pair"]["vocab"], 70 + 2 * i + j) for j, r in enumerate("ab"[:1 + i % 2])}
+        for d in drivers:
+            d.step(ids, end=list(ids))
+            counts.append(len(branches))
+        assert all(torch.equal(drivers[0].result(r), drivers[1].result(r)) for r in ids), f"step {i}"
+    assert all(d.runner.mixed_graphs.replays >= 4 for d in drivers)
+    assert branches and all(branches) and counts[4] > counts[3] and counts[5] == counts[4]      # the third step was captured
+
+
 def test_hip_libraries_are_the_ones_running(env):
     C.whole(env, "one")
     assert ops.backend().name == "hip" and any("libme_core" in p for p in ops.loaded_libraries())
