@@ -60,6 +60,9 @@ struct AttnArgs {
   int window;                   // 0: all keys
   int chunk;                    // > 0: a block mask (only the keys of the query's own block of `chunk` positions); window is then huge
   int tok_tile;                 // prefill: query tokens per workgroup
+  // decode in partitions: row r's head h is multiplied by sigmoid(head_gate[r * gate_stride + h]) behind the merge, or nullptr
+  const bf16_t* head_gate;
+  int64_t gate_stride;
   int part_size;                // decode: keys per partition (multiple of 32)
   int num_parts;                // decode: partitions launched
   int spread_heads;             // decode: grid (heads, sequences, partitions) instead of (sequences, heads, partitions)
@@ -1631,6 +1634,7 @@ __global__ void __launch_bounds__(128) attn_reduce_kernel(AttnArgs a) {
 #pragma unroll
   for (int p = 0; p < 16; ++p)
     first[p] = a.tmp_out[(row0 + (p < P ? p : 0)) * HD + (d0 < HD ? d0 : 0)];
+  const float gate = a.head_gate ? static_cast<float>(a.head_gate[(int64_t)b * a.gate_stride + hq]) : 0.f;
   if (threadIdx.x < 64) {
     const int p = threadIdx.x;
     const float mp = p < P ? a.tmp_m[row0 + p] : NEG;
@@ -1647,6 +1651,7 @@ __global__ void __launch_bounds__(128) attn_reduce_kernel(AttnArgs a) {
   }
   __syncthreads();
   const float inv = inv_s;
+  const float open = 1.0f / (1.0f + expf(-gate));
   for (int d = d0; d < HD; d += blockDim.x) {
     float o = 0.f;
     int p0 = 0;
@@ -1657,7 +1662,9 @@ __global__ void __launch_bounds__(128) attn_reduce_kernel(AttnArgs a) {
     }
 #pragma unroll 8
     for (int p = p0; p < P; ++p) o += wgt[p] * a.tmp_out[(row0 + p) * HD + d];
-    a.out[(int64_t)b * a.out_stride + (int64_t)hq * HD + d] = static_cast<bf16_t>(o * inv);
+    bf16_t r = static_cast<bf16_t>(o * inv);
+    if (a.head_gate) r = static_cast<bf16_t>(static_cast<float>(r) * open);        // rounded in between, as a kernel of its own reads it
+    a.out[(int64_t)b * a.out_stride + (int64_t)hq * HD + d] = r;
   }
 }
 
@@ -1697,6 +1704,7 @@ static int fill_common(AttnArgs& a, const void* q, int64_t q_stride, void* out, 
   a.seg_keys = 0; a.max_segs = 1; a.pf_scratch = nullptr; a.seq_of_token = nullptr; a.seq_base = 0;
   a.raw_k = a.raw_v = nullptr; a.q_w = a.k_w = nullptr; a.eps = 0.f; a.rope = nullptr;
   a.k_cache_w = a.v_cache_w = nullptr;
+  a.head_gate = nullptr; a.gate_stride = 0;
   a.softcap = softcap; a.lse_out = lse_out; a.sinks = sinks; a.slopes = slopes;
   return 0;
 }
@@ -1781,6 +1789,7 @@ static int launch_decode(AttnArgs& a, int num_seqs, int part_size, int num_parts
   ME_CHECK(num_parts == 1 || (part_size >= 32 && part_size % 32 == 0),
            "attention: partition size %d must be a multiple of 32", part_size);
   ME_CHECK(num_parts == 1 || scratch != nullptr, "attention: split decode needs scratch");
+  ME_CHECK(num_parts > 1 || a.head_gate == nullptr, "attention: gates join the merge of partitions");
   a.part_size = num_parts == 1 ? (1 << 30) : part_size;
   a.num_parts = num_parts;
   a.spread_heads = spread_heads ? 1 : 0;
@@ -1824,11 +1833,12 @@ extern "C" int me_attn_decode(const void* q, int64_t q_stride, void* out, int64_
                               int bt_stride, const int32_t* context_lens, int num_seqs, int Hq, int Hkv,
                               int page, float scale, int window, int part_size, int num_parts,
                               float* scratch, int spread_heads, float softcap, const float* sinks, const float* slopes,
-                              float* lse_out, hipStream_t stream) {
+                              float* lse_out, const void* head_gate, int64_t gate_stride, hipStream_t stream) {
   if (num_seqs == 0) return 0;
   AttnArgs a;
   if (fill_common(a, q, q_stride, out, out_stride, k_cache, v_cache, block_tables, bt_stride, context_lens,
                   num_seqs, Hq, Hkv, page, scale, window, softcap, sinks, slopes, lse_out)) return -1;
+  a.head_gate = (const bf16_t*)head_gate; a.gate_stride = gate_stride;
   return launch_decode(a, num_seqs, part_size, num_parts, scratch, spread_heads, false, stream);
 }
 
@@ -1845,7 +1855,8 @@ extern "C" int me_attn_decode_fused(const void* qkv, int64_t row_stride, void* o
                                     const int32_t* context_lens, int max_context, int num_seqs, int Hq, int Hkv,
                                     int page, float scale, int window, int part_size, int num_parts,
                                     float* scratch, int spread_heads, float softcap, const float* sinks,
-                                    const float* slopes, float* lse_out, int values_are_keys, hipStream_t stream) {
+                                    const float* slopes, float* lse_out, int values_are_keys, const void* head_gate, int64_t gate_stride,
+                                    hipStream_t stream) {
   if (num_seqs == 0) return 0;
   AttnArgs a;
   if (fill_common(a, qkv, row_stride, out, out_stride, k_cache, v_cache, block_tables, bt_stride, context_lens,
@@ -1858,6 +1869,7 @@ extern "C" int me_attn_decode_fused(const void* qkv, int64_t row_stride, void* o
   a.raw_k = (const bf16_t*)qkv + (int64_t)Hq * HD;
   a.raw_v = values_are_keys ? a.raw_k : a.raw_k + (int64_t)Hkv * HD;
   a.q_w = q_w; a.k_w = k_w; a.eps = eps; a.rope = rope;
+  a.head_gate = (const bf16_t*)head_gate; a.gate_stride = gate_stride;
   a.k_cache_w = (bf16_t*)k_cache; a.v_cache_w = (bf16_t*)v_cache;
   return launch_decode(a, num_seqs, part_size, num_parts, scratch, spread_heads, true, stream);
 }

@@ -288,8 +288,16 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __re
     const int m = m0 + 16 * mt + (idx >> 4), n = n0 + (idx & 15);
     if (m < M && n < N) {
       const float v = red[0][mt][idx] + red[1][mt][idx] + red[2][mt][idx] + red[3][mt][idx];
-      if (partials) partials[((int64_t)split * M + m) * N + n] = v;
-      else y[(int64_t)m * ldy + n] = from_f32<TO>(v);
+      if (partials) {
+        partials[((int64_t)split * M + m) * N + n] = v;
+      } else {
+        TO o = from_f32<TO>(v);
+        if (form.limit < 0.f) {                              // relu(v)^2 of the rounded sum, as the activation's kernel reads it
+          const float positive = fmaxf(to_f32<TO>(o), 0.f);
+          o = from_f32<TO>(positive * positive);
+        }
+        y[(int64_t)m * ldy + n] = o;
+      }
     }
   }
 }
@@ -459,12 +467,14 @@ extern "C" int me_gemm_rows_bf16(const void* x, int64_t ldx, const void* w, int6
 // y: bf16 or float32 [M, N]; or, when ksplit > 1, `partials` float32 [ksplit, M, N] (y unused).
 // gated: x is [M, 2K] and silu(x[:, :K]) * x[:, K:] is what is multiplied. act: w is a packed gate/up weight and y
 // is silu(gate) * up, [M, N / 2] (at most 16 rows, K not split, not together with gated); limit, alpha, bias: another
-// `GateForm` than that.
+// `GateForm` than that. Neither, and limit -1: y is relu(x . w^T)^2.
 extern "C" int me_gemm_skinny_bf16(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y,
                                    int64_t ldy, int out_dtype, float* partials, int ksplit, int M, int N,
                                    int K, int gated, int act, int wide, float limit, float alpha, const float* bias, hipStream_t stream) {
   if (M == 0 || N == 0) return 0;
-  ME_CHECK(act || (limit == 0.f && bias == nullptr), "skinny gemm: limits and biases belong to the gating epilogue");
+  ME_CHECK(act || ((limit == 0.f || (limit == -1.f && !gated && partials == nullptr)) && bias == nullptr),
+           "skinny gemm: limits and biases belong to the gating epilogue");
+  ME_CHECK(!act || limit >= 0.f, "skinny gemm: one activation in the epilogue");
   const GateForm form{limit, alpha, bias};
   // wide: the caller asks for the wide loads (large weights); they apply to one tile of tokens, K in whole steps of
   // 128, an ungated input and a weight under 2 GB, and are left out otherwise

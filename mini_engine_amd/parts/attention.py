@@ -285,7 +285,9 @@ class Attention(Mixer):
             packed = ops.add_bias(self.qkv.forward(x, out_dtype=torch.float32), self.qkv_bias, dtype)
         else:
             packed = self.qkv.forward(x)
-        gated = self.head_gate
+        gated, inside = self.head_gate, {}
+        if gated and getattr(ops.backend(), "gates_heads", False):
+            gated, inside = False, dict(head_gate=packed[:, self.gate_at:self.gate_at + Hq])
         extras = dict(keep_first=self.keep_first, softcap=self.score_cap)
         per_head = dict(sinks=self.sinks, slopes=self.slopes)
         same = dict(values_are_keys=True) if self.values_are_keys else {}
@@ -302,7 +304,7 @@ class Attention(Mixer):
             # only single tokens: norm, rotary, cache write and attention in one launch
             o = ops.decode_step_attention(qkv, qw, kw, eps, table, cache.k, cache.v, cache.page_size, grp.block_tables,
                                           step.context_lens, step.max_decode_context, self.scale, self.window,
-                                          Hq, Hkv, D, even_contexts=step.decode_contexts_even, chunk=self.chunk, **per_head, **same)
+                                          Hq, Hkv, D, even_contexts=step.decode_contexts_even, chunk=self.chunk, **per_head, **same, **inside)
             if gated:
                 ops.head_gate(o, packed[:, self.gate_at:self.gate_at + Hq], Hq, D)
             return self._project(o, packed)
@@ -335,7 +337,7 @@ class Attention(Mixer):
                                 step.seq_of_token, step.positions, step.prefill_cu, step.num_decodes,
                                 step.max_decode_context, self.scale, self.window, Hq, Hkv, D,
                                 max_prefill_context=step.max_prefill_context,
-                                even_contexts=step.decode_contexts_even, chunk=self.chunk, **extras, **per_head)
+                                even_contexts=step.decode_contexts_even, chunk=self.chunk, **extras, **per_head, **inside)
         if gated:
             ops.head_gate(o, packed[:, self.gate_at:self.gate_at + Hq], Hq, D)
         return self._project(o, packed)

@@ -83,7 +83,7 @@ class ActivatedMLP(FeedForward):
 
     def forward(self, x, defer_gate: bool = False):
         if not self.token_gate:
-            return self.down.forward(ops.activation(self.up.forward(x), self.activation), allow_partials=True)
+            return self.down.forward(ops.activated_linear(x, self.up.weight, self.activation), allow_partials=True)
         F = self.intermediate_size
         rows = ops.linear(x, self._packed)
         out = TokenGated(self.down.forward(ops.activation(rows[:, :F], self.activation), allow_partials=True), rows[:, F:F + 1])

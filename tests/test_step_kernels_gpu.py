@@ -4,7 +4,7 @@ import torch
 
 import kernel_twins as twin
 from mini_engine_amd.kernels import ops
-from test_kernels_gpu import DEV, close, hip
+from test_kernels_gpu import DEV, _attention_case, close, hip
 
 pytestmark = pytest.mark.gpu
 
@@ -290,3 +290,46 @@ def test_sums_and_norms_of_few_and_of_many_rows_are_the_same(n, parts, dtype):
     for a, b in zip(many[1:], few[1:]):
         close(a[500:], b, 1e-6 if dtype == torch.float32 else 8e-3)
     close(many[0], stream + 0.45 * (s1 * sums.sum(0) + rows.float()), 1e-6)
+
+
+@pytest.mark.parametrize("dtype,Hq,Hkv,D,page", [(torch.bfloat16, 16, 8, 128, 16), (torch.bfloat16, 6, 2, 32, 8), (torch.bfloat16, 4, 4, 256, 16), (torch.float32, 4, 2, 16, 16)])
+@pytest.mark.parametrize("seqs", [[(1, 1)], [(700, 1), (33, 1), (900, 1), (1, 1)], [(300, 1), (50, 50), (2, 2)], [(9, 9)], [(1500, 1)] * 40])
+def test_gated_heads_give_the_bits_of_a_gate_behind_the_attention(dtype, Hq, Hkv, D, page, seqs):
+    """Joined with the merge of a decode step's partitions, behind one partition, a mixed step or float32 in a kernel of its own; a gate that is
+    not a number or closes altogether reaches its own head only; the step in one launch the same."""
+    args = _attention_case(dtype, Hq, Hkv, D, page, seqs, seed=len(seqs))
+    T = args[0].shape[0]
+    g = torch.Generator(device=DEV).manual_seed(D)
+    gates = (3 * torch.randn(T, Hq + 9, device=DEV, generator=g)).to(dtype)[:, 3:3 + Hq]
+    gates[0, 1], gates[-1, 0], gates[-1, 2] = -200.0, float("nan"), float("inf")
+    for even in (False, True):
+        want = hip().paged_attention(*args, even_contexts=even)
+        hip().head_gate(want, gates, Hq, D)
+        got = hip().paged_attention(*args, even_contexts=even, head_gate=gates)
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.nan_to_num(got), torch.nan_to_num(want))
+        assert int(torch.isnan(got).sum()) == D
+    if dtype == torch.bfloat16 and all(n == 1 for _, n in seqs):
+        q, k_cache, v_cache, _, bt, ctx = args[:6]
+        rows = q._base
+        rows[:, Hq * D:] = torch.randn(T, 2 * Hkv * D, device=DEV, generator=g).to(dtype)
+        outs = [hip().decode_step_attention(rows, None, None, 0.0, None, k_cache.clone(), v_cache.clone(), page, bt, ctx, args[10], D ** -0.5, None, Hq, Hkv, D, **kw)
+                for kw in ({}, dict(head_gate=gates))]
+        hip().head_gate(outs[0], gates, Hq, D)
+        assert torch.equal(torch.nan_to_num(outs[0]), torch.nan_to_num(outs[1])) and int(torch.isnan(outs[1]).sum()) == D
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("kind", ["relu2", "silu"])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 8), (1, 3072, 1024), (7, 40, 136), (16, 8192, 1024), (17, 96, 256), (32, 3072, 1024), (33, 3072, 1024), (65, 3072, 1024), (300, 264, 128)])
+def test_an_activation_in_the_products_epilogue_gives_the_bits_of_one_behind_it(M, N, K, kind, dtype):
+    """Row counts on both sides of what the kernel for few rows takes, wide loads and others, rows of a wider tensor, a sum that is not a number
+    or not finite."""
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    x, w = (torch.randn(n, K + 8, device=DEV, generator=g).to(dtype)[:, :K] for n in (M, N))
+    x[0, 0], w[3, 0] = float("inf"), 0.0
+    want = hip().activation(hip().linear(x, w), kind)
+    got = hip().activated_linear(x, w, kind)
+    assert got.shape == (M, N) and got.dtype == dtype and got.is_contiguous()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.nan_to_num(got), torch.nan_to_num(want))
+    with pytest.raises(ops.KernelError):
+        hip().activated_linear(x, w[:, :K - 1], kind)
