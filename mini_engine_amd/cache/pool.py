@@ -13,6 +13,7 @@ import math
 
 import torch
 
+from ..kernels import ops
 from ..parts.base import CacheView
 
 _DTYPES = {"float32": torch.float32, "bfloat16": torch.bfloat16, "int32": torch.int32}
@@ -74,15 +75,18 @@ class CachePool:
             self.states.append(st)
             self.state_initial.append(first)
 
-    def reset_state(self, slots: torch.Tensor) -> None:
-        """Rows `slots` (int64, on the device) of every state tensor back to what a request starts from."""
-        for st, first in zip(self.states, self.state_initial):
-            if st is None:
-                continue
+    def reset_state(self, slots: list) -> None:
+        """Rows `slots` of every state tensor back to what a request starts from."""
+        kept = [(st, first) for st, first in zip(self.states, self.state_initial) if st is not None]
+        if kept and kept[0][0].is_cuda and all(st.element_size() == 4 for st, _ in kept):
+            ops.HipBackend().reset_rows([st for st, _ in kept], [first for _, first in kept], slots)
+            return
+        for st, first in kept:
+            index = torch.tensor(slots, dtype=torch.long, device=st.device)
             if first is None:
-                st.index_fill_(0, slots, 0)
+                st.index_fill_(0, index, 0)
             else:
-                st.index_copy_(0, slots, first.unsqueeze(0).expand((slots.numel(),) + tuple(first.shape)))
+                st.index_copy_(0, index, first.unsqueeze(0).expand((len(slots),) + tuple(first.shape)))
 
     def spare_page(self, group: int) -> int:
         return self.num_pages[group]

@@ -182,7 +182,7 @@ class DecodeGraphs:
             cap.put("state_slots", state)
             fresh = state[:B][pos[:B] == 0]
             if fresh.size:              # a request whose first token this is starts from empty state (outside the graph)
-                r.pool.reset_state(torch.tensor(fresh.tolist(), dtype=torch.long, device=r.device))
+                r.pool.reset_state(fresh.tolist())
         continues = self._continues(cap, reqs, pos, B)
         cap.last_starts = None                       # stays so if what follows raises
         if continues:

@@ -217,7 +217,7 @@ class ModelRunner:
             return
         fresh = [s for s, st in zip(slots_of, starts) if st == 0 and s >= 0]
         if fresh:
-            self.pool.reset_state(torch.tensor(fresh, dtype=torch.long, device=self.device))
+            self.pool.reset_state(fresh)
 
     # -- what the captured graphs share ----------------------------------------------------
     def graph_pool(self):

@@ -104,6 +104,7 @@ _CORE_PROTOS = {
     "me_token_shift": [P, L, I, P, I, P, L, P, P, P, P, L, I, P],
     "me_decay_rows_recurrence": [P, L, P, L, P, L, P, L, P, L, I, P, P, P, P, L, P, P, P, I, I, I, I, I, I, I, F, F, I, L, P, P],
     "me_linear_chunks": [P, L, P, L, P, L, P, L, P, P, P, P, P, L, P, P, P, I, I, I, I, I, I, L, P, L, P],
+    "me_reset_rows": [P, P, P, P, I, P, I, L, P],
     "me_sample": [P, L, P, P, P, P, I, I, P],
     "me_sample_static": [P, L, P, P, P, I, I, P],
 }
@@ -826,6 +827,19 @@ class HipBackend:
         _check(o.is_contiguous() and o.shape == (T, H * D) and gate.shape == (T, H) and gate.stride(1) == 1
                and gate.dtype == o.dtype, "head_gate: o [T, H * D] contiguous, gate [T, H] of its dtype")
         core().call("me_head_gate", o.data_ptr(), gate.data_ptr(), gate.stride(0), _code(o.dtype), T, H, D, _stream())
+
+    def reset_rows(self, tensors: list, firsts: list, rows: list) -> None:
+        """Rows `rows` of every tensor (whole rows of four-byte numbers, equally many in each) become its `firsts` row, or zeros (None): one
+        launch for all of them, with nothing to send ahead."""
+        for t, first in zip(tensors, firsts):
+            _check(t.element_size() == 4 and t.is_contiguous() and t.shape[0] == tensors[0].shape[0], "reset_rows: contiguous rows of four-byte numbers")
+            _check(first is None or (first.dtype == t.dtype and first.is_contiguous() and first.shape == t.shape[1:]), "reset_rows: a first row of the tensor's kind")
+        n = len(tensors)
+        if n == 0 or not rows:
+            return
+        width = [t.numel() // t.shape[0] for t in tensors]
+        core().call("me_reset_rows", (c_void_p * n)(*[t.data_ptr() for t in tensors]), (c_void_p * n)(*[_ptr(f) for f in firsts]),
+                    (c_int64 * n)(*width), (c_int64 * n)(*width), n, (c_int * len(rows))(*rows), len(rows), tensors[0].shape[0], _stream())
 
     # -- mixers with a state of fixed size -------------------------------------------------
     def causal_conv(self, x, weight, bias, state, state_slots, cu_seqlens, q_lens) -> torch.Tensor:

@@ -333,3 +333,21 @@ def test_an_activation_in_the_products_epilogue_gives_the_bits_of_one_behind_it(
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.nan_to_num(got), torch.nan_to_num(want))
     with pytest.raises(ops.KernelError):
         hip().activated_linear(x, w[:, :K - 1], kind)
+
+
+@pytest.mark.parametrize("widths,rows", [((1,), [0]), ((3, 4097, 16), [2, 5, 0]), ((70000, 5), [1]), (tuple(range(1, 71)), list(range(0, 140, 2))), ((8,), [])])
+def test_rows_of_many_tensors_go_back_to_what_they_start_from(widths, rows):
+    """More tensors and rows than one launch holds, rows that begin at no step of four numbers; the other rows stay."""
+    g = torch.Generator(device=DEV).manual_seed(len(widths))
+    tensors = [torch.randn(141, w, device=DEV, generator=g) for w in widths]
+    firsts = [torch.randn(w, device=DEV, generator=g) if i % 3 == 1 else None for i, w in enumerate(widths)]
+    want = [t.clone() for t in tensors]
+    for t, f in zip(want, firsts):
+        t[rows] = 0.0 if f is None else f
+    hip().reset_rows(tensors, firsts, rows)
+    assert all(torch.equal(a, b) for a, b in zip(tensors, want))
+    with pytest.raises(ops.KernelError):
+        hip().reset_rows(tensors, firsts, [0, 141])
+    with pytest.raises(ops.KernelError):
+        hip().reset_rows(tensors, firsts, [-1])
+    assert all(torch.equal(a, b) for a, b in zip(tensors, want))
