@@ -65,7 +65,7 @@ class SideBySide(Mixer):
     def forward(self, x, step, cache, state, terms: bool = False):
         """`terms`: return the two outputs unadded (`ScaledTerms`) for a consumer that forms the weighted sum itself."""
         give = lambda i: (cache if self._cache_of == i else None, state if self._state_of == i else None)
-        walks = self.captures_branches and x.is_cuda and ops.second_workspace.made(x.device)
+        walks = self.side_stream and self.captures_branches and x.is_cuda and ops.second_workspace.made(x.device)
         if (self.side_stream and few_tokens(x)) or (walks and torch.cuda.is_current_stream_capturing()):
             with side_branch(x.device, 1) as branch:
                 b = self.right.forward(x, step, *give(1))
