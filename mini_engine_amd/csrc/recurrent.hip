@@ -471,17 +471,22 @@ struct RecArgs {
   float* state; int64_t state_stride;               // [slots, H * N * P] view
   const int32_t* slots; const int32_t* cu;
   float* y; int64_t y_slice_stride;                 // [slices of N, T, H * P] float32
-  float* span_state; float* span_decay;             // scratch: [requests, spans, H, N, P], [requests, spans, H]
+  float* span_state; float* span_decay;             // scratch: [places, H, N, P], [places, H] (span_place)
   int H, G, N, P, span, max_spans;
   int silu;                                         // q, k and v pass silu on their way in
   const float* coef_a; const float* coef_b;         // a, b given per token and head, [T, H], or null
   float* keys;                                      // the summed keys' state [slots, H * N] (stride state_stride), or null: none
   float* key_dot; int64_t dot_slice_stride;         // n . q: [slices of N, T, H]
-  float* span_keys;                                 // scratch: [requests, spans, H, N]
+  float* span_keys;                                 // scratch: [places, H, N]
   SoftGates gates;                                  // a step of single tokens forms a and b itself (gates.i null: not)
 };
 
 #define REC_TB 8
+
+// Span c of request b has place cu[b] / span + b + c (whole division): the places of two requests never meet and there are at most
+// T / span + requests of them, however the tokens are shared out, so scratch made for a captured step holds every step of its
+// layout.
+__device__ __forceinline__ int64_t span_place(const RecArgs& a, int b, int c) { return a.cu[b] / a.span + b + c; }
 
 // HPB heads and PPB blocks of 64 columns per wave; CL = HPB * PPB columns per lane. KEYS: the waves of the first column
 // block also keep the summed keys of their NT rows, one row per lane; a batch's products with q meet in LDS, where eight
@@ -578,7 +583,7 @@ __global__ void __launch_bounds__(64) recurrence_kernel(RecArgs a) {
 #pragma unroll
   for (int j = 0; j < CL; ++j) {
     row[j] = a.state + (int64_t)a.slots[b] * a.state_stride + (int64_t)head[j] * a.N * a.P;
-    span_row[j] = PASS == 0 ? nullptr : a.span_state + (((int64_t)b * a.max_spans + c) * a.H + head[j]) * (int64_t)a.N * a.P;
+    span_row[j] = PASS == 0 ? nullptr : a.span_state + (span_place(a, b, c) * a.H + head[j]) * (int64_t)a.N * a.P;
     if (PASS == 1) {
 #pragma unroll
       for (int i = 0; i < NT; ++i) S[j][i] = 0.f;
@@ -597,7 +602,7 @@ __global__ void __launch_bounds__(64) recurrence_kernel(RecArgs a) {
   const bool my_key = keys && lane < NT && lane <= n_last;
   if (KEYS) {
     key_row = a.keys + (int64_t)a.slots[b] * a.state_stride + (int64_t)h0 * a.N + n0;
-    if (PASS != 0) span_key_row = a.span_keys + (((int64_t)b * a.max_spans + c) * a.H + h0) * (int64_t)a.N + n0;
+    if (PASS != 0) span_key_row = a.span_keys + (span_place(a, b, c) * a.H + h0) * (int64_t)a.N + n0;
     if (PASS != 1 && my_key) nk = (PASS == 0 ? key_row : span_key_row)[lane];
   }
   float skip[CL];
@@ -757,7 +762,7 @@ __global__ void __launch_bounds__(64) recurrence_kernel(RecArgs a) {
   }
   if (PASS == 1 && lane == 0 && blockIdx.y == 0 && slice == 0)
 #pragma unroll
-    for (int j = 0; j < HPB; ++j) a.span_decay[((int64_t)b * a.max_spans + c) * a.H + h0 + j] = total_decay[j];
+    for (int j = 0; j < HPB; ++j) a.span_decay[span_place(a, b, c) * a.H + h0 + j] = total_decay[j];
 }
 
 // in[0] = the request's state row; in[c + 1] = decay[c] * in[c] + end[c]. scratch[c] holds end[c] on entry and in[c] on
@@ -771,14 +776,15 @@ __global__ void recurrence_carry_kernel(RecArgs a) {
   if (e >= (key ? (a.keys ? (int64_t)a.H * a.N : 0) : per_req)) return;
   const int h = (int)(e / (key ? a.N : per_head));
   const int64_t len = a.cu[b + 1] - a.cu[b];
-  const int spans = (int)((len + a.span - 1) / a.span);
+  const int spans = (int)min((len + a.span - 1) / a.span, (int64_t)a.max_spans);       // (none that the passes were not launched for)
   if (spans <= 0) return;
   float carry = (key ? a.keys : a.state)[(int64_t)a.slots[b] * a.state_stride + e];
   for (int c = 0; c < spans; ++c) {
-    float* at = key ? a.span_keys + ((int64_t)b * a.max_spans + c) * a.H * a.N + e : a.span_state + ((int64_t)b * a.max_spans + c) * per_req + e;
+    const int64_t place = span_place(a, b, c);
+    float* at = key ? a.span_keys + place * a.H * a.N + e : a.span_state + place * per_req + e;
     const float ended = *at;
     *at = carry;
-    carry = a.span_decay[((int64_t)b * a.max_spans + c) * a.H + h] * carry + ended;
+    carry = a.span_decay[place * a.H + h] * carry + ended;
   }
 }
 
@@ -973,8 +979,8 @@ static int launch_recurrence(RecArgs& a, int num_seqs, int spans, int one_by_one
 }
 
 // spans <= 1: every request's tokens in one pass. Otherwise the tokens are cut into spans of `span` tokens that run
-// side by side (at most `spans` per request), and scratch holds spans * H * N * P + spans * H floats per request.
-// keys: the summed keys beside the states, in the same state rows (see RecArgs); scratch then holds spans * H * N more.
+// side by side (at most `spans` per request), and scratch holds `places` = T / span + num_seqs times H * N * P + H floats.
+// keys: the summed keys beside the states, in the same state rows (see RecArgs); scratch then holds places * H * N more.
 // one_by_one: a single pass (spans <= 1) takes the form for short requests. columns: 1, or 2: a lane keeps two columns of the state (two blocks of 64 columns of one head where P > 64, else
 // the same columns of two neighbouring heads of one group, which needs an even number of heads per group).
 extern "C" int me_linear_recurrence(const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
@@ -982,7 +988,7 @@ extern "C" int me_linear_recurrence(const void* q, int64_t q_stride, const void*
                                     const float* dt_bias, const float* rate, const float* skip, float* state,
                                     int64_t state_stride, const int32_t* slots, const int32_t* cu, float* y,
                                     int64_t y_slice_stride, int num_seqs, int H, int G, int N, int P, int rows_per_wave,
-                                    int columns, int silu, int span, int spans, int one_by_one, float* scratch, const float* coef_a,
+                                    int columns, int silu, int span, int spans, int64_t places, int one_by_one, float* scratch, const float* coef_a,
                                     const float* coef_b, float* keys, float* key_dot, int64_t dot_slice_stride, const void* gate_i,
                                     const void* gate_f, int64_t gate_stride, const float* bias_i, const float* bias_f, float cap,
                                     float* gate_m, int64_t gate_m_stride, hipStream_t stream) {
@@ -995,7 +1001,7 @@ extern "C" int me_linear_recurrence(const void* q, int64_t q_stride, const void*
   ME_CHECK((keys != nullptr) == (key_dot != nullptr) && (keys == nullptr || columns == 1), "recurrence: summed keys with one column per lane");
   ME_CHECK(dt == nullptr || (dt_bias && rate), "recurrence: step sizes need their bias and rates");
   ME_CHECK((int64_t)num_seqs * H <= 2147483647ll, "recurrence: too many (request, head) pairs");
-  ME_CHECK(spans <= 1 || (span >= 1 && scratch != nullptr), "recurrence: spans need a length and scratch");
+  ME_CHECK(spans <= 1 || (span >= 1 && scratch != nullptr && places >= num_seqs), "recurrence: spans need a length and scratch");
   const bool two_heads = columns == 2 && P <= 64;
   ME_CHECK(columns == 1 || columns == 2, "recurrence: 1 or 2 columns per lane");
   ME_CHECK(!two_heads || (H / G) % 2 == 0, "recurrence: two heads per wave need an even number of heads per group");
@@ -1006,8 +1012,8 @@ extern "C" int me_linear_recurrence(const void* q, int64_t q_stride, const void*
   a.H = H; a.G = G; a.N = N; a.P = P; a.span = span > 0 ? span : 1; a.max_spans = spans > 1 ? spans : 1;
   a.silu = silu;
   a.span_state = scratch;
-  a.span_decay = scratch ? scratch + (int64_t)num_seqs * a.max_spans * H * N * P : nullptr;
-  a.span_keys = scratch && keys ? a.span_decay + (int64_t)num_seqs * a.max_spans * H : nullptr;
+  a.span_decay = scratch ? scratch + places * H * N * P : nullptr;
+  a.span_keys = scratch && keys ? a.span_decay + places * H : nullptr;
   a.coef_a = coef_a; a.coef_b = coef_b; a.keys = keys; a.key_dot = key_dot; a.dot_slice_stride = dot_slice_stride;
   a.gates.i = gate_i; a.gates.f = gate_f; a.gates.stride = gate_stride; a.gates.bias_i = bias_i; a.gates.bias_f = bias_f;
   a.gates.cap = cap; a.gates.m = gate_m; a.gates.m_stride = gate_m_stride;

@@ -13,6 +13,17 @@ class GroupStep:
     slot_mapping: torch.Tensor      # int32 [T] page_id * page_size + offset of each new token
 
 
+class TokenCounts(list):
+    """A step's new tokens per request, on the host. `longest`: no request of any step that runs through the same launches brings
+    more tokens. A step launched one by one is its own measure; a captured one stands for every step of its layout, whose requests
+    may share the tokens out otherwise, so what a launch covers goes by `longest` (`ops.longest_request`), never by the counts
+    that the layout happened to be captured with. Those may choose between forms that are right for any counts."""
+
+    def __init__(self, counts=(), longest: int = 0):
+        super().__init__(counts)
+        self.longest = max(longest, max(counts, default=0))
+
+
 @dataclass
 class StepContext:
     num_tokens: int
@@ -30,7 +41,7 @@ class StepContext:
     state_slots: torch.Tensor | None = None          # int32 [B]
     first_chunk: torch.Tensor | None = None          # int32 [B]: 1 if the request's tokens start at position 0
     # host copies, for parts that decide launches on the host
-    q_lens: list = field(default_factory=list)
+    q_lens: TokenCounts = field(default_factory=TokenCounts)
     starts: list = field(default_factory=list)
     # what one layer call leaves for later calls of the same step, by name (values of this step's tokens that a
     # later layer blends into its own); filled and read while the step runs, also while it is captured

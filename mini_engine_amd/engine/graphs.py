@@ -20,7 +20,7 @@ import numpy as np
 import torch
 
 from ..kernels import ops
-from .context import GroupStep, StepContext
+from .context import GroupStep, StepContext, TokenCounts
 from .packing import StepLayout, context_of, pack_step, views_of
 
 PENDING = -1      # the runner's marker for a token that is still on the device (runner.PENDING)
@@ -98,7 +98,7 @@ class _Captured:
             decode_contexts_even=self.even,
             groups=[GroupStep(self.view(f"bt{g}").view(B, self.MB), self.view(f"slots{g}")) for g in range(self.G)],
             state_slots=self.view("state_slots"), first_chunk=self.view("first_chunk"),
-            q_lens=[1] * B, starts=[0] * B)
+            q_lens=TokenCounts([1] * B), starts=[0] * B)
 
     def upload(self):
         i = self.flip
@@ -517,7 +517,7 @@ class MixedGraphs:
         r = self.runner
         layout = cap.layout
         tokens, rows = views_of(layout, cap.dev)
-        h, residual = r.model.forward(tokens, context_of(layout, cap.dev, q_lens, first), r.pool.views, r.pool.states)
+        h, residual = r.model.forward(tokens, context_of(layout, cap.dev, q_lens, first, layout.longest), r.pool.views, r.pool.states)
         if not layout.rows:
             return None
         return r.model.logits(h, residual, rows[:layout.rows], out=out)

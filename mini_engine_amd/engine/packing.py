@@ -16,7 +16,7 @@ from dataclasses import dataclass
 
 import numpy as np
 
-from .context import GroupStep, StepContext
+from .context import GroupStep, StepContext, TokenCounts
 
 
 def _pad4(n: int) -> int:
@@ -41,6 +41,11 @@ class StepLayout:
     @property
     def num_seqs(self) -> int:
         return self.decode_rows + self.prefill_reqs
+
+    @property
+    def longest(self) -> int:
+        """The most tokens that one request of a step of this layout can bring (the others bring one at least)."""
+        return max(1 if self.decode_rows else 0, self.prefill_tokens - (self.prefill_reqs - 1) if self.prefill_reqs else 0)
 
     def segments(self) -> tuple:
         """({name: (offset, size)}, total size) of the packed array."""
@@ -90,6 +95,8 @@ def pack_step(layout: StepLayout, out: np.ndarray, token_lists: list, starts: li
     all_start = starts[:Dn] + [0] * pad_rows + starts[Dn:] + [0] * pad_req
     all_ctx = [s + 1 for s in starts[:Dn]] + [0] * pad_rows + [s + q for s, q in zip(starts[Dn:], q_lens[Dn:])] + [pad_tokens] * pad_req
     B, T = layout.num_seqs, layout.num_tokens
+    if max(all_q) > layout.longest:                        # launches captured for the layout would not cover the request
+        raise ValueError(f"a request of {max(all_q)} tokens in a layout whose longest has {layout.longest}")
     cu = np.zeros(B + 1, dtype=np.int64)
     np.cumsum(all_q, out=cu[1:])
 
@@ -155,8 +162,9 @@ def pack_step(layout: StepLayout, out: np.ndarray, token_lists: list, starts: li
     return all_q, all_start
 
 
-def context_of(layout: StepLayout, dev, q_lens: list | None = None, starts: list | None = None) -> StepContext:
-    """The `StepContext` whose tensors are views into the packed array `dev` (on the device)."""
+def context_of(layout: StepLayout, dev, q_lens: list | None = None, starts: list | None = None, longest: int = 0) -> StepContext:
+    """The `StepContext` whose tensors are views into the packed array `dev` (on the device). `longest`: see `TokenCounts`; a step
+    that is launched for its whole layout names the layout's."""
     seg, _ = layout.segments()
 
     def view(name):
@@ -171,7 +179,7 @@ def context_of(layout: StepLayout, dev, q_lens: list | None = None, starts: list
         decode_contexts_even=layout.even, max_prefill_context=layout.prefill_ctx,
         groups=[GroupStep(view(f"bt{g}").view(B, mb), view(f"slots{g}")) for g, mb in enumerate(layout.max_blocks)],
         state_slots=view("state_slots"), first_chunk=view("first_chunk"),
-        q_lens=list(q_lens) if q_lens is not None else [], starts=list(starts) if starts is not None else [])
+        q_lens=TokenCounts(q_lens if q_lens is not None else [], longest), starts=list(starts) if starts is not None else [])
 
 
 def views_of(layout: StepLayout, dev) -> tuple:

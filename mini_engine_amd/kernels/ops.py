@@ -82,7 +82,7 @@ _CORE_PROTOS = {
     "me_activation": [P, L, P, I, I, L, I, P],
     "me_head_gate": [P, P, L, I, L, I, I, P],
     "me_causal_conv": [P, L, I, P, P, P, L, P, P, I, I, P, L, I, I, I, P],
-    "me_linear_recurrence": [P, L, P, L, P, L, I, P, L, P, P, P, P, P, L, P, P, P, L, I, I, I, I, I, I, I, I, I, I, I, P,
+    "me_linear_recurrence": [P, L, P, L, P, L, I, P, L, P, P, P, P, P, L, P, P, P, L, I, I, I, I, I, I, I, I, I, I, L, I, P,
                              P, P, P, P, L, P, P, L, P, P, F, P, L, P],
     "me_soft_gates": [P, P, L, I, P, P, F, P, L, P, P, P, P, P, I, I, P],
     "me_memory_readout": [P, I, L, P, P, F, P, L, I, P, P, L, I, I, F, P, P, L, P, P, F, P, L, P, P],
@@ -847,7 +847,7 @@ class HipBackend:
         continued from its state: x a row view [T, C]; weight float32 [C, taps] (the last tap is the current
         token's); state a float32 view [slots, C * (taps - 1)] (per channel the inputs before the request's next
         token, oldest first), rows `state_slots`; it moves on by this step's tokens. `q_lens`: the requests' token
-        counts on the host (the launch is sized by the longest). Returns [T, C]."""
+        counts on the host (the launch is sized by `longest_request`). Returns [T, C]."""
         T, C = x.shape
         taps = weight.shape[1]
         B = state_slots.numel()
@@ -859,8 +859,8 @@ class HipBackend:
                "causal_conv: metadata must be int32, one token count per request")
         out = torch.empty((T, C), dtype=x.dtype, device=x.device)
         core().call("me_causal_conv", x.data_ptr(), x.stride(0), _code(x.dtype), weight.data_ptr(), _ptr(bias),
-                    state.data_ptr(), state.stride(0), state_slots.data_ptr(), cu_seqlens.data_ptr(), max(q_lens),
-                    conv_tokens_per_thread(T, B, max(q_lens), taps, C), out.data_ptr(), T, B, C, taps, _stream())
+                    state.data_ptr(), state.stride(0), state_slots.data_ptr(), cu_seqlens.data_ptr(), longest_request(q_lens),
+                    conv_tokens_per_thread(T, B, longest_request(q_lens), taps, C), out.data_ptr(), T, B, C, taps, _stream())
         return out
 
     def linear_recurrence(self, q, k, v, state, state_slots, cu_seqlens, q_lens, H: int, G: int, N: int, P: int,
@@ -905,7 +905,7 @@ class HipBackend:
             core().call("me_linear_recurrence", q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
                         _code(dtype), _ptr(dt), 0 if dt is None else dt.stride(0), _ptr(decay), _ptr(dt_bias), _ptr(rate), _ptr(skip),
                         state.data_ptr(), state.stride(0), state_slots.data_ptr(), cu_seqlens.data_ptr(), y.data_ptr(), T * H * P,
-                        B, H, G, N, P, 0, 1, int(silu), 0, 1, 0, None,
+                        B, H, G, N, P, 0, 1, int(silu), 0, 1, 0, 0, None,
                         *(none if gates is None else (None, None, key_state.data_ptr(), dot.data_ptr(), T * H)),
                         *(no_gates if gates is None else gates.args()), _stream())
             return y if gates is None else MemoryReads(y, dot, None, gates)
@@ -929,12 +929,13 @@ class HipBackend:
             i, f, stride, bi, bf, cap, m, m_stride = gates.args()
             core().call("me_soft_gates", i, f, stride, _code(dtype), bi, bf, cap, m, m_stride, state_slots.data_ptr(), cu_seqlens.data_ptr(),
                         factors[0].data_ptr(), factors[1].data_ptr(), factors[2].data_ptr(), B, H, _stream())
-        scratch = _scratch(B * spans * (H * N * P + H + (H * N if gates is not None else 0)), v.device, "recurrence") if spans > 1 else None
+        places = T // span + B if spans > 1 else 0        # spans of all requests, however the tokens are shared out among them
+        scratch = _scratch(places * (H * N * P + H + (H * N if gates is not None else 0)), v.device, "recurrence") if spans > 1 else None
         y = torch.empty((slices, T, H * P) if slices > 1 else (T, H * P), dtype=torch.float32, device=v.device)
         core().call("me_linear_recurrence", q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
                     _code(dtype), _ptr(dt), 0 if dt is None else dt.stride(0), _ptr(decay), _ptr(dt_bias), _ptr(rate), _ptr(skip),
                     state.data_ptr(), state.stride(0), state_slots.data_ptr(), cu_seqlens.data_ptr(), y.data_ptr(), T * H * P,
-                    B, H, G, N, P, per_wave, columns, int(silu), span, spans, recurrence_one_by_one(q_lens, H * -(-P // 64) * slices // columns, per_wave), _ptr(scratch),
+                    B, H, G, N, P, per_wave, columns, int(silu), span, spans, places, recurrence_one_by_one(q_lens, H * -(-P // 64) * slices // columns, per_wave), _ptr(scratch),
                     *(none if gates is None else (factors[0].data_ptr(), factors[1].data_ptr(), key_state.data_ptr(), dot.data_ptr(), T * H)),
                     *no_gates, _stream())
         return y if gates is None else MemoryReads(y, dot, factors[2], gates)
@@ -1909,6 +1910,12 @@ def wide_head_partitions(part: int, parts: int, base: int, max_context: int) -> 
     return part, parts
 
 
+def longest_request(q_lens) -> int:
+    """What launches over requests are sized by: no request of a step that runs through them brings more tokens. `q_lens`: the step's
+    counts, with a `longest` of their own where the launches are kept for steps of other counts (`TokenCounts`)."""
+    return max(getattr(q_lens, "longest", 0), max(q_lens, default=0))
+
+
 def conv_tokens_per_thread(T: int, B: int, longest: int, taps: int, C: int) -> int:
     """Tokens that a thread of the short convolution takes: 8 at once (two to four taps), or a walk over 32. The grid has
     workgroups for every 8 (32) tokens of the longest request in each of the B requests, whether the request has them or
@@ -1972,16 +1979,15 @@ def recurrence_spans(q_lens: list, waves_per_request: int, most_spans: int = 819
     carries the state on, then each span again from the state before it, which costs the work twice and pays as soon
     as the spans are many. Spans of RECURRENCE_MIN_SPAN tokens or more (shorter ones spend their time on reading and
     writing states), as many as bring the launch to RECURRENCE_WAVES waves, for steps whose longest request has two
-    spans or more."""
-    longest = max(q_lens, default=0)
+    spans or more. A captured launch has as many spans a request as the longest of its layout could fill (`longest_request`)."""
+    longest, most = max(q_lens, default=0), longest_request(q_lens)
     if longest < 2 * RECURRENCE_MIN_SPAN:
         return 0, 1
     total = sum(q_lens)
     want = max(1, RECURRENCE_WAVES // max(1, waves_per_request))        # spans over all requests
-    span = max(RECURRENCE_MIN_SPAN, -(-total // want), -(-longest // most_spans))    # a launch holds `most_spans` spans a request
+    span = max(RECURRENCE_MIN_SPAN, -(-total // want), -(-most // most_spans))    # a launch holds `most_spans` spans a request
     span = -(-span // 16) * 16
-    spans = -(-longest // span)
-    return (span, spans) if spans >= 2 else (0, 1)
+    return (span, -(-most // span)) if longest > span else (0, 1)
 
 
 EXPERT_SKINNY_MAX_ROWS = 24       # mean rows per expert up to which the 16-row tiles of the streaming kernel are taken

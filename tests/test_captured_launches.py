@@ -1,0 +1,131 @@
+"""What a captured step's launches are sized by: a graph is kept for a layout, and every step of that layout runs through it, however
+its tokens are shared out among its requests. Recorded on the CPU, without a kernel."""
+import random
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from mini_engine_amd.engine.graphs import MixedGraphs
+from mini_engine_amd.engine.packing import exact_layout
+from mini_engine_amd.kernels import ops
+
+# what was captured first, what comes after: steps of one layout, some padded, some exact, some beside decoding requests
+STEPS = [(319, [[70], [120], [64], [127]]), (319, [[1, 1, 40, 30], [1, 1, 5, 65], [1, 1, 2, 101]]), (2048, [[300, 340], [500, 140], [260, 400], [400, 240]]),
+         (319, [[1030, 1018], [1900, 148], [2046, 2], [3, 2045]]), (2048, [[130], [250], [200]]), (2048, [[130, 128, 142], [2, 2, 396], [396, 2, 2]])]
+
+
+class Recorder:
+    """In the place of the kernels' library: takes down what is launched."""
+
+    def __init__(self):
+        self.calls = []
+
+    def call(self, name, *args):
+        self.calls.append((name, args))
+
+
+def graphs(max_tokens):
+    g = MixedGraphs.__new__(MixedGraphs)
+    g.max_rows, g.capture, g.max_tokens, g.max_exact_tokens = 64, False, max_tokens, 12 * max_tokens
+    g.runner = SimpleNamespace(vocab_size=100, device=torch.device("cpu"), manager=SimpleNamespace(page_size=16), max_positions=8192)
+    return g
+
+
+def layout_of(g, lens):
+    tables = [[[0] * -(-n // 16) for n in lens]]
+    return g.padded(exact_layout(lens, [0] * len(lens), tables, len(lens), lambda *a: False))
+
+
+def captured(g, lens, monkeypatch):
+    """The context with which the step's forward pass is captured."""
+    seen = []
+    g.runner.model = SimpleNamespace(forward=lambda tokens, step, *rest: (seen.append(step), (None, None))[1], logits=lambda *a, **k: torch.zeros(64, 4))
+    g.runner.pool = SimpleNamespace(spare_page=lambda i: 500, spare_state_slot=63, views=None, states=None)
+    g.runner.zero_fresh_state = lambda *a: None
+    g.replays = 0
+    layout = layout_of(g, lens)
+    cap = SimpleNamespace(layout=layout, dev=torch.zeros(layout.segments()[1], dtype=torch.int32), events=[None], replays=0, graph=None,
+                          staging=lambda: (0, torch.zeros(layout.segments()[1], dtype=torch.int32)))
+    tables = [[list(range(-(-n // 16))) for n in lens]]
+    g.run(cap, [[0] * n for n in lens], [0] * len(lens), tables, list(range(len(lens))), [], None)
+    return seen[0]
+
+
+def divisions(layout, given):
+    """The given steps, as they are padded to the layout, and others of it."""
+    out = [[1] * layout.decode_rows + [n for n in lens if n > 1] + [layout.prefill_tokens - sum(n for n in lens if n > 1)] * (
+        layout.prefill_reqs - sum(1 for n in lens if n > 1)) for lens in given]
+    rng = random.Random(layout.prefill_tokens)
+    for _ in range(50):
+        cuts = sorted(rng.sample(range(1, layout.prefill_tokens), layout.prefill_reqs - 1))
+        out.append([1] * layout.decode_rows + [b - a for a, b in zip([0] + cuts, cuts + [layout.prefill_tokens])])
+    return out
+
+
+@pytest.mark.parametrize("limit,steps", STEPS, ids=[str(s[1][0]) for s in STEPS])
+@pytest.mark.parametrize("dtype,gated", [(torch.bfloat16, False), (torch.float32, False), (torch.bfloat16, True)], ids=["bfloat16", "float32", "gates"])
+def test_launches_cover_every_step_of_the_layout(monkeypatch, limit, steps, dtype, gated):
+    """Captured with the first step, the convolution's and the recurrence's launches cover the tokens of every other one, and the
+    scratch of the spans holds all of them."""
+    core = Recorder()
+    scratch = {}
+
+    def scratch_of(n, device, use="decode"):
+        scratch[use] = n
+        return torch.zeros(1)
+
+    monkeypatch.setattr(ops, "core", lambda: core)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_scratch", scratch_of)
+    g = graphs(limit)
+    layout = layout_of(g, steps[0])
+    assert all(layout_of(g, lens) == layout for lens in steps)
+    step = captured(g, steps[0], monkeypatch)
+    assert list(step.q_lens) == divisions(layout, steps)[0]
+    T, B, H, N, P, C, taps = layout.num_tokens, layout.num_seqs, 2, 160, 8, 8, 4          # 160 rows: in spans in both types
+    rows = lambda w: torch.empty(T, w, dtype=dtype)
+    state = torch.empty(64, H * N * P + H * N + H)
+    slots, cu = torch.zeros(B, dtype=torch.int32), torch.zeros(B + 1, dtype=torch.int32)
+    backend = ops.HipBackend()
+    backend.causal_conv(rows(C), torch.empty(C, taps), None, torch.empty(64, C * (taps - 1)), slots, cu, step.q_lens)
+    kw = dict(decay=torch.empty(H))
+    if gated:
+        kw = dict(gates=ops.SoftGates(rows(H), rows(H), torch.empty(H), torch.empty(H), 15.0, state[:, H * N * P + H * N:], slots),
+                  key_state=state[:, H * N * P: H * N * P + H * N])
+    backend.linear_recurrence(rows(H * N), rows(H * N), rows(H * P), state[:, :H * N * P], slots, cu, step.q_lens, H, H, N, P, **kw)
+    called = {name: args for name, args in core.calls}
+    conv, rec = called["me_causal_conv"], called["me_linear_recurrence"]
+    max_tokens = conv[9]
+    span, spans, places = rec[27:30]
+    for lens in divisions(layout, steps):
+        assert len(lens) == B and sum(lens) == T
+        assert max_tokens >= max(lens)
+        if spans > 1:
+            assert span * spans >= max(lens)
+            at = 0
+            for b, n in enumerate(lens):
+                assert at // span + b + -(-n // span) <= (places if b == B - 1 else (at + n) // span + b + 1)
+                at += n
+    if spans > 1:
+        assert scratch["recurrence"] >= places * (H * N * P + H + (H * N if gated else 0))
+
+
+def test_a_request_longer_than_the_layout_is_refused():
+    """The host's check in front of a replay."""
+    import numpy as np
+    from dataclasses import replace
+    from mini_engine_amd.engine import packing
+
+    layout = exact_layout([5, 3], [0, 0], [[[0], [1]]], 0, lambda *a: False)
+    assert layout.longest == 7 and exact_layout([1, 1], [0, 0], [[[0], [1]]], 0, lambda *a: False).longest == 1
+    pack = lambda l: packing.pack_step(l, np.zeros(l.segments()[1], dtype=np.int32), [[0] * 5, [0] * 3], [0, 0], [[[0], [1]]], [0, 1], [], 16, [9], 9, 100)
+    pack(layout)
+    with pytest.raises(ValueError, match="longest"):
+        pack(type("Short", (type(layout),), {"longest": 4})(**layout.__dict__))
+
+
+def test_counts_of_a_step_launched_alone_are_its_own_measure():
+    from mini_engine_amd.engine.context import TokenCounts
+    assert ops.longest_request([3, 9, 1]) == 9 and ops.longest_request([]) == 0
+    assert ops.longest_request(TokenCounts([3, 9])) == 9 and ops.longest_request(TokenCounts([3, 9], 11)) == 11
