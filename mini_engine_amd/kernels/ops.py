@@ -2034,7 +2034,7 @@ def linear_chunks_take(dtype, H: int, N: int, P: int, q_lens) -> bool:
     token 278 / 362, one of 300 among 200 535 / 242; 16 of 700 685 / 320."""
     if dtype != torch.bfloat16 or N > 128:
         return False
-    longest, count = max(q_lens), len(q_lens)
+    longest, count = max(q_lens, default=0), len(q_lens)
     if count * H * -(-P // 64) <= LINEAR_CHUNKS_FEW:
         return longest >= LINEAR_CHUNKS_MIN_TOKENS
     return longest >= (LINEAR_CHUNKS_MIN_TOKENS_MORE if count < LINEAR_CHUNKS_MANY else LINEAR_CHUNKS_MIN_TOKENS_MANY)

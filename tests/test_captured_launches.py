@@ -129,3 +129,16 @@ def test_counts_of_a_step_launched_alone_are_its_own_measure():
     from mini_engine_amd.engine.context import TokenCounts
     assert ops.longest_request([3, 9, 1]) == 9 and ops.longest_request([]) == 0
     assert ops.longest_request(TokenCounts([3, 9])) == 9 and ops.longest_request(TokenCounts([3, 9], 11)) == 11
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rows_without_a_request_launch_nothing_for_any(monkeypatch, dtype):
+    """Padding rows alone: the recurrence goes to the library with no requests, which then has nothing to do."""
+    core = Recorder()
+    monkeypatch.setattr(ops, "core", lambda: core)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    rows = lambda w: torch.empty(3, w, dtype=dtype)
+    assert not ops.linear_chunks_take(dtype, 2, 16, 8, [])
+    y = ops.HipBackend().linear_recurrence(rows(32), rows(32), rows(16), torch.empty(4, 256), torch.zeros(0, dtype=torch.int32),
+                                           torch.zeros(1, dtype=torch.int32), [], 2, 2, 16, 8, decay=torch.empty(2))
+    assert y.shape == (3, 16) and [(name, args[19]) for name, args in core.calls] == [("me_linear_recurrence", 0)]
