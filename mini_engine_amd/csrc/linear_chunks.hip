@@ -21,6 +21,7 @@ struct LinArgs {
   const int32_t* slots; const int32_t* cu;
   float* y;
   int H, G, N, P, silu, num_seqs, col_blocks;
+  int64_t from, upto;                                        // the places that scratch holds now (me_linear_chunks)
 };
 
 // Floats of a chunk: of a group q [tokens, rows], k [rows, tokens] and their products; of a head F, c, (a_{j+1} ... a_16) b_j, c_16 (with
@@ -39,7 +40,7 @@ linear_chunk_kernel(LinArgs a, float* __restrict__ group_chunks, float* __restri
   __shared__ __align__(16) float sq[C][ROW], sk[C][ROW];
   __shared__ float sl[C], sb[C];
   const int tid = threadIdx.x, lane = tid & 63;
-  const int64_t place = blockIdx.x;
+  const int64_t slot = blockIdx.x, place = a.from + slot;
   const int b = chunk_request(a.cu, a.num_seqs, place, lane);
   if (b < 0) return;
   const int begin = a.cu[b], at = (int)(place - chunk_place(a.cu, b)) * C, n_tok = min(C, a.cu[b + 1] - begin - at);
@@ -75,7 +76,7 @@ linear_chunk_kernel(LinArgs a, float* __restrict__ group_chunks, float* __restri
 #pragma unroll
       for (int e = 0; e < 4; ++e) dot[e] = fmaf(qi[e], kj[e], dot[e]);
     }
-    float* out = group_chunks + (place * a.G + g) * (int64_t)linear_group_floats(NR);
+    float* out = group_chunks + (slot * a.G + g) * (int64_t)linear_group_floats(NR);
     out[32 * NR + (j >> 2) * 64 + i * 4 + (j & 3)] = (dot[0] + dot[1]) + (dot[2] + dot[3]);
     for (int e = tid; e < C * NR / 4; e += 256) {
       const int tile = e >> 6, four = e >> 4 & 3, low = e & 15;
@@ -89,7 +90,7 @@ linear_chunk_kernel(LinArgs a, float* __restrict__ group_chunks, float* __restri
   }
 
   const int h = blockIdx.y - a.G;
-  float* out = head_chunks + (place * a.H + h) * linear_head_floats(a.col_blocks);
+  float* out = head_chunks + (slot * a.H + h) * linear_head_floats(a.col_blocks);
   // token j's -log of the decay and its factor b
   if (tid < C) {
     float l = 0.f, f = j < n_tok ? 1.f : 0.f;
@@ -150,9 +151,12 @@ linear_chunk_walk_kernel(LinArgs a, const float* __restrict__ group_chunks, cons
   const int slot = blockIdx.x >> 3, group = slot / a.col_blocks * 8 + (blockIdx.x & 7), cb = slot % a.col_blocks;
   if (group >= groups) return;
   const int b = group / a.H, h = group % a.H;
-  const int begin = __builtin_amdgcn_readfirstlane(a.cu[b]), n_tok = __builtin_amdgcn_readfirstlane(a.cu[b + 1]) - begin;
-  if (n_tok <= 0) return;
-  const int count = (n_tok + C - 1) / C;
+  // of the request the chunks whose places scratch holds; the state waits in its row between two walks
+  const int all_begin = __builtin_amdgcn_readfirstlane(a.cu[b]), all_tok = __builtin_amdgcn_readfirstlane(a.cu[b + 1]) - all_begin;
+  const int all_place = __builtin_amdgcn_readfirstlane((int)chunk_place(a.cu, b));
+  const int first = max((int)a.from - all_place, 0), count = min((all_tok + C - 1) / C, (int)a.upto - all_place) - first;
+  if (all_tok <= 0 || count <= 0) return;
+  const int begin = all_begin + C * first, n_tok = min(all_tok - C * first, C * count);
   const int p = cb * 16 + col, pc = min(p, a.P - 1);
   const bool live = p < a.P;
   float* srow = a.state + (int64_t)a.slots[b] * a.state_stride + (int64_t)h * a.N * a.P;
@@ -166,7 +170,7 @@ linear_chunk_walk_kernel(LinArgs a, const float* __restrict__ group_chunks, cons
       S[t][e] = n < a.N ? srow[(int64_t)n * a.P + pc] : 0.f;
     }
   const float skip = a.skip ? a.skip[h] : 0.f;
-  const int64_t place = __builtin_amdgcn_readfirstlane((int)chunk_place(a.cu, b));
+  const int64_t place = all_place + first - (int)a.from;
   const int64_t group_pace = (int64_t)a.G * linear_group_floats(NR), head_pace = a.H * linear_head_floats(a.col_blocks);
   const float* of_group = group_chunks + place * group_pace + (int64_t)(h / (a.H / a.G)) * linear_group_floats(NR);
   const float* of_head = head_chunks + place * head_pace + h * linear_head_floats(a.col_blocks);
@@ -269,8 +273,9 @@ linear_chunk_walk_kernel(LinArgs a, const float* __restrict__ group_chunks, cons
   }
 }
 
-// chunks: scratch of (T / 16 + num_seqs) (G linear_group_floats + H linear_head_floats) floats, for N rounded up to 32, 64 or 128; `room`:
-// how many it has.
+// chunks: scratch of `room` floats; a place takes G linear_group_floats + H linear_head_floats of them, for N rounded up to 32, 64 or 128.
+// There are T / 16 + num_seqs places; those that scratch does not hold at once are laid out and walked one part behind the other, with
+// the same bits.
 extern "C" int me_linear_chunks(const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v, int64_t v_stride,
                                 const void* dt, int64_t dt_stride, const float* decay, const float* dt_bias, const float* rate, const float* skip,
                                 float* state, int64_t state_stride, const int32_t* slots, const int32_t* cu, float* y, int num_seqs, int H,
@@ -281,23 +286,27 @@ extern "C" int me_linear_chunks(const void* q, int64_t q_stride, const void* k, 
   ME_CHECK((dt != nullptr) != (decay != nullptr) && (dt == nullptr || (dt_bias && rate)), "linear_chunks: fixed decays, or step sizes with bias and rates");
   const int64_t places = T / DC_TOKENS + num_seqs, groups = (int64_t)num_seqs * H;
   const int col_blocks = (P + 15) / 16, NR = N <= 32 ? 32 : N <= 64 ? 64 : 128;
-  const int64_t in_groups = places * G * linear_group_floats(NR);
+  const int64_t group_floats = (int64_t)G * linear_group_floats(NR), head_floats = H * linear_head_floats(col_blocks);
+  const int64_t held = room / (group_floats + head_floats), part = held < places ? held : places;
   ME_CHECK(places <= 2147483647ll && (int64_t)H + G <= 65535 && (groups + 7) / 8 * 8 * col_blocks <= 2147483647ll, "linear_chunks: too many tokens, heads or columns");
-  ME_CHECK(chunks != nullptr && (uintptr_t)chunks % 16 == 0 && room >= in_groups + places * H * linear_head_floats(col_blocks), "linear_chunks: scratch too small");
+  ME_CHECK(chunks != nullptr && (uintptr_t)chunks % 16 == 0 && part >= 1, "linear_chunks: scratch too small");
   LinArgs a;
   a.q = q; a.k = k; a.v = v; a.dt = dt; a.q_stride = q_stride; a.k_stride = k_stride; a.v_stride = v_stride; a.dt_stride = dt_stride;
   a.decay = decay; a.dt_bias = dt_bias; a.rate = rate; a.skip = skip; a.state = state; a.state_stride = state_stride; a.slots = slots; a.cu = cu;
   a.y = y; a.H = H; a.G = G; a.N = N; a.P = P; a.silu = silu; a.num_seqs = num_seqs; a.col_blocks = col_blocks;
-  const dim3 pgrid((unsigned)places, H + G);
   const unsigned wgrid = (unsigned)((groups + 7) / 8 * 8 * col_blocks);
 #define LC(NR)                                                                                                                        \
   do {                                                                                                                                \
     constexpr int WAVES = NR >= 64 ? 4 : 2;                                                                                           \
-    linear_chunk_kernel<bf16_t, NR><<<pgrid, 256, 0, stream>>>(a, chunks, chunks + in_groups);                                        \
-    linear_chunk_walk_kernel<bf16_t, NR, WAVES><<<wgrid, 64 * WAVES, 0, stream>>>(a, chunks, chunks + in_groups, (int)groups);        \
+    linear_chunk_kernel<bf16_t, NR><<<dim3((unsigned)(a.upto - a.from), H + G), 256, 0, stream>>>(a, chunks, heads);                  \
+    linear_chunk_walk_kernel<bf16_t, NR, WAVES><<<wgrid, 64 * WAVES, 0, stream>>>(a, chunks, heads, (int)groups);                     \
   } while (0)
-  if (NR == 32) LC(32); else if (NR == 64) LC(64); else LC(128);
+  float* heads = chunks + part * group_floats;
+  for (a.from = 0; a.from < places; a.from = a.upto) {
+    a.upto = a.from + part < places ? a.from + part : places;
+    if (NR == 32) LC(32); else if (NR == 64) LC(64); else LC(128);
+    ME_LAUNCH_CHECK();
+  }
 #undef LC
-  ME_LAUNCH_CHECK();
   return 0;
 }

@@ -911,12 +911,13 @@ class HipBackend:
             return y if gates is None else MemoryReads(y, dot, None, gates)
         if gates is None and linear_chunks_take(dtype, H, N, P, q_lens):
             NR = 32 if N <= 32 else 64 if N <= 64 else 128
-            room = (T // 16 + B) * (G * (32 * NR + 256) + H * (304 + 256 * -(-P // 16)))
+            place = G * (32 * NR + 256) + H * (304 + 256 * -(-P // 16))
+            room = min((T // 16 + B) * place, max(LINEAR_CHUNKS_FLOATS, place))
             chunks = _scratch(room, v.device, "recurrence")
             y = torch.empty((T, H * P), dtype=torch.float32, device=v.device)
             core().call("me_linear_chunks", q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), _ptr(dt),
                         0 if dt is None else dt.stride(0), _ptr(decay), _ptr(dt_bias), _ptr(rate), _ptr(skip), state.data_ptr(), state.stride(0),
-                        state_slots.data_ptr(), cu_seqlens.data_ptr(), y.data_ptr(), B, H, G, N, P, int(silu), T, chunks.data_ptr(), chunks.numel(),
+                        state_slots.data_ptr(), cu_seqlens.data_ptr(), y.data_ptr(), B, H, G, N, P, int(silu), T, chunks.data_ptr(), room,
                         _stream())
             return y
         per_wave = recurrence_rows_per_wave(N)
@@ -2023,6 +2024,11 @@ LINEAR_CHUNKS_FEW = 256
 LINEAR_CHUNKS_MIN_TOKENS_MORE = 64       # ... with more of them and fewer than LINEAR_CHUNKS_MANY requests,
 LINEAR_CHUNKS_MANY = 64
 LINEAR_CHUNKS_MIN_TOKENS_MANY = 128      # ... and with that many
+# Scratch that a step's chunks are laid out in, part by part if they are more: 128 MiB (`_scratch` holds up to half as much again), which
+# is about 4,900 tokens of 16 heads of 128 x 128 at once. Without a bound it grows with the step (840 MB for 16,384 tokens of
+# 32 such heads). us, 16 heads, parts of 64 MiB / 128 / 256 / one part: 8 requests of up to 350 tokens 60 / 60 / 60 / 60, 4,096 tokens 194 / 181 /
+# 181 / 181, 4 requests of 2,048 301 / 257 / 224 / 224, 16 of 700 345 / 322 / 339 / 317, 16,384 tokens, which no cache holds, 813 / 775 / 893 / 944.
+LINEAR_CHUNKS_FLOATS = 1 << 25
 
 
 def linear_chunks_take(dtype, H: int, N: int, P: int, q_lens) -> bool:

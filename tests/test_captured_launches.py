@@ -142,3 +142,23 @@ def test_rows_without_a_request_launch_nothing_for_any(monkeypatch, dtype):
     y = ops.HipBackend().linear_recurrence(rows(32), rows(32), rows(16), torch.empty(4, 256), torch.zeros(0, dtype=torch.int32),
                                            torch.zeros(1, dtype=torch.int32), [], 2, 2, 16, 8, decay=torch.empty(2))
     assert y.shape == (3, 16) and [(name, args[19]) for name, args in core.calls] == [("me_linear_recurrence", 0)]
+
+
+@pytest.mark.parametrize("lens", [[16384], [2048] * 8, [30] * 600, [1] * 300 + [9000, 4000]])
+@pytest.mark.parametrize("H,G,N,P", [(16, 16, 128, 128), (32, 1, 128, 64), (32, 32, 128, 128), (4000, 4000, 128, 128)])
+def test_scratch_for_chunks_does_not_grow_with_the_step(monkeypatch, lens, H, G, N, P):
+    """However many tokens a step has, the chunks' scratch is what the rule names, or one place where that is more."""
+    core, asked = Recorder(), []
+    monkeypatch.setattr(ops, "core", lambda: core)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_scratch", lambda n, device, use="decode": (asked.append((n, use)), torch.zeros(1))[1])
+    T, B = sum(lens), len(lens)
+    rows = lambda w: torch.empty(1, w, dtype=torch.bfloat16).expand(T, w)
+    monkeypatch.setattr(ops, "linear_chunks_take", lambda *a: True)
+    ops.HipBackend().linear_recurrence(rows(G * N), rows(G * N), rows(H * P), torch.empty(1, H * N * P), torch.zeros(B, dtype=torch.int32),
+                                       torch.zeros(B + 1, dtype=torch.int32), lens, H, G, N, P, decay=torch.empty(H))
+    (name, args), ((room, use),) = core.calls[-1], asked
+    place = G * (32 * 128 + 256) + H * (304 + 256 * (P // 16))
+    assert name == "me_linear_chunks" and use == "recurrence" and args[-2] == room
+    assert place <= room <= max(ops.LINEAR_CHUNKS_FLOATS, place) and (room // place >= T // 16 + B or room >= ops.LINEAR_CHUNKS_FLOATS)
+    assert ops.LINEAR_CHUNKS_FLOATS * 4 * 3 // 2 <= 192 << 20

@@ -48,6 +48,21 @@ def test_chunks_against_the_twin(monkeypatch, selective, lens, H, G, N, P):
 
 
 @pytest.mark.parametrize("selective", [False, True])
+@pytest.mark.parametrize("lens,H,G,N,P", [([130, 2, 80], 8, 8, 128, 64), ([1, 15, 16, 17, 0, 200], 6, 3, 20, 12), ([400], 4, 1, 64, 37), ([48, 1] * 35, 2, 1, 16, 8)])
+def test_chunks_in_parts_give_the_same_bits(monkeypatch, selective, lens, H, G, N, P):
+    """Scratch for some places only, down to one: parts that end inside a request, between two and in places that nobody has."""
+    monkeypatch.setattr(ops, "linear_chunks_take", lambda *a: True)
+    args, kw, start = _case(lens, H, G, N, P, selective)
+    want_state = start.clone()
+    want = _run(hip(), args, kw, want_state, lens, (H, G, N, P))
+    place = G * (32 * (32 if N <= 32 else 64 if N <= 64 else 128) + 256) + H * (304 + 256 * -(-P // 16))
+    for places in (1, 2, 3, 4, 7, 11, sum(lens) // 16 + len(lens) - 1):
+        monkeypatch.setattr(ops, "LINEAR_CHUNKS_FLOATS", places * place + 5)
+        state = start.clone()
+        assert torch.equal(_run(hip(), args, kw, state, lens, (H, G, N, P)), want) and torch.equal(state, want_state)
+
+
+@pytest.mark.parametrize("selective", [False, True])
 def test_what_is_not_a_number_stays_behind_its_token(monkeypatch, selective):
     """A value, key or query that is not finite reaches its own token and later ones and no token in front of it, in its chunk or
     another; a value only its own column, a head's step size only its head."""
