@@ -78,8 +78,9 @@ class CachePool:
     def reset_state(self, slots: list) -> None:
         """Rows `slots` of every state tensor back to what a request starts from."""
         kept = [(st, first) for st, first in zip(self.states, self.state_initial) if st is not None]
-        if kept and kept[0][0].is_cuda and all(st.element_size() == 4 for st, _ in kept):
-            ops.HipBackend().reset_rows([st for st, _ in kept], [first for _, first in kept], slots)
+        in_one_launch = getattr(ops.backend(), "reset_rows", None) if kept and kept[0][0].is_cuda else None
+        if in_one_launch is not None and all(st.element_size() == 4 for st, _ in kept):
+            in_one_launch([st for st, _ in kept], [first for _, first in kept], slots)
             return
         for st, first in kept:
             index = torch.tensor(slots, dtype=torch.long, device=st.device)

@@ -351,3 +351,22 @@ def test_rows_of_many_tensors_go_back_to_what_they_start_from(widths, rows):
     with pytest.raises(ops.KernelError):
         hip().reset_rows(tensors, firsts, [-1])
     assert all(torch.equal(a, b) for a, b in zip(tensors, want))
+
+
+@pytest.mark.parametrize("takes", [True, False])
+def test_states_go_back_through_the_backend_in_use(takes):
+    """The pool asks whichever backend is installed; one without a kernel for it leaves the rows to plain tensor operations."""
+    from types import SimpleNamespace
+    from mini_engine_amd.cache.pool import CachePool
+    pool, calls = CachePool.__new__(CachePool), []
+    pool.states = [torch.ones(5, 7, device=DEV), None, torch.ones(5, 2, 3, device=DEV)]
+    pool.state_initial = [None, None, torch.full((2, 3), 4.0, device=DEV)]
+    want = [t if t is None else t.clone() for t in pool.states]
+    want[0][[1, 3]], want[2][[1, 3]] = 0.0, 4.0
+    ops.set_backend(SimpleNamespace(reset_rows=lambda *a: (calls.append(a[2]), hip().reset_rows(*a))) if takes else SimpleNamespace())
+    try:
+        pool.reset_state([3, 1])
+    finally:
+        ops.set_backend(None)
+    assert calls == ([[3, 1]] if takes else [])
+    assert torch.equal(pool.states[0], want[0]) and torch.equal(pool.states[2], want[2])
