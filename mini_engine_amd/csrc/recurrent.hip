@@ -853,7 +853,7 @@ __global__ void __launch_bounds__(256) recurrence_step_kernel(RecArgs a) {
 #pragma unroll
     for (int i = 0; i < HB; ++i)
       if (r + i < r1) {
-        const float next = fmaf(sk[r + i], bv, da * held[i]);
+        const float next = fmaf(da, held[i], sk[r + i] * bv);       // the state's share is rounded once, with the sum
         acc = fmaf(next, sq[r + i], acc);
         if (on) __builtin_nontemporal_store(next, &row[(int64_t)(r + i) * a.P]);
       }
@@ -930,7 +930,7 @@ __global__ void __launch_bounds__(256) recurrence_step_few_kernel(RecArgs a) {
     if (r < r1) {
       f32x4 next;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) next[e] = fmaf(sk[r], bv[e], da * held[i][e]);
+      for (int e = 0; e < 4; ++e) next[e] = fmaf(da, held[i][e], sk[r] * bv[e]);
       if (on) __builtin_nontemporal_store(next, reinterpret_cast<f32x4*>(row + (int64_t)r * a.P));
       *reinterpret_cast<f32x4*>(&made[r][four]) = next;
     }

@@ -56,6 +56,22 @@ def test_both_forms_of_the_step_give_the_same_bits(B, H, G, N, P, selective, dty
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,H,N,P", [(3, 4, 64, 64), (1, 2, 100, 36), (5, 2, 33, 37), (2, 2, 150, 64), (70, 8, 64, 64), (30, 4, 128, 256), (90, 4, 128, 256)])
+def test_the_state_moves_on_with_one_rounding_of_its_own_share(B, H, N, P, dtype):
+    """a S + b k v^T: k v^T rounded, then a S added to it in one rounding, in every form of the step (for few requests, for many, past
+    the caches and through them): the bits that a request's state has had from the step on, and those of float64 rounded once (which
+    differs from a single rounding for sums within 2^-29 of a tie only, none of them here)."""
+    g = torch.Generator(device=DEV).manual_seed(B * N + P)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    q, k, v = (rnd(B, w).to(dtype) for w in (H * N, H * N, H * P))
+    decay, state = torch.rand(H, device=DEV, generator=g), rnd(B, H * N * P)
+    added = k.float().view(B, H, N, 1) * v.float().view(B, H, 1, P)
+    want = (decay.double().view(1, H, 1, 1) * state.double().view(B, H, N, P) + added.double()).float()
+    hip().linear_recurrence(q, k, v, state, torch.arange(B, device=DEV).int(), torch.arange(B + 1, device=DEV).int(), [1] * B, H, H, N, P, decay=decay)
+    assert torch.equal(state.view(B, H, N, P), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("kind", ["silu_before", "sigmoid_behind", "silu_behind"])
 @pytest.mark.parametrize("n,parts", [(1023, 1), (1024, 1), (1025, 2), (2048, 1), (2049, 1), (4097, 3), (8192, 1), (8200, 1)])
 def test_gated_norm_widths(n, parts, kind, dtype):
