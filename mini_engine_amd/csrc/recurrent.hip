@@ -812,13 +812,14 @@ __device__ __forceinline__ void step_factors(const RecArgs& a, int b, int h, flo
   }
 }
 
-// A step of single tokens (token b is request b's): the state streams through once, past the caches, which do not hold it until the
-// next step (64 requests, 16 heads of 128 x 128: 31.4 -> 24.7 us, 5.4 TB/s). One workgroup of four waves per
+// A step of single tokens (token b is request b's): the state streams through once, with PAST past the caches, which do not
+// hold it until the next step (where: me_linear_recurrence; 64 requests, 32 heads of 128 x 64: 32.2 -> 25.5 us, 5.3 TB/s). One workgroup of four waves per
 // (request, head, 64 columns); each wave takes a quarter of the N rows, and the four partial outputs meet in LDS.
 // HB: rows that a wave asks for at once and holds until they are written back, the first of them before it meets the others: a quarter of 128 rows is one trip to
 // memory instead of four behind each other (8 requests, 16 heads of 128 x 128, 16.8 MB read and written: 10.4 -> 8.1 us).
-template <typename TX, int HB>
+template <typename TX, int HB, bool PAST>
 __global__ void __launch_bounds__(256) recurrence_step_kernel(RecArgs a) {
+  auto state_at = [](const float* at) { return PAST ? __builtin_nontemporal_load(at) : *at; };
   extern __shared__ float kq[];                       // k[N], q[N], then 4 x 64 partial outputs
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int b = blockIdx.x / a.H, h = blockIdx.x - b * a.H;
@@ -835,7 +836,7 @@ __global__ void __launch_bounds__(256) recurrence_step_kernel(RecArgs a) {
   const int r0 = wave * per, r1 = r0 + per < a.N ? r0 + per : a.N;
   float held[HB];
 #pragma unroll
-  for (int i = 0; i < HB; ++i) held[i] = __builtin_nontemporal_load(&row[(int64_t)max(min(r0 + i, r1 - 1), 0) * a.P]);
+  for (int i = 0; i < HB; ++i) held[i] = state_at(&row[(int64_t)max(min(r0 + i, r1 - 1), 0) * a.P]);
   for (int i = threadIdx.x; i < a.N; i += 256) {
     float kk = to_f32<TX>(((const TX*)a.k)[(int64_t)b * a.k_stride + (int64_t)g * a.N + i]);
     float qq = to_f32<TX>(((const TX*)a.q)[(int64_t)b * a.q_stride + (int64_t)g * a.N + i]);
@@ -855,11 +856,14 @@ __global__ void __launch_bounds__(256) recurrence_step_kernel(RecArgs a) {
       if (r + i < r1) {
         const float next = fmaf(da, held[i], sk[r + i] * bv);       // the state's share is rounded once, with the sum
         acc = fmaf(next, sq[r + i], acc);
-        if (on) __builtin_nontemporal_store(next, &row[(int64_t)(r + i) * a.P]);
+        if (on) {
+          if (PAST) __builtin_nontemporal_store(next, &row[(int64_t)(r + i) * a.P]);
+          else row[(int64_t)(r + i) * a.P] = next;
+        }
       }
     if (r + HB < r1) {
 #pragma unroll
-      for (int i = 0; i < HB; ++i) held[i] = __builtin_nontemporal_load(&row[(int64_t)min(r + HB + i, r1 - 1) * a.P]);
+      for (int i = 0; i < HB; ++i) held[i] = state_at(&row[(int64_t)min(r + HB + i, r1 - 1) * a.P]);
     }
   }
   part[wave * 64 + lane] = acc;
@@ -1036,13 +1040,21 @@ extern "C" int me_linear_recurrence(const void* q, int64_t q_stride, const void*
       return 0;
     }
     const size_t lds = (size_t)(2 * N + 256) * sizeof(float);
-#define REC_STEP(HB)                                                                                   \
+    // Which states pass the caches. us, through / past them, fourteen layers' states in turn, rows x columns and MB of a layer: 128 x 64 25 14.0 / 10.1, 67 32 / 25.5, 134 58 / 50; 128
+    // x 128 25 14.9 / 12.7, 134 64 / 62, beside summed keys 21 14.1 / 12.6, 67 39.5 / 44; 128 x 256 25 15.5 / 13.6, 42 24.7 / 25.3, 67 38.5 / 42.5,
+    // 134 68 / 86; 256 x 512 50 26 / 30, 134 65 / 96; 64 x 64 with keys 0.5 5.4 / 5.7, 4.2 6.6 / 6.5. Rows of more than 64 columns are
+    // shared between workgroups, which then reach the same memory at different times.
+    const int64_t bytes = (int64_t)num_seqs * H * N * P * 4;
+    const bool past = bytes >= (4 << 20) && (P <= 64 || bytes <= 26000000 || (P <= 128 && N <= 128 && keys == nullptr));
+#define REC_STEP_AT(HB, PAST)                                                                          \
   do {                                                                                                 \
-    if (dtype == ME_F32) recurrence_step_kernel<float, HB><<<grid, dim3(256), lds, stream>>>(a);       \
-    else recurrence_step_kernel<bf16_t, HB><<<grid, dim3(256), lds, stream>>>(a);                      \
+    if (dtype == ME_F32) recurrence_step_kernel<float, HB, PAST><<<grid, dim3(256), lds, stream>>>(a); \
+    else recurrence_step_kernel<bf16_t, HB, PAST><<<grid, dim3(256), lds, stream>>>(a);                \
   } while (0)
+#define REC_STEP(HB) do { if (past) REC_STEP_AT(HB, true); else REC_STEP_AT(HB, false); } while (0)
     if (N <= 32) REC_STEP(8); else if (N <= 64) REC_STEP(16); else REC_STEP(32);
 #undef REC_STEP
+#undef REC_STEP_AT
     ME_LAUNCH_CHECK();
     return 0;
   }
