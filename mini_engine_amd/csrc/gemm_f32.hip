@@ -2,7 +2,7 @@
 // (v_mfma_f32_16x16x32_bf16: products exact, sums float32). The 32-bit path's product for any number of rows (reference
 // layers/linear.py:26,45: F.linear).
 //
-// An operand is the exact sum of three bfloat16 numbers (`Thirds`), and of the nine products of two operands' thirds the six
+// An operand of 2^-110 or more is the exact sum of three bfloat16 numbers (`Thirds`; smaller ones: F32_SMALLEST), and of the nine products of two operands' thirds the six
 // largest are formed, the smallest first; the other three are below 2^-24 of the product. A float32 matrix instruction does
 // 256 operations a cycle and compute unit, six of these 683. Weights that came as bfloat16, as most checkpoints
 // hold them, have one third only: a wave that sees no bit in the lower halves of its 32 k of weights leaves out the three products
@@ -31,6 +31,12 @@
 
 
 #define F32_ROW_GROUP 8
+// What three bfloat16 parts cannot give, an infinity, a value that rounds up to one and one below 2^-110, whose last bits are below the
+// smallest bfloat16 of 2^-133, shows in the sums: they are not finite, or small. Sums that are not finite, and those below this,
+// are formed again (end of the kernel): from here up a value that lost what is below 2^-134 moves a sum by less than float32's own
+// rounding as long as its terms' operands add up to less than 2^46. Sums of zero stay: operands below 2^-134 count as zeros where
+// none of a sum's terms has larger ones.
+#define F32_SMALLEST 0x1f800000u                   // 2^-64
 
 // A lane's 8 values of one row as sums of three bfloat16 numbers each: the value rounded, what that leaves rounded, and the rest,
 // which has no more than 8 bits: the three add up to the value exactly. The remainders come from the dot product of two
@@ -59,14 +65,6 @@ __device__ __forceinline__ void f32_thirds(const f32x4 (&v)[2], Thirds& t) {
   }
   t.high = high.v;
   if (ALL) { t.mid = mid.v; t.low = low.v; }
-}
-
-// One output in plain multiply-adds (see the end of the kernel).
-__device__ __forceinline__ float f32_plain_dot(const float* x, const float* w, int K) {
-  float v = 0.f;
-#pragma unroll 1
-  for (int k = 0; k < K; ++k) v = fmaf(x[k], w[k], v);
-  return v;
 }
 
 // 16 bytes per lane and load into LDS at lds_addr + 1024 j + 16 lane for load j of a group of two or four; its memory is base +
@@ -218,6 +216,9 @@ gemm_f32_kernel(const float* __restrict__ x, int64_t ldx, const float* __restric
     __syncthreads();                             // all blocks have been read: LDS takes the sums
   }
 
+  // What the parts cannot give (F32_SMALLEST): a bit for each of a thread's outputs that is formed again below.
+  static_assert(TM * 4 <= 256 && NI <= 8, "four outputs of every sixteen features to a thread");
+  uint32_t again = 0;
   f32x4 (*merge)[4][TM * 4] = reinterpret_cast<f32x4 (*)[4][TM * 4]>(f32_lds);
   // a lane holds features 4 g .. 4 g + 3 of row r: the waves' sums meet 16 features at a time through LDS
 #pragma unroll
@@ -226,13 +227,17 @@ gemm_f32_kernel(const float* __restrict__ x, int64_t ldx, const float* __restric
     for (int i = 0; i < MI; ++i) merge[n & 1][wave][(16 * i + r) * 4 + g] = acc[i][n];
     __syncthreads();                             // the buffer of the round before is free again two rounds on
     for (int e = tid; e < TM * 4; e += 256) {
-      f32x4 v = (merge[n & 1][0][e] + merge[n & 1][1][e]) + (merge[n & 1][2][e] + merge[n & 1][3][e]);
+      const f32x4 v = (merge[n & 1][0][e] + merge[n & 1][1][e]) + (merge[n & 1][2][e] + merge[n & 1][3][e]);
       const int m = m0 + e / 4, f = n0 + 16 * n + (e & 3) * 4;
       if (m < M) {
-        // an infinity has no thirds (its rest is not a number), so what came out as not a number is formed once more
+        bool odd = false;                        // (as whole numbers the sizes of floats have their order)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (v[j] != v[j] && f + j < N) v[j] = f32_plain_dot(x + (int64_t)m * ldx, w + (int64_t)(f + j) * ldw, K);
+        for (int j = 0; j < 4; ++j) odd |= (f32_bits(v[j]) & 0x7fffffffu) - F32_SMALLEST >= 0x7f800000u - F32_SMALLEST;
+        if (__builtin_expect(odd, 0)) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (f + j < N && v[j] != 0.f && !(fabsf(v[j]) >= __uint_as_float(F32_SMALLEST) && fabsf(v[j]) < INFINITY)) again |= 1u << (4 * n + j);
+        }
         float* at = y + (int64_t)m * ldy + f;
         if (vec_out && f + 3 < N) *reinterpret_cast<f32x4*>(at) = v;
         else {
@@ -241,6 +246,34 @@ gemm_f32_kernel(const float* __restrict__ x, int64_t ldx, const float* __restric
             if (f + j < N) at[j] = v[j];
         }
       }
+    }
+  }
+
+  // These once more, 16 x 16 outputs at a time, on the float32 matrix instructions: blocks and chains as above, all by the wave that has
+  // the outputs, a lane's 4 consecutive k of a row straight from memory. The others keep their bits. (300 rows of 151936 x 1024, one of which is
+  // not a number, 0.51 -> 2.4 ms.)
+#pragma unroll 1
+  for (int n = 0; n < NI; ++n) {
+    const uint32_t mine = again >> (4 * n) & 15u;
+    if (__ballot(mine != 0) == 0) continue;
+    const float *xr = x0 + (int64_t)min(16 * wave + r, M - 1 - m0) * ldx, *wr = w0 + (int64_t)min(16 * n + r, N - 1 - n0) * ldw;
+    f32x4 chain[4] = {};
+#pragma unroll 1
+    for (int k0 = 4 * g; k0 - 4 * g < K; k0 += k0 & 16 ? 112 : 16)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int k = k0 + 32 * c + j, at = min(k, K - 1);
+          chain[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(k < K ? wr[at] : 0.f, k < K ? xr[at] : 0.f, chain[c], 0, 0, 0);
+        }
+    // a lane holds features 4 g .. 4 g + 3 of row r, and stored those of 4 (lane % 4) on of row lane / 4
+    const f32x4 v = (chain[0] + chain[1]) + (chain[2] + chain[3]);
+    const int from = (lane & 3) * 16 + (lane >> 2);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float o = __shfl(v[j], from);
+      if (mine >> j & 1) y[(int64_t)(m0 + tid / 4) * ldy + n0 + 16 * n + (tid & 3) * 4 + j] = o;
     }
   }
 }

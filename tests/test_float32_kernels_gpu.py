@@ -74,6 +74,52 @@ def test_product_by_parts(M, N, K):
         assert torch.allclose(got[rows, N // 2].double()[inside], want[inside], rtol=1e-5)
 
 
+@pytest.mark.parametrize("M,N,K", [(2, 40, 32), (19, 33, 100), (50, 150, 516), (130, 64, 300)])
+@pytest.mark.parametrize("power", [-100, -110, -118, -126, -133])
+def test_product_of_tiny_values(M, N, K, power):
+    """Values whose last bits lie below what a part can hold: as near to 64 bits as float32 sums are, and rows of other sizes in the
+    same launch keep their bits."""
+    g = torch.Generator(device=DEV).manual_seed(M * K)
+    usual = torch.randn(M, K, device=DEV, generator=g)
+    w = torch.randn(N, K, device=DEV, generator=g)
+    x = usual.clone()
+    x[::2] = (usual[::2].double() * 2.0 ** power).float()
+    for few in (x, x.flip(0)):
+        # of the sum of the products' sizes as in test_product_by_parts, and half a step of 2^-149 for every product and sum
+        bound = 2.0 ** -24 * (12 * -(-K // 128) + 5) * (few.double().abs() @ w.double().abs().T) + 2.0 ** -149 * K
+        for tile in TILES:
+            y = _product(few, w, tile)
+            assert bool(((y.double() - few.double() @ w.double().T).abs() <= bound).all()), tile
+    # both operands tiny where the other is not
+    some = torch.zeros(M, K, device=DEV)
+    some[:, ::2] = x[:, ::2]
+    v = (w.double() * torch.where(torch.arange(K, device=DEV) % 2 == 1, 2.0 ** power, 1.0)).float()
+    for tile in TILES:
+        assert torch.equal(_product(x, w, tile)[1::2], _product(usual, w, tile)[1::2])
+        y, want = _product(some + x * 0.25, v, tile), (some + x * 0.25).double() @ v.double().T
+        size = (some + x * 0.25).double().abs() @ v.double().abs().T
+        assert bool(((y.double() - want).abs() <= 2.0 ** -24 * (12 * -(-K // 128) + 5) * size + 2.0 ** -149 * K).all())
+
+
+@pytest.mark.parametrize("tile", TILES)
+def test_product_near_overflow(tile):
+    """A sum that float32 holds, though a value rounds up to an infinity in bfloat16 or the product of the rounded values is one; and one
+    that float32 does not hold, whose neighbours keep their bits."""
+    g = torch.Generator(device=DEV).manual_seed(5)
+    x, w = torch.randn(70, 200, device=DEV, generator=g), torch.randn(90, 200, device=DEV, generator=g)
+    x[:3] = w[:3] = 0.0
+    x[0, 7], w[0, 7] = 3.4e38, 0.99                       # rounds up to an infinity
+    x[1, 50], w[1, 50] = 1.999 * 2.0 ** 64, 1.999 * 2.0 ** 62          # 2^65 * 2^63
+    x[2, 199], w[2, 199] = 2.0 ** 100, -2.0 ** 100
+    y = _product(x, w, tile)
+    assert abs(y[0, 0].double() / (x[0, 7].double() * w[0, 7].double()) - 1) < 2.0 ** -23
+    assert abs(y[1, 1].double() / (x[1, 50].double() * w[1, 50].double()) - 1) < 2.0 ** -23
+    assert float(y[2, 2]) == -float("inf")
+    other = x.clone()
+    other[:3] = torch.randn(3, 200, device=DEV, generator=g)
+    assert torch.equal(y[3:, 3:], _product(other, w, tile)[3:, 3:])
+
+
 @pytest.mark.parametrize("Hq,Hkv,D,page", [(4, 2, 16, 4), (3, 1, 80, 8), (6, 2, 112, 16), (2, 2, 128, 12), (4, 4, 96, 64)])
 @pytest.mark.parametrize("extra", [{}, {"window": 20}, {"window": 37, "keep_first": 5}, {"chunk": 24}, {"softcap": 3.0}])
 def test_attention_tiles(Hq, Hkv, D, page, extra):
