@@ -43,6 +43,9 @@ class StepContext:
     # host copies, for parts that decide launches on the host
     q_lens: TokenCounts = field(default_factory=TokenCounts)
     starts: list = field(default_factory=list)
+    # the step is being captured, or it is the run in front of a capture, which is launched the same way so that whatever a
+    # capture refuses to make (handles and workspaces of a further stream) is there
+    captured: bool = False
     # what one layer call leaves for later calls of the same step, by name (values of this step's tokens that a
     # later layer blends into its own); filled and read while the step runs, also while it is captured
     shared: dict = field(default_factory=dict)

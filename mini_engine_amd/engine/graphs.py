@@ -89,7 +89,7 @@ class _Captured:
         o, size = self.seg[name]
         return self.dev[o:o + size]
 
-    def context(self) -> StepContext:
+    def context(self, captured: bool = False) -> StepContext:
         B = self.bucket
         return StepContext(
             num_tokens=B, num_seqs=B, num_decodes=B, positions=self.view("positions"),
@@ -98,7 +98,7 @@ class _Captured:
             decode_contexts_even=self.even,
             groups=[GroupStep(self.view(f"bt{g}").view(B, self.MB), self.view(f"slots{g}")) for g in range(self.G)],
             state_slots=self.view("state_slots"), first_chunk=self.view("first_chunk"),
-            q_lens=TokenCounts([1] * B), starts=[0] * B)
+            q_lens=TokenCounts([1] * B), starts=[0] * B, captured=captured)
 
     def upload(self):
         i = self.flip
@@ -286,7 +286,7 @@ class DecodeGraphs:
 
     def _forward(self, cap: _Captured, out=None):
         r = self.runner
-        h, residual = r.model.forward(cap.view("tokens"), cap.context(), r.pool.views, r.pool.states)
+        h, residual = r.model.forward(cap.view("tokens"), cap.context(self.capture), r.pool.views, r.pool.states)
         return r.model.logits(h, residual, cap.view("rows"), out=out)
 
     def _capture(self, cap: _Captured) -> bool:
@@ -418,17 +418,25 @@ class MixedGraphs:
         self.capture_after = capture_after
         self.max_graphs = max_graphs
         self.max_tokens = host_bound_tokens(runner.model) if max_tokens is None else max_tokens
-        branches = max_tokens is None and any(getattr(part, "captures_branches", False) for part in runner.model.parts())
-        self.max_exact_tokens = (BRANCHES_LAYOUT_FACTOR if branches else EXACT_LAYOUT_FACTOR) * self.max_tokens
+        self.max_exact_tokens = EXACT_LAYOUT_FACTOR * self.max_tokens
+        self.branching = [part for part in runner.model.parts() if hasattr(part, "captures_branches")]
+        self.max_branches_tokens = (BRANCHES_LAYOUT_FACTOR if max_tokens is None else EXACT_LAYOUT_FACTOR) * self.max_tokens
         self.captured: dict = {}
         self.sightings: dict = {}
         self.pool = runner.graph_pool() if capture else None
         self.replays = 0
 
+    def pays(self, tokens: int) -> bool:
+        """Whether a step of so many tokens is worth a replay at all; what the model's parts put on further streams counts as it is
+        switched now."""
+        if tokens < self.max_exact_tokens:
+            return True
+        return tokens < self.max_branches_tokens and any(part.captures_branches for part in self.branching)
+
     def padded(self, exact: StepLayout) -> StepLayout | None:
         r = self.runner
         tokens = exact.decode_rows + exact.prefill_tokens
-        if (exact.prefill_reqs == 0 or exact.rows > self.max_rows or tokens >= self.max_exact_tokens or r.vocab_size is None
+        if (exact.prefill_reqs == 0 or exact.rows > self.max_rows or r.vocab_size is None or not self.pays(tokens)
                 or not (r.device.type == "cuda" or not self.capture)):
             return None
         ps = r.manager.page_size
@@ -517,7 +525,7 @@ class MixedGraphs:
         r = self.runner
         layout = cap.layout
         tokens, rows = views_of(layout, cap.dev)
-        h, residual = r.model.forward(tokens, context_of(layout, cap.dev, q_lens, first, layout.longest), r.pool.views, r.pool.states)
+        h, residual = r.model.forward(tokens, context_of(layout, cap.dev, q_lens, first, layout.longest, self.capture), r.pool.views, r.pool.states)
         if not layout.rows:
             return None
         return r.model.logits(h, residual, rows[:layout.rows], out=out)

@@ -162,7 +162,8 @@ def pack_step(layout: StepLayout, out: np.ndarray, token_lists: list, starts: li
     return all_q, all_start
 
 
-def context_of(layout: StepLayout, dev, q_lens: list | None = None, starts: list | None = None, longest: int = 0) -> StepContext:
+def context_of(layout: StepLayout, dev, q_lens: list | None = None, starts: list | None = None, longest: int = 0,
+               captured: bool = False) -> StepContext:
     """The `StepContext` whose tensors are views into the packed array `dev` (on the device). `longest`: see `TokenCounts`; a step
     that is launched for its whole layout names the layout's."""
     seg, _ = layout.segments()
@@ -179,7 +180,7 @@ def context_of(layout: StepLayout, dev, q_lens: list | None = None, starts: list
         decode_contexts_even=layout.even, max_prefill_context=layout.prefill_ctx,
         groups=[GroupStep(view(f"bt{g}").view(B, mb), view(f"slots{g}")) for g, mb in enumerate(layout.max_blocks)],
         state_slots=view("state_slots"), first_chunk=view("first_chunk"),
-        q_lens=TokenCounts(q_lens if q_lens is not None else [], longest), starts=list(starts) if starts is not None else [])
+        q_lens=TokenCounts(q_lens if q_lens is not None else [], longest), starts=list(starts) if starts is not None else [], captured=captured)
 
 
 def views_of(layout: StepLayout, dev) -> tuple:

@@ -53,7 +53,6 @@ class SideBySide(Mixer):
         self._cache_of = 0 if needs[0] is not None else (1 if needs[1] is not None else None)
         self._state_of = 0 if states[0] is not None else (1 if states[1] is not None else None)
         self.capturable = getattr(left, "capturable", True) and getattr(right, "capturable", True)
-        self.captures_branches = self.side_stream and getattr(right, "walks", False)
         left.defer_bias = right.defer_bias = True         # an output bias joins the weighted sum's kernel (`Biased`)
 
     def cache_need(self):
@@ -62,11 +61,15 @@ class SideBySide(Mixer):
     def state_need(self):
         return None if self._state_of is None else (self.left, self.right)[self._state_of].state_need()
 
+    @property
+    def captures_branches(self) -> bool:
+        """Whether captured steps of any size have the right mixer on a second stream."""
+        return self.side_stream and getattr(self.right, "walks", False)
+
     def forward(self, x, step, cache, state, terms: bool = False):
         """`terms`: return the two outputs unadded (`ScaledTerms`) for a consumer that forms the weighted sum itself."""
         give = lambda i: (cache if self._cache_of == i else None, state if self._state_of == i else None)
-        walks = self.side_stream and self.captures_branches and x.is_cuda and ops.second_workspace.made(x.device)
-        if (self.side_stream and few_tokens(x)) or (walks and torch.cuda.is_current_stream_capturing()):
+        if (self.side_stream and few_tokens(x)) or (step.captured and self.captures_branches and x.is_cuda and ops.second_workspace.made(x.device)):
             with side_branch(x.device, 1) as branch:
                 b = self.right.forward(x, step, *give(1))
             a = self.left.forward(x, step, *give(0))

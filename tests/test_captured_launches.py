@@ -27,7 +27,7 @@ class Recorder:
 
 def graphs(max_tokens):
     g = MixedGraphs.__new__(MixedGraphs)
-    g.max_rows, g.capture, g.max_tokens, g.max_exact_tokens = 64, False, max_tokens, 12 * max_tokens
+    g.max_rows, g.capture, g.max_tokens, g.max_exact_tokens, g.max_branches_tokens = 64, False, max_tokens, 12 * max_tokens, 0
     g.runner = SimpleNamespace(vocab_size=100, device=torch.device("cpu"), manager=SimpleNamespace(page_size=16), max_positions=8192)
     return g
 
@@ -109,6 +109,36 @@ def test_launches_cover_every_step_of_the_layout(monkeypatch, limit, steps, dtyp
                 at += n
     if spans > 1:
         assert scratch["recurrence"] >= places * (H * N * P + H + (H * N if gated else 0))
+
+
+def test_reach_of_captures_follows_the_branches_switch():
+    """Twice as many tokens as otherwise, while a part that may put work on a further stream does."""
+    g = graphs(319)
+    g.max_exact_tokens, g.max_branches_tokens = 6 * 319, 12 * 319
+    part = SimpleNamespace(captures_branches=True)
+    g.branching = [SimpleNamespace(captures_branches=False), part]
+    takes = lambda n: layout_of(g, [n]) is not None
+    assert takes(1913) and takes(1914) and takes(3827) and not takes(3828)
+    part.captures_branches = False
+    assert takes(1913) and not takes(1914)
+
+
+def test_the_run_in_front_of_a_capture_is_launched_as_the_capture_is(monkeypatch):
+    """Both forward passes have the context that puts work on further streams; a step launched one by one has not."""
+    import contextlib
+    from mini_engine_amd.engine import graphs as module
+    from mini_engine_amd.engine.packing import context_of
+    g, seen = graphs(319), []
+    monkeypatch.setattr(module.torch.cuda, "CUDAGraph", lambda: SimpleNamespace(replay=lambda: seen.append("replay")))
+    monkeypatch.setattr(module.torch.cuda, "graph", lambda graph, pool: contextlib.nullcontext())
+    monkeypatch.setattr(module.torch.cuda, "synchronize", lambda: None)
+    layout = layout_of(g, [70])
+    g.capture, g.pool = True, None
+    g.runner.model = SimpleNamespace(forward=lambda tokens, step, *rest: (seen.append(step.captured), (None, None))[1], logits=lambda *a, **k: None)
+    g.runner.pool = SimpleNamespace(views=None, states=[torch.zeros(2)])
+    cap = SimpleNamespace(layout=layout, dev=torch.zeros(layout.segments()[1], dtype=torch.int32))
+    module.capture_graph(g.runner, None, lambda: g._forward(cap, None, [70, 58], [0, 0]))
+    assert seen == [True, True] and not context_of(layout, cap.dev).captured
 
 
 def test_a_request_longer_than_the_layout_is_refused():

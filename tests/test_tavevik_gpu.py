@@ -260,7 +260,8 @@ def test_prompts_of_captured_steps_run_both_mixers_beside_each_other(tavevik_fol
         for part in runner.model.parts():
             if isinstance(part, hybrid.SideBySide):
                 assert part.captures_branches
-                part.captures_branches = beside
+                part.side_stream = beside
+                assert part.captures_branches == beside
         drivers.append(helpers.Driver(runner, manager))
     for i in range(6):
         ids = {f"{r}{i}": helpers.random_ids(90, C.CONFIGS["pair"]["vocab"], 70 + 2 * i + j) for j, r in enumerate("ab"[:1 + i % 2])}
@@ -269,7 +270,34 @@ def test_prompts_of_captured_steps_run_both_mixers_beside_each_other(tavevik_fol
             counts.append(len(branches))
         assert all(torch.equal(drivers[0].result(r), drivers[1].result(r)) for r in ids), f"step {i}"
     assert all(d.runner.mixed_graphs.replays >= 4 for d in drivers)
-    assert branches and all(branches) and counts[4] > counts[3] and counts[5] == counts[4]      # the third step was captured
+    # every branch of a capture has run once in front of it, launched by itself
+    assert branches and sum(branches) * 2 == len(branches) and counts[4] > counts[3] and counts[5] == counts[4]      # the third step was captured
+
+
+def test_products_of_a_captured_branch_may_go_through_torch(tavevik_folders, monkeypatch):
+    """Where the direct library call offers nothing for a shape, torch's route makes its handle and workspace for the second stream in the
+    run in front of the capture, not in the capture, which refuses that."""
+    linear, through_torch = ops.HipBackend.linear, []
+
+    def other(self, x, w, out_dtype=None, allow_partials=False, out=None):
+        if x.dim() != 2 or x.dtype != torch.bfloat16 or w.dtype != x.dtype or out is not None or out_dtype not in (None, x.dtype):
+            return linear(self, x, w, out_dtype, allow_partials, out)
+        through_torch.append((torch.cuda.current_stream().cuda_stream, torch.cuda.is_current_stream_capturing()))
+        return torch.matmul(x, w.t())
+
+    monkeypatch.setattr(ops.HipBackend, "linear", other)
+    drivers = []
+    for graphs in (True, False):
+        runner, manager, _ = Env(tavevik_folders, torch.bfloat16, graphs=graphs).runner("pair", 200, 4)
+        drivers.append(helpers.Driver(runner, manager))
+    for i in range(5):
+        ids = {f"a{i}": helpers.random_ids(90, C.CONFIGS["pair"]["vocab"], 90 + i)}
+        for d in drivers:
+            d.step(ids, end=list(ids))
+        got, want = (d.result(f"a{i}") for d in drivers)
+        assert float((got - want).abs().max() / want.abs().max()) <= TOL[torch.bfloat16]
+    assert drivers[0].runner.mixed_graphs.replays >= 3
+    assert len({stream for stream, captured in through_torch if captured}) == 2
 
 
 def test_hip_libraries_are_the_ones_running(env):
