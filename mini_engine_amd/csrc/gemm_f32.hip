@@ -23,8 +23,11 @@
 // Measured (us, weights from bfloat16 / with all bits; in brackets the float32 matrix instructions on operands read straight from
 // memory, the 32-bit product before): 300 rows of 4096 x 1024 22 / 27 (43), 1024 x 2048 16 / 20 (25), 6144 x 1024 26 / 34 (57), 1024
 // x 3072 22 / 28 (37), 151936 x 1024 540 / 738 (1,263). Few rows: 16 of 4096 x 1024 7.1 / 7.4 (8.4), of 1024 x 3072 10.9 / 12.4
-// (16.2), one row of 6144 x 1024 8.8 / 9.2 (10.1), of 12288 x 4096 46 / 46 (56), of 1024 x 3072, where 64 workgroups have a
-// compute unit each and a block's chain of conversions and products is what is waited for, 11.2 / 12.4 (10.4). Error against 64
+// (16.2), one row of 6144 x 1024 8.4 / 8.4 (9.7 / 9.2), of 4096 x 1024 6.5 / 6.7 (6.5), of 12288 x 4096 46 / 46 (56). Behind the product before, for
+// one to four rows: few workgroups, a compute unit each, where a block's chain of conversions and products is what is waited for: one row of
+// 1024 x 2048 7.4 / 8.2 (7.2), 1024 x 3072 10.2 / 11.3 (9.8), 512 x 4096 13.0 / 14.6 (11.4); four rows 7.4 / 8.2 (8.0), 10.3 / 11.4 (11.0), 13.0 / 14.7 (12.9). A form of
+// its own for them would give a token other bits alone than among others; reading a block ahead of its use, deeper rings and a
+// second wave to split the features were no faster. Error against 64
 // bits over 1,024 / 2,048 / 3,072 / 12,288 terms 1.7 / 2.4 / 2.9 / 6.1e-7 of the result's norm with bfloat16 weights, 2.3 / 3.4 / 4.2 /
 // 9.0e-7 with all bits (2.9 / 4.1 / 5.0 / 9.9e-7).
 #include "common.h"
@@ -84,8 +87,12 @@ __device__ __forceinline__ void f32_wait_lds() { asm volatile("s_waitcnt lgkmcnt
 
 // RING: blocks of a wave that wait in LDS or are on their way there; 0: operands that are no whole 16-byte pieces, every value
 // loaded by itself straight into registers (the same sums).
+// Tiles of 32 x 64 and 64 x 32 are held to 256 registers, of which matrix instructions then use the ordinary ones: the sums are not copied
+// to others and back around every block (300 rows, weights from bfloat16 / with all bits, 4096 x 1024 19.9 -> 18.8 / 25.3 -> 24.7 us, 1024 x 2048
+// 14.8 -> 13.5 / 20.2 -> 20.3, 1024 x 3072 20.1 -> 18.4 / 28.2 -> 28.5). Smaller ones with all bits lose by it (512 x 4096 14.6 -> 15.1), larger ones
+// have more sums than that.
 template <int TM, int TN, int RING>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, TM * TN == 2048 ? 2 : 1)
 gemm_f32_kernel(const float* __restrict__ x, int64_t ldx, const float* __restrict__ w, int64_t ldw, float* __restrict__ y,
                 int64_t ldy, int M, int N, int K, int m_tiles, int n_tiles, int vec_out) {
   constexpr int MI = TM / 16, NI = TN / 16;
