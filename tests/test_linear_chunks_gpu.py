@@ -89,3 +89,31 @@ def test_rule():
     assert take([16]) and take([16] * 8) and not take([15]) and not take([16] * 8, H=32) and take([64] * 8, H=32)
     assert not take([64] + [1] * 300) and take([300] + [1] * 200) and take([128] * 64)
     assert not take([300], N=130) and not take([300], dtype=torch.float32)
+
+
+@pytest.mark.parametrize("pattern", [[300], [15, 1, 16, 17], [100, 7, 63, 64], [1, 130, 40], [8, 31, 33, 200]], ids=str)
+def test_cuts_and_neighbours_on_both_sides_of_the_rule(tmp_path, monkeypatch, pattern):
+    """Portions and requests beside them decide which form a step takes. However a prompt is cut, its logits are as near to the plain
+    evaluation as with the other form alone: both round to bfloat16 in the same places, so their errors are draws of one size, and the
+    largest over a prompt's logits differs by less than half."""
+    import helpers
+    import sigosun_cases as S
+    from mini_engine_amd.cache.manager import CacheManager
+    from mini_engine_amd.engine.runner import ModelRunner
+    from mini_engine_amd.weights.loader import load_model
+
+    folder = S.make_folder("real", str(tmp_path))
+    model = load_model(folder, DEV, torch.bfloat16, 512)
+    ids = {r: helpers.random_ids(n, S.CONFIGS["real"]["vocab"], n) for r, n in (("long", 300), ("short", 70), ("last", 180))}
+    take, took, errors = ops.linear_chunks_take, [], []
+    for chunks in (True, False):
+        monkeypatch.setattr(ops, "linear_chunks_take", lambda *a: chunks and (took.append(take(*a)) or took[-1]))
+        manager = CacheManager(64, 16, ModelRunner.windows_of(model), num_state_slots=4, enable_prefix_caching=False)
+        driver = helpers.Driver(ModelRunner(model, manager, torch.bfloat16, DEV, 512), manager)
+        for step in helpers.cuts_schedule({r: len(t) for r, t in ids.items()}, pattern):
+            driver.step({r: ids[r][a:b] for r, (a, b) in step.items()})
+        got = {r: driver.result(r).double() for r in ids}
+        errors.append({r: max(float((got[r] - w).norm() / w.norm()) for w in [S.plain_logits(folder, t).double()]) for r, t in ids.items()})
+    assert True in took
+    for r in ids:
+        assert errors[0][r] <= 1.5 * errors[1][r], errors
