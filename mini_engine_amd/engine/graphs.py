@@ -352,7 +352,9 @@ SMALL_STEP_FLOPS = 1.0e14
 # launches leave gaps between kernels of a few microseconds each): a 2,048-token prompt at the 0.6B sizes 5.40 -> 5.08 ms.
 EXACT_LAYOUT_FACTOR = 6
 # Twice as far for a model with mixers side by side of which one walks: they run beside each other in captured steps only
-# (`SideBySide`), which pays whatever bounds the step launched one by one.
+# (`SideBySide`), which pays beyond what the host bounds. At the 0.6B sizes (3,828 tokens) one prompt breaks even there: eager / replayed with
+# branches, ms, 2,500 tokens 15.1 / 13.5, 3,500 20.2 / 18.8, 3,800 21.2 / 21.4, 4,096 22.5 / 23.8; at the 8B sizes (768 tokens) they
+# would gain on (12 layers, 2,048 tokens 16.5 / 15.9).
 BRANCHES_LAYOUT_FACTOR = 12
 
 
@@ -405,7 +407,7 @@ class MixedGraphs:
     over the padded step.
 
     Steps beyond `max_tokens` and up to `max_exact_tokens` (six times as many: up to there the host's launches
-    still leave gaps between the GPU's kernels; more where a capture holds branches) take a layout with the step's own token and request counts and
+    still leave gaps between the GPU's kernels; `max_branches_tokens` where a capture holds branches) take a layout with the step's own token and request counts and
     only the context cap and the rows of logits rounded, if nobody decodes in them: prompts of one length alone, or
     a long prompt's portions under a fixed budget, come up again and again exactly so, and nothing is lost to
     padding when they do not."""
