@@ -976,7 +976,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 //           the rows inside one), and the exchange leaves 4 ks + (g ^ (n & 3)): the pieces of the
 //           four ks steps stay 64 bytes apart.
 //   values  [2 halves of 16 keys][128 channels][32 B]: an instruction is 32 channel rows of one half,
-//           so with pages of 16 keys it reads one page; piece (g & 1) of a row lies at (g & 1) ^ (channel >> 3 & 1).
+//           so with pages of 16 keys it reads one page. A read of 16 bytes a lane is worked off for lanes 0-3, 12-15 and 20-27
+//           together, then for 4-11, 16-19 and 28-31 and so on: rows n of one piece and their neighbours of the other
+//           then lie in 16 different bank groups as they are (with the pieces of every second 8 rows exchanged, which
+//           16 lanes in a row would want, each read of values took 8 cycles instead of 4).
 // A block that reaches beyond the context (the last one of a sequence), or back into pages behind a window that
 // may have been given back (the first one of a tile, with pages of 16 keys), is loaded into registers, zeroed where
 // it must not be used, and written to the same places.
@@ -986,6 +989,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #define DMA_VHALF 4096
 #define DMA_BUF (DMA_KBYTES + 2 * DMA_VHALF)
 #define DMA_NB 3                       // buffers: three workgroups of a compute unit hold 3 x 3 x 16.5 KB of its 160 KB
+#define PIPE_NB 4                      // ... of the pipelined form, of which a compute unit runs two workgroups: its requests go out late in a block
 
 // 64 x 16 bytes from gbase + voff (bytes, per lane) to LDS at lds_addr + 16 * lane. The write to m0 needs one wait
 // state before an instruction that reads it for an LDS address.
@@ -1000,52 +1004,19 @@ __device__ __forceinline__ void dma16(const bf16_t* gbase, uint32_t voff, uint32
 template <int N>
 __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
-// Keeps the reads of a whole operand array where they are written: without it the compiler moves every read
-// down to the product that uses it and waits for each in turn.
-template <int N>
-__device__ __forceinline__ void pin_operands(bf16x8 (&x)[N]) {
-#pragma unroll
-  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(x[i]));
-}
-template <int N, int M>
-__device__ __forceinline__ void pin_operands(bf16x8 (&x)[N][M]) {
-#pragma unroll
-  for (int i = 0; i < N; ++i)
-#pragma unroll
-    for (int j = 0; j < M; ++j) asm volatile("" : "+v"(x[i][j]));
-}
-
-// Reads of 16 bytes at addr + 512 i that the compiler does not know to be reads: it neither moves them to their
-// use nor waits for them, so lds_reads_done() has to stand between them and the first use of what they return.
-// Until then the values must stay in the registers they were read into (a copy or a spill made by the compiler in
-// between would move what the registers held before): only for a kernel with registers to spare, which the form
-// with two waves per SIMD is (205 of 256; its test compares it bit for bit with the form that reads as usual).
-template <int I>
-__device__ __forceinline__ void lds_read16_ahead(uint32_t addr, bf16x8 (&x)[DT]) {
-  if constexpr (I < DT) {
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(x[I]) : "v"(addr), "n"(512 * I));
-    lds_read16_ahead<I + 1>(addr, x);
-  }
-}
-__device__ __forceinline__ void lds_reads_done(bf16x8 (&x)[DT]) {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  pin_operands(x);
-}
-
-// A wave in its softmax goes first when the SIMD chooses whose instruction to issue: its vector instructions are
-// what the next products wait for, while a wave that is issuing products needs a slot only every 16 cycles
-// (with two waves per SIMD: 2,048 tokens over 8,192 keys 151 -> 142 us, 512 over 8,192 55.0 -> 53.7 us, a prompt of
-// 2,048 tokens 45.7 -> 44.1 us; with three it changes nothing).
+// A wave in its softmax goes first when the SIMD chooses whose instruction to issue.
 __device__ __forceinline__ void softmax_priority(bool on) {
   if (on) __builtin_amdgcn_s_setprio(1); else __builtin_amdgcn_s_setprio(0);
 }
 
 struct DmaPages { int k, v; };   // the page of this wave's two key instructions and of its two value instructions
 
-template <int CT, int W, bool WINDOW>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, W))) attn_prefill_dma_kernel(AttnArgs a) {
+// With three waves to a SIMD (168 registers each): launches of so many workgroups that the third wave fills the others' waits
+// (`prefill_waves`). It reads operands where it uses them.
+template <bool WINDOW>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) attn_prefill_dma_kernel(AttnArgs a) {
   extern __shared__ __align__(16) unsigned char pf_lds[];   // [NB][DMA_BUF]
-  constexpr int NB = DMA_NB, PD = NB - 1;                   // PD: blocks asked for ahead of the one in use
+  constexpr int CT = 2, NB = DMA_NB, PD = NB - 1;                   // PD: blocks asked for ahead of the one in use
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, g = lane >> 4;
@@ -1084,9 +1055,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, W))
   const uint32_t lds0 = (uint32_t)(uintptr_t)pf_lds;
   // what a lane names in memory, relative to its instruction's first byte, and where it reads its operands
   const uint32_t voff_k = (lane >> 4) * 256 + (((lane & 15) ^ (lane >> 4)) * 16);
-  const uint32_t voff_v = ((lane >> 1) * a.page + (((lane & 1) ^ ((lane >> 4) & 1)) * 8)) * 2;
+  const uint32_t voff_v = ((lane >> 1) * a.page + ((lane & 1) * 8)) * 2;
   const uint32_t rd_k = (n >> 2) * DMA_KINST + (n & 3) * 256 + ((g ^ (n & 3)) * 16);
-  const uint32_t rd_v = DMA_KBYTES + (g >> 1) * DMA_VHALF + n * 32 + (((g & 1) ^ (n >> 3)) * 16);
+  const uint32_t rd_v = DMA_KBYTES + (g >> 1) * DMA_VHALF + n * 32 + ((g & 1) * 16);
   const int kg0 = 8 * ((2 * wave) & 3) + 4 * (wave >> 1);   // first key of this wave's first key instruction; the second: + 8
   const int vh = wave >> 1, vrow0 = 64 * (wave & 1);        // this wave's value instructions: half vh, channel rows vrow0 + 32 j
   const uint32_t page_elems = (uint32_t)(a.Hkv * a.page * HD);                 // elements of a page, keys and values alike
@@ -1126,7 +1097,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, W))
       }
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const int key0 = t0 + 16 * vh + 8 * ((lane & 1) ^ ((lane >> 4) & 1));
+        const int key0 = t0 + 16 * vh + 8 * (lane & 1);
         const int nv = held(key0) ? L - key0 : 0;    // (a piece of 8 keys lies wholly before or behind first_held)
         const bf16x8 vv = ld8(reinterpret_cast<const bf16_t*>(reinterpret_cast<const unsigned char*>(gv + (int64_t)32 * j * a.page) + voff_v));
         u32x4 w = __builtin_bit_cast(u32x4, vv);
@@ -1203,67 +1174,30 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, W))
       const unsigned char* kb = pf_lds + cur * DMA_BUF + rd_k;
       f32x4 st[CT][2];
       bf16x8 pb[CT];
-      if constexpr (W == 2) {
-        // With 256 registers to a wave all of a block's key operands are asked for before the first score product,
-        // and its value operands before the softmax, which takes longer than they do: one LDS latency for each,
-        // not one for every pair of reads.
-        bf16x8 ka[2][KS];
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
+      for (int tt = 0; tt < 2; ++tt) {
 #pragma unroll
-          for (int ks = 0; ks < KS; ++ks)
-            ka[tt][ks] = *reinterpret_cast<const bf16x8*>(kb + tt * 4 * DMA_KINST + 64 * ks);
-        pin_operands(ka);
+        for (int ct = 0; ct < CT; ++ct) st[ct][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-#pragma unroll
-          for (int ct = 0; ct < CT; ++ct) st[ct][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct)
-              st[ct][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[tt][ks], qb[ct][ks], st[ct][tt], 0, 0, 0);
-        }
-        bf16x8 va[DT];
-        lds_read16_ahead<0>(lds0 + cur * DMA_BUF + rd_v, va);
-        softmax_priority(true);
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct)
-          block_softmax<FULL>(a, st[ct], t0, col_lo[ct], col_hi[ct], slope[ct], m[ct], l[ct], acc[ct], g, pb[ct]);
-        softmax_priority(false);
-        lds_reads_done(va);
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+        for (int ks = 0; ks < KS; ++ks) {
+          const bf16x8 ka = *reinterpret_cast<const bf16x8*>(kb + tt * 4 * DMA_KINST + 64 * ks);
 #pragma unroll
           for (int ct = 0; ct < CT; ++ct)
-            acc[ct][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[dt], pb[ct], acc[ct][dt], 0, 0, 0);
-      } else {
-        // With 168 registers the operands are read where they are used, and the third wave fills the waits.
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-#pragma unroll
-          for (int ct = 0; ct < CT; ++ct) st[ct][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int ks = 0; ks < KS; ++ks) {
-            const bf16x8 ka = *reinterpret_cast<const bf16x8*>(kb + tt * 4 * DMA_KINST + 64 * ks);
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct)
-              st[ct][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qb[ct][ks], st[ct][tt], 0, 0, 0);
-          }
+            st[ct][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qb[ct][ks], st[ct][tt], 0, 0, 0);
         }
-        softmax_priority(true);
+      }
+      softmax_priority(true);
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+        block_softmax<FULL>(a, st[ct], t0, col_lo[ct], col_hi[ct], slope[ct], m[ct], l[ct], acc[ct], g, pb[ct]);
+      softmax_priority(false);
+      const unsigned char* vb = pf_lds + cur * DMA_BUF + rd_v;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const bf16x8 va = *reinterpret_cast<const bf16x8*>(vb + 512 * dt);
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct)
-          block_softmax<FULL>(a, st[ct], t0, col_lo[ct], col_hi[ct], slope[ct], m[ct], l[ct], acc[ct], g, pb[ct]);
-        softmax_priority(false);
-        const unsigned char* vb = pf_lds + cur * DMA_BUF + rd_v;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          const bf16x8 va = *reinterpret_cast<const bf16x8*>(vb + 512 * dt);
-#pragma unroll
-          for (int ct = 0; ct < CT; ++ct)
-            acc[ct][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb[ct], acc[ct][dt], 0, 0, 0);
-        }
+          acc[ct][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb[ct], acc[ct][dt], 0, 0, 0);
       }
       cur = cur == NB - 1 ? 0 : cur + 1;
     };
@@ -1277,6 +1211,341 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, W))
     }
     for (; k < end_full; ++k) block_step(std::true_type{}, k);
     for (; k < nblk; ++k) block_step(std::false_type{}, k);
+
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      const float ls = column_sum(l[ct]);
+      if (valid[ct] && tr.nseg > 1) {
+        float* p = a.pf_scratch + (((int64_t)tq[ct] * a.Hq + head[ct]) * a.max_segs + seg) * (HD + 2);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+          *reinterpret_cast<f32x4*>(p + 16 * dt + 4 * g) = acc[ct][dt];
+        if (g == 0) { p[HD] = m[ct]; p[HD + 1] = ls; }
+      } else if (valid[ct]) {
+        const float dn = with_sink(a, head[ct], m[ct], ls);
+        const float inv = dn > 0.f ? 1.f / dn : 0.f;
+        if (a.lse_out != nullptr && g == 0) a.lse_out[(int64_t)tq[ct] * a.Hq + head[ct]] = natural_lse(m[ct], ls);
+        bf16_t* o = a.out + tq[ct] * a.out_stride + (int64_t)head[ct] * HD + 4 * g;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+          bf16x4 r;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) r[i] = static_cast<bf16_t>(acc[ct][dt][i] * inv);
+          *reinterpret_cast<bf16x4*>(o + 16 * dt) = r;
+        }
+      }
+    }
+  }
+}
+
+// The pipelined kernel's softmax in two parts. The block's scores as the softmax takes them: capped, biased, masked.
+template <bool FULL>
+__device__ __forceinline__ void block_scores(const AttnArgs& a, const f32x4 (&st)[2], int t0, int col_lo, int col_hi, float slope, int g,
+                                             float (&sv)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) sv[i] = st[i >> 2][i & 3];
+  cap_scores(a, sv);
+  distance_scores(slope, t0 + 8 * g, col_hi, sv);
+  if (!FULL) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int j = t0 + 8 * g + i;
+      sv[i] = (j <= col_hi && j >= col_lo) ? sv[i] : NEG;
+    }
+  }
+}
+// Moves a column's reference point where a score lies more than RESCALE_STEP above it, as `block_softmax` does, with one test for
+// all of the wave's columns.
+template <int CT>
+__device__ __forceinline__ void follow_maxima(float c, const float (&sv)[CT][8], float (&m)[CT], float (&l)[CT], f32x4 (&acc)[CT][DT]) {
+  float bm[CT];
+  bool rose = false;
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) {
+    bm[ct] = NEG;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) bm[ct] = fmaxf(bm[ct], sv[ct][i]);
+    rose |= bm[ct] > 0.5f * NEG && bm[ct] * c > m[ct] + RESCALE_STEP;
+  }
+  if (__builtin_expect(__any(rose), 0)) {
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      const float top = max_over_groups(bm[ct]);
+      const float m_blk = top > 0.5f * NEG ? top * c : NEG;
+      if (m_blk > m[ct] + RESCALE_STEP) {
+        const float alpha = __builtin_amdgcn_exp2f(m[ct] - m_blk);
+        l[ct] *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+          acc[ct][dt][0] *= alpha; acc[ct][dt][1] *= alpha; acc[ct][dt][2] *= alpha; acc[ct][dt][3] *= alpha;
+        }
+        m[ct] = m_blk;
+      }
+    }
+  }
+}
+
+// The same as a software pipeline, with two waves to a SIMD (256 registers each): while a block's softmax is formed its successor's
+// scores are multiplied, a product beside every number, so that a wave's vector instructions run in the shade of its own matrix
+// instructions (a product holds the issue port of its SIMD for 8 of its 16 cycles). Walked one block after the other, a wave alone on
+// its SIMD took 0.86 us for a block of 32 keys and two column tiles, of which its 32 products are 0.22, two on a SIMD 0.95 us for both;
+// so 0.64 and 0.80. The order of a column's sums is the same, and so are the bits. What bounds it now is the SIMD's issue port (two
+// waves: 0.6 us a block with their scalar and LDS instructions beside it) and, in launches of a few hundred workgroups, 6 us around the
+// blocks and how evenly they are cut. us, before / now, 16 query and 8 key heads: 512 tokens 13.8 / 12.1, 2,048 40.5 / 39.3, three
+// prompts of up to 2,048 68 / 59.6, 512 over 8,192 keys 75 / 66, two prompts of 2,048 and 1,075 under a window of 512
+// 30.8 / 28.1; 32 and 8 heads: 800 tokens 20.1 / 17.4, 2,048 63.8 / 60.
+template <int CT, bool WINDOW>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) attn_prefill_pipe_kernel(AttnArgs a) {
+  extern __shared__ __align__(16) unsigned char pf_lds[];   // [NB][DMA_BUF]
+  constexpr int NB = PIPE_NB, PD = NB - 1;                  // PD: blocks asked for ahead of the one whose softmax is formed
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, g = lane >> 4;
+  const int kvh = blockIdx.x % a.Hkv;
+  const int x = gridDim.x / a.Hkv - 1 - blockIdx.x / a.Hkv;
+  int lo_b = 0, hi_b = a.num_seqs - 1;
+  while (lo_b < hi_b) {
+    const int mid = (lo_b + hi_b + 1) >> 1;
+    if (a.cu_seqlens[mid] / a.tok_tile + mid <= x) lo_b = mid; else hi_b = mid - 1;
+  }
+  const int b = lo_b;
+  const int q0 = a.cu_seqlens[b], q_len = a.cu_seqlens[b + 1] - q0;
+  const int tok0 = (x - (q0 / a.tok_tile + b)) * a.tok_tile;
+  if (tok0 >= q_len) return;
+  const int L = a.context_lens[b];
+  const int start = L - q_len;
+  const int32_t* bt = a.block_tables + (int64_t)b * a.bt_stride;
+  const TileRange tr = tile_range(a, tok0, q_len, L);
+  const int ncols = tr.tile_tokens * a.G;
+  const int seg = blockIdx.z;
+  if (seg >= tr.nseg) return;
+  const int seg_lo = a.seg_keys > 0 ? tr.tile_base + seg * a.seg_keys : tr.tile_base;
+  const int seg_hi = (a.seg_keys > 0 && seg + 1 < tr.nseg) ? seg_lo + a.seg_keys : (1 << 30);
+  const int last = min(tr.pos_last, seg_hi - 1);   // the same key range for every wave of the workgroup
+  const int nblk = (last - seg_lo) / 32 + 1;
+  // With a window, pages wholly behind it may have been given back: from the page that holds the tile's first
+  // visible key on, every page is held (pages are 16 keys or more, so this is a multiple of 16).
+  // (Without a window all of this is known when the kernel is compiled: the tests below cost the common case 2-7 %.)
+  const int first_held = WINDOW ? (tr.tile_lo >> a.page_shift) << a.page_shift : 0;
+  auto held = [&](int key) { return !WINDOW || key >= first_held; };
+
+  const uint32_t lds0 = (uint32_t)(uintptr_t)pf_lds;
+  // what a lane names in memory, relative to its instruction's first byte, and where it reads its operands
+  const uint32_t voff_k = (lane >> 4) * 256 + (((lane & 15) ^ (lane >> 4)) * 16);
+  const uint32_t voff_v = ((lane >> 1) * a.page + ((lane & 1) * 8)) * 2;
+  const uint32_t rd_k = (n >> 2) * DMA_KINST + (n & 3) * 256 + ((g ^ (n & 3)) * 16);
+  const uint32_t rd_v = DMA_KBYTES + (g >> 1) * DMA_VHALF + n * 32 + ((g & 1) * 16);
+  const int kg0 = 8 * ((2 * wave) & 3) + 4 * (wave >> 1);   // first key of this wave's first key instruction; the second: + 8
+  const int vh = wave >> 1, vrow0 = 64 * (wave & 1);        // this wave's value instructions: half vh, channel rows vrow0 + 32 j
+  const uint32_t page_elems = (uint32_t)(a.Hkv * a.page * HD);                 // elements of a page, keys and values alike
+  const bf16_t* k_head = a.k_cache + (int64_t)kvh * a.page * HD;
+  const bf16_t* v_head = a.v_cache + ((int64_t)kvh * HD + vrow0) * a.page;
+
+  // The pages of 32 blocks are held by the wave's lanes, one for every 16 keys, and a block's are read from there: asked
+  // for block by block with scalar loads, each block waited for the entries it had just asked for on behalf of the next one
+  // (scalar loads return in any order, so that there is no waiting for the older ones alone).
+  auto usable = [&](int key) { return key < L && held(key); };
+  auto ask_pages = [&](int t0) { const int key = t0 + 16 * lane; return bt[usable(key) ? key >> a.page_shift : 0]; };
+  auto settle_pages = [&](int t0, int raw) { return usable(t0 + 16 * lane) ? raw : 0; };
+  struct Source { const bf16_t *k, *v; uint32_t buf; };               // where this wave's pieces of a block come from, the buffer they go to
+  auto source = [&](int t0, int k, int pages, uint32_t buf) -> Source {
+    const uint32_t kpage = __builtin_amdgcn_readlane(pages, (2 * k + (wave & 1)) & 63);
+    const uint32_t vpage = __builtin_amdgcn_readlane(pages, (2 * k + vh) & 63);
+    return {k_head + (uint64_t)kpage * page_elems + (uint32_t)((t0 + kg0) & (a.page - 1)) * HD,
+            v_head + (uint64_t)vpage * page_elems + (uint32_t)((t0 + 16 * vh) & (a.page - 1)), buf};
+  };
+  auto whole = [&](int t0) { return t0 + 32 <= L && held(t0); };      // the memory system fills LDS: every row of the block may be used
+  auto ask_piece = [&](const Source& from, int j) {                   // 0, 1: this wave's keys, 2, 3: its values
+    if (j < 2) dma16(from.k + 8 * j * HD, voff_k, lds0 + from.buf + (2 * wave + j) * DMA_KINST);
+    else dma16(from.v + (int64_t)32 * (j - 2) * a.page, voff_v, lds0 + from.buf + DMA_KBYTES + vh * DMA_VHALF + (vrow0 / 32 + j - 2) * 1024);
+  };
+  auto stage_part = [&](const Source& from, int t0) {                 // a block that is not whole, through registers
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const bf16x8 z = zero8();
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int key = t0 + kg0 + 8 * j + (lane >> 4);
+      // rows of a page that is held may be read beyond the context; without a page, page 0 is read
+      const bool mapped = t0 + kg0 + 8 * j < L && held(t0 + kg0);
+      const bf16_t* src = mapped ? from.k + 8 * j * HD : k_head;
+      const bf16x8 kk = ld8(reinterpret_cast<const bf16_t*>(reinterpret_cast<const unsigned char*>(src) + voff_k));
+      *reinterpret_cast<bf16x8*>(pf_lds + from.buf + (2 * wave + j) * DMA_KINST + 16 * lane) = (key < L && held(key)) ? kk : z;
+    }
+    const bf16_t* vsrc = usable(t0 + 16 * vh) ? from.v : v_head;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int key0 = t0 + 16 * vh + 8 * (lane & 1);
+      const int nv = held(key0) ? L - key0 : 0;    // (a piece of 8 keys lies wholly before or behind first_held)
+      const bf16x8 vv = ld8(reinterpret_cast<const bf16_t*>(reinterpret_cast<const unsigned char*>(vsrc + (int64_t)32 * j * a.page) + voff_v));
+      u32x4 w = __builtin_bit_cast(u32x4, vv);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] &= (2 * i < nv ? 0x0000ffffu : 0u) | (2 * i + 1 < nv ? 0xffff0000u : 0u);
+      *reinterpret_cast<u32x4*>(pf_lds + from.buf + DMA_KBYTES + vh * DMA_VHALF + (vrow0 / 32 + j) * 1024 + 16 * lane) = w;
+    }
+  };
+
+  // every wave runs every round (a wave without columns in a round masks everything and writes nothing)
+  for (int c_base = 0; c_base < ncols; c_base += 4 * 16 * CT) {
+    const int first_pages = ask_pages(seg_lo);
+    const bool active = c_base + wave * 16 * CT < ncols;
+    const int c0 = active ? c_base + wave * 16 * CT : 0;
+    bf16x8 qb[CT][KS];
+    int col_lo[CT], col_hi[CT];
+    int64_t tq[CT];
+    int head[CT];
+    bool valid[CT];
+    float slope[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      const int cc = c0 + 16 * ct + n;
+      valid[ct] = active && cc < ncols;
+      const int tl = valid[ct] ? cc / a.G : 0;
+      const int hh = valid[ct] ? cc - tl * a.G : 0;
+      tq[ct] = q0 + tok0 + tl;
+      head[ct] = kvh * a.G + hh;
+      const int pos = start + tok0 + tl;
+      col_hi[ct] = valid[ct] ? pos : -1;
+      slope[ct] = column_slope(a, head[ct], valid[ct]);
+      col_lo[ct] = WINDOW ? lower_edge(a, pos) : 0;
+      load_q(a.q + tq[ct] * a.q_stride + (int64_t)head[ct] * HD, valid[ct], g, qb[ct]);
+    }
+    const int c_last = min(ncols, c0 + 16 * CT) - 1;
+    const int pos_first = start + tok0 + c0 / a.G, pos_last = start + tok0 + c_last / a.G;
+    const int full_hi = active ? pos_first - 31 : -(1 << 30);
+    const int full_lo = WINDOW ? lower_edge(a, pos_last) : 0;
+    float m[CT], l[CT];
+    f32x4 acc[CT][DT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      m[ct] = NEG; l[ct] = 0.f;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) acc[ct][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+
+    pf_barrier();                                    // the round before has finished with every buffer
+    int pages = settle_pages(seg_lo, first_pages), more_pages = 0;
+#pragma unroll
+    for (int k = 0; k < PD; ++k)
+      if (k < nblk) {
+        const Source from = source(seg_lo + 32 * k, k, pages, k * DMA_BUF);
+        if (whole(seg_lo + 32 * k)) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) ask_piece(from, j);
+        } else {
+          stage_part(from, seg_lo + 32 * k);
+        }
+      }
+    f32x4 st[CT][2];                                 // the scores of the block whose softmax comes next
+    bf16x8 ka[2][KS];
+    auto read_keys = [&](uint32_t buf) {
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+          ka[tt][ks] = *reinterpret_cast<const bf16x8*>(pf_lds + buf + rd_k + tt * 4 * DMA_KINST + 64 * ks);
+    };
+    // product i of a block's scores: the chains of the key tiles and column tiles beside each other (one alone waits for itself)
+    auto score = [&](f32x4 (&s)[CT][2], int i) {
+      const int ct = i % CT, tt = i / CT % 2, ks = i / CT / 2;
+      s[ct][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[tt][ks], qb[ct][ks], ks ? s[ct][tt] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+    };
+    static_assert(KS == 4 && DT == 8, "a score product beside every number of the softmax, a request behind every second row of value products");
+    const float c = a.scale * 1.4426950408889634f;
+    uint32_t cur = 0;                                // the buffer of the block whose softmax is formed
+    if (PD <= nblk) dma_wait<4 * (PD - 1)>(); else dma_wait<0>();
+    pf_barrier();
+    read_keys(0);
+#pragma unroll
+    for (int i = 0; i < 8 * CT; ++i) score(st, i);
+    // Step k: the softmax of block k beside the scores of block k + 1 (MORE: there is one), then block k's values, and the request
+    // for block k + PD. FULL: every key of block k is visible to every column of this wave. STEADY: block k + PD is there and whole;
+    // such a step has no branch but for a maximum that rises and for the next 32 pages, its requests go out between the value products
+    // (in front of the softmax all waves of the workgroup would wait until the memory pipe has taken them). Blocks are walked
+    // in ascending order, so a wave's FULL blocks come first and form a loop of their own; every wave passes the same barriers in any loop.
+    auto block_step = [&](auto full_tag, auto steady_tag, auto more_tag, int k) {
+      constexpr bool FULL = decltype(full_tag)::value, STEADY = decltype(steady_tag)::value, MORE = decltype(more_tag)::value;
+      const int t0 = seg_lo + 32 * k, next = k + PD, t_next = t0 + 32 * PD;
+      const uint32_t nxt = cur == (NB - 1) * DMA_BUF ? 0 : cur + DMA_BUF, to = cur == 0 ? (NB - 1) * DMA_BUF : cur - DMA_BUF;
+      if constexpr (MORE) {
+        // block k + 1 has landed: at most the PD - 2 blocks asked for after it are still on their way
+        if (STEADY || next <= nblk) dma_wait<4 * (PD - 2)>(); else dma_wait<0>();
+        pf_barrier();                                // ... for every wave, and the buffer of block k - 1 is free
+        read_keys(nxt);
+      }
+      bf16x8 va[DT];
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) va[dt] = *reinterpret_cast<const bf16x8*>(pf_lds + cur + rd_v + 512 * dt);
+      __builtin_amdgcn_sched_barrier(0);
+      if (STEADY || (MORE && next < nblk)) {
+        // (stored whether they have changed or not: a store in each branch would put them into scratch memory)
+        int now = pages, later = more_pages;
+        if (__builtin_expect((next & 31) == 31, 0)) { asm volatile("" ::: "memory"); later = ask_pages(t_next + 32); }
+        if (__builtin_expect((next & 31) == 0, 0)) { asm volatile("" ::: "memory"); now = settle_pages(t_next, later); }
+        pages = now; more_pages = later;
+        if constexpr (!STEADY) {
+          const Source from = source(t_next, next, pages, to);
+          if (whole(t_next)) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) ask_piece(from, j);
+          } else {
+            stage_part(from, t_next);
+          }
+        }
+      }
+      float sv[CT][8];
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) block_scores<FULL>(a, st[ct], t0, col_lo[ct], col_hi[ct], slope[ct], g, sv[ct]);
+      follow_maxima<CT>(c, sv, m, l, acc);
+      f32x4 sn[CT][2];
+      bf16x8 pb[CT];
+      float psum[CT], p[CT][8];
+#pragma unroll
+      for (int i = 0; i < 8 * CT; ++i) {
+        const int ct = i % CT, e = i / CT;
+        if constexpr (MORE) score(sn, i);
+        // a masked score is NEG: while the column has seen no key m is NEG too, and exp2(NEG * c - NEG) is not 0, hence the select
+        float v = __builtin_amdgcn_exp2f(fmaf(sv[ct][e], c, -m[ct]));
+        if (!FULL) v = sv[ct][e] > 0.5f * NEG ? v : 0.f;
+        p[ct][e] = v;
+        psum[ct] = e ? psum[ct] + v : v;
+        if (e & 1) { pb[ct][e - 1] = static_cast<bf16_t>(p[ct][e - 1]); pb[ct][e] = static_cast<bf16_t>(v); }
+      }
+      Source from;
+      if constexpr (STEADY) from = source(t_next, next, pages, to);
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) l[ct] += psum[ct];
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+          acc[ct][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[dt], pb[ct], acc[ct][dt], 0, 0, 0);
+        if (STEADY && (dt & 1)) {
+          __builtin_amdgcn_sched_barrier(0);
+          ask_piece(from, dt >> 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      if constexpr (MORE) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) { st[ct][0] = sn[ct][0]; st[ct][1] = sn[ct][1]; }
+        cur = nxt;
+      }
+    };
+    // blocks [first_full, end_full) lie wholly inside every column's range of this wave: behind the window's lower
+    // edge (if there is a window) and before the diagonal
+    const std::true_type yes;
+    const std::false_type no;
+    const int end_full = full_hi >= seg_lo ? min(nblk, (full_hi - seg_lo) / 32 + 1) : 0;
+    int k = 0;
+    if constexpr (WINDOW) {
+      const int first_full = full_lo > seg_lo ? min(end_full, (full_lo - seg_lo + 31) / 32) : 0;
+      for (; k < min(first_full, nblk - 1); ++k) block_step(no, no, yes, k);
+    }
+    const int end_steady = min(end_full, min(nblk, (L - seg_lo) / 32) - PD);       // (a block behind the tile's first is always held)
+    for (; k < end_steady; ++k) block_step(yes, yes, yes, k);
+    for (; k < min(end_full, nblk - 1); ++k) block_step(yes, no, yes, k);
+    for (; k < nblk - 1; ++k) block_step(no, no, yes, k);
+    block_step(no, no, no, k);
 
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
@@ -1760,13 +2029,24 @@ extern "C" int me_attn_prefill(const void* q, int64_t q_stride, void* out, int64
   // caller knows the launches for which that pays.
   if (through_lds && shared == 1 && page >= 16 && (int64_t)Hkv * page * HD < (1ll << 31)) {
     const bool three = ct == 2 && waves == 3;
-#define DMA_LAUNCH(CTV, WV)                                                                                    \
-  do {                                                                                                         \
-    if (window != 0) attn_prefill_dma_kernel<CTV, WV, true><<<grid, dim3(256), DMA_NB * DMA_BUF, stream>>>(a);  \
-    else attn_prefill_dma_kernel<CTV, WV, false><<<grid, dim3(256), DMA_NB * DMA_BUF, stream>>>(a);            \
-  } while (0)
-    if (three) DMA_LAUNCH(2, 3); else if (ct == 2) DMA_LAUNCH(2, 2); else DMA_LAUNCH(1, 2);
-#undef DMA_LAUNCH
+    if (three) {
+      if (window != 0) attn_prefill_dma_kernel<true><<<grid, dim3(256), DMA_NB * DMA_BUF, stream>>>(a);
+      else attn_prefill_dma_kernel<false><<<grid, dim3(256), DMA_NB * DMA_BUF, stream>>>(a);
+    } else {
+      static bool allowed = false;                     // more LDS than a kernel may have unasked
+      if (!allowed) {
+        for (const void* kernel : {(const void*)attn_prefill_pipe_kernel<1, false>, (const void*)attn_prefill_pipe_kernel<1, true>,
+                                   (const void*)attn_prefill_pipe_kernel<2, false>, (const void*)attn_prefill_pipe_kernel<2, true>}) {
+          const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, PIPE_NB * DMA_BUF);
+          ME_CHECK(e == hipSuccess, "attention: cannot get %d bytes of LDS", PIPE_NB * DMA_BUF);
+        }
+        allowed = true;
+      }
+#define PIPE_LAUNCH(CTV, WIN) attn_prefill_pipe_kernel<CTV, WIN><<<grid, dim3(256), PIPE_NB * DMA_BUF, stream>>>(a)
+      if (ct == 2) { if (window != 0) PIPE_LAUNCH(2, true); else PIPE_LAUNCH(2, false); }
+      else { if (window != 0) PIPE_LAUNCH(1, true); else PIPE_LAUNCH(1, false); }
+#undef PIPE_LAUNCH
+    }
   } else
 #endif
   if (through_lds) {

@@ -472,6 +472,24 @@ def test_attention_prefill_lds_filled_by_the_loads_themselves(monkeypatch, Hq, H
         close(direct, twin.paged_attention(*args), 1.5e-2)
 
 
+@pytest.mark.parametrize("col_tiles", [1, 2])
+@pytest.mark.parametrize("page,window", [(16, None), (64, None), (16, 1100)])
+def test_attention_prefill_pipelined_walk(monkeypatch, col_tiles, page, window):
+    """Walks of one to a few blocks (the pipeline's four buffers), and walks that pass the 32nd and the 64th block, where the next
+    pages are taken up: bit for bit what the form that stages through registers gives, a maximum rising in the middle."""
+    seqs = [(n, min(n, 40)) for n in (1, 31, 32, 64, 65, 96, 97, 128, 129, 160, 991, 1023, 1024, 1025, 1056, 1057, 2047, 2049, 2080, 2113)]
+    monkeypatch.setattr(ops, "PREFILL_SEGMENT_KEYS", 0)
+    monkeypatch.setattr(ops, "prefill_col_tiles", lambda *a: col_tiles)
+    for peak in (None, 1030):
+        args = _attention_case(torch.bfloat16, 4, 2, 128, page, seqs, window=window, seed=page + col_tiles, peak=peak)
+        forms = []
+        for form in (1, 2):
+            monkeypatch.setattr(ops, "PREFILL_THROUGH_LDS", form)
+            forms.append(hip().paged_attention(*args, max_prefill_context=2113))
+        assert not torch.isnan(forms[0]).any() and torch.equal(*forms)
+        close(forms[0], twin.paged_attention(*args), 1.5e-2)
+
+
 def test_attention_prefill_segments_chosen_automatically():
     """A short chunk at the end of a long context is cut by the engine's own rule."""
     seqs = [(2500, 33), (1100, 2)]
