@@ -52,6 +52,59 @@ __device__ __forceinline__ void tile_barrier() {
 enum { REGION_W0 = 0, REGION_X0 = 1, REGION_W1 = 2, REGION_X1 = 3 };
 #define TILE_INT(v) std::integral_constant<int, v>{}
 
+// Writes a wave's sums: its rows are m0 + 16 j of the lane, its features begin at n0 (ACT: its gated features).
+template <int MI, int NI, bool ACT, typename TO>
+__device__ __forceinline__ void tile_store(const f32x4 (&acc)[NI][MI], TO* __restrict__ out, int64_t ldy, int M, int N, int m0, int n0, int g,
+                                           const GateForm& form, int rounded) {
+  constexpr int NH = NI / 2;
+  constexpr bool PAIRED = sizeof(TO) == 2;
+  const int I = N / 2, F = ACT ? I : N;
+#pragma unroll
+  for (int j = 0; j < MI; ++j) {
+    const int m = m0 + 16 * j;
+    if (m >= M) continue;
+    TO* row = out + (int64_t)m * ldy;
+#pragma unroll
+    for (int h = 0; h < (ACT ? 1 : 2); ++h) {
+      const int f0 = ACT ? n0 : n0 + h * (8 * NI);
+      auto value = [&](int i, int e, int f) {
+        if constexpr (ACT) {
+          float gate = acc[i][j][e], up = acc[NH + i][j][e];
+          if (rounded) { gate = (float)(bf16_t)gate; up = (float)(bf16_t)up; }
+          if (form.bias) { gate += form.bias[f]; up += form.bias[I + f]; }
+          return rounded ? gate_value<false>(gate, up, form) : gate_value<true>(gate, up, form);
+        } else {
+          return acc[h * NH + i][j][e];
+        }
+      };
+#pragma unroll
+      for (int i = 0; i < NH; ++i) {
+        if constexpr (!PAIRED) {
+          const int f = f0 + 16 * i + 4 * g;
+          if (f < F) *reinterpret_cast<f32x4*>(row + f) = acc[h * NH + i][j];
+        } else if (i / 2 < NH / 2) {
+          if (i & 1) continue;                                       // i and i + 1: 8 consecutive features (F is in eights)
+          const int f = f0 + 16 * i + 8 * g;
+          if (f < F) {
+            bf16x8 r;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) r[e] = (bf16_t)value(i + e / 4, e & 3, f + e);
+            *reinterpret_cast<bf16x8*>(row + f) = r;
+          }
+        } else {
+          const int f = f0 + 16 * i + 4 * g;
+          if (f < F) {
+            bf16x4 r;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r[e] = (bf16_t)value(i, e, f + e);
+            *reinterpret_cast<bf16x4*>(row + f) = r;
+          }
+        }
+      }
+    }
+  }
+}
+
 // WGM x WGN waves, each with MI tiles of 16 rows x NI tiles of 16 features (both even). ACT: w is a packed gate/up weight
 // [2 I, K] (gate rows first, N = 2 I); the first half of a wave's features are gates, the second their ups, and what is
 // written is their gated product [M, I] (reference layers/activation.py:5-7), formed from the unrounded sums as the other
@@ -226,52 +279,150 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __rest
   step(k + 1, TILE_INT(2));
   if (PING && !late) tile_barrier();
 
-  TO* out = y + (int64_t)blockIdx.z * M * ldy;
-  const int F = ACT ? I : N;
+  tile_store<MI, NI, ACT>(acc, y + (int64_t)blockIdx.z * M * ldy, ldy, M, N, m0 + wm * (16 * MI) + n, n0 + wn * (ACT ? 8 * NI : 16 * NI), g, form, rounded);
+}
+
+// The same by four waves for launches of one workgroup to a compute unit, which no other fills the waits of: whole steps of 64 of K in
+// a ring of RING_STAGES, a barrier a step. A wave reads the next step's operands and asks for the step behind the ring between its
+// products, so that neither stands in a row of its own: 16 products of 128 x 64 beside 12 reads and 6 requests take about what the requests take
+// (24 KB a step at the 64 bytes a cycle that reach a compute unit; 5 stages are 12 % faster than 4 and 5 % than 6). In quarters, with four barriers
+// a step and the reads in front of the products, a step took 0.29-0.48 us whatever the tile; now 0.17 for 64 x 64, 0.31 for 64 x 128, 0.49 for 128 x
+// 128. us of a launch in a chain, the library / quarters / this: 2,048 rows of 1024 x 2048 16.4 / 14.0 / 11.9, of 1024 x 3072 19.3 / 19.5 / 16.8,
+// 700 rows 10.2 / 10.7 / 8.4 and 13.9 / 15.1 / 11.5, 800 rows of 4096 x 4096 39.9 / 38.9 / 32.9; the same bits (K in one order).
+#define RING_STAGES 5
+template <int WGM, int WGN, int MI, int NI, bool ACT, typename TO>
+__global__ void __launch_bounds__(WGM* WGN * 64, 1)
+gemm_ring_kernel(const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ w, int64_t ldw, TO* __restrict__ y, int64_t ldy,
+                 int M, int N, int steps_per_split, int all_steps, int m_tiles, int n_tiles, int group_m, GateForm form, int rounded) {
+  extern __shared__ __align__(16) unsigned char tile_lds[];          // [ST][STAGE]
+  constexpr int NW = WGM * WGN, TM = WGM * MI * 16, TN = WGN * NI * 16, NH = NI / 2, ST = RING_STAGES;
+  constexpr int STAGE = (TM + TN) * 128;
+  constexpr bool PAIRED = sizeof(TO) == 2;
+  constexpr int XS = TM / 8 / NW, WS = TN / 8 / NW, PIECES = XS + WS;   // a wave's pieces of 8 rows of a stage: rows, then features
+  static_assert(TM / 8 % NW == 0 && TN / 8 % NW == 0 && PIECES * (ST - 2) < 64, "whole pieces, and what the counter of loads can tell apart");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, g = lane >> 4;
+  const int tiles = m_tiles * n_tiles, per_xcd = (tiles + 7) >> 3;
+  const int t = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if ((blockIdx.x >> 3) >= per_xcd || t >= tiles) return;
+  const int group = t / (group_m * n_tiles), rest = t % (group_m * n_tiles);
+  const int in_group = min(group_m, m_tiles - group * group_m);
+  const int mt = group * group_m + rest % in_group, nt = rest / in_group;
+  const int I = N / 2;                                               // ACT only
+  const int m0 = mt * TM, n0 = nt * (ACT ? TN / 2 : TN);
+  const int first = blockIdx.z * steps_per_split;
+  const int steps = min(steps_per_split, all_steps - first);          // one or more
+
+  uint32_t off[PIECES];                                               // what a lane names in memory for each piece
+  const int r8 = lane >> 3, c8 = lane & 7;
 #pragma unroll
-  for (int j = 0; j < MI; ++j) {
-    const int m = m0 + wm * (16 * MI) + 16 * j + n;
-    if (m >= M) continue;
-    TO* row = out + (int64_t)m * ldy;
-#pragma unroll
-    for (int h = 0; h < (ACT ? 1 : 2); ++h) {
-      const int f0 = ACT ? n0 + wn * (8 * NI) : n0 + wn * (16 * NI) + h * (8 * NI);
-      auto value = [&](int i, int e, int f) {
-        if constexpr (ACT) {
-          float gate = acc[i][j][e], up = acc[NH + i][j][e];
-          if (rounded) { gate = (float)(bf16_t)gate; up = (float)(bf16_t)up; }
-          if (form.bias) { gate += form.bias[f]; up += form.bias[I + f]; }
-          return rounded ? gate_value<false>(gate, up, form) : gate_value<true>(gate, up, form);
-        } else {
-          return acc[h * NH + i][j][e];
-        }
-      };
-#pragma unroll
-      for (int i = 0; i < NH; ++i) {
-        if constexpr (!PAIRED) {
-          const int f = f0 + 16 * i + 4 * g;
-          if (f < F) *reinterpret_cast<f32x4*>(row + f) = acc[h * NH + i][j];
-        } else if (i / 2 < NH / 2) {
-          if (i & 1) continue;                                       // i and i + 1: 8 consecutive features (F is in eights)
-          const int f = f0 + 16 * i + 8 * g;
-          if (f < F) {
-            bf16x8 r;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) r[e] = (bf16_t)value(i + e / 4, e & 3, f + e);
-            *reinterpret_cast<bf16x8*>(row + f) = r;
-          }
-        } else {
-          const int f = f0 + 16 * i + 4 * g;
-          if (f < F) {
-            bf16x4 r;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) r[e] = (bf16_t)value(i, e, f + e);
-            *reinterpret_cast<bf16x4*>(row + f) = r;
-          }
-        }
-      }
-    }
+  for (int q = 0; q < XS; ++q) {
+    const int R = 8 * (wave + NW * q) + r8;
+    off[q] = (uint32_t)((int64_t)min(m0 + R, M - 1) * ldx * 2 + 16 * (c8 ^ ((R >> 1) & 7)));
   }
+#pragma unroll
+  for (int q = 0; q < WS; ++q) {
+    const int R = 8 * (wave + NW * q) + r8, owner = R / (16 * NI), h = R % (16 * NI) / (8 * NI);
+    int f = R % (8 * NI);                                             // laid out as in `gemm_tile_kernel`
+    if (PAIRED && (f >> 5) < NH / 2) f = (f & ~31) + 8 * ((f & 15) >> 2) + 4 * ((f >> 4) & 1) + (f & 3);
+    const int64_t row = ACT ? (int64_t)h * I + min(n0 + owner * (8 * NI) + f, I - 1) : min(n0 + owner * (16 * NI) + h * (8 * NI) + f, N - 1);
+    off[XS + q] = (uint32_t)(row * ldw * 2 + 16 * (c8 ^ ((R >> 1) & 7)));
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)tile_lds + 1024 * wave;
+  const bf16_t* xa = x + (int64_t)first * 64;                         // of the step that is asked for next
+  const bf16_t* wa = w + (int64_t)first * 64;
+  auto ask_piece = [&](uint32_t slot, int q) {
+    if (q < XS) tile_dma16(xa, off[q], lds0 + slot + NW * q * 1024);
+    else tile_dma16(wa, off[q], lds0 + slot + TM * 128 + NW * (q - XS) * 1024);
+  };
+  const int wm = wave / WGN, wn = wave % WGN, swizzle = (n >> 1) & 7;
+  uint32_t rd_x[2], rd_w[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    rd_x[s] = (wm * (16 * MI) + n) * 128 + (((4 * s + g) ^ swizzle) * 16);
+    rd_w[s] = (TM + wn * (16 * NI) + n) * 128 + (((4 * s + g) ^ swizzle) * 16);
+  }
+  struct Operands { bf16x8 x[MI][2], w[NI][2]; } one, two;
+  constexpr int READS = 2 * (NI + MI), PRODUCTS = 2 * NI * MI;
+  auto read_one = [&](uint32_t slot, Operands& o, int r) {            // in the order of use
+    const int s = r / (NI + MI), q = r % (NI + MI);
+    if (q < NI) o.w[q][s] = *reinterpret_cast<const bf16x8*>(tile_lds + slot + rd_w[s] + q * 2048);
+    else o.x[q - NI][s] = *reinterpret_cast<const bf16x8*>(tile_lds + slot + rd_x[s] + (q - NI) * 2048);
+  };
+  f32x4 acc[NI][MI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < MI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto next_slot = [&](uint32_t s) { return s == (ST - 1) * STAGE ? 0u : s + STAGE; };
+
+  const int early = min(ST - 1, steps);
+#pragma unroll
+  for (int s = 0; s < ST - 1; ++s)
+    if (s < early) {
+#pragma unroll
+      for (int q = 0; q < PIECES; ++q) ask_piece(s * STAGE, q);
+      xa += 64; wa += 64;
+    }
+  // waits until no more than the last `count` steps asked for are on their way
+  auto wait = [&](int count) {
+    if (count <= 0) tile_wait<0>();
+    else if (count == 1) tile_wait<PIECES>();
+    else if (count == 2) tile_wait<2 * PIECES>();
+    else tile_wait<3 * PIECES>();
+  };
+  static_assert(ST - 2 == 3, "`wait` knows up to three steps");
+  wait(early - 1);
+  tile_barrier();
+#pragma unroll
+  for (int r = 0; r < READS; ++r) read_one(0, one, r);
+  // The first operands are there before the loop, where the compiler then counts the reads of LDS alone and waits for as many as it needs.
+  __builtin_amdgcn_s_waitcnt(0xC07F);                                 // lgkmcnt(0)
+  uint32_t slot = 0, free_slot = (ST - 1) * STAGE;                    // where step k is; where step k + ST - 1 goes, which held step k - 1
+  int k = 0;
+  // Why no wait is missing: step k + 1 has been waited for by every wave that asked for part of it before the barrier of step k, behind
+  // which it is read. A wave passes that barrier with its products of step k - 1 behind it, so with its reads of that step done: the
+  // requests of step k overwrite what nobody reads any more.
+  auto step = [&](const Operands& cur, Operands& nxt, auto asks, auto more) {
+    uint32_t s1 = 0;
+    if constexpr (decltype(more)::value) { tile_barrier(); s1 = next_slot(slot); }
+#pragma unroll
+    for (int c = 0; c < PRODUCTS; ++c) {
+      const int s = c / (NI * MI), i = c / MI % NI, j = c % MI;
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.w[i][s], cur.x[j][s], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (decltype(more)::value) {
+#pragma unroll
+        for (int r = c * READS / PRODUCTS; r < (c + 1) * READS / PRODUCTS; ++r) read_one(s1, nxt, r);
+      }
+      if constexpr (decltype(asks)::value) {
+#pragma unroll
+        for (int q = c * PIECES / PRODUCTS; q < (c + 1) * PIECES / PRODUCTS; ++q) ask_piece(free_slot, q);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (decltype(asks)::value) { xa += 64; wa += 64; }
+    if constexpr (decltype(more)::value) { free_slot = slot; slot = s1; }
+    ++k;
+  };
+  const std::true_type yes;
+  const std::false_type no;
+  auto steady = [&](const Operands& cur, Operands& nxt) { tile_wait<PIECES * (ST - 3)>(); step(cur, nxt, yes, yes); };
+  auto ending = [&](const Operands& cur, Operands& nxt) {             // near the end: what is left decides
+    if (k + 1 < steps) {
+      wait(min(ST - 3, steps - 2 - k));
+      if (k + ST - 1 < steps) step(cur, nxt, yes, yes); else step(cur, nxt, no, yes);
+    } else {
+      step(cur, nxt, no, no);
+    }
+  };
+  while (k + ST < steps) { steady(one, two); steady(two, one); }
+  while (k < steps) {
+    ending(one, two);
+    if (k < steps) ending(two, one);
+  }
+  tile_store<MI, NI, ACT>(acc, y + (int64_t)blockIdx.z * M * ldy, ldy, M, N, m0 + wm * (16 * MI) + n, n0 + wn * (ACT ? 8 * NI : 16 * NI), g, form, rounded);
 }
 
 // y: [M, N] of out_dtype (ksplit 1), or float32 partial sums [ksplit, M, N] with ldy = N; act: w is a packed gate/up weight
@@ -295,9 +446,9 @@ extern "C" int me_gemm_tile_bf16(const void* x, int64_t ldx, const void* w, int6
   const int steps = K / 64, per_split = (steps + ksplit - 1) / ksplit;
   ME_CHECK((int64_t)(ksplit - 1) * per_split <= steps - 2, "tile gemm: %d slices leave one of %d steps with fewer than two", ksplit, steps);
   const GateForm form{limit, alpha, bias};
-#define TILE_LAUNCH(WGM, WGN, MI, NI, ACT, TO)                                                                                       \
+#define TILE_LAUNCH(KERNEL, WGM, WGN, MI, NI, ACT, TO)                                                                               \
   do {                                                                                                                               \
-    auto kernel = gemm_tile_kernel<WGM, WGN, MI, NI, ACT, TO>;                                                                       \
+    auto kernel = KERNEL<WGM, WGN, MI, NI, ACT, TO>;                                                                                 \
     if (lds > 65536) {                                         /* more than a kernel may have unasked */                             \
       static bool allowed = false;                                                                                                   \
       if (!allowed) {                                                                                                                \
@@ -309,31 +460,47 @@ extern "C" int me_gemm_tile_bf16(const void* x, int64_t ldx, const void* w, int6
     kernel<<<grid, WGM * WGN * 64, lds, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, ldw, (TO*)y, ldy, M, N, per_split, steps, \
                                                   (int)m_tiles, (int)n_tiles, (int)(m_tiles < 8 ? m_tiles : 8), form, act == 2);               \
   } while (0)
-#define TILE(WGM, WGN, MI, NI)                                                                                        \
+#define TILE_KIND(KERNEL, WGM, WGN, MI, NI)                                                                           \
+  do {                                                                                                                \
+    if (act) TILE_LAUNCH(KERNEL, WGM, WGN, MI, NI, true, bf16_t);                                                     \
+    else if (out_dtype == ME_F32) TILE_LAUNCH(KERNEL, WGM, WGN, MI, NI, false, float);                                \
+    else TILE_LAUNCH(KERNEL, WGM, WGN, MI, NI, false, bf16_t);                                                        \
+  } while (0)
+// RING: the steps from which a tile of four waves goes through the ring where the launch has at most a workgroup to a compute unit (0: never).
+// Below 16 steps the quarters are level or ahead (8 steps a slice, 128 rows of 1024 x 2048 in tiles of 128 x 64 6.3 / 6.7 us). Tiles of 128 x 128, whose ring
+// fills a compute unit's LDS, gain from 32 steps on and up to 248 workgroups (16 steps 12.3 / 16.5 with 256 of them, 32 steps 20.2 / 23.2,
+// with 208 19.5 / 18.5).
+#define TILE(WGM, WGN, MI, NI, RING)                                                                                  \
   if (tile_rows == WGM * MI * 16 && tile_features == WGN * NI * 16) {                                                 \
     const int64_t m_tiles = ((int64_t)M + tile_rows - 1) / tile_rows;                                                 \
     const int64_t n_tiles = act ? ((int64_t)N / 2 + tile_features / 2 - 1) / (tile_features / 2) : ((int64_t)N + tile_features - 1) / tile_features; \
     const int64_t blocks = (m_tiles * n_tiles + 7) / 8 * 8;                                                           \
     ME_CHECK(blocks < (1ll << 31) && 8 * n_tiles < (1ll << 31) && ksplit <= 65535, "tile gemm: too many tiles");      \
     const dim3 grid((unsigned)blocks, 1, (unsigned)ksplit);                                                           \
+    if constexpr (RING > 0)                                                                                           \
+      if (m_tiles * n_tiles * ksplit <= (RING >= 32 ? 248 : 256) && per_split >= RING) {                              \
+        const size_t lds = (size_t)(tile_rows + tile_features) * 128 * RING_STAGES;                                   \
+        TILE_KIND(gemm_ring_kernel, WGM, WGN, MI, NI);                                                                \
+        ME_LAUNCH_CHECK();                                                                                            \
+        return 0;                                                                                                     \
+      }                                                                                                               \
     const size_t lds = (size_t)(tile_rows + tile_features) * 256;                                                     \
-    if (act) TILE_LAUNCH(WGM, WGN, MI, NI, true, bf16_t);                                                             \
-    else if (out_dtype == ME_F32) TILE_LAUNCH(WGM, WGN, MI, NI, false, float);                                        \
-    else TILE_LAUNCH(WGM, WGN, MI, NI, false, bf16_t);                                                                \
+    TILE_KIND(gemm_tile_kernel, WGM, WGN, MI, NI);                                                                    \
     ME_LAUNCH_CHECK();                                                                                                \
     return 0;                                                                                                         \
   }
-  TILE(2, 4, 8, 4)     // 256 x 256
-  TILE(4, 2, 4, 6)     // 256 x 192
-  TILE(2, 4, 6, 4)     // 192 x 256
-  TILE(2, 4, 4, 4)     // 128 x 256
-  TILE(4, 2, 4, 4)     // 256 x 128
-  TILE(4, 2, 2, 6)     // 128 x 192
-  TILE(2, 2, 4, 4)     // 128 x 128
-  TILE(2, 2, 2, 4)     // 64 x 128
-  TILE(2, 2, 4, 2)     // 128 x 64
-  TILE(2, 2, 2, 2)     // 64 x 64
+  TILE(2, 4, 8, 4, 0)     // 256 x 256
+  TILE(4, 2, 4, 6, 0)     // 256 x 192
+  TILE(2, 4, 6, 4, 0)     // 192 x 256
+  TILE(2, 4, 4, 4, 0)     // 128 x 256
+  TILE(4, 2, 4, 4, 0)     // 256 x 128
+  TILE(4, 2, 2, 6, 0)     // 128 x 192
+  TILE(2, 2, 4, 4, 32)     // 128 x 128
+  TILE(2, 2, 2, 4, 16)     // 64 x 128
+  TILE(2, 2, 4, 2, 16)     // 128 x 64
+  TILE(2, 2, 2, 2, 16)     // 64 x 64
 #undef TILE
+#undef TILE_KIND
 #undef TILE_LAUNCH
   ME_CHECK(false, "tile gemm: no tile of %d rows x %d features", tile_rows, tile_features);
 }

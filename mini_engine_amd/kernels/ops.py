@@ -262,13 +262,13 @@ def library_product(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, sp
 
 
 def _tile_product(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, slices: int = 1, gated: int = 0, form: tuple = (0.0, 1.0),
-                  bias: torch.Tensor | None = None) -> torch.Tensor:
+                  bias: torch.Tensor | None = None, tile: tuple | None = None) -> torch.Tensor:
     """x [M, K] . w[N, K]^T by csrc/gemm_tile.hip into y: [M, N], float32 partial sums [slices, M, N], or with `gated` (1: formed
-    from the unrounded sums, 2: from the sums rounded to bfloat16) [M, N / 2]."""
+    from the unrounded sums, 2: from the sums rounded to bfloat16) [M, N / 2]. `tile`: in place of `tile_choice`'s."""
     M, K = x.shape
     N = w.shape[0]
     core().call("me_gemm_tile_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), y.shape[-1], _code(y.dtype), slices,
-                M, N, K, gated, *form, _ptr(bias), *tile_choice(M, N, K, slices, gated > 0)[0], _stream())
+                M, N, K, gated, *form, _ptr(bias), *(tile or tile_choice(M, N, K, slices, gated > 0)[0]), _stream())
     return y
 
 
@@ -682,6 +682,9 @@ class HipBackend:
             return y
         mid = mid_takes(M, N, K, False) == 1
         tiles = tile_fits(x, w) and (out is None or out.data_ptr() % 16 == 0)      # an `out` may begin anywhere
+        ring = ring_tile(M, N, K) if tiles and not (mid and N * K > RING_MAX_WEIGHT_OF_MID) else None
+        if ring is not None:
+            return _tile_product(x, w, new(), tile=ring)
         if mid and not (mid_crowded(M, N, 1) and tiles):
             y = new()
             core().call("me_gemm_mid_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N,
@@ -1764,6 +1767,41 @@ def tile_takes(M: int, N: int, K: int) -> bool:
         return True
     rounds = -(-(-(-M // rows) * -(-N // features)) // _COMPUTE_UNITS)
     return tile in ((256, 128), (256, 192)) and M * N >= TILE_FILL * rounds * _COMPUTE_UNITS * rows * features
+
+
+RING_TILES = ((64, 64), (64, 128), (128, 64), (128, 128))
+RING_MAX_WEIGHT_OF_MID = 1 << 22          # beyond, the tiled kernel of csrc/gemm_mid.hip keeps what it has: 7.2 / 6.6 us over 6144 x 1024
+
+
+@lru_cache(maxsize=4096)
+def ring_tile(M: int, N: int, K: int) -> tuple | None:
+    """The tile by which M rows (more than 64) against a bfloat16 weight [N, K] go through the ring of csrc/gemm_tile.hip, one workgroup to
+    a compute unit, or None. The smallest tile that gives one round of workgroups, for a step of it is the shortest (0.17 us for 64 x 64, 0.31 for 64 x
+    128, 0.49 for 128 x 128); over a K of 4,096 and more 128 x 64 before 64 x 128 (300 rows of 4096 x 4096 27.8 / 23.4). Timed against
+    what had these products, the library or older kernels, in a chain with weights from memory (us, theirs / this), 65 to 3,123 rows:
+    up to a K of 2,048 ahead in 58 of 60 products, by 1.15 on average (128 rows of 4096 x 1024 7.0 / 6.4, 700 of 1024 x 2048 10.8 / 9.0, 2,048 15.3 /
+    12.6, 128 of 12288 x 2048 15.9 / 13.4), but not with tiles of 128 x 128 over a K below 2,048 (800 rows of 4096 x 1024 11.7 / 12.1); below 4,096
+    where six tenths of the compute units have a tile (2,048 rows of 1024 x 3072 20.9 / 17.5, 700 14.2 / 12.1); beyond, where the rows and features fill
+    seven tenths of a round (800 of 4096 x 4096 40.0 / 33.6, 640 of 6144 x 4096 41.1 / 33.2, 1,563 of 2048 x 6144 55.2 / 47.4, 700 of 2560 x 9728
+    64.4 / 53.3; below that behind as often as ahead: 640 of 4096 x 4096 35.2 / 38.0, 700 of 4096 x 12288 87 / 99), with tiles of 64 x 64 up to 4,096
+    (256 rows of 4096 x 12288 54.5 / 60.5). The bits are those of the library's kernels that add up K in one piece; over a K beyond
+    16,384, where it takes others, the library keeps it."""
+    if M <= 64 or K < 1024 or K > 16384:
+        return None
+    order = RING_TILES if K < 4096 else (RING_TILES[0], RING_TILES[2], RING_TILES[1], RING_TILES[3])
+    for tile in order:
+        tiles = -(-M // tile[0]) * -(-N // tile[1])
+        if tiles <= (_COMPUTE_UNITS if tile != (128, 128) else _COMPUTE_UNITS - 8):
+            break
+    else:
+        return None
+    if K <= 2048:
+        return None if tile == (128, 128) and K < 2048 else tile
+    if K < 4096:
+        return tile if tiles >= 0.6 * _COMPUTE_UNITS else None
+    if tile == (64, 64) and K > 4096:
+        return None
+    return tile if M * N >= 0.7 * _COMPUTE_UNITS * tile[0] * tile[1] else None
 
 
 def tile_fits(x: torch.Tensor, w: torch.Tensor, slices: int = 1) -> bool:

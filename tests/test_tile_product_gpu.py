@@ -183,3 +183,35 @@ def test_what_the_kernel_refuses():
     for args in ((x[:, :96], w[:, :96], y, 1, (64, 64)), (x, w, y, 1, (64, 96)), (x, w, y.float(), 2, (64, 64)), (x, w[:60], y[:, :60], 1, (64, 64))):
         with pytest.raises(ops.KernelError):
             _launch(*args)
+
+
+@pytest.mark.parametrize("tile", [(64, 64), (64, 128), (128, 64), (128, 128)], ids=lambda t: f"{t[0]}x{t[1]}")
+@pytest.mark.parametrize("steps", [16, 17, 32, 33, 35])
+def test_tiles_in_one_round_go_round_the_ring(tile, steps):
+    """Launches of one workgroup to a compute unit walk K through a ring of stages: from its fewest steps on, with an odd count and a
+    row, a feature piece and a stride beside the tile's, every kind of output; bit for bit what a launch of many rounds gives the same rows."""
+    rows, features = tile
+    M, N, K = 2 * rows + 5, 3 * features - 16, 64 * steps
+    x, w = _operands(M, N, K, 8)
+    many = torch.cat([x] * (1 + 300 * rows * features // (M * N)))                          # more than 256 tiles
+    many = many[:many.shape[0] - many.shape[0] % rows + 3]
+    ref = x.double() @ w.double().t()
+    for dtype, slices, gated in ((torch.bfloat16, 1, 0), (torch.float32, 1, 0), (torch.float32, 2, 0), (torch.bfloat16, 1, 1), (torch.bfloat16, 1, 2)):
+        outs = []
+        for rows_in in (x, many):
+            shape = (rows_in.shape[0], N // 2 if gated else N)
+            y = torch.full(shape if slices == 1 else (slices, *shape), float("nan"), dtype=dtype, device=DEV)
+            _launch(rows_in, w, y, slices, tile, gated)
+            outs.append(y[..., :M, :])
+        assert torch.equal(*outs)
+        if not gated:
+            close(outs[0] if slices == 1 else outs[0].sum(0), ref, 4e-3 if dtype == torch.bfloat16 else 2e-5)
+
+
+@pytest.mark.parametrize("M,N,K,route", [(65, 4096, 1024, TILE), (256, 4096, 1024, TILE), (700, 1024, 2048, TILE), (2048, 1024, 3072, TILE), (300, 1024, 3072, LIBRARY),
+                                         (800, 4096, 4096, TILE), (640, 4096, 4096, LIBRARY), (256, 4096, 6144, LIBRARY), (90, 4100, 1024, MID)])
+def test_each_product_of_one_round_runs_where_the_rule_sends_it(monkeypatch, M, N, K, route):
+    x, w = _operands(M, N, K)
+    y, ran = _products(monkeypatch, lambda: hip().linear(x, w))
+    assert ran == [route] and (ops.ring_tile(M, N, K) is not None) == (route == TILE or N % 8 > 0)
+    close(y, x.double() @ w.double().t(), 4e-3)
