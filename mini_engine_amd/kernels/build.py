@@ -2,17 +2,20 @@
 
 Two kinds of library: ``libme_core.so`` (every kernel that takes its sizes at run
 time) and ``libme_attn_d<D>.so`` (the MFMA attention kernels, specialised per
-head size). A library is rebuilt when the hash of its sources and flags differs
+head size); beside them ``me_calls.so``, a Python module through which their entry points are called. A library is rebuilt when the hash of its sources and flags differs
 from the one recorded beside it. Libraries live in ``mini_engine_amd/lib`` when
 that folder can be written, else in a per-user folder under the temp directory.
 """
 from __future__ import annotations
 
 import hashlib
+import importlib.machinery
+import importlib.util
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 import threading
 import time
@@ -33,6 +36,7 @@ CORE_SOURCES = ["elementwise.hip", "rope_kv.hip", "attention_simple.hip",
                 "streams.hip"]
 ATTN_SOURCE = "attention_mfma.hip"
 HEADERS = ["common.h", "errors.inc", "sampling.h", "chunks.h"]
+CALLS_SOURCE = "calls.cpp"
 # Head sizes that build_all() compiles ahead of use; any other multiple of 16 up to 512 is compiled when a model first needs it.
 DEFAULT_HEAD_DIMS = (16, 32, 48, 64, 80, 128, 256)
 CAPPED_HEAD_DIMS = (32, 64, 128)          # ... of the variant with a cap on the scores
@@ -200,11 +204,36 @@ def attention_library(head_dim: int, force: bool = False, score_cap: bool = Fals
     return _ensure(f"libme_attn_d{head_dim}{'c' * score_cap}{'d' * distance}.so", [ATTN_SOURCE], flags, force)
 
 
+def calls_library(force: bool = False) -> str | None:
+    """The Python module of csrc/calls.cpp, for the interpreter that runs; None where it is not built and cannot be (no compiler, no
+    headers of Python): the entry points are then called through ctypes."""
+    include = sysconfig.get_paths()["include"]
+    extra = ["-x", "c++", "-I", include, "-DME_PYTHON=" + str(sysconfig.get_config_var("SOABI")).replace("-", "_")]
+    digest = _hash([CALLS_SOURCE], extra)
+    if not force:
+        for d in _lib_dirs():
+            if _up_to_date(os.path.join(d, "me_calls.so"), digest):
+                return os.path.join(d, "me_calls.so")
+    if hipcc_path() is None or not os.path.isfile(os.path.join(include, "Python.h")):
+        return None
+    return _ensure("me_calls.so", [CALLS_SOURCE], extra, force)
+
+
+def calls_module():
+    path = calls_library()
+    if path is None:
+        return None
+    loader = importlib.machinery.ExtensionFileLoader("me_calls", path)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("me_calls", loader))
+    loader.exec_module(module)
+    return module
+
+
 def build_all(head_dims=DEFAULT_HEAD_DIMS, force: bool = True) -> list:
     """Compile every library (used by the repository's build check)."""
-    libs = [core_library(force=force)]
+    libs = [core_library(force=force), calls_library(force=force)]
     with ThreadPoolExecutor(max_workers=4) as pool:
         libs += list(pool.map(lambda d: attention_library(d, force=force), head_dims))
         libs += list(pool.map(lambda d: attention_library(d, force=force, score_cap=True), CAPPED_HEAD_DIMS))
         libs += list(pool.map(lambda d: attention_library(d, force=force, distance=True), DISTANCE_HEAD_DIMS))
-    return libs
+    return [lib for lib in libs if lib]

@@ -41,21 +41,40 @@ def _code(dtype: torch.dtype) -> int:
 # --------------------------------------------------------------------------- libraries
 
 class _Lib:
+    """A kernel library. `fns`: its entry points by name; `call(name, *args)` raises where one does not return 0. Both go through
+    the native module (csrc/calls.cpp) where it is built, which takes a sixth of ctypes' time a call, otherwise through ctypes."""
+
     def __init__(self, path: str, protos: dict):
         self.path = path
         self.cdll = ctypes.CDLL(path)
         self.cdll.me_last_error.restype = c_char_p
+        native = _native_calls()
         self.fns = {}
         for name, argtypes in protos.items():
             fn = getattr(self.cdll, name)
             fn.argtypes = argtypes
             fn.restype = c_int
+            if native is not None:
+                fn = native.bind(ctypes.cast(fn, c_void_p).value, "".join(_KINDS[t] for t in argtypes), fn)
             self.fns[name] = fn
         self.protos = protos
+        if native is not None:
+            self.call = native.caller(self.fns, self._failed)
+
+    def _failed(self, name: str):
+        raise KernelError(f"{name}: {self.cdll.me_last_error().decode()}")
 
     def call(self, name: str, *args):
         if self.fns[name](*args) != 0:
-            raise KernelError(f"{name}: {self.cdll.me_last_error().decode()}")
+            self._failed(name)
+
+
+_KINDS = {c_void_p: "p", c_int: "i", c_int64: "i", ctypes.c_size_t: "i", c_float: "f"}
+
+
+@lru_cache(maxsize=1)
+def _native_calls():
+    return build.calls_module()
 
 
 P, I, L, F = c_void_p, c_int, c_int64, c_float
@@ -407,8 +426,8 @@ class HipBackend:
         layers/rotary_embedding.py:20-25, csrc/kv_cache.cu:10-31.)"""
         T = qkv.shape[0]
         width = (Hq + (2 * Hkv if store and not values_are_keys else Hkv)) * D
-        _check(qkv.dim() == 2 and qkv.stride(1) == 1 and qkv.shape[1] == width,
-               f"qk_norm_rope_store: rows must be [T, {width}] with unit inner stride, got {tuple(qkv.shape)}")
+        if not (qkv.dim() == 2 and qkv.stride(1) == 1 and qkv.shape[1] == width):
+            raise KernelError(f"qk_norm_rope_store: rows must be [T, {width}] with unit inner stride, got {tuple(qkv.shape)}")
         for w in (q_weight, k_weight):
             _check(w is None or (w.dtype == torch.float32 and w.shape == (D,) and w.is_contiguous()),
                    "qk_norm_rope_store: norm weights must be float32 [D]")
@@ -623,9 +642,12 @@ class HipBackend:
         from large tiles up to 256 rows and from the library as a strided batch up to 1,024 over larger weights
         (library_splits).
         `out` (not with allow_partials): a contiguous [M, N] tensor of the output dtype to write into."""
-        _check(x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1], f"linear: {tuple(x.shape)} x {tuple(w.shape)}^T")
-        _check(x.dtype == w.dtype, f"linear: activation {x.dtype} and weight {w.dtype} differ")
-        _check(x.stride(1) == 1 and w.stride(1) == 1, "linear: rows must be contiguous")
+        if not (x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1]):       # (messages are formed where they are needed)
+            raise KernelError(f"linear: {tuple(x.shape)} x {tuple(w.shape)}^T")
+        if x.dtype != w.dtype:
+            raise KernelError(f"linear: activation {x.dtype} and weight {w.dtype} differ")
+        (xs, x1), (ws, w1) = x.stride(), w.stride()
+        _check(x1 == 1 and w1 == 1, "linear: rows must be contiguous")
         M, K = x.shape
         N = w.shape[0]
         out_dtype = out_dtype or x.dtype
@@ -639,8 +661,7 @@ class HipBackend:
             core().call("me_gemm_f32", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N,
                         M, N, K, *f32_tile(M, N), _stream())
             return y
-        aligned = (K % 8 == 0 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
-                   and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+        aligned = K % 8 == 0 and xs % 8 == 0 and ws % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
         if not aligned:
             y = new()
             core().call("me_gemm_tiled", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N,
@@ -681,7 +702,9 @@ class HipBackend:
                         _code(out_dtype), None, 1, M, N, K, 0, 0, skinny_wide(N, K), 0.0, 1.0, None, _stream())
             return y
         mid = mid_takes(M, N, K, False) == 1
-        tiles = tile_fits(x, w) and (out is None or out.data_ptr() % 16 == 0)      # an `out` may begin anywhere
+        # `tile_fits` of what is left to ask, and an `out` may begin anywhere
+        tiles = (K % 64 == 0 and K >= 128 and N % 8 == 0 and M * xs < 1 << 31 and N * ws < 1 << 31
+                 and (out is None or out.data_ptr() % 16 == 0))
         ring = ring_tile(M, N, K) if tiles and not (mid and N * K > RING_MAX_WEIGHT_OF_MID) else None
         if ring is not None:
             return _tile_product(x, w, new(), tile=ring)
@@ -703,14 +726,17 @@ class HipBackend:
         rows, `gated_linear_tiles`). For the row counts `gated_linear_fuses` admits. `bias` (float32 [2 I]) joins the sums
         first; `clamp` (limit, alpha): the form of `glu_clamped` in place of silu(gate) * up. Returns [M, I].
         (reference layers/linear.py:29-45, layers/activation.py:5-7.)"""
-        _check(gated_linear_fuses(x, w), "gated_linear: bfloat16, few rows, see gated_linear_fuses")
-        M, K = x.shape
+        M = x.shape[0]
+        as_tiles = (x.dtype == torch.bfloat16 and x.dim() == 2 and M > GATED_EPILOGUE_MAX_M and gated_linear_tiles(M, w) and x.shape[1] == w.shape[1]
+                    and x.stride(1) == 1 and tile_fits(x, w))
+        _check(as_tiles or gated_linear_fuses(x, w), "gated_linear: bfloat16, few rows, see gated_linear_fuses")
+        K = x.shape[1]
         N = w.shape[0]
         y = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         _check(bias is None or (bias.dtype == torch.float32 and bias.shape == (N,) and bias.is_contiguous()), "gated_linear: bias float32 [2 I]")
         _check(clamp is None or clamp[0] > 0, "gated_linear: the limit must be positive")
         form = (0.0, 1.0) if clamp is None else (float(clamp[0]), float(clamp[1]))
-        if M > GATED_EPILOGUE_MAX_M and gated_linear_tiles(M, w) and tile_fits(x, w):
+        if as_tiles:
             # the gates as those forms that had these rows before this kernel make them: rounded where the gating was a kernel
             # of its own behind the product
             return _tile_product(x, w, y, gated=1 if mid_takes(M, N, K, False) == 1 else 2, form=form, bias=bias)
@@ -1807,10 +1833,11 @@ def ring_tile(M: int, N: int, K: int) -> tuple | None:
 def tile_fits(x: torch.Tensor, w: torch.Tensor, slices: int = 1) -> bool:
     """Whether csrc/gemm_tile.hip can compute x . w^T in that many slices of K: K in two steps of 64 or more for each, whole
     16-byte pieces in every row, 32-bit offsets."""
-    K, steps = x.shape[1], x.shape[1] // 64
-    return (K % 64 == 0 and w.shape[0] % 8 == 0 and (slices - 1) * -(-steps // slices) <= steps - 2
-            and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and x.shape[0] * x.stride(0) < 1 << 31 and w.shape[0] * w.stride(0) < 1 << 31)
+    (M, K), N = x.shape, w.shape[0]
+    steps, xs, ws = K // 64, x.stride(0), w.stride(0)
+    return (K % 64 == 0 and N % 8 == 0 and (slices - 1) * -(-steps // slices) <= steps - 2
+            and xs % 8 == 0 and ws % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and M * xs < 1 << 31 and N * ws < 1 << 31)
 
 
 def mid_crowded(M: int, N: int, slices: int) -> bool:
@@ -1889,6 +1916,7 @@ def _cheapest_partition(base: int, ctx: int, sizes: tuple) -> int:
     return min(sizes, key=lambda p: (_decode_partition_cost(base, ctx, p), -p))
 
 
+@lru_cache(maxsize=1024)      # a step asks once per layer
 def decode_partitions(num_seqs: int, Hq: int, Hkv: int, max_context: int, even: bool = False) -> tuple:
     """(keys per partition, number of partitions) for the split decode kernel.
 
@@ -2125,6 +2153,8 @@ def gated_linear_rows(rows: int, w: torch.Tensor) -> bool:
     # gating in its epilogue is still ahead of the two up to 8 rows over a K of 4,096
     takes = skinny_takes(rows, N, K) or (rows <= 8 and K <= 4096 and N < LIBRARY_MIN_N and rows <= SKINNY_MAX_M)
     aligned = N % 2 == 0 and K % 8 == 0 and w.stride(1) == 1 and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0
+    if rows > 256:
+        return False                     # (`mid_takes`)
     if rows > GATED_EPILOGUE_MAX_M:
         # the kernel for a few hundred rows over a small weight gates in its epilogue too, in place of a kernel of
         # its own behind it; and from 17 rows on, where the skinny kernel would have the product itself
@@ -2148,7 +2178,7 @@ def norm_linear_fuses(x: torch.Tensor, w: torch.Tensor) -> bool:
     bfloat16 weight that the unsplit skinny kernel would take, one or two rows, a weight of at most
     NORM_FUSE_MAX_WEIGHT elements. Every workgroup forms the normed rows for itself, which costs each about
     2 us; the norm kernel costs 3 us in a chain of decode kernels, so it pays for one and two rows only."""
-    if not FUSE_NORM_INTO_LINEAR or w.dtype != torch.bfloat16 or w.dim() != 2 or x.dim() not in (2, 3):
+    if not FUSE_NORM_INTO_LINEAR or x.dim() not in (2, 3) or x.shape[-2] > NORM_FUSE_MAX_M or w.dtype != torch.bfloat16 or w.dim() != 2:
         return False
     S = x.shape[0] if x.dim() == 3 else 1
     M, K = x.shape[-2], x.shape[-1]
