@@ -484,7 +484,15 @@ __device__ __forceinline__ float shape_token(const DrArgs& a, int lane, int nr_r
 
 // One wave per (token, head): the shaped values of every token at once, for a recurrence kernel that then only streams
 // them (decay_walk_kernel): pre_q, pre_k, pre_d [T, H, NR] and pre_x [T, H], float32. The rows of a (token, head) lie in the
-// order in which that kernel's lanes take them: row n at (n mod row_groups) NR / row_groups + n / row_groups.
+// order in which that kernel's lanes take them (walk_place).
+// Lane rg of the RG lanes of a column keeps rows rg, rg + RG, ...: its i-th row lies among the i / 4-th four of all lanes, so that
+// the lanes of a column read 16-byte pieces side by side (a lane's rows in one run met each bank RL / 4 times: 128 rows over 16
+// lanes, 44 % of the LDS cycles).
+template <int NR, int RG>
+__host__ __device__ constexpr int walk_place(int rg, int i) {
+  constexpr int RL = NR / RG;
+  return RL < 4 ? rg * RL + i : i / 4 * (RG * 4) + rg * 4 + i % 4;
+}
 template <typename TX, int NR, int RULE>
 __global__ void __launch_bounds__(64) decay_prepare_kernel(DrArgs a, int row_groups, float* __restrict__ pre_q, float* __restrict__ pre_k,
                                                            float* __restrict__ pre_d, float* __restrict__ pre_x) {
@@ -506,14 +514,16 @@ __global__ void __launch_bounds__(64) decay_prepare_kernel(DrArgs a, int row_gro
   }
   const float beta = (RULE == 1 || RULE == 3) ? to_f32<TX>(bp[t * a.beta_stride + h]) : 0.f;
   const float x = shape_token<PER, RULE>(a, lane, NR, q, k, d, base, bonus, RULE != 0 ? a.rate[h] : 0.f, beta);
+  // each lane takes the value that belongs in its place, so that a wave's stores are whole lines
   const int64_t at = (t * a.H + h) * NR;
+  const int from = row_groups == 16 ? (NR == 32 ? lane % 2 * 16 + lane / 2 : lane % 4 * 16 + lane / 4) : (lane & ~15) + lane % 4 * 4 + lane / 4 % 4;
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
-    const int n = lane + 64 * i;
-    if (n < NR) {
-      const int64_t to = at + n % row_groups * (NR / row_groups) + n / row_groups;
-      pre_q[to] = q[i]; pre_k[to] = k[i];
-      if (RULE != 3) pre_d[to] = d[i];
+    const float qv = __shfl(q[i], from), kv = __shfl(k[i], from), dv = RULE == 3 ? 0.f : __shfl(d[i], from);
+    const int64_t to = at + lane + 64 * i;
+    if (lane + 64 * i < NR) {
+      pre_q[to] = qv; pre_k[to] = kv;
+      if (RULE != 3) pre_d[to] = dv;
     }
   }
   if (lane == 0) {
@@ -660,25 +670,20 @@ __global__ void __launch_bounds__(64) decay_rows_kernel(DrArgs a) {
 }
 
 // The same walk over values that decay_prepare_kernel has shaped: portions of many tokens. What bounds it is the number of
-// instructions of a wave per token (a request's tokens are a chain, the chip has few waves per SIMD, and a lone wave of a SIMD
-// issues one instruction in eight cycles or so), so a batch of eight tokens is one piece of code without a branch: the exchange
+// instructions of a wave per token (a request's tokens are a chain, and the chip has few waves per SIMD, each of which issues an instruction
+// in four cycles), so a batch of eight tokens is one piece of code without a branch: the exchange
 // and the output sum of a token overlap the next token's reads and updates, and shared values are brought in 16-byte pieces that
-// go to LDS as they are. With W = 4 four waves hold the same columns: each of them carries the state through every token,
-// but forms, exchanges and stores the outputs of every fourth only, and brings a quarter of the shared values; batches
-// are twice as long, for eight tokens take less time than the next eight need to come from memory (the bound of the rules with
-// short chains: about 105 ns a token whatever their instructions), and tokens are read from LDS two or three ahead. The sums are
-// those of decay_rows_kernel in the same order. With the kernel that shapes the values, 2,048 tokens beside 1,075, one wave /
-// four: delta rule, 4 heads of 128 x 128, 344 / 265 us, bonus rule, 16 heads of 64 x 64, 230 / 143 us.
-template <typename TX, int NR, int RG, int RULE, int W>
-__global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const float* __restrict__ pre_q, const float* __restrict__ pre_k,
-                                                            const float* __restrict__ pre_d, const float* __restrict__ pre_x) {
-  constexpr int TB = W == 4 ? 16 : DR_TB;       // tokens of a batch: with more of them on their way than a trip to memory takes
+// go to LDS as they are. The sums are those of decay_rows_kernel in the same order.
+template <typename TX, int NR, int RG, int RULE>
+__global__ void __launch_bounds__(64) decay_walk_kernel(DrArgs a, const float* __restrict__ pre_q, const float* __restrict__ pre_k,
+                                                        const float* __restrict__ pre_d, const float* __restrict__ pre_x) {
+  constexpr int TB = DR_TB;
   constexpr int AHEAD = NR <= 64 ? 3 : NR <= 128 ? 2 : 1;    // tokens whose shared values are read from LDS ahead
   constexpr int PC = 64 / RG;            // columns per wave
   constexpr int RL = NR / RG;            // rows per lane
   constexpr int PIECES = TB * NR / 4; // 16-byte pieces of a batch's q, k or decays
-  constexpr int ROUNDS = (PIECES + 64 * W - 1) / (64 * W);
-  constexpr int VALUES = TB * PC, VROUNDS = (VALUES + 64 * W - 1) / (64 * W);
+  constexpr int ROUNDS = (PIECES + 63) / 64;
+  constexpr int VALUES = TB * PC, VROUNDS = (VALUES + 63) / 64;
   constexpr bool ROWS = RULE != 3;
   constexpr bool SHARED_V = NR <= 128;   // the columns' values go through LDS too; with 256 rows a lane asks for its own
   // A lane that holds 64 rows has no registers left over: the last batch shares the code around the others and the loads of a
@@ -688,8 +693,7 @@ __global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const floa
   __shared__ f32x4 sq[2][PIECES], sk[2][PIECES], sd[ROWS ? 2 : 1][ROWS ? PIECES : 1];
   __shared__ __align__(16) float sv[2][SHARED_V ? VALUES : 1];              // [column][token]
   __shared__ float sx[2][TB], sh[2][TB];               // the tokens' own numbers; their heads' decays (RULE 3)
-  const int tid = threadIdx.x, lane = W == 1 ? tid : tid & 63;
-  const int wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = threadIdx.x;
   const int col_blocks = (a.P + PC - 1) / PC;
   const int cb = blockIdx.x % col_blocks;
   const int h = (blockIdx.x / col_blocks) % a.H;
@@ -718,16 +722,16 @@ __global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const floa
   int place[VROUNDS];
 #pragma unroll
   for (int r = 0; r < ROUNDS; ++r) {
-    const int e = min(tid + 64 * W * r, PIECES - 1);
+    const int e = min(lane + 64 * r, PIECES - 1);
     piece[r] = (uint32_t)((e / (NR / 4) * a.H * (NR / 4) + e % (NR / 4)) * 16);
   }
 #pragma unroll
   for (int r = 0; r < VROUNDS; ++r) {
-    const int e = min(tid + 64 * W * r, VALUES - 1);
+    const int e = min(lane + 64 * r, VALUES - 1);
     column[r] = min(cb * PC + e % PC, a.P - 1);
     place[r] = e % PC * TB + e / PC;
   }
-  const int my_token = tid & (TB - 1);
+  const int my_token = lane & (TB - 1);
   const uint32_t own = (uint32_t)(my_token * a.H * 4);
   auto at = [](const void* base, uint32_t bytes) { return reinterpret_cast<const char*>(base) + bytes; };
   // the next batch on its way; of a batch that is not whole, tokens behind the last are read from the last one and not used
@@ -736,7 +740,7 @@ __global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const floa
     if (SHARED_V) {
 #pragma unroll
       for (int r = 0; r < VROUNDS; ++r)
-        nv[r] = values[(int64_t)min(t0 + min(tid + 64 * W * r, VALUES - 1) / PC, n_tok - 1) * a.v_stride + column[r]];
+        nv[r] = values[(int64_t)min(t0 + min(lane + 64 * r, VALUES - 1) / PC, n_tok - 1) * a.v_stride + column[r]];
     } else if (!TIGHT) {
 #pragma unroll
       for (int j = 0; j < TB; ++j) nv[j] = values[(int64_t)min(t0 + j, n_tok - 1) * a.v_stride + pc];
@@ -760,7 +764,7 @@ __global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const floa
     }
 #pragma unroll
     for (int r = 0; r < ROUNDS; ++r) {
-      const int e = min(tid + 64 * W * r, PIECES - 1);
+      const int e = min(lane + 64 * r, PIECES - 1);
       const int64_t from = (head0 + (int64_t)min(t0 + e / (NR / 4), n_tok - 1) * a.H) * NR + e % (NR / 4) * 4;
       nq[r] = *reinterpret_cast<const f32x4*>(pre_q + from);
       nk[r] = *reinterpret_cast<const f32x4*>(pre_k + from);
@@ -775,33 +779,34 @@ __global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const floa
     }
   };
   struct Shared { float q[RL], k[RL], d[RL], x; };
-  auto read = [&](int buf, int j, Shared& o, bool reads_out) {
-    const float* aq = reinterpret_cast<const float*>(&sq[buf][0]) + j * NR + rg * RL;
-    const float* ak = reinterpret_cast<const float*>(&sk[buf][0]) + j * NR + rg * RL;
-    const float* ad = reinterpret_cast<const float*>(&sd[ROWS ? buf : 0][0]) + j * NR + rg * RL;
+  auto read = [&](int buf, int j, Shared& o) {
+    const float* aq = reinterpret_cast<const float*>(&sq[buf][0]) + j * NR + walk_place<NR, RG>(rg, 0);
+    const float* ak = reinterpret_cast<const float*>(&sk[buf][0]) + j * NR + walk_place<NR, RG>(rg, 0);
+    const float* ad = reinterpret_cast<const float*>(&sd[ROWS ? buf : 0][0]) + j * NR + walk_place<NR, RG>(rg, 0);
 #pragma unroll
     for (int i = 0; i < RL; ++i) {
-      if (reads_out) o.q[i] = aq[i];
-      o.k[i] = ak[i];
-      if (ROWS) o.d[i] = ad[i];
+      const int e = walk_place<NR, RG>(0, i);
+      o.q[i] = aq[e];
+      o.k[i] = ak[e];
+      if (ROWS) o.d[i] = ad[e];
     }
     if (!ROWS) o.d[0] = sh[buf][j];
-    o.x = RULE == 2 || (RULE == 0 && !reads_out) ? 0.f : sx[buf][j];
+    o.x = RULE == 2 ? 0.f : sx[buf][j];
   };
-  // the state behind a token and, where this wave is to give it, the token's output
-  auto token = [&](const Shared& o, float v, bool reads_out) {
+  // the state behind a token and the token's output
+  auto token = [&](const Shared& o, float v) {
     float y = 0.f;
     if (RULE == 0) {
 #pragma unroll
       for (int i = 0; i < RL; ++i) {
-        if (reads_out) y = fmaf(o.q[i], S[i], y);
+        y = fmaf(o.q[i], S[i], y);
         S[i] = fmaf(o.d[i], S[i], o.k[i] * v);
       }
     } else if (RULE == 2) {
 #pragma unroll
       for (int i = 0; i < RL; ++i) {
         S[i] = fmaf(o.d[i], S[i], o.k[i] * v);
-        if (reads_out) y = fmaf(o.q[i], S[i], y);
+        y = fmaf(o.q[i], S[i], y);
       }
     } else {
       float dot = 0.f;
@@ -815,10 +820,9 @@ __global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const floa
 #pragma unroll
       for (int i = 0; i < RL; ++i) {
         S[i] = fmaf(o.k[i], u, S[i]);
-        if (reads_out) y = fmaf(S[i], o.q[i], y);
+        y = fmaf(S[i], o.q[i], y);
       }
     }
-    if (!reads_out) return 0.f;
     y = group_sum<RG>(y);
     if (RULE == 0) y = fmaf(o.x, v, y);          // the current token's own term: v_p * sum_n q_n bonus_n k_n
     return y;
@@ -829,8 +833,8 @@ __global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const floa
   auto next_batch = [&](float (&v)[TB]) {
 #pragma unroll
     for (int r = 0; r < ROUNDS; ++r) {
-      const int e = tid + 64 * W * r;
-      if (PIECES % (64 * W) == 0 || e < PIECES) {
+      const int e = lane + 64 * r;
+      if (PIECES % 64 == 0 || e < PIECES) {
         sq[buf][e] = nq[r]; sk[buf][e] = nk[r];
         if (ROWS) sd[ROWS ? buf : 0][e] = nd[r];
       }
@@ -841,16 +845,14 @@ __global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const floa
     } else
 #pragma unroll
     for (int r = 0; r < VROUNDS; ++r)
-      if (VALUES % (64 * W) == 0 || tid + 64 * W * r < VALUES) sv[buf][place[r]] = to_f32<TX>(nv[r]);
-    if (tid < TB) {
-      sx[buf][tid] = nx;
-      if (!ROWS) sh[buf][tid] = nh;
+      if (VALUES % 64 == 0 || lane + 64 * r < VALUES) sv[buf][place[r]] = to_f32<TX>(nv[r]);
+    if (lane < TB) {
+      sx[buf][lane] = nx;
+      if (!ROWS) sh[buf][lane] = nh;
     }
     asm volatile("" ::: "memory");
     fetch(t0 + TB);
-    // the batch is in LDS; the other buffer, which the next batch will take, has been read by all (one wave needs no
-    // barrier: what its lanes write to LDS, its lanes read behind it)
-    if (W > 1) __syncthreads(); else asm volatile("" ::: "memory");
+    asm volatile("" ::: "memory");         // (one wave needs no barrier: what its lanes write to LDS, its lanes read behind it)
     if (SHARED_V) {
 #pragma unroll
       for (int j = 0; j < TB; ++j) v[j] = sv[buf][lane / RG * TB + j];
@@ -860,70 +862,283 @@ __global__ void __launch_bounds__(64 * W) decay_walk_kernel(DrArgs a, const floa
 #define DR_LAST_BATCH                                             \
   _Pragma("unroll 1") for (int j = 0; t0 + j < n_tok; ++j) {      \
     Shared o;                                                     \
-    read(buf, j, o, true);                                        \
+    read(buf, j, o);                                              \
     float vj = v[0];                                              \
     _Pragma("unroll") for (int i = 1; i < TB; ++i) vj = i == j ? v[i] : vj; \
-    const float y = token(o, vj, true);                           \
+    const float y = token(o, vj);                                 \
     if (live && rg == 0) out[(int64_t)(t0 + j) * (a.H * a.P)] = y; \
   }
-  auto walk = [&](auto which) {                  // a wave's whole batches: it gives the outputs of tokens which, which + W, ... of each
-    constexpr int ME = decltype(which)::value, MINE = TB / W;
-    for (; t0 + (TIGHT ? 1 : TB) <= n_tok; t0 += TB, buf ^= 1) {
-      float v[TB], y[MINE];
-      next_batch(v);
-      if (TIGHT && t0 + TB > n_tok) {
-        DR_LAST_BATCH
-        continue;
-      }
-      Shared o[AHEAD + 1];                       // a token's values are read while those before it are worked on
+  fetch(0);
+  for (; t0 + (TIGHT ? 1 : TB) <= n_tok; t0 += TB, buf ^= 1) {
+    float v[TB], y[TB];
+    next_batch(v);
+    if (TIGHT && t0 + TB > n_tok) {
+      DR_LAST_BATCH
+      continue;
+    }
+    Shared o[AHEAD + 1];                         // a token's values are read while those before it are worked on
 #pragma unroll
-      for (int j = 0; j < AHEAD; ++j) read(buf, j, o[j], j % W == ME);
+    for (int j = 0; j < AHEAD; ++j) read(buf, j, o[j]);
 #pragma unroll
-      for (int j = 0; j < TB; ++j) {
-        if (j + AHEAD < TB) read(buf, j + AHEAD, o[(j + AHEAD) % (AHEAD + 1)], (j + AHEAD) % W == ME);
-        const float yj = token(o[j % (AHEAD + 1)], v[j], j % W == ME);
-        if (j % W == ME) y[j / W] = yj;
-      }
-      // the first four lanes of a column hold the same bits (the others have added in another order): lane rg of them stores
-      // the wave's output i0 + rg
-      constexpr int ST = RG < 4 ? (RG < MINE ? RG : MINE) : (MINE < 4 ? MINE : 4);
-      if (live && rg < ST) {
+    for (int j = 0; j < TB; ++j) {
+      if (j + AHEAD < TB) read(buf, j + AHEAD, o[(j + AHEAD) % (AHEAD + 1)]);
+      y[j] = token(o[j % (AHEAD + 1)], v[j]);
+    }
+    // the first four lanes of a column hold the same bits (the others have added in another order): lane rg of them stores
+    // output i0 + rg
+    constexpr int ST = RG < 4 ? RG : 4;
+    if (live && rg < ST) {
 #pragma unroll
-        for (int i0 = 0; i0 < MINE; i0 += ST) {
-          float mine = y[i0];
+      for (int i0 = 0; i0 < TB; i0 += ST) {
+        float mine = y[i0];
 #pragma unroll
-          for (int i = 1; i < ST; ++i) mine = rg == i ? y[i0 + i] : mine;
-          out[(int64_t)(t0 + ME + W * (i0 + rg)) * (a.H * a.P)] = mine;
-        }
+        for (int i = 1; i < ST; ++i) mine = rg == i ? y[i0 + i] : mine;
+        out[(int64_t)(t0 + i0 + rg) * (a.H * a.P)] = mine;
       }
     }
-  };
-  static_assert(W == 1 || W == 4, "each wave's walk is code of its own");
-  fetch(0);
-  if (W == 1 || wave == 0) walk(std::integral_constant<int, 0>{});
-  else if (wave == 1) walk(std::integral_constant<int, 1 % W>{});
-  else if (wave == 2) walk(std::integral_constant<int, 2 % W>{});
-  else walk(std::integral_constant<int, 3 % W>{});
+  }
   if (!TIGHT && t0 < n_tok) {
     float v[TB];
     next_batch(v);
-    if (wave == 0) DR_LAST_BATCH                 // its outputs and the state behind it are the first wave's
+    DR_LAST_BATCH
   }
 #undef DR_LAST_BATCH
-  if (live && wave == 0) {
+  if (live) {
 #pragma unroll
     for (int i = 0; i < RL; ++i)
       if (i * RG + rg < a.N) srow[(int64_t)(i * RG + rg) * a.P + p] = S[i];
   }
 }
 
-// Workgroups up to which four waves share the walk of a column group: beyond, the waves of one SIMD share its instructions, and
-// the state carried four times costs more than it saves. us, one wave / four, requests of 1,100 tokens, bonus and delta rule: 128 rows, 256
-// workgroups 159 / 131 and 185 / 158, 320 (two on some compute units) 182 / 198 and 205 / 216, 512 187 / 211 and 213 / 234; 64 rows, 512
-// workgroups 122 / 98 and 154 / 150, 768 143 / 126 and 178 / 184, 832 156 / 170 and 188 / 257. Of 128 rows the delta rules keep it up to
-// 384: between a layer's other launches three prompts of 1,100 tokens over 4 heads take 195 / 188 us. With 256 rows the
-// batches' LDS leaves no room for longer ones, and without them four waves gain nothing (624 / 650).
-template <int NR, int RULE> constexpr unsigned dr_shared_max() { return NR <= 64 ? 768 : NR <= 128 ? (RULE == 1 || RULE == 3 ? 384 : 256) : 0; }
+// 64 x 16 bytes from base + voff (bytes, per lane) to LDS at lds_addr + 16 * lane. The write to m0 needs one wait
+// state before an instruction that reads it for an LDS address.
+__device__ __forceinline__ void walk_request(uint32_t lds_addr, uint32_t voff, const void* base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(base) : "memory");
+}
+
+// The walk where compute units are left over: four waves hold the same four columns: each of them carries the state through every
+// token, but forms, exchanges and stores the outputs of every fourth only, and brings a quarter of the shared values. What bounds it
+// is a wave's instructions for a token, the delta rules' also the sum over the column's lanes, four exchanges of which each waits for the one
+// before (152 cycles of a token's 200 at 128 rows); so everything else is kept out of the way. A batch's rows go to LDS past the registers, without
+// a branch in front of what is waited for; reads from LDS run seven tokens ahead (three waited for them: 64 rows 157 us for one request of 2,048
+// tokens, 109 so) and on into the next batch, behind the one barrier of a batch; the delta rules' reads and an output's exchanges stand between
+// the sum's exchanges. With the kernel that shapes the values, 2,048 tokens beside 1,075, against register copies, two barriers' worth of waiting for
+// a batch's outputs and values, and reads two or three tokens ahead: delta rule, 4 heads of 128 x 128, 262 -> 227 us, bonus rule, 16 heads of 64 x 64,
+// 150 -> 134 (one wave to a column group 344 and 230). Up to 64 rows batches of 32 tokens, held to the registers that let three workgroups onto a
+// compute unit (768 workgroups of 1,100 tokens 141 -> 130 us, 512 132 -> 135).
+template <typename TX, int NR, int RULE>
+__global__ void __launch_bounds__(256, NR <= 64 ? 3 : 2) decay_walk_shared_kernel(DrArgs a, const float* __restrict__ pre_q, const float* __restrict__ pre_k,
+                                                                const float* __restrict__ pre_d, const float* __restrict__ pre_x) {
+  constexpr int RG = 16, W = 4, PC = 4, RL = NR / RG;
+  constexpr int TB = NR <= 64 ? 32 : 16;      // tokens of a batch
+  constexpr int AHEAD = 7;               // tokens whose shared values are read from LDS ahead
+  constexpr int PIECES = TB * NR / 4, ROUNDS = (PIECES + 255) / 256;
+  constexpr bool ROWS = RULE != 3;
+  constexpr bool DELTA = RULE == 1 || RULE == 3;
+  constexpr int KINDS = ROWS ? 3 : 2;
+  __shared__ f32x4 rows[2][KINDS][PIECES];               // q, k, decays
+  __shared__ f32x4 sv[2][PC][TB / 4], sx[2][TB / 4], sh[2][TB / 4];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col_blocks = (a.P + PC - 1) / PC;
+  const int cb = blockIdx.x % col_blocks;
+  const int h = (blockIdx.x / col_blocks) % a.H;
+  const int b = blockIdx.x / (col_blocks * a.H);
+  const int begin = __builtin_amdgcn_readfirstlane(a.cu[b]);
+  const int n_tok = __builtin_amdgcn_readfirstlane(a.cu[b + 1]) - begin;
+  if (n_tok <= 0) return;
+  const int64_t first = begin;
+  const int p = cb * PC + lane / RG;
+  const int rg = lane % RG;
+  const bool live = p < a.P;
+  const int pc = live ? p : a.P - 1;
+  float* srow = a.state + (int64_t)a.slots[b] * a.state_stride + (int64_t)h * a.N * a.P;
+  float S[RL];
+#pragma unroll
+  for (int i = 0; i < RL; ++i) S[i] = (i * RG + rg < a.N) ? srow[(int64_t)(i * RG + rg) * a.P + pc] : 0.f;
+
+  // What a thread brings of a batch: pieces of the rows, which go to LDS past the registers; the first threads one column's
+  // value of one token each, the third wave's (and the fourth's) one token's number (and decay). Addresses are a batch's own, the same
+  // for all lanes, and a lane's bytes behind it; of a batch that is not whole, tokens behind the last are read from the last
+  // one and not used.
+  const int my_token = tid & (TB - 1), my_column = min(cb * PC + (tid / TB) % PC, a.P - 1);
+  TX nv;
+  float nx = 0.f;
+  const uint32_t rows_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)&rows[0][0][0];
+  auto request = [&](int t0, int buf) {          // (behind the last batch: the last token's once more; a branch here would wait for nv)
+    t0 = min(t0, n_tok - 1);
+    const int last = n_tok - 1 - t0;
+    const int64_t row = (first + t0) * a.H + h;
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r) {
+      const int e0 = 64 * wave + 256 * r;
+      if (PIECES % 256 == 0 || e0 < PIECES) {
+        const int e = e0 + lane;
+        const uint32_t from = (uint32_t)((min(e / (NR / 4), last) * a.H * (NR / 4) + e % (NR / 4)) * 16);
+        const uint32_t to = rows_base + (uint32_t)((buf * KINDS * PIECES + e0) * 16);
+        walk_request(to, from, pre_q + row * NR);
+        walk_request(to + PIECES * 16, from, pre_k + row * NR);
+        if (ROWS) walk_request(to + 2 * PIECES * 16, from, pre_d + row * NR);
+      }
+    }
+    const int t = min(my_token, last);
+    nv = ((const TX*)a.v + (first + t0) * a.v_stride + h * a.P)[(int64_t)t * a.v_stride + my_column];
+    if (RULE != 2) nx = ((!ROWS && wave == 3 ? pre_d : pre_x) + row)[t * a.H];
+  };
+  // The requested batch is in LDS for all waves behind this, and nobody reads from the other buffer any more.
+  auto arrive = [&](int buf) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (wave < TB * PC / 64) reinterpret_cast<float*>(&sv[buf][0][0])[tid] = to_f32<TX>(nv);
+    if (wave == 2 && RULE != 2 && lane < TB) reinterpret_cast<float*>(&sx[buf][0])[lane] = nx;
+    if (wave == 3 && !ROWS && lane < TB) reinterpret_cast<float*>(&sh[buf][0])[lane] = nx;
+    __syncthreads();
+  };
+  struct Rows { float q[RL], k[RL], d[RL], x; };         // (x: RULE 0's number, which goes to the output)
+  struct Numbers { float v[4], x[4], h[4]; };   // of four tokens: the column's value, the delta rules' number and (RULE 3) decay
+  auto read_rows = [&](int buf, int j, float (&to)[RL], int kind) {
+    const float* f = reinterpret_cast<const float*>(&rows[buf][kind][0]) + j * NR + walk_place<NR, RG>(rg, 0);
+#pragma unroll
+    for (int i = 0; i < RL; ++i) to[i] = f[walk_place<NR, RG>(0, i)];
+  };
+  auto read_x = [&](int buf, int j) { return RULE == 0 ? reinterpret_cast<const float*>(&sx[buf][0])[j] : 0.f; };
+  auto read_numbers = [&](int buf, int g, Numbers& o) {
+    const f32x4 v = sv[buf][lane / RG][g];
+    f32x4 x = {0.f, 0.f, 0.f, 0.f}, hh = x;
+    if (DELTA) x = sx[buf][g];           // (a register of a read that nobody uses is given away at once, and its next owner waits for the read)
+    if (!ROWS) hh = sh[buf][g];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { o.v[i] = v[i]; o.x[i] = x[i]; o.h[i] = hh[i]; }
+  };
+  auto exchange = [&](float y, int step) {
+    return y + (step == 0 ? dpp_f<0xB1>(y) : step == 1 ? dpp_f<0x4E>(y) : step == 2 ? dpp_f<0x124>(y) : dpp_f<0x128>(y));
+  };
+  // One token: the state behind it and, where this wave is to give it, the lane's part of its output. `beside(step)` is what
+  // is issued in front of the exchanges of the delta rules' sum, each of which waits for the one before it.
+  auto token = [&](const Rows& o, float v, float x, float hd, bool reads_out, auto beside) {
+    float y = 0.f;
+    if (!DELTA) {
+      beside(0); beside(1); beside(2); beside(3);
+#pragma unroll
+      for (int i = 0; i < RL; ++i) {
+        if (RULE == 0 && reads_out) y = fmaf(o.q[i], S[i], y);
+        S[i] = fmaf(o.d[i], S[i], o.k[i] * v);
+        if (RULE == 2 && reads_out) y = fmaf(o.q[i], S[i], y);
+      }
+    } else {
+      float dot = 0.f;
+#pragma unroll
+      for (int i = 0; i < RL; ++i) {
+        S[i] *= ROWS ? o.d[i] : hd;
+        dot = fmaf(S[i], o.k[i], dot);
+      }
+#pragma unroll
+      for (int step = 0; step < 4; ++step) {
+        __builtin_amdgcn_sched_barrier(0);
+        beside(step);
+        __builtin_amdgcn_sched_barrier(0);
+        dot = exchange(dot, step);
+      }
+      const float u = x * (v - dot);
+#pragma unroll
+      for (int i = 0; i < RL; ++i) {
+        S[i] = fmaf(o.k[i], u, S[i]);
+        if (reads_out) y = fmaf(S[i], o.q[i], y);
+      }
+    }
+    return y;
+  };
+  float* out = a.y + first * (int64_t)(a.H * a.P) + h * a.P;
+  int t0 = 0, buf = 0;
+  request(0, 0);
+  arrive(0);
+  request(TB, 1);
+  auto walk = [&](auto which) {                  // the whole batches; this wave gives the outputs of tokens ME, ME + W, ... of each
+    constexpr int ME = decltype(which)::value;
+    if (TB > n_tok) return;
+    Rows o[AHEAD + 1];
+    constexpr int NUMS = AHEAD <= 4 ? 2 : 4;     // groups of four tokens whose numbers are held
+    Numbers num[NUMS];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) {
+      read_rows(0, j, o[j].k, 1);
+      if (ROWS) read_rows(0, j, o[j].d, 2);
+      if (j % W == ME) read_rows(0, j, o[j].q, 0), o[j].x = read_x(0, j);
+    }
+#pragma unroll
+    for (int g = 0; 4 * g < AHEAD; ++g) read_numbers(0, g, num[g]);
+    const uint32_t to_mine = (uint32_t)((ME + W * rg) * (a.H * a.P) + p);
+    for (; t0 + TB <= n_tok; t0 += TB, buf ^= 1) {
+      float y[4], part = 0.f;
+#pragma unroll
+      for (int j = 0; j < TB; ++j) {
+        if (j == TB - AHEAD) {                   // from here on the next batch is read
+          arrive(buf ^ 1);
+          request(t0 + 2 * TB, buf);
+        }
+        const int from = j + AHEAD < TB ? buf : buf ^ 1, jn = (j + AHEAD) % TB;
+        Rows& next = o[(j + AHEAD) % (AHEAD + 1)];
+        const bool waits = DELTA && j % 16 > 0 && (j - 1) % W == ME;     // an output whose exchanges go beside this token's
+        const Numbers& n = num[j / 4 % NUMS];
+        const float yj = token(o[j % (AHEAD + 1)], n.v[j % 4], n.x[j % 4], n.h[j % 4], j % W == ME, [&](int step) {
+          if (step == 1) read_rows(from, jn, next.k, 1);
+          if (step == 2 && ROWS) read_rows(from, jn, next.d, 2);
+          if (step == 3 && jn % W == ME) read_rows(from, jn, next.q, 0), next.x = read_x(from, jn);
+          if (step == (ROWS ? 3 : 2) && jn % 4 == 0) read_numbers(from, jn / 4, num[(j + AHEAD) / 4 % NUMS]);
+          asm volatile("" ::: "memory");         // the reads stay here (the compiler would sink them to where they are used)
+          if (waits) part = exchange(part, step);
+        });
+        if (waits) y[(j - 1) / W % 4] = part;
+        if (j % W == ME) {
+          part = yj;
+          if (!DELTA || j % 16 == 15) {
+            part = group_sum<RG>(part);
+            if (RULE == 0) part = fmaf(o[j % (AHEAD + 1)].x, n.v[j % 4], part);   // the token's own term: v_p * sum_n q_n bonus_n k_n
+            y[j / W % 4] = part;
+          }
+        }
+        // the first four lanes of a column hold the same bits (the others have added in another order): lane rg of them stores
+        // the wave's output rg of sixteen tokens
+        if (j % 16 == 15) {
+          float mine = y[0];
+#pragma unroll
+          for (int i = 1; i < 4; ++i) mine = rg == i ? y[i] : mine;
+          if (live && rg < 4) (out + (int64_t)(t0 + j - 15) * (a.H * a.P))[to_mine] = mine;
+        }
+      }
+    }
+  };
+  if (wave == 0) walk(std::integral_constant<int, 0>{});
+  else if (wave == 1) walk(std::integral_constant<int, 1>{});
+  else if (wave == 2) walk(std::integral_constant<int, 2>{});
+  else walk(std::integral_constant<int, 3>{});
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // no request outlives its workgroup's LDS
+  if (wave != 0) return;
+  // a last batch that is not whole, which lies in LDS: its outputs and the state behind it are the first wave's
+  for (int j = 0; t0 + j < n_tok; ++j) {
+    Rows o;
+    read_rows(buf, j, o.q, 0);
+    read_rows(buf, j, o.k, 1);
+    if (ROWS) read_rows(buf, j, o.d, 2);
+    const float v = reinterpret_cast<const float*>(&sv[buf][lane / RG][0])[j];
+    const float x = RULE == 2 ? 0.f : reinterpret_cast<const float*>(&sx[buf][0])[j];
+    const float hd = ROWS ? 0.f : reinterpret_cast<const float*>(&sh[buf][0])[j];
+    float y = group_sum<RG>(token(o, v, x, hd, true, [](int) {}));
+    if (RULE == 0) y = fmaf(x, v, y);
+    if (live && rg == 0) (out + (int64_t)(t0 + j) * (a.H * a.P))[p] = y;
+  }
+  if (live) {
+#pragma unroll
+    for (int i = 0; i < RL; ++i)
+      if (i * RG + rg < a.N) srow[(int64_t)(i * RG + rg) * a.P + p] = S[i];
+  }
+}
+
+// Workgroups up to which four waves share the walk of a column group: as many as are in flight at once by their LDS and registers, three
+// to a compute unit up to 64 rows, two of 128. us with the kernel that shapes the values, requests of 1,100 tokens, one wave / four, bonus and
+// delta rule: 64 rows, 512 workgroups 122 / 94 and 162 / 140, 768 146 / 126 and 185 / 185, 832 157 / 157 and 193 / 228; 128 rows, 256
+// workgroups 150 / 104 and 179 / 139, 384 167 / 134 and 197 / 181, 512 169 / 144 and 202 / 199, 576 197 / 206 and 242 / 276. With 256 rows
+// the batches' LDS leaves no room for longer ones, and without them four waves gain nothing (624 / 650).
+template <int NR> constexpr unsigned dr_shared_max() { return NR <= 64 ? 768 : NR <= 128 ? 512 : 0; }
 template <typename TX, int NR, int RG, bool PRE>
 static void launch_decay_rows(const DrArgs& a, int rule, int num_seqs, int64_t T, float* pre, hipStream_t stream) {
   constexpr int PC = 64 / RG;
@@ -935,10 +1150,10 @@ static void launch_decay_rows(const DrArgs& a, int rule, int num_seqs, int64_t T
 #define DR_RULE(R)                                                                       \
   do {                                                                                   \
     decay_prepare_kernel<TX, NR, R><<<pgrid, block, 0, stream>>>(a, RG, pq, pk, pd, px); \
-    constexpr bool SHARES = RG == 16 && dr_shared_max<NR, R>() > 0;                      \
-    if (SHARES && grid.x <= dr_shared_max<NR, R>())                                      \
-      decay_walk_kernel<TX, NR, RG, R, SHARES ? 4 : 1><<<grid, 256, 0, stream>>>(a, pq, pk, pd, px); \
-    else decay_walk_kernel<TX, NR, RG, R, 1><<<grid, block, 0, stream>>>(a, pq, pk, pd, px); \
+    constexpr bool SHARES = RG == 16 && dr_shared_max<NR>() > 0;                         \
+    const bool shared = SHARES && grid.x <= dr_shared_max<NR>() && (int64_t)a.H * a.P < (1 << 27);  \
+    if constexpr (SHARES) { if (shared) decay_walk_shared_kernel<TX, NR, R><<<grid, 256, 0, stream>>>(a, pq, pk, pd, px); } \
+    if (!shared) decay_walk_kernel<TX, NR, RG, R><<<grid, block, 0, stream>>>(a, pq, pk, pd, px);  \
   } while (0)
     if (rule == 0) DR_RULE(0); else if (rule == 1) DR_RULE(1); else if (rule == 2) DR_RULE(2); else DR_RULE(3);
 #undef DR_RULE

@@ -81,3 +81,34 @@ def test_waves_that_share_a_walk(H, N, P, count, rule):
             state = start.clone()
             assert torch.equal(run(lo, lo + n, [i], [n], state), y[lo:lo + n]) and torch.equal(state[i], together[i])
         lo += n
+
+
+@pytest.mark.parametrize("T", [15, 16, 31, 32, 63, 64, 97, 128])
+@pytest.mark.parametrize("N,rule", [(32, "bonus"), (64, "delta"), (64, "gated"), (128, "delta"), (128, "delta_head"), (100, "bonus")])
+def test_whole_batches_of_the_shared_walk(monkeypatch, N, rule, T):
+    """Requests that end with a batch of the four waves, just before or behind one, the one behind them read ahead: the same bits as in
+    pieces of seven tokens, none of which holds a whole batch, and as beside so many requests that one wave walks alone."""
+    monkeypatch.setattr(ops, "decay_row_groups", lambda *a: (16, True))
+    g = torch.Generator(device=DEV).manual_seed(N + T)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    H, P, crowd = 2, 64, 26
+    wide = H if rule == "delta_head" else H * N
+    q, k, v, raw, beta = (rnd(T, n).to(torch.bfloat16) for n in (H * N, H * N, H * P, wide, H))
+    kw = dict(base=rnd(wide) - 1)
+    kw.update(dict(bonus=rnd(wide)) if rule == "bonus" else dict(rate=rnd(H).abs() + 0.1))
+    if rule.startswith("delta"):
+        kw.update(unit_eps=1e-6, q_scale=N ** -0.5)
+    start = rnd(1, H * N * P)
+
+    def run(rows, state):
+        lens = [r.shape[0] for r in rows]
+        at = torch.cat(rows)
+        more = dict(kw, beta=beta[at]) if rule.startswith("delta") else kw
+        return hip().decay_rows_recurrence(q[at], k[at], v[at], raw[at], state, torch.arange(len(rows), dtype=torch.int32, device=DEV),
+                                           torch.tensor([0] + lens, dtype=torch.int32, device=DEV).cumsum(0, dtype=torch.int32), lens, H, H, N, P, rule, **more)
+
+    every = torch.arange(T, device=DEV)
+    whole, pieces, many = start.clone(), start.clone(), start.repeat(crowd, 1)
+    y = run([every], whole)
+    assert torch.equal(torch.cat([run([every[lo:lo + 7]], pieces) for lo in range(0, T, 7)]), y) and torch.equal(pieces, whole)
+    assert torch.equal(run([every] * crowd, many).view(crowd, T, H * P), y.expand(crowd, T, H * P)) and torch.equal(many, whole.expand(crowd, -1))
