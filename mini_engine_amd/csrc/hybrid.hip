@@ -675,8 +675,8 @@ __global__ void __launch_bounds__(64) decay_rows_kernel(DrArgs a) {
 // and the output sum of a token overlap the next token's reads and updates, and shared values are brought in 16-byte pieces that
 // go to LDS as they are. The sums are those of decay_rows_kernel in the same order.
 template <typename TX, int NR, int RG, int RULE>
-__global__ void __launch_bounds__(64) decay_walk_kernel(DrArgs a, const float* __restrict__ pre_q, const float* __restrict__ pre_k,
-                                                        const float* __restrict__ pre_d, const float* __restrict__ pre_x) {
+__device__ __forceinline__ void walk_alone(const DrArgs& a, const float* __restrict__ pre_q, const float* __restrict__ pre_k,
+                                           const float* __restrict__ pre_d, const float* __restrict__ pre_x) {
   constexpr int TB = DR_TB;
   constexpr int AHEAD = NR <= 64 ? 3 : NR <= 128 ? 2 : 1;    // tokens whose shared values are read from LDS ahead
   constexpr int PC = 64 / RG;            // columns per wave
@@ -927,8 +927,8 @@ __device__ __forceinline__ void walk_request(uint32_t lds_addr, uint32_t voff, c
 // 150 -> 134 (one wave to a column group 344 and 230). Up to 64 rows batches of 32 tokens, held to the registers that let three workgroups onto a
 // compute unit (768 workgroups of 1,100 tokens 141 -> 130 us, 512 132 -> 135).
 template <typename TX, int NR, int RULE>
-__global__ void __launch_bounds__(256, NR <= 64 ? 3 : 2) decay_walk_shared_kernel(DrArgs a, const float* __restrict__ pre_q, const float* __restrict__ pre_k,
-                                                                const float* __restrict__ pre_d, const float* __restrict__ pre_x) {
+__device__ __forceinline__ void walk_shared(const DrArgs& a, const float* __restrict__ pre_q, const float* __restrict__ pre_k,
+                                            const float* __restrict__ pre_d, const float* __restrict__ pre_x) {
   constexpr int RG = 16, W = 4, PC = 4, RL = NR / RG;
   constexpr int TB = NR <= 64 ? 32 : 16;      // tokens of a batch
   constexpr int AHEAD = 7;               // tokens whose shared values are read from LDS ahead
@@ -1056,16 +1056,14 @@ __global__ void __launch_bounds__(256, NR <= 64 ? 3 : 2) decay_walk_shared_kerne
     constexpr int ME = decltype(which)::value;
     if (TB > n_tok) return;
     Rows o[AHEAD + 1];
-    constexpr int NUMS = AHEAD <= 4 ? 2 : 4;     // groups of four tokens whose numbers are held
-    Numbers num[NUMS];
+    Numbers num[2];                              // of the four tokens under way and the next four
 #pragma unroll
     for (int j = 0; j < AHEAD; ++j) {
       read_rows(0, j, o[j].k, 1);
       if (ROWS) read_rows(0, j, o[j].d, 2);
       if (j % W == ME) read_rows(0, j, o[j].q, 0), o[j].x = read_x(0, j);
     }
-#pragma unroll
-    for (int g = 0; 4 * g < AHEAD; ++g) read_numbers(0, g, num[g]);
+    read_numbers(0, 0, num[0]);
     const uint32_t to_mine = (uint32_t)((ME + W * rg) * (a.H * a.P) + p);
     for (; t0 + TB <= n_tok; t0 += TB, buf ^= 1) {
       float y[4], part = 0.f;
@@ -1078,12 +1076,12 @@ __global__ void __launch_bounds__(256, NR <= 64 ? 3 : 2) decay_walk_shared_kerne
         const int from = j + AHEAD < TB ? buf : buf ^ 1, jn = (j + AHEAD) % TB;
         Rows& next = o[(j + AHEAD) % (AHEAD + 1)];
         const bool waits = DELTA && j % 16 > 0 && (j - 1) % W == ME;     // an output whose exchanges go beside this token's
-        const Numbers& n = num[j / 4 % NUMS];
+        const Numbers& n = num[j / 4 % 2];
         const float yj = token(o[j % (AHEAD + 1)], n.v[j % 4], n.x[j % 4], n.h[j % 4], j % W == ME, [&](int step) {
           if (step == 1) read_rows(from, jn, next.k, 1);
           if (step == 2 && ROWS) read_rows(from, jn, next.d, 2);
           if (step == 3 && jn % W == ME) read_rows(from, jn, next.q, 0), next.x = read_x(from, jn);
-          if (step == (ROWS ? 3 : 2) && jn % 4 == 0) read_numbers(from, jn / 4, num[(j + AHEAD) / 4 % NUMS]);
+          if (step == (ROWS ? 3 : 2) && j % 4 == 0) read_numbers(j + 4 < TB ? buf : buf ^ 1, (j / 4 + 1) % (TB / 4), num[(j / 4 + 1) % 2]);
           asm volatile("" ::: "memory");         // the reads stay here (the compiler would sink them to where they are used)
           if (waits) part = exchange(part, step);
         });
@@ -1133,6 +1131,14 @@ __global__ void __launch_bounds__(256, NR <= 64 ? 3 : 2) decay_walk_shared_kerne
   }
 }
 
+// W: the waves that hold a column group, one or four.
+template <typename TX, int NR, int RG, int RULE, int W>
+__global__ void __launch_bounds__(64 * W, W == 1 ? 1 : NR <= 64 ? 3 : 2) decay_walk_kernel(DrArgs a, const float* __restrict__ pre_q, const float* __restrict__ pre_k,
+                                                                                           const float* __restrict__ pre_d, const float* __restrict__ pre_x) {
+  if constexpr (W == 1) walk_alone<TX, NR, RG, RULE>(a, pre_q, pre_k, pre_d, pre_x);
+  else walk_shared<TX, NR, RULE>(a, pre_q, pre_k, pre_d, pre_x);
+}
+
 // Workgroups up to which four waves share the walk of a column group: as many as are in flight at once by their LDS and registers, three
 // to a compute unit up to 64 rows, two of 128. us with the kernel that shapes the values, requests of 1,100 tokens, one wave / four, bonus and
 // delta rule: 64 rows, 512 workgroups 122 / 94 and 162 / 140, 768 146 / 126 and 185 / 185, 832 157 / 157 and 193 / 228; 128 rows, 256
@@ -1151,9 +1157,9 @@ static void launch_decay_rows(const DrArgs& a, int rule, int num_seqs, int64_t T
   do {                                                                                   \
     decay_prepare_kernel<TX, NR, R><<<pgrid, block, 0, stream>>>(a, RG, pq, pk, pd, px); \
     constexpr bool SHARES = RG == 16 && dr_shared_max<NR>() > 0;                         \
-    const bool shared = SHARES && grid.x <= dr_shared_max<NR>() && (int64_t)a.H * a.P < (1 << 27);  \
-    if constexpr (SHARES) { if (shared) decay_walk_shared_kernel<TX, NR, R><<<grid, 256, 0, stream>>>(a, pq, pk, pd, px); } \
-    if (!shared) decay_walk_kernel<TX, NR, RG, R><<<grid, block, 0, stream>>>(a, pq, pk, pd, px);  \
+    if (SHARES && grid.x <= dr_shared_max<NR>() && (int64_t)a.H * a.P < (1 << 27))       \
+      decay_walk_kernel<TX, NR, RG, R, SHARES ? 4 : 1><<<grid, SHARES ? 256 : 64, 0, stream>>>(a, pq, pk, pd, px); \
+    else decay_walk_kernel<TX, NR, RG, R, 1><<<grid, block, 0, stream>>>(a, pq, pk, pd, px); \
   } while (0)
     if (rule == 0) DR_RULE(0); else if (rule == 1) DR_RULE(1); else if (rule == 2) DR_RULE(2); else DR_RULE(3);
 #undef DR_RULE
