@@ -202,11 +202,14 @@ class GatedDelta(Mixer):
         blocks["a" if decay_rank is None else "a1"] = num_heads if decay_rank is None else decay_rank
         if gate_rank is not None:
             blocks["g1"] = gate_rank
-        self.block_starts, at = {}, 0                       # block name -> its first row
+        # block name -> its first row as `finalize` lays the blocks out: the low-rank inputs' at whole steps of 8, so that the products
+        # that read them take views of the packed result (rows that start at whole steps of 16 bytes) and no copies
+        self.blocks, self.block_starts, at = blocks, {}, 0
         for name, size in blocks.items():
+            at = -(-at // 8) * 8 if name in ("a1", "g1") else at
             self.block_starts[name] = at
             at += size
-        self.add_child("in_proj", Linear(hidden_size, at, parts=blocks))
+        self.add_child("in_proj", Linear(hidden_size, sum(blocks.values()), parts=blocks))
         self.decay_rank, self.gate_rank = decay_rank, gate_rank
         self.add_param("conv_weight", ParamSpec((self.channels, taps), init=_taps, dtype="float32"))
         if decay_rank is not None:
@@ -227,8 +230,14 @@ class GatedDelta(Mixer):
         self.rate = torch.exp(self.A_log.float()).contiguous()
         self.wide_norm = self.norm_weight.float().repeat(self.num_heads).contiguous()
         w = self.in_proj.weight
-        if w.shape[0] % 8:                  # the packed rows in whole steps of 8: views of them keep 16-byte row strides
-            self.in_proj.weight = torch.cat((w, w.new_zeros(8 - w.shape[0] % 8, w.shape[1])), 0).contiguous()
+        if w.shape[0] == sum(self.blocks.values()):
+            # blocks at their starts, rows in whole steps of 8 (views of them keep 16-byte row strides), zeros between
+            rows = -(-(self.block_starts[next(reversed(self.blocks))] + next(reversed(self.blocks.values()))) // 8) * 8
+            if rows != w.shape[0]:
+                laid = w.new_zeros(rows, w.shape[1])
+                for name, block in zip(self.blocks, w.split(list(self.blocks.values()))):
+                    laid[self.block_starts[name]:self.block_starts[name] + block.shape[0]] = block
+                self.in_proj.weight = laid
 
     def forward(self, x, step, cache, state):
         H, G, N, P = self.num_heads, self.key_heads, self.key_dim, self.value_dim
