@@ -227,80 +227,132 @@ __device__ __forceinline__ void select_token(const float* __restrict__ logits, i
   }
 }
 
-// The largest of a wave's values, in every lane: rotations inside rows of 16 lanes, then the four rows' results (a maximum is the
+// A wave holds one token, an expert to a lane, or with LANES = 32 two of them, a half wave each. Of a token's lanes: the largest of
+// their values, in every lane: rotations inside rows of 16 lanes, then the rows' results (a maximum is the
 // same whatever the order; no trip through LDS).
-__device__ __forceinline__ float wave_largest(float v) {
+template <int LANES>
+__device__ __forceinline__ float lanes_largest(float v) {
   v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, true)));
   v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xF, 0xF, true)));
   v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xF, 0xF, true)));
   v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xF, 0xF, true)));
   const int i = __float_as_int(v);
-  return fmaxf(fmaxf(__int_as_float(__builtin_amdgcn_readlane(i, 0)), __int_as_float(__builtin_amdgcn_readlane(i, 16))),
-               fmaxf(__int_as_float(__builtin_amdgcn_readlane(i, 32)), __int_as_float(__builtin_amdgcn_readlane(i, 48))));
+  const float low = fmaxf(__int_as_float(__builtin_amdgcn_readlane(i, 0)), __int_as_float(__builtin_amdgcn_readlane(i, 16)));
+  const float high = fmaxf(__int_as_float(__builtin_amdgcn_readlane(i, 32)), __int_as_float(__builtin_amdgcn_readlane(i, 48)));
+  return LANES == 64 ? fmaxf(low, high) : (threadIdx.x & 32) ? high : low;
+}
+// ... their sum, as wave_sum adds (a second half wave of zeros changes nothing there)
+template <int LANES>
+__device__ __forceinline__ float lanes_sum(float v) {
+#pragma unroll
+  for (int off = LANES / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, ME_WAVE);
+  return v;
+}
+// ... which of them say yes
+template <int LANES>
+__device__ __forceinline__ unsigned long long lanes_ballot(bool yes) {
+  const unsigned long long all = __ballot(yes);
+  return LANES == 64 ? all : (threadIdx.x & 32) ? all >> 32 : all & 0xffffffffull;
+}
+// The largest of `per` neighbouring lanes (2, 4, 8 or 16 of them, aligned), in each of them.
+__device__ __forceinline__ float group_largest(float v, int per) {
+  if (per >= 2) v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true)));     // quad_perm [1, 0, 3, 2]
+  if (per >= 4) v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, true)));     // quad_perm [2, 3, 0, 1]
+  if (per >= 8) v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, true)));    // row_half_mirror
+  if (per >= 16) v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, true)));   // row_mirror
+  return v;
 }
 
-// select_token for up to 64 experts, one to a lane: scores stay in registers, and a race's winner is the lowest lane that holds
-// the wave's largest value. The same choice and the same weights; `x`: the token's logit of expert `lane`. chosen: where
-// the ids also go in LDS, or null.
-__device__ __forceinline__ void select_token64(float x, int64_t t, int E, const RouteRule& r, int32_t* __restrict__ ids,
-                                               float* __restrict__ weights, int32_t* chosen) {
-  const int lane = threadIdx.x & 63;
+// select_token for up to LANES experts, one to a lane: scores stay in registers, and a race's winner is the lowest lane that holds
+// the largest value. The same choice and the same weights; `x`: the token's logit of the lane's expert. live: whether there is a
+// token here. chosen: where the ids also go in LDS, or null.
+template <int LANES>
+__device__ __forceinline__ void select_lanes(float x, int64_t t, bool live, int E, const RouteRule& r, int32_t* __restrict__ ids,
+                                             float* __restrict__ weights, int32_t* chosen) {
+  const int lane = threadIdx.x & (LANES - 1), first = threadIdx.x & (63 & ~(LANES - 1));     // first: the token's first lane
   const bool on = lane < E;
   const int per = E / r.group_count;
   float s = x;
   if (r.sigmoid == 1) {
     s = 1.0f / (1.0f + expf(-x));
   } else if (r.sigmoid == 0) {
-    const float hi = wave_largest(on ? x : -INFINITY);
+    const float hi = lanes_largest<LANES>(on ? x : -INFINITY);
     const float p = on ? expf(x - hi) : 0.f;
-    s = p / wave_sum(p);
+    s = p / lanes_sum<LANES>(p);
   }
   float m = on ? (r.correction ? s + r.correction[lane] : s) : -INFINITY;
   if (r.group_count > 1 && r.group_keep < r.group_count) {
     const int count = r.group_top < per ? r.group_top : per;
-    const bool group = lane < r.group_count;
-    float total = 0.f, pv = INFINITY;
-    int pi = -1;
-    bool more = true;
-    for (int c = 0; c < count; ++c) {
-      float bv = -INFINITY;
-      int bi = -1;
-      for (int j = 0; j < per; ++j) {
-        const float v = __shfl(m, group ? lane * per + j : 0, ME_WAVE);
-        const bool behind = v < pv || (v == pv && j > pi);
-        if (behind && (bi < 0 || v > bv)) { bv = v; bi = j; }
+    if (per <= 16 && (per & (per - 1)) == 0) {         // a group's lanes meet in exchanges inside a row; each holds what it comes to
+      const int shift = __builtin_ctz(per), base = lane >> shift << shift;
+      float total = 0.f;
+      bool race = on && m == m;                        // (what is no number is in no race)
+      for (int c = 0; c < count; ++c) {
+        const float best = group_largest(race ? m : -INFINITY, per);
+        const uint32_t in = (uint32_t)(lanes_ballot<LANES>(race && m == best) >> base) & ((1u << per) - 1u);
+        if (in) total += best;
+        if (in && lane == base + __ffs(in) - 1) race = false;
       }
-      more = more && bi >= 0;
-      if (more) { total += bv; pv = bv; pi = bi; }
+      bool kept = on && total == INFINITY;
+      for (int k = 0; k < r.group_keep; ++k) {
+        const float hi = lanes_largest<LANES>(on && !kept ? total : -INFINITY);
+        const unsigned long long best = lanes_ballot<LANES>(on && !kept && total == hi);
+        if (lane >> shift == (best ? (__ffsll(best) - 1) >> shift : 0)) kept = true;
+      }
+      if (on && !kept) m = -INFINITY;
+    } else {
+      const bool group = lane < r.group_count;
+      float total = 0.f, pv = INFINITY;
+      int pi = -1;
+      bool more = true;
+      for (int c = 0; c < count; ++c) {
+        float bv = -INFINITY;
+        int bi = -1;
+        for (int j = 0; j < per; ++j) {
+          const float v = __shfl(m, first + (group ? lane * per + j : 0), ME_WAVE);
+          const bool behind = v < pv || (v == pv && j > pi);
+          if (behind && (bi < 0 || v > bv)) { bv = v; bi = j; }
+        }
+        more = more && bi >= 0;
+        if (more) { total += bv; pv = bv; pi = bi; }
+      }
+      bool kept = group && total == INFINITY;
+      for (int k = 0; k < r.group_keep; ++k) {
+        const float hi = lanes_largest<LANES>(group && !kept ? total : -INFINITY);
+        const unsigned long long best = lanes_ballot<LANES>(group && !kept && total == hi);
+        if (lane == (best ? __ffsll(best) - 1 : 0)) kept = true;
+      }
+      const unsigned long long in = lanes_ballot<LANES>(kept);
+      if (on && !((in >> (lane / per)) & 1)) m = -INFINITY;
     }
-    bool kept = group && total == INFINITY;
-    for (int k = 0; k < r.group_keep; ++k) {
-      const float hi = wave_largest(group && !kept ? total : -INFINITY);
-      const unsigned long long best = __ballot(group && !kept && total == hi);
-      if (lane == (best ? __ffsll(best) - 1 : 0)) kept = true;
-    }
-    const unsigned long long in = __ballot(kept);
-    if (on && !((in >> (lane / per)) & 1)) m = -INFINITY;
   }
   float total = 0.f;
   int mine = 0;              // lane j keeps the j-th choice
   for (int j = 0; j < r.top; ++j) {
-    const float hi = wave_largest(m > -INFINITY ? m : -INFINITY);
+    const float hi = lanes_largest<LANES>(m > -INFINITY ? m : -INFINITY);
     const unsigned long long best = __ballot(m > -INFINITY && m == hi);
-    const int bi = best ? __ffsll(best) - 1 : 0;
+    int bi;
+    if (LANES == 64) {
+      bi = best ? __ffsll(best) - 1 : 0;
+      total += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), bi));
+    } else {                 // both halves' winners, the same in all lanes
+      const int low = (uint32_t)best ? __ffs((uint32_t)best) - 1 : 0, high = (uint32_t)(best >> 32) ? __ffs((uint32_t)(best >> 32)) - 1 : 0;
+      const float s_low = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), low)), s_high = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), 32 + high));
+      bi = first ? high : low;
+      total += first ? s_high : s_low;
+    }
     if (lane == bi) m = -INFINITY;
     if (lane == j) mine = bi;
-    total += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), bi));
   }
-  const float sm = __shfl(s, mine, ME_WAVE);
+  const float sm = __shfl(s, first + mine, ME_WAVE);
   float weight = r.normalise ? sm / (total + 1e-20f) : sm;
   if (r.sigmoid == 2) {                    // softmax over the chosen logits
     const float z = lane < r.top ? sm : -INFINITY;
-    const float hi = wave_largest(z);
+    const float hi = lanes_largest<LANES>(z);
     const float p = lane < r.top ? expf(z - hi) : 0.f;
-    weight = p / wave_sum(p);
+    weight = p / lanes_sum<LANES>(p);
   }
-  if (lane < r.top) {
+  if (live && lane < r.top) {
     ids[t * r.top + lane] = mine;
     weights[t * r.top + lane] = r.scale * weight;
     if (chosen != nullptr) chosen[t * r.top + lane] = mine;
@@ -316,7 +368,7 @@ moe_select_kernel(const float* __restrict__ logits, int64_t T, int E, RouteRule 
   const int64_t t = (int64_t)blockIdx.x * 4 + wave;
   if (t >= T) return;
   if (E <= 64) {
-    select_token64((threadIdx.x & 63) < E ? logits[t * E + (threadIdx.x & 63)] : 0.f, t, E, rule, ids, weights, nullptr);
+    select_lanes<64>((threadIdx.x & 63) < E ? logits[t * E + (threadIdx.x & 63)] : 0.f, t, true, E, rule, ids, weights, nullptr);
     return;
   }
   float* s = reinterpret_cast<float*>(route_lds) + (size_t)wave * (2 * E + rule.group_count);
@@ -405,12 +457,24 @@ moe_sort_kernel(int32_t* __restrict__ ids, int P, int routed, int E, int max_til
   const int32_t* pairs = ids;                        // where the pairs' ids are read
   if (logits && routed <= 64) {
     int32_t* chosen = P <= MOE_LDS_PAIRS ? reinterpret_cast<int32_t*>(route_lds) : nullptr;
-    const int T = P / rule.top, at = min(lane, routed - 1);
-    float next = wave < T ? logits[(int64_t)wave * routed + at] : 0.f;
-    for (int t = wave; t < T; t += waves) {
-      const float x = next;
-      if (t + waves < T) next = logits[(int64_t)(t + waves) * routed + at];
-      select_token64(x, t, routed, rule, ids, weights, chosen);
+    const int T = P / rule.top;
+    if (routed <= 32) {
+      const int at = min(lane & 31, routed - 1);
+      float next = logits[(int64_t)min(2 * wave + (lane >> 5), T - 1) * routed + at];
+      for (int t0 = 2 * wave; t0 < T; t0 += 2 * waves) {
+        const int t = t0 + (lane >> 5);
+        const float x = next;
+        next = logits[(int64_t)min(t + 2 * waves, T - 1) * routed + at];
+        select_lanes<32>(x, t, t < T, routed, rule, ids, weights, chosen);
+      }
+    } else {
+      const int at = min(lane, routed - 1);
+      float next = wave < T ? logits[(int64_t)wave * routed + at] : 0.f;
+      for (int t = wave; t < T; t += waves) {
+        const float x = next;
+        if (t + waves < T) next = logits[(int64_t)(t + waves) * routed + at];
+        select_lanes<64>(x, t, true, routed, rule, ids, weights, chosen);
+      }
     }
     if (chosen) pairs = chosen; else __threadfence_block();
   } else if (logits) {

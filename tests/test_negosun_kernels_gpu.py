@@ -154,3 +154,28 @@ def test_route_and_run_experts(E, top, count, keep, F, K):
         want = hip().routed_experts(x, ids, w, gate_up, down)
         assert torch.equal(got, want), f"T={T}: the fused choice differs from the separate one"
     assert ops.moe_sort_chooses(64, 256, 8) and not ops.moe_sort_chooses(65, 32, 1) and not ops.moe_sort_chooses(8, 512, 1)
+
+
+@pytest.mark.parametrize("kind,group_top", [("softmax", 1), ("sigmoid", 2), ("chosen", 3)])
+@pytest.mark.parametrize("E,top,count,keep", [(32, 4, 4, 2), (24, 3, 3, 2), (20, 4, 4, 2), (32, 6, 16, 5), (32, 8, 2, 1), (7, 7, 1, 1), (1, 1, 1, 1),
+                                              (64, 6, 4, 2), (33, 4, 3, 2), (48, 5, 24, 9)])
+def test_two_tokens_to_a_wave_choose_alike(E, top, count, keep, kind, group_top):
+    """Up to 32 experts the kernel that orders the pairs holds two tokens in a wave; groups of 2, 4, 8 or 16 meet in exchanges, others
+    in reads of other lanes. Logits that are small whole numbers, so that many are equal: ids as the plain reference chooses them, and
+    the same bits as by the kernel that only chooses."""
+    g = torch.Generator().manual_seed(E + top)
+    K = 64
+    router = torch.randint(-1, 2, (E, K), generator=g).float()
+    if kind == "chosen":                   # (the plain reference of this rule knows neither groups nor corrections)
+        count = keep = 1
+    correction = torch.randint(-2, 3, (E,), generator=g).float() / 4 if kind == "sigmoid" else None
+    rule = lambda device: ops.RouteRule(kind, None if correction is None else correction.to(device), group_top, kind == "sigmoid", 1.3)
+    gate_up, down = torch.randn(E, 16, K, device=DEV).bfloat16(), torch.randn(E, K, 8, device=DEV).bfloat16()
+    for T in (1, 2, 31, 33, 64):
+        x = torch.randint(0, 2, (T, K), generator=g) * (torch.rand(T, K, generator=g) < 0.1)
+        ids, w = hip().moe_route(x.to(DEV).bfloat16(), router.to(DEV), top, count, keep, rule(DEV))
+        want_ids, want_w = twin.moe_route(x.bfloat16(), router, top, count, keep, rule("cpu"))
+        assert torch.equal(ids.cpu(), want_ids.int())
+        close(w.cpu(), want_w, 1e-5)
+        got = hip().route_and_run_experts(x.to(DEV).bfloat16(), router.to(DEV), top, count, keep, gate_up, down, rule(DEV))
+        assert torch.equal(got, hip().routed_experts(x.to(DEV).bfloat16(), ids, w, gate_up, down, routed=E))
