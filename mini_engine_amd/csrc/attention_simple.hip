@@ -133,7 +133,8 @@ attn_simple_kernel(const T* __restrict__ q, int64_t q_stride, T* __restrict__ ou
 // products and sums), up to 16 tokens of one request and one head to a workgroup. attn_simple reads every key row and value row
 // once per token from a thread of its own; here they are read once per 16 tokens in pieces of 16 bytes, and what bounds a
 // workgroup is its chain of blocks (64 matrix instructions of 32 cycles for 16 keys at head size 128). A prompt of 300 tokens,
-// 16 heads of 128: 279 -> 25 us. A decoding row fills one of 16 columns, but reads its keys in pieces of 16 bytes with four waves
+// 16 heads of 128: 279 -> 25 us; with a workgroup for each request of a tile and no more (for each of its rows, most found nothing to do and held
+// 34 KB of LDS meanwhile), the longest tiles first, and what each wave counts worked out once a row, 23.3 -> 18.3, of 1,000 tokens 106 -> 72. A decoding row fills one of 16 columns, but reads its keys in pieces of 16 bytes with four waves
 // where attn_simple has a lane walk a key's row: one row over 60 / 512 / 4,096 keys 22 / 138 / 1,128 -> 8 / 21 / 136 us, 64 rows
 // over 300 / 2,048 keys 122 / 893 -> 55 / 300, a prompt of 16 tokens 10.0 -> 10.3. Larger heads would need more registers than a wave has and stay with attn_simple, as do
 // odd head sizes and pages.
@@ -145,25 +146,33 @@ attn_simple_kernel(const T* __restrict__ q, int64_t q_stride, T* __restrict__ ou
 // are, so a token's bits do not depend on the others of its tile, i.e. on how the request was cut.
 // Values of keys that a token does not see meet a probability of zero; where such a value is not a finite number it is
 // taken out of the product and joined by hand for the tokens that do see it.
+#define F32_WAVES 4
 template <int NS>        // head size / 16
-__global__ void __launch_bounds__(256, 2)       // two waves to a SIMD asked for: without it head size 96 took 276 registers and scratch, now 151
+__global__ void __launch_bounds__(64 * F32_WAVES, 2)       // two waves to a SIMD asked for: without it head size 96 took 276 registers and scratch, now 151
 attn_f32_kernel(const float* __restrict__ q, int64_t q_stride, float* __restrict__ out, int64_t out_stride,
                 const float* __restrict__ k_cache, const float* __restrict__ v_cache, const int32_t* __restrict__ block_tables,
                 int bt_stride, const int32_t* __restrict__ seq_of_token, const int32_t* __restrict__ positions,
                 const int32_t* __restrict__ context_lens, int num_tokens, int Hq, int Hkv, int page, float scale, int window,
                 int keep_first, float softcap, const float* __restrict__ sinks, const float* __restrict__ slopes) {
   constexpr int D = 16 * NS;
-  __shared__ float merge_acc[4][16][D + 4];
-  __shared__ float merge_m[4][16], merge_l[4][16];
-  // the workgroup's rows: from row blockIdx.z of a tile of 16, if a request's rows in the tile begin there, to the last of them
+  __shared__ float merge_acc[F32_WAVES][16][D + 4];
+  __shared__ float merge_m[F32_WAVES][16], merge_l[F32_WAVES][16], merge_a[F32_WAVES][16], merge_inv[16];
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int tile = blockIdx.x * 16, z = blockIdx.z, r0 = tile + z;
-  if (r0 >= num_tokens) return;
-  const int b = __builtin_amdgcn_readfirstlane(seq_of_token[r0]);
-  if (z > 0 && seq_of_token[r0 - 1] == b) return;
-  const bool mine = col < 16 - z && r0 + col < num_tokens && seq_of_token[min(r0 + col, num_tokens - 1)] == b;
-  const int h = blockIdx.y, kvh = h / (Hq / Hkv);
+  // heads side by side, the last tiles (a prompt's longest) first: what a compute unit takes beside one of them is short
+  const int h = blockIdx.x, tile = (gridDim.y - 1 - blockIdx.y) * 16;
+  // the tile's runs of rows of one request, by the row at which each begins; this workgroup takes every gridDim.z-th of them
+  const int at_row = tile + col;
+  const int whose = seq_of_token[min(at_row, num_tokens - 1)], before = seq_of_token[max(min(at_row, num_tokens - 1) - 1, 0)];
+  const uint32_t begins = (uint32_t)__ballot(at_row < num_tokens && (col == 0 || whose != before)) & 0xffffu;
+  const int in_tile = min(16, num_tokens - tile);
+  const int nth = (begins >> col & 1) ? __popc(begins & ((1u << col) - 1u)) : -1;          // the run that begins at this lane's row
+  for (int run = blockIdx.z; run < __popc(begins); run += gridDim.z) {
+  const int z = __builtin_ctzll(__ballot(nth == run)), r0 = tile + z;
+  const int rows = (begins >> (z + 1) ? z + 1 + __builtin_ctz(begins >> (z + 1)) : in_tile) - z;
+  const int b = __builtin_amdgcn_readlane(whose, z);
+  const bool mine = col < rows;
+  const int kvh = h / (Hq / Hkv);
   const int row = mine ? r0 + col : r0;
   const int32_t* bt = block_tables + (int64_t)b * bt_stride;
 
@@ -196,7 +205,7 @@ attn_f32_kernel(const float* __restrict__ q, int64_t q_stride, float* __restrict
 
   // this wave's next block of 16 keys at or behind kb (a multiple of 16 that is this wave's) in which some token sees a key
   auto next_block = [&](int kb) {
-    if (kb >= kept_most && kb + 16 <= lo_least) kb += ((lo_least - 16 - kb) / 64 + 1) * 64;
+    if (kb >= kept_most && kb + 16 <= lo_least) kb += ((lo_least - 16 - kb) / (16 * F32_WAVES) + 1) * (16 * F32_WAVES);
     return kb;
   };
   auto page_of = [&](int j) { return bt[min(j, hi_most - 1) / page]; };      // hi_most > 0 wherever this is asked
@@ -206,14 +215,14 @@ attn_f32_kernel(const float* __restrict__ q, int64_t q_stride, float* __restrict
 #pragma unroll
     for (int i = 0; i < NS; ++i) fk[i] = *reinterpret_cast<const f32x4*>(kr + 16 * i);
   };
-  int kb = next_block(16 * wave);
+  int kb = next_block(16 * wave);            // (block i of 16 keys belongs to wave i mod F32_WAVES)
   int pk = 0, pv = 0;
   if (kb < hi_most) {
     pk = page_of(kb + col); pv = page_of(kb + 4 * g);
     fetch_keys(kb, pk);
   }
   while (kb < hi_most) {
-    const int kn = next_block(kb + 64);
+    const int kn = next_block(kb + 16 * F32_WAVES);
     // four keys of a page lie side by side in every dimension's row of values; a group of four that begins behind the last
     // key any token sees is read from the last such group of the table's reach instead and zeroed below
     const int j0 = kb + 4 * g;
@@ -302,20 +311,28 @@ attn_f32_kernel(const float* __restrict__ q, int64_t q_stride, float* __restrict
 #pragma unroll
   for (int i = 0; i < NS; ++i) *reinterpret_cast<f32x4*>(&merge_acc[wave][col][16 * i + 4 * g]) = acc[i];
   __syncthreads();
-  for (int e = tid; e < 16 * D; e += 256) {
-    const int c = e / D, d = e % D;
-    if (c >= 16 - z || r0 + c >= num_tokens || seq_of_token[r0 + c] != b) continue;
+  if (tid < 16) {                                // what each wave's numbers count, once a row
     float top = sinks != nullptr ? sinks[h] : -INFINITY;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) top = fmaxf(top, merge_m[w][c]);
-    float sum = sinks != nullptr ? expf(sinks[h] - top) : 0.f, o = 0.f;
+    for (int w = 0; w < F32_WAVES; ++w) top = fmaxf(top, merge_m[w][tid]);
+    float sum = sinks != nullptr ? expf(sinks[h] - top) : 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const float a = merge_m[w][c] == -INFINITY ? 0.f : expf(merge_m[w][c] - top);
-      sum += a * merge_l[w][c];
-      o += a * merge_acc[w][c][d];
+    for (int w = 0; w < F32_WAVES; ++w) {
+      const float a = merge_m[w][tid] == -INFINITY ? 0.f : expf(merge_m[w][tid] - top);
+      sum += a * merge_l[w][tid];
+      merge_a[w][tid] = a;
     }
-    out[(int64_t)(r0 + c) * out_stride + (int64_t)h * D + d] = o * (sum > 0.f ? 1.f / sum : 0.f);
+    merge_inv[tid] = sum > 0.f ? 1.f / sum : 0.f;
+  }
+  __syncthreads();
+  for (int e = tid; e < rows * D; e += 64 * F32_WAVES) {
+    const int c = e / D, d = e % D;
+    float o = 0.f;
+#pragma unroll
+    for (int w = 0; w < F32_WAVES; ++w) o += merge_a[w][c] * merge_acc[w][c][d];
+    out[(int64_t)(r0 + c) * out_stride + (int64_t)h * D + d] = o * merge_inv[c];
+  }
+  if (run + gridDim.z < __popc(begins)) __syncthreads();       // the numbers in LDS have been read
   }
 }
 
@@ -323,7 +340,7 @@ extern "C" int me_attn_simple(const void* q, int64_t q_stride, void* out, int64_
                               const void* k_cache, const void* v_cache, const int32_t* block_tables,
                               int bt_stride, const int32_t* seq_of_token, const int32_t* positions,
                               const int32_t* context_lens, int64_t num_tokens, int Hq, int Hkv, int D, int page, float scale, int window,
-                              int keep_first, float softcap, const float* sinks, const float* slopes, hipStream_t stream) {
+                              int keep_first, float softcap, const float* sinks, const float* slopes, int num_seqs, hipStream_t stream) {
   if (num_tokens == 0) return 0;
   ME_CHECK(Hq >= 1 && Hkv >= 1 && Hq % Hkv == 0, "attention: %d query heads are not a multiple of %d key heads", Hq, Hkv);
   ME_CHECK(D >= 1 && D <= AS_CHANNELS * AS_THREADS, "attention (float32 path): head_dim %d outside 1..%d", D, AS_CHANNELS * AS_THREADS);
@@ -331,9 +348,9 @@ extern "C" int me_attn_simple(const void* q, int64_t q_stride, void* out, int64_
   ME_CHECK(keep_first >= 0 && softcap >= 0.f, "attention: keep_first and softcap must not be negative");
   dim3 grid(num_tokens, Hq), block(AS_THREADS);
   size_t lds = (size_t)(D + AS_THREADS) * sizeof(float);
-  if (dtype == ME_F32 && D % 16 == 0 && D <= 128 && page % 4 == 0 && num_tokens <= 2147483647ll - 16 && Hq <= 65535 &&
+  if (dtype == ME_F32 && D % 16 == 0 && D <= 128 && page % 4 == 0 && num_tokens <= 65535 * 16 &&
       (uintptr_t)k_cache % 16 == 0 && (uintptr_t)v_cache % 16 == 0) {
-    const dim3 tiles((unsigned)((num_tokens + 15) / 16), Hq, 16);
+    const dim3 tiles(Hq, (unsigned)((num_tokens + 15) / 16), num_seqs < 1 ? 1 : num_seqs < 16 ? num_seqs : 16), block(64 * F32_WAVES);
 #define AS_F32(NS) case NS: attn_f32_kernel<NS><<<tiles, block, 0, stream>>>((const float*)q, q_stride, (float*)out, out_stride,          \
         (const float*)k_cache, (const float*)v_cache, block_tables, bt_stride, seq_of_token, positions, context_lens, (int)num_tokens, \
         Hq, Hkv, page, scale, window, keep_first, softcap, sinks, slopes); break

@@ -86,7 +86,7 @@ _CORE_PROTOS = {
     "me_gate_mul": [P, L, P, F, F, P, I, L, I, P],
     "me_qk_norm_rope_store": [P, I, L, L, P, P, F, P, L, L, P, P, P, P, I, I, I, I, I, I, P],
     "me_store_kv": [P, P, I, L, L, L, P, P, P, I, I, I, P],
-    "me_attn_simple": [P, L, P, L, I, P, P, P, I, P, P, P, L, I, I, I, I, F, I, I, F, P, P, P],
+    "me_attn_simple": [P, L, P, L, I, P, P, P, I, P, P, P, L, I, I, I, I, F, I, I, F, P, P, I, P],
     "me_attn_tail": [P, L, P, L, P, I, P, P, P, I, P, P, P, L, I, I, I, I, F, I, I, F, P, P, P],
     "me_gemm_tiled": [P, L, P, L, P, L, I, I, I, I, P],
     "me_gemm_f32": [P, L, P, L, P, L, I, I, I, I, I, P],
@@ -521,7 +521,7 @@ class HipBackend:
             core().call("me_attn_simple", q.data_ptr(), q.stride(0), out.data_ptr(), out.stride(0), _code(q.dtype),
                         k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr(), block_tables.stride(0),
                         seq_of_token.data_ptr(), positions.data_ptr(), context_lens.data_ptr(), T, Hq, Hkv, D, page,
-                        float(scale), win, int(keep_first or 0), float(softcap or 0.0), _ptr(sinks), _ptr(slopes), _stream())
+                        float(scale), win, int(keep_first or 0), float(softcap or 0.0), _ptr(sinks), _ptr(slopes), context_lens.numel(), _stream())
             if head_gate is not None:
                 self.head_gate(out, head_gate, Hq, D)
             return out

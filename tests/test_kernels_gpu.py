@@ -499,6 +499,20 @@ def test_attention_prefill_segments_chosen_automatically():
         close(hip().paged_attention(*args, max_prefill_context=2500), twin.paged_attention(*args), 1.5e-2)
 
 
+@pytest.mark.parametrize("D", [16, 96, 128])
+@pytest.mark.parametrize("seqs", [[(300, 300)], [(40, 1)] * 17 + [(33, 7), (50, 50)], [(20, 20), (9, 2)], [(16, 16)] * 3, [(70, 3)] * 11])
+def test_float32_attention_takes_every_run_of_a_tile(seqs, D):
+    """A workgroup for each run of a request's rows in a tile of 16, at most as many as there are requests: prompts alone, single rows
+    beside prompts, several prompts in a tile; and rows in such an order that a tile holds more runs than there are requests, which
+    give the same bits."""
+    args = list(_attention_case(torch.float32, 6, 3, D, 16, seqs, window=25, seed=D))
+    got = hip().paged_attention(*args)
+    close(got, twin.paged_attention(*args), 1e-5)
+    order = torch.randperm(got.shape[0], generator=torch.Generator().manual_seed(D)).to(DEV)
+    args[0], args[6], args[7] = args[0][order].contiguous(), args[6][order].contiguous(), args[7][order].contiguous()
+    assert torch.equal(hip().paged_attention(*args), got[order])
+
+
 def test_attention_generic_path_takes_odd_sizes():
     """Head size 24 and page 5 are outside the matrix-core kernel: the generic kernel takes them."""
     for dtype in (torch.float32, torch.bfloat16):
