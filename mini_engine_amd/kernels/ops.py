@@ -2066,7 +2066,7 @@ SORT_CHOOSES_MAX_TOKENS = 64
 
 def moe_sort_chooses(T: int, E: int, group_count: int) -> bool:
     """Whether the kernel that orders the (token, choice) pairs also makes the choice: up to SORT_CHOOSES_MAX_TOKENS tokens
-    (its one workgroup takes them 16 at a time, a wave each) and as many experts as leave its 16 waves their scratch
+    (its one workgroup of 16 waves takes them 16 at a time, up to 32 experts 32) and as many experts as leave its 16 waves their scratch
     memory."""
     return T <= SORT_CHOOSES_MAX_TOKENS and 16 * (2 * E + group_count) * 4 <= 40 * 1024
 
