@@ -12,6 +12,7 @@ import hashlib
 import importlib.machinery
 import importlib.util
 import os
+import platform
 import shutil
 import subprocess
 import sys
@@ -206,7 +207,9 @@ def attention_library(head_dim: int, force: bool = False, score_cap: bool = Fals
 
 def calls_library(force: bool = False) -> str | None:
     """The Python module of csrc/calls.cpp, for the interpreter that runs; None where it is not built and cannot be (no compiler, no
-    headers of Python): the entry points are then called through ctypes."""
+    headers of Python, a machine with another calling convention)."""
+    if platform.machine() != "x86_64":
+        return None
     include = sysconfig.get_paths()["include"]
     extra = ["-x", "c++", "-I", include, "-DME_PYTHON=" + str(sysconfig.get_config_var("SOABI")).replace("-", "_")]
     digest = _hash([CALLS_SOURCE], extra)
@@ -220,13 +223,19 @@ def calls_library(force: bool = False) -> str | None:
 
 
 def calls_module():
-    path = calls_library()
-    if path is None:
+    """That module, loaded; None where there is none, where it does not compile or cannot be loaded (said once on stderr): the entry
+    points are then called through ctypes."""
+    try:
+        path = calls_library()
+        if path is None:
+            return None
+        loader = importlib.machinery.ExtensionFileLoader("me_calls", path)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("me_calls", loader))
+        loader.exec_module(module)
+        return module
+    except (BuildError, ImportError, OSError) as e:
+        _log(f"entry points are called through ctypes, without me_calls.so: {e}")
         return None
-    loader = importlib.machinery.ExtensionFileLoader("me_calls", path)
-    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("me_calls", loader))
-    loader.exec_module(module)
-    return module
 
 
 def build_all(head_dims=DEFAULT_HEAD_DIMS, force: bool = True) -> list:

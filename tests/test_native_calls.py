@@ -66,3 +66,36 @@ def test_what_is_no_plain_number_goes_to_ctypes(library):
             lib.call("me_mixed", *bad)
     with pytest.raises(KeyError):
         lib.call("me_unknown")
+
+
+@pytest.fixture()
+def fresh(monkeypatch, tmp_path):
+    """A folder of libraries of its own in which nothing is built, and no module kept from before."""
+    monkeypatch.setattr(build, "PKG_LIB", str(tmp_path / "lib"))
+    monkeypatch.setattr(build, "_fallback", str(tmp_path / "none"))
+    (tmp_path / "lib").mkdir()
+    ops._native_calls.cache_clear()
+    yield tmp_path
+    ops._native_calls.cache_clear()
+
+
+def _compiler(tmp_path, line):
+    path = tmp_path / "hipcc"
+    path.write_text(f"#!/bin/sh\n{line}\n")
+    path.chmod(0o755)
+    return str(path)
+
+
+@pytest.mark.parametrize("why", ["does not compile", "cannot be loaded", "another machine", "no compiler"])
+def test_without_the_module_the_entry_points_are_called_through_ctypes(monkeypatch, fresh, library, why):
+    if why == "another machine":
+        monkeypatch.setattr(build.platform, "machine", lambda: "aarch64")
+    # (what "links" writes is no library)
+    lines = {"does not compile": "echo no headers >&2; exit 1", "cannot be loaded": 'while [ $# -gt 1 ]; do [ "$1" = -o ] && echo x > "$2"; shift; done'}
+    monkeypatch.setattr(build, "hipcc_path", lambda: None if why == "no compiler" else _compiler(fresh, lines.get(why, "exit 1")))
+    assert build.calls_module() is None
+    lib = ops._Lib(library, PROTOS)
+    lib.call("me_none")
+    assert isinstance(lib.fns["me_none"], ctypes._CFuncPtr)
+    with pytest.raises(ops.KernelError, match="me_many: 0.5 0 9 1 7 -9"):
+        lib.call("me_many", 0.5, *range(10), 1.0, 2.0, 3.0, 4.0, 5.0, 6.0, 7.0, -9)
