@@ -1536,16 +1536,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     const std::true_type yes;
     const std::false_type no;
     const int end_full = full_hi >= seg_lo ? min(nblk, (full_hi - seg_lo) / 32 + 1) : 0;
-    int k = 0;
+    int k = 0, first_full = 0;
     if constexpr (WINDOW) {
-      const int first_full = full_lo > seg_lo ? min(end_full, (full_lo - seg_lo + 31) / 32) : 0;
+      first_full = full_lo > seg_lo ? min(end_full, (full_lo - seg_lo + 31) / 32) : 0;
       for (; k < min(first_full, nblk - 1); ++k) block_step(no, no, yes, k);
     }
     const int end_steady = min(end_full, min(nblk, (L - seg_lo) / 32) - PD);       // (a block behind the tile's first is always held)
     for (; k < end_steady; ++k) block_step(yes, yes, yes, k);
     for (; k < min(end_full, nblk - 1); ++k) block_step(yes, no, yes, k);
     for (; k < nblk - 1; ++k) block_step(no, no, yes, k);
-    block_step(no, no, no, k);
+    // (a segment's last block is mostly wholly visible: masked, a score that is no number would vanish there and nowhere else)
+    if (k >= first_full && k < end_full) block_step(yes, no, no, k); else block_step(no, no, no, k);
 
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {

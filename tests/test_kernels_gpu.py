@@ -490,6 +490,30 @@ def test_attention_prefill_pipelined_walk(monkeypatch, col_tiles, page, window):
         close(forms[0], twin.paged_attention(*args), 1.5e-2)
 
 
+@pytest.mark.parametrize("col_tiles", [1, 2])
+@pytest.mark.parametrize("segment,window", [(64, None), (96, None), (0, None), (64, 200), (0, 200)])
+def test_attention_prefill_shows_what_is_no_number(monkeypatch, col_tiles, segment, window):
+    """A key that is not a number, in a block in front of a segment's last, in the last one and in a tile's diagonal: the form
+    whose loads fill LDS themselves shows it in the same tokens as the one that stages through registers, whose segments' last blocks
+    are like any other, and in every token from a tile and a block behind the key on that sees it."""
+    monkeypatch.setattr(ops, "PREFILL_SEGMENT_KEYS", segment)
+    monkeypatch.setattr(ops, "prefill_col_tiles", lambda *a: col_tiles)
+    L, page, Hq, Hkv = 420, 16, 4, 2
+    for bad, value in ((10, float("nan")), (40, float("nan")), (95, float("nan")), (130, float("nan")), (191, float("inf")), (200, float("nan"))):
+        args = _attention_case(torch.bfloat16, Hq, Hkv, 128, page, [(L, L)], window=window, seed=bad)
+        args[1][int(args[4][0, bad // page]), 1, bad % page, 5] = value
+        forms = []
+        for form in (1, 2):
+            monkeypatch.setattr(ops, "PREFILL_THROUGH_LDS", form)
+            forms.append(hip().paged_attention(*args, max_prefill_context=L).view(L, Hq, 128))
+        assert torch.equal(torch.isnan(forms[0]), torch.isnan(forms[1]))
+        assert torch.equal(forms[0].nan_to_num(7.0), forms[1].nan_to_num(7.0))
+        # a tile is at most 64 tokens (128 columns of 2 heads), a block 32 keys: these tokens' waves see the key's block whole
+        behind = forms[0][bad + 64 + 32: L if window is None else bad + window - 64 - 32]
+        if value != value:
+            assert torch.isnan(behind[:, 2:]).all() and not torch.isnan(forms[0][:bad]).any() and not torch.isnan(forms[0][:, :2]).any()
+
+
 def test_attention_prefill_segments_chosen_automatically():
     """A short chunk at the end of a long context is cut by the engine's own rule."""
     seqs = [(2500, 33), (1100, 2)]
