@@ -147,37 +147,45 @@ attn_simple_kernel(const T* __restrict__ q, int64_t q_stride, T* __restrict__ ou
 // Values of keys that a token does not see meet a probability of zero; where such a value is not a finite number it is
 // taken out of the product and joined by hand for the tokens that do see it.
 #define F32_WAVES 4
-template <int NS>        // head size / 16
+template <int NS, bool MANY>        // NS: head size / 16; MANY: a tile may hold more runs of rows than workgroups are sent to it (a loop, which costs a single row 3 %)
 __global__ void __launch_bounds__(64 * F32_WAVES, 2)       // two waves to a SIMD asked for: without it head size 96 took 276 registers and scratch, now 151
 attn_f32_kernel(const float* __restrict__ q, int64_t q_stride, float* __restrict__ out, int64_t out_stride,
                 const float* __restrict__ k_cache, const float* __restrict__ v_cache, const int32_t* __restrict__ block_tables,
                 int bt_stride, const int32_t* __restrict__ seq_of_token, const int32_t* __restrict__ positions,
                 const int32_t* __restrict__ context_lens, int num_tokens, int Hq, int Hkv, int page, float scale, int window,
-                int keep_first, float softcap, const float* __restrict__ sinks, const float* __restrict__ slopes) {
+                int keep_first, float softcap, const float* __restrict__ sinks, const float* __restrict__ slopes, int runs) {
   constexpr int D = 16 * NS;
   __shared__ float merge_acc[F32_WAVES][16][D + 4];
   __shared__ float merge_m[F32_WAVES][16], merge_l[F32_WAVES][16], merge_a[F32_WAVES][16], merge_inv[16];
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // heads side by side, the last tiles (a prompt's longest) first: what a compute unit takes beside one of them is short
-  const int h = blockIdx.x, tile = (gridDim.y - 1 - blockIdx.y) * 16;
-  // the tile's runs of rows of one request, by the row at which each begins; this workgroup takes every gridDim.z-th of them
-  const int at_row = tile + col;
-  const int whose = seq_of_token[min(at_row, num_tokens - 1)], before = seq_of_token[max(min(at_row, num_tokens - 1) - 1, 0)];
+  // The heads of a key head, a tile and a run of its rows share keys: one such unit after the other goes to each XCD (consecutive
+  // workgroups go to the XCDs in turn; with all heads side by side those of a key head were on as many XCDs, 64 decoding rows over 2,048
+  // keys, 32 and 8 heads of 128, 580 us, now 430). The first tile, which holds the decoding rows, is asked for first, then the last tiles (a
+  // prompt's longest): what a compute unit takes beside one of them is short (5 decoding rows beside 200 tokens, 4 and 2 heads of 64, 13.5 -> 11.1 us).
+  const uint32_t tiles = (uint32_t)(num_tokens + 15) >> 4, unit = (blockIdx.z * 65535 + blockIdx.y) * 8 + (blockIdx.x & 7);
+  const uint32_t place = unit / (uint32_t)Hkv, first_run = place / tiles, rank = place - first_run * tiles;
+  if (first_run >= (uint32_t)runs) return;
+  const int kvh = unit - place * Hkv, h = kvh * (Hq / Hkv) + (blockIdx.x >> 3);
+  const int tile = (rank == 0 ? 0 : tiles - rank) * 16;
+  // the tile's runs of rows of one request, by the row at which each begins; this workgroup takes every `runs`-th of them
+  const int at_row = tile + col, here = min(at_row, num_tokens - 1);
+  const int whose = seq_of_token[here], before = seq_of_token[max(here - 1, 0)], where = positions[here];
   const uint32_t begins = (uint32_t)__ballot(at_row < num_tokens && (col == 0 || whose != before)) & 0xffffu;
   const int in_tile = min(16, num_tokens - tile);
   const int nth = (begins >> col & 1) ? __popc(begins & ((1u << col) - 1u)) : -1;          // the run that begins at this lane's row
-  for (int run = blockIdx.z; run < __popc(begins); run += gridDim.z) {
+  int run = first_run;
+  if (run >= __popc(begins)) return;
+  do {
   const int z = __builtin_ctzll(__ballot(nth == run)), r0 = tile + z;
   const int rows = (begins >> (z + 1) ? z + 1 + __builtin_ctz(begins >> (z + 1)) : in_tile) - z;
   const int b = __builtin_amdgcn_readlane(whose, z);
   const bool mine = col < rows;
-  const int kvh = h / (Hq / Hkv);
   const int row = mine ? r0 + col : r0;
   const int32_t* bt = block_tables + (int64_t)b * bt_stride;
 
   // what this lane's token sees, [lo, hi) and [0, kept) as in attn_simple, and the reach of the tile's tokens together
-  const int pos = positions[row];
+  const int pos = __shfl(where, mine ? z + col : z, ME_WAVE);
   const int hi = min(pos + 1, context_lens[b]);
   const int lo = window > 0 ? max(0, pos - window + 1) : (window < 0 ? pos - pos % (-window) : 0);
   const int kept = (window > 0 && keep_first > 0) ? min(min(keep_first, lo), hi) : 0;
@@ -311,29 +319,47 @@ attn_f32_kernel(const float* __restrict__ q, int64_t q_stride, float* __restrict
 #pragma unroll
   for (int i = 0; i < NS; ++i) *reinterpret_cast<f32x4*>(&merge_acc[wave][col][16 * i + 4 * g]) = acc[i];
   __syncthreads();
-  if (tid < 16) {                                // what each wave's numbers count, once a row
+  // what each wave's numbers count in a row
+  auto weigh = [&](int c, float (&count)[F32_WAVES]) {
     float top = sinks != nullptr ? sinks[h] : -INFINITY;
 #pragma unroll
-    for (int w = 0; w < F32_WAVES; ++w) top = fmaxf(top, merge_m[w][tid]);
+    for (int w = 0; w < F32_WAVES; ++w) top = fmaxf(top, merge_m[w][c]);
     float sum = sinks != nullptr ? expf(sinks[h] - top) : 0.f;
 #pragma unroll
     for (int w = 0; w < F32_WAVES; ++w) {
-      const float a = merge_m[w][tid] == -INFINITY ? 0.f : expf(merge_m[w][tid] - top);
-      sum += a * merge_l[w][tid];
-      merge_a[w][tid] = a;
+      count[w] = merge_m[w][c] == -INFINITY ? 0.f : expf(merge_m[w][c] - top);
+      sum += count[w] * merge_l[w][c];
     }
-    merge_inv[tid] = sum > 0.f ? 1.f / sum : 0.f;
-  }
-  __syncthreads();
-  for (int e = tid; e < rows * D; e += 64 * F32_WAVES) {
-    const int c = e / D, d = e % D;
+    return sum > 0.f ? 1.f / sum : 0.f;
+  };
+  auto put = [&](int c, int d, const float (&count)[F32_WAVES], float inv) {
     float o = 0.f;
 #pragma unroll
-    for (int w = 0; w < F32_WAVES; ++w) o += merge_a[w][c] * merge_acc[w][c][d];
-    out[(int64_t)(r0 + c) * out_stride + (int64_t)h * D + d] = o * merge_inv[c];
+    for (int w = 0; w < F32_WAVES; ++w) o += count[w] * merge_acc[w][c][d];
+    out[(int64_t)(r0 + c) * out_stride + (int64_t)h * D + d] = o * inv;
+  };
+  float count[F32_WAVES];
+  if (rows == 1) {                               // (a thread for every number: no second trip through LDS; 60 keys 6.3 -> 6.2 us)
+    const float inv = weigh(0, count);
+    if (tid < D) put(0, tid, count, inv);
+  } else {                                       // once a row
+    if (tid < 16) {
+      merge_inv[tid] = weigh(tid, count);
+#pragma unroll
+      for (int w = 0; w < F32_WAVES; ++w) merge_a[w][tid] = count[w];
+    }
+    __syncthreads();
+    for (int e = tid; e < rows * D; e += 64 * F32_WAVES) {
+      const int c = e / D;
+#pragma unroll
+      for (int w = 0; w < F32_WAVES; ++w) count[w] = merge_a[w][c];
+      put(c, e % D, count, merge_inv[c]);
+    }
   }
-  if (run + gridDim.z < __popc(begins)) __syncthreads();       // the numbers in LDS have been read
-  }
+  if (!MANY) return;
+  run += runs;
+  if (run < __popc(begins)) __syncthreads();       // the numbers in LDS have been read
+  } while (run < __popc(begins));
 }
 
 extern "C" int me_attn_simple(const void* q, int64_t q_stride, void* out, int64_t out_stride, int dtype,
@@ -348,14 +374,19 @@ extern "C" int me_attn_simple(const void* q, int64_t q_stride, void* out, int64_
   ME_CHECK(keep_first >= 0 && softcap >= 0.f, "attention: keep_first and softcap must not be negative");
   dim3 grid(num_tokens, Hq), block(AS_THREADS);
   size_t lds = (size_t)(D + AS_THREADS) * sizeof(float);
-  if (dtype == ME_F32 && D % 16 == 0 && D <= 128 && page % 4 == 0 && num_tokens <= 65535 * 16 &&
-      (uintptr_t)k_cache % 16 == 0 && (uintptr_t)v_cache % 16 == 0) {
-    const dim3 tiles(Hq, (unsigned)((num_tokens + 15) / 16), num_seqs < 1 ? 1 : num_seqs < 16 ? num_seqs : 16), block(64 * F32_WAVES);
-#define AS_F32(NS) case NS: attn_f32_kernel<NS><<<tiles, block, 0, stream>>>((const float*)q, q_stride, (float*)out, out_stride,          \
-        (const float*)k_cache, (const float*)v_cache, block_tables, bt_stride, seq_of_token, positions, context_lens, (int)num_tokens, \
-        Hq, Hkv, page, scale, window, keep_first, softcap, sinks, slopes); break
+  const int runs = num_seqs < 1 ? 1 : num_seqs < 16 ? num_seqs : 16;
+  const int64_t units = (num_tokens + 15) / 16 * runs * Hkv;           // see `attn_f32_kernel`
+  if (dtype == ME_F32 && D % 16 == 0 && D <= 128 && page % 4 == 0 && num_tokens <= 2147483647ll - 16 && units < (1ll << 31) &&
+      Hq / Hkv < (1 << 20) &&       (uintptr_t)k_cache % 16 == 0 && (uintptr_t)v_cache % 16 == 0) {
+    const int64_t eights = (units + 7) / 8;
+    const dim3 tiles((unsigned)(Hq / Hkv * 8), (unsigned)(eights < 65535 ? eights : 65535), (unsigned)((eights + 65534) / 65535)), block(64 * F32_WAVES);
+    const bool many = runs > 1 && runs < 16;
+#define AS_ARGS <<<tiles, block, 0, stream>>>((const float*)q, q_stride, (float*)out, out_stride, (const float*)k_cache, (const float*)v_cache, \
+        block_tables, bt_stride, seq_of_token, positions, context_lens, (int)num_tokens, Hq, Hkv, page, scale, window, keep_first, softcap, sinks, slopes, runs)
+#define AS_F32(NS) case NS: if (many) attn_f32_kernel<NS, true> AS_ARGS; else attn_f32_kernel<NS, false> AS_ARGS; break
     switch (D / 16) { AS_F32(1); AS_F32(2); AS_F32(3); AS_F32(4); AS_F32(5); AS_F32(6); AS_F32(7); AS_F32(8); }
 #undef AS_F32
+#undef AS_ARGS
   } else if (dtype == ME_F32)
     attn_simple_kernel<float><<<grid, block, lds, stream>>>(
         (const float*)q, q_stride, (float*)out, out_stride, (const float*)k_cache, (const float*)v_cache,

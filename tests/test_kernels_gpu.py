@@ -537,6 +537,30 @@ def test_float32_attention_takes_every_run_of_a_tile(seqs, D):
     assert torch.equal(hip().paged_attention(*args), got[order])
 
 
+def test_float32_attention_of_more_tokens_than_a_grid_row_has_tiles():
+    """More than 65,535 tiles of 16 tokens in one call: the same kernel, so the same bits as the rows in two calls."""
+    D, Hq, Hkv, page, lens = 16, 2, 1, 16, (1, 700, 1048560)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    T, pages = sum(lens), [-(-n // page) for n in lens]
+    q, k, v = rnd(T, Hq * D), rnd(sum(pages), Hkv, page, D), rnd(sum(pages), Hkv, D, page)
+    tables = torch.zeros(len(lens), max(pages), dtype=torch.int32)
+    for i, n in enumerate(pages):
+        tables[i, :n] = torch.arange(n) + sum(pages[:i])
+    tables, ctx = tables.to(DEV), torch.tensor(lens, dtype=torch.int32, device=DEV)
+    of = torch.repeat_interleave(torch.arange(len(lens), dtype=torch.int32), torch.tensor(lens)).to(DEV)
+    at = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens]).to(DEV)
+    rows = lambda lo, hi: hip().paged_attention(q[lo:hi], k, v, page, tables, ctx, of[lo:hi], at[lo:hi], None, 0, 0, D ** -0.5, 20, Hq, Hkv, D)
+    whole = rows(0, T)
+    assert torch.equal(whole[:600000], rows(0, 600000)) and torch.equal(whole[600000:], rows(600000, T))
+    some = torch.randint(701 + 20, T, (50,), generator=torch.Generator().manual_seed(1)).tolist()
+    keys, values = k[sum(pages[:2]):, 0].reshape(-1, D).double(), v[sum(pages[:2]):, 0].transpose(1, 2).reshape(-1, D).double()
+    for r in some:
+        p = r - 701
+        score = (q[r].double().view(Hq, D) @ keys[p - 19:p + 1].t()) * D ** -0.5
+        close(whole[r].view(Hq, D), torch.softmax(score, -1) @ values[p - 19:p + 1], 1e-5)
+
+
 def test_attention_generic_path_takes_odd_sizes():
     """Head size 24 and page 5 are outside the matrix-core kernel: the generic kernel takes them."""
     for dtype in (torch.float32, torch.bfloat16):
