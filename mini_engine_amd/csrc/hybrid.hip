@@ -925,7 +925,10 @@ __device__ __forceinline__ void walk_request(uint32_t lds_addr, uint32_t voff, c
 // the sum's exchanges. With the kernel that shapes the values, 2,048 tokens beside 1,075, against register copies, two barriers' worth of waiting for
 // a batch's outputs and values, and reads two or three tokens ahead: delta rule, 4 heads of 128 x 128, 262 -> 227 us, bonus rule, 16 heads of 64 x 64,
 // 150 -> 134 (one wave to a column group 344 and 230). Up to 64 rows batches of 32 tokens, held to the registers that let three workgroups onto a
-// compute unit (768 workgroups of 1,100 tokens 141 -> 130 us, 512 132 -> 135).
+// compute unit (768 workgroups of 1,100 tokens 141 -> 130 us, 512 132 -> 135). What is left of a request behind its whole batches, or all of a
+// short one, all four waves walk too, four tokens in a piece (16 heads of 64 x 64, bonus rule, one request of 16 / 31 / 63 / 127 tokens 9.5 / 12.0 / 14.3 /
+// 18.5 us by one wave with nothing read ahead, 8.1 / 9.5 / 12.0 / 16.0 so; batches of 16 tokens through registers, which have nothing left of 16, 7.8 / 11.4
+// / 13.6 / 18.1), and behind the last batch no rows are asked for (one of 2,048 tokens 118 -> 110 us).
 template <typename TX, int NR, int RULE>
 __device__ __forceinline__ void walk_shared(const DrArgs& a, const float* __restrict__ pre_q, const float* __restrict__ pre_k,
                                             const float* __restrict__ pre_d, const float* __restrict__ pre_x) {
@@ -965,22 +968,24 @@ __device__ __forceinline__ void walk_shared(const DrArgs& a, const float* __rest
   TX nv;
   float nx = 0.f;
   const uint32_t rows_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)&rows[0][0][0];
-  auto request = [&](int t0, int buf) {          // (behind the last batch: the last token's once more; a branch here would wait for nv)
+  auto request = [&](int t0, int buf) {
+    const bool more = t0 < n_tok;                // (behind the last batch no rows, but the last token's values: a branch around them would wait for nv)
     t0 = min(t0, n_tok - 1);
     const int last = n_tok - 1 - t0;
     const int64_t row = (first + t0) * a.H + h;
+    if (more)
 #pragma unroll
-    for (int r = 0; r < ROUNDS; ++r) {
-      const int e0 = 64 * wave + 256 * r;
-      if (PIECES % 256 == 0 || e0 < PIECES) {
-        const int e = e0 + lane;
-        const uint32_t from = (uint32_t)((min(e / (NR / 4), last) * a.H * (NR / 4) + e % (NR / 4)) * 16);
-        const uint32_t to = rows_base + (uint32_t)((buf * KINDS * PIECES + e0) * 16);
-        walk_request(to, from, pre_q + row * NR);
-        walk_request(to + PIECES * 16, from, pre_k + row * NR);
-        if (ROWS) walk_request(to + 2 * PIECES * 16, from, pre_d + row * NR);
+      for (int r = 0; r < ROUNDS; ++r) {
+        const int e0 = 64 * wave + 256 * r;
+        if (PIECES % 256 == 0 || e0 < PIECES) {
+          const int e = e0 + lane;
+          const uint32_t from = (uint32_t)((min(e / (NR / 4), last) * a.H * (NR / 4) + e % (NR / 4)) * 16);
+          const uint32_t to = rows_base + (uint32_t)((buf * KINDS * PIECES + e0) * 16);
+          walk_request(to, from, pre_q + row * NR);
+          walk_request(to + PIECES * 16, from, pre_k + row * NR);
+          if (ROWS) walk_request(to + 2 * PIECES * 16, from, pre_d + row * NR);
+        }
       }
-    }
     const int t = min(my_token, last);
     nv = ((const TX*)a.v + (first + t0) * a.v_stride + h * a.P)[(int64_t)t * a.v_stride + my_column];
     if (RULE != 2) nx = ((!ROWS && wave == 3 ? pre_d : pre_x) + row)[t * a.H];
@@ -1051,7 +1056,7 @@ __device__ __forceinline__ void walk_shared(const DrArgs& a, const float* __rest
   int t0 = 0, buf = 0;
   request(0, 0);
   arrive(0);
-  request(TB, 1);
+  if (TB < n_tok) request(TB, 1);
   auto walk = [&](auto which) {                  // the whole batches; this wave gives the outputs of tokens ME, ME + W, ... of each
     constexpr int ME = decltype(which)::value;
     if (TB > n_tok) return;
@@ -1109,21 +1114,56 @@ __device__ __forceinline__ void walk_shared(const DrArgs& a, const float* __rest
   else if (wave == 1) walk(std::integral_constant<int, 1>{});
   else if (wave == 2) walk(std::integral_constant<int, 2>{});
   else walk(std::integral_constant<int, 3>{});
+  // A last batch that is not whole, which lies in LDS, four tokens at a time, whose rows are read while the four before them are
+  // worked on; each wave gives the output of one of the four. (Rows behind the last token are there, and not used.)
+  auto rest = [&](auto which) {
+    constexpr int ME = decltype(which)::value;
+    const int left = n_tok - t0;
+    if (left <= 0) return;
+    struct Four { float k[4][RL], d[4][RL], q[RL], x; };
+    Four f[2];
+    Numbers num[2];
+    auto read_four = [&](int g, Four& o, Numbers& n) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        read_rows(buf, 4 * g + j, o.k[j], 1);
+        if (ROWS) read_rows(buf, 4 * g + j, o.d[j], 2);
+      }
+      read_rows(buf, 4 * g + ME, o.q, 0);
+      o.x = read_x(buf, 4 * g + ME);
+      read_numbers(buf, g, n);
+    };
+    auto four = [&](int g, const Four& o, const Numbers& n) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (4 * g + j >= left) return;
+        Rows r;
+#pragma unroll
+        for (int i = 0; i < RL; ++i) { r.k[i] = o.k[j][i]; if (ROWS) r.d[i] = o.d[j][i]; r.q[i] = o.q[i]; }
+        float y = token(r, n.v[j], n.x[j], n.h[j], j == ME, [](int) {});
+        if (j != ME) continue;
+        y = group_sum<RG>(y);
+        if (RULE == 0) y = fmaf(o.x, n.v[j], y);
+        if (live && rg == 0) (out + (int64_t)(t0 + 4 * g + j) * (a.H * a.P))[p] = y;
+      }
+    };
+    read_four(0, f[0], num[0]);
+#pragma unroll 1
+    for (int g = 0; 4 * g < left; g += 2) {
+      read_four(g + 1, f[1], num[1]);
+      asm volatile("" ::: "memory");
+      four(g, f[0], num[0]);
+      read_four(min(g + 2, TB / 4 - 1), f[0], num[0]);
+      asm volatile("" ::: "memory");
+      four(g + 1, f[1], num[1]);
+    }
+  };
+  if (wave == 0) rest(std::integral_constant<int, 0>{});
+  else if (wave == 1) rest(std::integral_constant<int, 1>{});
+  else if (wave == 2) rest(std::integral_constant<int, 2>{});
+  else rest(std::integral_constant<int, 3>{});
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // no request outlives its workgroup's LDS
   if (wave != 0) return;
-  // a last batch that is not whole, which lies in LDS: its outputs and the state behind it are the first wave's
-  for (int j = 0; t0 + j < n_tok; ++j) {
-    Rows o;
-    read_rows(buf, j, o.q, 0);
-    read_rows(buf, j, o.k, 1);
-    if (ROWS) read_rows(buf, j, o.d, 2);
-    const float v = reinterpret_cast<const float*>(&sv[buf][lane / RG][0])[j];
-    const float x = RULE == 2 ? 0.f : reinterpret_cast<const float*>(&sx[buf][0])[j];
-    const float hd = ROWS ? 0.f : reinterpret_cast<const float*>(&sh[buf][0])[j];
-    float y = group_sum<RG>(token(o, v, x, hd, true, [](int) {}));
-    if (RULE == 0) y = fmaf(x, v, y);
-    if (live && rg == 0) (out + (int64_t)(t0 + j) * (a.H * a.P))[p] = y;
-  }
   if (live) {
 #pragma unroll
     for (int i = 0; i < RL; ++i)
@@ -1143,8 +1183,10 @@ __global__ void __launch_bounds__(64 * W, W == 1 ? 1 : NR <= 64 ? 3 : 2) decay_w
 // to a compute unit up to 64 rows, two of 128. us with the kernel that shapes the values, requests of 1,100 tokens, one wave / four, bonus and
 // delta rule: 64 rows, 512 workgroups 122 / 94 and 162 / 140, 768 146 / 126 and 185 / 185, 832 157 / 157 and 193 / 228; 128 rows, 256
 // workgroups 150 / 104 and 179 / 139, 384 167 / 134 and 197 / 181, 512 169 / 144 and 202 / 199, 576 197 / 206 and 242 / 276. With 256 rows
-// the batches' LDS leaves no room for longer ones, and without them four waves gain nothing (624 / 650).
-template <int NR> constexpr unsigned dr_shared_max() { return NR <= 64 ? 768 : NR <= 128 ? 512 : 0; }
+// the batches' LDS leaves no room for longer ones, and without them four waves gain nothing (624 / 650). Of 128 rows requests of
+// fewer than 64 tokens on average (`mean`) share up to 256 workgroups (384 of them, bonus rule, 16 tokens 11.3 / 12.4, 32 14.2 / 14.9, 48 17.1 /
+// 17.2, 64 20.2 / 19.8, 95 27.2 / 24.9).
+template <int NR> static unsigned dr_shared_max(int64_t mean) { return NR <= 64 ? 768 : NR > 128 ? 0 : mean >= 64 ? 512 : 256; }
 template <typename TX, int NR, int RG, bool PRE>
 static void launch_decay_rows(const DrArgs& a, int rule, int num_seqs, int64_t T, float* pre, hipStream_t stream) {
   constexpr int PC = 64 / RG;
@@ -1156,8 +1198,8 @@ static void launch_decay_rows(const DrArgs& a, int rule, int num_seqs, int64_t T
 #define DR_RULE(R)                                                                       \
   do {                                                                                   \
     decay_prepare_kernel<TX, NR, R><<<pgrid, block, 0, stream>>>(a, RG, pq, pk, pd, px); \
-    constexpr bool SHARES = RG == 16 && dr_shared_max<NR>() > 0;                         \
-    if (SHARES && grid.x <= dr_shared_max<NR>() && (int64_t)a.H * a.P < (1 << 27))       \
+    constexpr bool SHARES = RG == 16 && NR <= 128;                                       \
+    if (SHARES && grid.x <= dr_shared_max<NR>(T / num_seqs) && (int64_t)a.H * a.P < (1 << 27))       \
       decay_walk_kernel<TX, NR, RG, R, SHARES ? 4 : 1><<<grid, SHARES ? 256 : 64, 0, stream>>>(a, pq, pk, pd, px); \
     else decay_walk_kernel<TX, NR, RG, R, 1><<<grid, block, 0, stream>>>(a, pq, pk, pd, px); \
   } while (0)

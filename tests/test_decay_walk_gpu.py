@@ -112,3 +112,31 @@ def test_whole_batches_of_the_shared_walk(monkeypatch, N, rule, T):
     y = run([every], whole)
     assert torch.equal(torch.cat([run([every[lo:lo + 7]], pieces) for lo in range(0, T, 7)]), y) and torch.equal(pieces, whole)
     assert torch.equal(run([every] * crowd, many).view(crowd, T, H * P), y.expand(crowd, T, H * P)) and torch.equal(many, whole.expand(crowd, -1))
+
+
+@pytest.mark.parametrize("rule", ["bonus", "delta_head"])
+@pytest.mark.parametrize("n", [63, 64, 130])
+def test_shared_walk_of_128_rows_by_the_requests_length(n, rule):
+    """Between 256 and 512 workgroups requests of 64 tokens and more on average share their columns' walk, shorter ones do not: the same bits as each
+    request alone, whose 128 workgroups always do, remainders of a batch included."""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    H, N, P, count = 8, 128, 64, 3
+    T, wide = n * count, H if rule == "delta_head" else H * N
+    q, k, v, raw, beta = (rnd(T, m).to(torch.bfloat16) for m in (H * N, H * N, H * P, wide, H))
+    kw = dict(base=rnd(wide) - 1)
+    kw.update(dict(bonus=rnd(wide)) if rule == "bonus" else dict(rate=rnd(H).abs() + 0.1, unit_eps=1e-6, q_scale=N ** -0.5))
+    start = rnd(count, H * N * P)
+
+    def run(lo, hi, which, state):
+        lens = [n] * len(which)
+        more = dict(kw, beta=beta[lo:hi]) if rule == "delta_head" else kw
+        cu = torch.arange(len(which) + 1, dtype=torch.int32, device=DEV) * n
+        return hip().decay_rows_recurrence(q[lo:hi], k[lo:hi], v[lo:hi], raw[lo:hi], state, torch.tensor(which, dtype=torch.int32, device=DEV), cu,
+                                           lens, H, H, N, P, rule, **more)
+
+    together = start.clone()
+    y = run(0, T, [0, 1, 2], together)
+    for i in range(count):
+        state = start.clone()
+        assert torch.equal(run(i * n, i * n + n, [i], state), y[i * n:i * n + n]) and torch.equal(state[i], together[i])
