@@ -705,7 +705,8 @@ class HipBackend:
         # `tile_fits` of what is left to ask, and an `out` may begin anywhere
         tiles = (K % 64 == 0 and K >= 128 and N % 8 == 0 and M * xs < 1 << 31 and N * ws < 1 << 31
                  and (out is None or out.data_ptr() % 16 == 0))
-        ring = ring_tile(M, N, K) if tiles and not (mid and N * K > RING_MAX_WEIGHT_OF_MID) else None
+        # (rows may overlap, one row stand for all: `gemm_mid` takes them)
+        ring = ring_tile(M, N, K) if tiles and xs >= K and ws >= K and not (mid and N * K > RING_MAX_WEIGHT_OF_MID) else None
         if ring is not None:
             return _tile_product(x, w, new(), tile=ring)
         if mid and not (mid_crowded(M, N, 1) and tiles):

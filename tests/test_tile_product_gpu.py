@@ -215,3 +215,18 @@ def test_each_product_of_one_round_runs_where_the_rule_sends_it(monkeypatch, M, 
     y, ran = _products(monkeypatch, lambda: hip().linear(x, w))
     assert ran == [route] and (ops.ring_tile(M, N, K) is not None) == (route == TILE or N % 8 > 0)
     close(y, x.double() @ w.double().t(), 4e-3)
+
+
+@pytest.mark.parametrize("M,N,K", [(100, 1024, 1024), (256, 2048, 1024), (128, 1024, 2048)])
+def test_rows_that_overlap_are_taken_as_before(M, N, K):
+    """One row that stands for all of them (an expanded view), and rows that begin inside the one before: the kernel for a few hundred
+    rows reads them; the ring, which would refuse them, does not get them. For more rows both refuse."""
+    x, w = _operands(M, N, K)
+    base = torch.randn(8 * M + K, device=DEV).bfloat16()
+    for rows in (x[:1].expand(M, K), base.as_strided((M, K), (8, 1))):
+        assert ops.ring_tile(M, N, K) is not None
+        close(hip().linear(rows, w), rows.double() @ w.double().t(), 4e-3)
+    features = w[:1].expand(N, K)
+    close(hip().linear(x, features), x.double() @ features.double().t(), 4e-3)
+    with pytest.raises(ops.KernelError):
+        hip().linear(x[:1].expand(600, K), w)
