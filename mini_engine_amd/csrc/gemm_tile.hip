@@ -285,7 +285,7 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __rest
 // The same by four waves for launches of one workgroup to a compute unit, which no other fills the waits of: whole steps of 64 of K in
 // a ring of RING_STAGES, a barrier a step. A wave reads the next step's operands and asks for the step behind the ring between its
 // products, so that neither stands in a row of its own: 16 products of 128 x 64 beside 12 reads and 6 requests take about what the requests take
-// (24 KB a step at the 64 bytes a cycle that reach a compute unit; 5 stages are 12 % faster than 4 and 5 % than 6). In quarters, with four barriers
+// (24 KB a step at the 64 bytes a cycle that reach a compute unit; 2,048 rows of 1024 x 2048 with 4 / 5 / 6 stages 12.9 / 11.9 / 12.5 us). In quarters, with four barriers
 // a step and the reads in front of the products, a step took 0.29-0.48 us whatever the tile; now 0.17 for 64 x 64, 0.31 for 64 x 128, 0.49 for 128 x
 // 128. us of a launch in a chain, the library / quarters / this: 2,048 rows of 1024 x 2048 16.4 / 14.0 / 11.9, of 1024 x 3072 19.3 / 19.5 / 16.8,
 // 700 rows 10.2 / 10.7 / 8.4 and 13.9 / 15.1 / 11.5, 800 rows of 4096 x 4096 39.9 / 38.9 / 32.9; the same bits (K in one order).
@@ -425,6 +425,15 @@ gemm_ring_kernel(const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __rest
   tile_store<MI, NI, ACT>(acc, y + (int64_t)blockIdx.z * M * ldy, ldy, M, N, m0 + wm * (16 * MI) + n, n0 + wn * (ACT ? 8 * NI : 16 * NI), g, form, rounded);
 }
 
+// Whether a launch of so many tiles (times slices of K), each of `per_split` steps, goes through the ring: tiles of four waves where there is at
+// most a workgroup to a compute unit. Below 16 steps the quarters are level or ahead (8 steps a slice, 128 rows of 1024 x 2048 in tiles of 128 x
+// 64 6.3 / 6.7 us). Tiles of 128 x 128, whose ring fills a compute unit's LDS, gain from 32 steps on and up to 248 workgroups (16 steps 12.3 /
+// 16.5 with 256 of them, 32 steps 20.2 / 23.2, with 208 19.5 / 18.5).
+extern "C" int me_gemm_tile_rings(int tile_rows, int tile_features, int64_t tiles, int per_split) {
+  const bool large = tile_rows == 128 && tile_features == 128;
+  return tile_rows * tile_features <= 128 * 128 && tile_rows <= 128 && tile_features <= 128 && tiles <= (large ? 248 : 256) && per_split >= (large ? 32 : 16);
+}
+
 // y: [M, N] of out_dtype (ksplit 1), or float32 partial sums [ksplit, M, N] with ldy = N; act: w is a packed gate/up weight
 // [N = 2 I, K] and y is the gated product [M, I] (bfloat16, ksplit 1) in the form that limit, alpha and bias give (`GateForm`);
 // 1: of the unrounded sums, 2: of the sums rounded to bfloat16.
@@ -466,10 +475,7 @@ extern "C" int me_gemm_tile_bf16(const void* x, int64_t ldx, const void* w, int6
     else if (out_dtype == ME_F32) TILE_LAUNCH(KERNEL, WGM, WGN, MI, NI, false, float);                                \
     else TILE_LAUNCH(KERNEL, WGM, WGN, MI, NI, false, bf16_t);                                                        \
   } while (0)
-// RING: the steps from which a tile of four waves goes through the ring where the launch has at most a workgroup to a compute unit (0: never).
-// Below 16 steps the quarters are level or ahead (8 steps a slice, 128 rows of 1024 x 2048 in tiles of 128 x 64 6.3 / 6.7 us). Tiles of 128 x 128, whose ring
-// fills a compute unit's LDS, gain from 32 steps on and up to 248 workgroups (16 steps 12.3 / 16.5 with 256 of them, 32 steps 20.2 / 23.2,
-// with 208 19.5 / 18.5).
+// RING: whether the tile has a form that goes through the ring.
 #define TILE(WGM, WGN, MI, NI, RING)                                                                                  \
   if (tile_rows == WGM * MI * 16 && tile_features == WGN * NI * 16) {                                                 \
     const int64_t m_tiles = ((int64_t)M + tile_rows - 1) / tile_rows;                                                 \
@@ -477,8 +483,8 @@ extern "C" int me_gemm_tile_bf16(const void* x, int64_t ldx, const void* w, int6
     const int64_t blocks = (m_tiles * n_tiles + 7) / 8 * 8;                                                           \
     ME_CHECK(blocks < (1ll << 31) && 8 * n_tiles < (1ll << 31) && ksplit <= 65535, "tile gemm: too many tiles");      \
     const dim3 grid((unsigned)blocks, 1, (unsigned)ksplit);                                                           \
-    if constexpr (RING > 0)                                                                                           \
-      if (m_tiles * n_tiles * ksplit <= (RING >= 32 ? 248 : 256) && per_split >= RING) {                              \
+    if constexpr (RING)                                                                                               \
+      if (me_gemm_tile_rings(tile_rows, tile_features, m_tiles * n_tiles * ksplit, per_split)) {                      \
         const size_t lds = (size_t)(tile_rows + tile_features) * 128 * RING_STAGES;                                   \
         TILE_KIND(gemm_ring_kernel, WGM, WGN, MI, NI);                                                                \
         ME_LAUNCH_CHECK();                                                                                            \
@@ -489,16 +495,16 @@ extern "C" int me_gemm_tile_bf16(const void* x, int64_t ldx, const void* w, int6
     ME_LAUNCH_CHECK();                                                                                                \
     return 0;                                                                                                         \
   }
-  TILE(2, 4, 8, 4, 0)     // 256 x 256
-  TILE(4, 2, 4, 6, 0)     // 256 x 192
-  TILE(2, 4, 6, 4, 0)     // 192 x 256
-  TILE(2, 4, 4, 4, 0)     // 128 x 256
-  TILE(4, 2, 4, 4, 0)     // 256 x 128
-  TILE(4, 2, 2, 6, 0)     // 128 x 192
-  TILE(2, 2, 4, 4, 32)     // 128 x 128
-  TILE(2, 2, 2, 4, 16)     // 64 x 128
-  TILE(2, 2, 4, 2, 16)     // 128 x 64
-  TILE(2, 2, 2, 2, 16)     // 64 x 64
+  TILE(2, 4, 8, 4, false)     // 256 x 256
+  TILE(4, 2, 4, 6, false)     // 256 x 192
+  TILE(2, 4, 6, 4, false)     // 192 x 256
+  TILE(2, 4, 4, 4, false)     // 128 x 256
+  TILE(4, 2, 4, 4, false)     // 256 x 128
+  TILE(4, 2, 2, 6, false)     // 128 x 192
+  TILE(2, 2, 4, 4, true)     // 128 x 128
+  TILE(2, 2, 2, 4, true)     // 64 x 128
+  TILE(2, 2, 4, 2, true)     // 128 x 64
+  TILE(2, 2, 2, 2, true)     // 64 x 64
 #undef TILE
 #undef TILE_KIND
 #undef TILE_LAUNCH

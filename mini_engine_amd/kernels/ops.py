@@ -94,6 +94,7 @@ _CORE_PROTOS = {
     "me_gemm_rows_bf16": [P, L, P, L, P, L, I, P, I, I, I, I, I, P],
     "me_gemm_skinny_norm_bf16": [P, I, I, P, P, P, F, P, L, P, L, I, I, I, I, I, P],
     "me_gemm_mid_bf16": [P, L, P, L, P, L, I, I, I, I, I, I, F, F, P, P],
+    "me_gemm_tile_rings": [I, I, L, I],
     "me_gemm_tile_bf16": [P, L, P, L, P, L, I, I, I, I, I, I, F, F, P, I, I, P],
     "me_gemm_library_bf16": [P, L, P, L, P, L, I, P, ctypes.c_size_t, I, I, I, I, P],
     "me_add_rms_norm": [P, I, I, L, P, P, P, P, L, I, F, P],

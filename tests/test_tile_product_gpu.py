@@ -185,27 +185,39 @@ def test_what_the_kernel_refuses():
             _launch(*args)
 
 
+def _rings(tile, M, N, steps, slices=1, gated=False):
+    tiles = -(-M // tile[0]) * (-(-(N // 2) // (tile[1] // 2)) if gated else -(-N // tile[1]))
+    return bool(ops.core().fns["me_gemm_tile_rings"](*tile, tiles * slices, -(-steps // slices)))
+
+
 @pytest.mark.parametrize("tile", [(64, 64), (64, 128), (128, 64), (128, 128)], ids=lambda t: f"{t[0]}x{t[1]}")
-@pytest.mark.parametrize("steps", [16, 17, 32, 33, 35])
-def test_tiles_in_one_round_go_round_the_ring(tile, steps):
-    """Launches of one workgroup to a compute unit walk K through a ring of stages: from its fewest steps on, with an odd count and a
-    row, a feature piece and a stride beside the tile's, every kind of output; bit for bit what a launch of many rounds gives the same rows."""
+@pytest.mark.parametrize("extra", [-1, 0, 1, 3])
+def test_tiles_in_one_round_go_round_the_ring(tile, extra):
+    """Launches of one workgroup to a compute unit walk K through a ring of stages: from its fewest steps on and with one fewer, where they do not,
+    in slices of K with a shorter last one, with an odd count and a row, a feature piece and a stride beside the tile's, every kind of
+    output; bit for bit what a launch of many rounds gives the same rows."""
     rows, features = tile
-    M, N, K = 2 * rows + 5, 3 * features - 16, 64 * steps
-    x, w = _operands(M, N, K, 8)
-    many = torch.cat([x] * (1 + 300 * rows * features // (M * N)))                          # more than 256 tiles
-    many = many[:many.shape[0] - many.shape[0] % rows + 3]
-    ref = x.double() @ w.double().t()
-    for dtype, slices, gated in ((torch.bfloat16, 1, 0), (torch.float32, 1, 0), (torch.float32, 2, 0), (torch.bfloat16, 1, 1), (torch.bfloat16, 1, 2)):
-        outs = []
-        for rows_in in (x, many):
-            shape = (rows_in.shape[0], N // 2 if gated else N)
-            y = torch.full(shape if slices == 1 else (slices, *shape), float("nan"), dtype=dtype, device=DEV)
-            _launch(rows_in, w, y, slices, tile, gated)
-            outs.append(y[..., :M, :])
-        assert torch.equal(*outs)
-        if not gated:
-            close(outs[0] if slices == 1 else outs[0].sum(0), ref, 4e-3 if dtype == torch.bfloat16 else 2e-5)
+    fewest = 32 if tile == (128, 128) else 16
+    M, N = 2 * rows + 5, 3 * features - 16
+    for slices in (1, 2):
+        steps = slices * fewest + extra
+        K = 64 * steps
+        x, w = _operands(M, N, K, 8)
+        many = torch.cat([x] * (1 + 300 * rows * features // (M * N)))                          # more than 256 tiles
+        many = many[:many.shape[0] - many.shape[0] % rows + 3]
+        assert _rings(tile, M, N, steps, slices) == (-(-steps // slices) >= fewest) and not _rings(tile, many.shape[0], N, steps, slices)
+        ref = x.double() @ w.double().t()
+        for dtype, gated in ((torch.bfloat16, 0), (torch.float32, 0), (torch.bfloat16, 1), (torch.bfloat16, 2)) if slices == 1 else ((torch.float32, 0),):
+            assert _rings(tile, M, N, steps, slices, gated > 0) == (extra >= 0 or slices == 2)
+            outs = []
+            for rows_in in (x, many):
+                shape = (rows_in.shape[0], N // 2 if gated else N)
+                y = torch.full(shape if slices == 1 else (slices, *shape), float("nan"), dtype=dtype, device=DEV)
+                _launch(rows_in, w, y, slices, tile, gated)
+                outs.append(y[..., :M, :])
+            assert torch.equal(*outs)
+            if not gated:
+                close(outs[0] if slices == 1 else outs[0].sum(0), ref, 4e-3 if dtype == torch.bfloat16 else 2e-5)
 
 
 @pytest.mark.parametrize("M,N,K,route", [(65, 4096, 1024, TILE), (256, 4096, 1024, TILE), (700, 1024, 2048, TILE), (2048, 1024, 3072, TILE), (300, 1024, 3072, LIBRARY),
