@@ -256,18 +256,14 @@ class GatedDelta(Mixer):
         return self.o.forward(o, allow_partials=True)
 
 
-# Steps of so many rows copy the low-rank inputs although views would do: without the copies' time the walk begins in front of the
-# left mixer's large tiles, which find no room beside it, now in front and now behind from one length to the next. One prompt of Tavevik's
-# 0.6B sizes, copies / views, ms: 300 tokens 3.95 / 3.85, 980 6.48 / 6.34, 1,024 6.74 / 6.79, 1,300 8.28 / 8.67, 1,500 9.27 / 9.73, 1,740 10.21 /
-# 10.71, 1,780 10.87 / 10.49, 1,820 10.36 / 10.65, 2,048 11.80 / 11.49, 2,300 12.72 / 12.53; 30 decoding requests 2.98 / 2.84.
-COPIED_ROWS = range(1024, 2048)
-
-
 def _rows(rows: torch.Tensor, start: int, width: int) -> torch.Tensor:
     """Columns [start, start + width) of packed rows as an operand of a product: a view where the products take one
-    (their rows start at whole steps of 16 bytes), else, and for steps of COPIED_ROWS rows, a copy."""
+    (their rows start at whole steps of 16 bytes), else a copy. A copy takes 2.7 us and its product 4.2 us with either. Beside another
+    mixer the step's time also moves by up to 5 % with where the walk's and the other mixer's kernels meet: at Tavevik's 0.6B sizes one prompt of
+    700 tokens 5.61 / 5.48 ms with copies / views, of 1,150 7.68 / 7.80, of 1,500 9.06 / 9.47, of 1,740 10.64 / 10.94, of 1,780 11.24 / 10.88, of 2,048
+    11.92 / 11.77, of 2,300 13.32 / 13.04, two of 2,048 and 1,075 14.28 / 14.00; at its 1.7B sizes views are ahead throughout."""
     view = rows[:, start:start + width]
-    if (start * rows.element_size()) % 16 == 0 and (rows.stride(0) * rows.element_size()) % 16 == 0 and rows.shape[0] not in COPIED_ROWS:
+    if (start * rows.element_size()) % 16 == 0 and (rows.stride(0) * rows.element_size()) % 16 == 0:
         return view
     return view.contiguous()
 

@@ -305,3 +305,13 @@ def test_launch_rule_of_the_recurrence():
                 assert not prepared and rg in (1, 4) and (rg == 4 or N <= 64)
                 rg, prepared = ops.decay_row_groups(B, H, N, P_, 700)
                 assert prepared and rg in (4, 16) and (rg == 4 or B * H * -(-P_ // 4) <= 4096)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_thin_pairs_read_views_of_the_packed_rows(dtype):
+    """At every number of rows, where the columns begin and the rows follow each other at whole steps of 16 bytes; else a copy."""
+    from mini_engine_amd.parts import hybrid
+    for T in (1, 30, 1023, 1024, 1500, 2047, 2048):
+        rows = torch.zeros(T, 40, dtype=dtype)
+        assert hybrid._rows(rows, 8, 16).data_ptr() == rows[:, 8:].data_ptr()
+        assert hybrid._rows(rows, 9, 16).is_contiguous() and hybrid._rows(rows[:, :39].contiguous(), 8, 16).is_contiguous()
