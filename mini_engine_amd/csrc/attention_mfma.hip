@@ -1004,15 +1004,11 @@ __device__ __forceinline__ void dma16(const bf16_t* gbase, uint32_t voff, uint32
 template <int N>
 __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
-// A wave in its softmax goes first when the SIMD chooses whose instruction to issue.
-__device__ __forceinline__ void softmax_priority(bool on) {
-  if (on) __builtin_amdgcn_s_setprio(1); else __builtin_amdgcn_s_setprio(0);
-}
-
 struct DmaPages { int k, v; };   // the page of this wave's two key instructions and of its two value instructions
 
 // With three waves to a SIMD (168 registers each): launches of so many workgroups that the third wave fills the others' waits
-// (`prefill_waves`). It reads operands where it uses them.
+// (`prefill_waves`). It reads operands where it uses them. No wave goes in front of another (with the priority raised for its softmax
+// 40 prompts of 300 tokens, 32 and 8 heads, took 85.4 us, without 81.8; one of 16,384, 16 and 8 heads, 1,024, 1,014).
 template <bool WINDOW>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) attn_prefill_dma_kernel(AttnArgs a) {
   extern __shared__ __align__(16) unsigned char pf_lds[];   // [NB][DMA_BUF]
@@ -1186,11 +1182,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
             st[ct][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qb[ct][ks], st[ct][tt], 0, 0, 0);
         }
       }
-      softmax_priority(true);
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct)
         block_softmax<FULL>(a, st[ct], t0, col_lo[ct], col_hi[ct], slope[ct], m[ct], l[ct], acc[ct], g, pb[ct]);
-      softmax_priority(false);
       const unsigned char* vb = pf_lds + cur * DMA_BUF + rd_v;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {

@@ -1896,7 +1896,12 @@ def prefill_waves(max_context: int, num_tokens: int, num_seqs: int, Hq: int, Hkv
     2,048 workgroups or more, and the prompts start at their beginning (the longest context at most twice the mean
     number of new tokens per sequence): tiles of all lengths are then under way at once and the third wave fills
     the others' waits. Portions over a long prefix, whose tiles are equally long and walk the same keys together,
-    run better with two waves and 205 registers, and so do launches of few workgroups."""
+    run better with two, and so do launches of few workgroups (16 and 8 heads, three / two: a prompt of 4,096 tokens 132 / 95 us, of
+    8,192 303 / 276, sixteen of 512 48.5 / 42.4). From 2,048 workgroups on the line was drawn against a form with two waves
+    that the pipeline has replaced since; against the pipeline three waves are ahead at many short prompts (40 of 300 tokens, 32 and 8 heads 81.8 /
+    86.1; 16 of 600, 64 and 8 heads 167.9 / 166.8; 16 of 512, 32 and 8 heads 71.7 / 70.4) and behind at long ones (one of 16,384 tokens, 16 and 8
+    heads 1,014 / 970, 8 of 2,048 176 / 163, one of 8,192, 32 and 8 heads 523 / 498, of 6,144, 64 and 8 heads 594 / 565): a line by
+    length as well is not drawn yet."""
     if col_tiles != 2 or max_segs != 1 or num_seqs < 1 or max_context <= 0:
         return 2
     group = max(1, Hq // max(1, Hkv))
