@@ -445,8 +445,8 @@ __device__ __forceinline__ int count_one(int* counter, int e, int common) {
 // With `logits` (few tokens) the workgroup first makes the choice itself, a wave per one or two tokens in turn, and writes ids and
 // weights: the launch of `moe_select` is saved. What bounds it is the length of one workgroup's way: up to 64 experts the
 // choice runs in registers with a wave's next token on its way (up to 32 experts its next two), the ids stay in LDS (up to MOE_LDS_PAIRS of them), and one wave adds up the classes' places by
-// exchanges (32 tokens, 32 experts, 4 of 4 groups: 20.5 us with races through LDS and one thread adding up, 9.4 with a wave per token
-// and groups that read each other's lanes through LDS, 6.1 so; the same without a choice 2.5).
+// exchanges (32 tokens, 4 of 32 experts, all groups kept: 20.5 us with races through LDS and one thread adding up, 7.6 with a wave per token, 6.2
+// with two to a wave; in 2 of 4 groups 10.2 with groups that read each other's lanes through LDS, 6.9 with exchanges in a row; without a choice 2.5).
 __global__ void __launch_bounds__(1024)
 moe_sort_kernel(int32_t* __restrict__ ids, int P, int routed, int E, int max_tiles, int tile_rows, int32_t* __restrict__ order,
                 int32_t* __restrict__ offsets, int32_t* __restrict__ tile_expert, int32_t* __restrict__ tile_row,
