@@ -1801,28 +1801,28 @@ RING_TILES = ((64, 64), (64, 128), (128, 64), (128, 128))
 RING_MAX_WEIGHT_OF_MID = 1 << 22          # beyond, the tiled kernel of csrc/gemm_mid.hip keeps what it has: 7.2 / 6.6 us over 6144 x 1024
 
 
-RING_FILL = 0.78
-
-
 @lru_cache(maxsize=4096)
 def ring_tile(M: int, N: int, K: int) -> tuple | None:
     """The tile by which M rows (more than 64) against a bfloat16 weight [N, K] go through the ring of csrc/gemm_tile.hip, one workgroup to
     a compute unit, or None. The smallest tile that gives one round of workgroups, for a step of it is the shortest (0.17 us for 64 x 64, 0.31 for 64 x
     128, 0.49 for 128 x 128); over a K of 4,096 and more 128 x 64 before 64 x 128 (300 rows of 4096 x 4096 27.8 / 23.4).
 
-    Timed against what had these products, the library or older kernels (us, theirs / this). Up to a K of 1,536 ahead at every fill, but not with
+    Against what had these products, the library or older kernels (us, theirs / this). Up to a K of 1,536 ahead at every fill, but not with
     tiles of 128 x 128 (800 rows of 4096 x 1024 11.7 / 12.1). Tiles of 64 x 64 are ahead up to a K of 2,048 (700 rows of 1024 x 2048 10.8 / 9.0, 128 of 12288 x
     2048 15.9 / 13.4), below 4,096 where six tenths of the compute units have a tile (900 rows of 1024 x 3072 16.7 / 16.1, 300 of 2048 x 3072 17.2 / 15.8), of 4,096
-    where the rows and features fill seven tenths of a round (128 rows of 6144 x 4096 3.4 us a layer); beyond, 256 rows of 4096 x 12288 54.5 / 60.5. The
-    larger tiles take the same time however empty their round is, and the library's grows by a step where its own tiles need another round: in whole
-    prompts, by which a layer's product gets faster (slower: -), 1024 x 2048 at 1,060 / 1,136 / 1,212 / 1,288 / 1,364 / 1,440 / 1,516 rows -0.7 / -1.2 / -1.3 / -0.3 /
-    0.3 / -0.1 / -0.3 us, at 1,592 / 1,744 / 1,896 / 2,048 1.3 / 1.1 / 2.1 / 1.6; 2048 x 2048 at 560 / 700 / 760 -0.7 / -1.1 / -0.6, at 820 / 900 / 1,000 1.1 / 2.0 / 1.5;
-    2048 x 6144 at 1,500 / 1,536 rows -8.1 / -10.9, at 1,600 / 1,700 / 1,850 7.2 / 9.8 / 6.5; 6144 x 4096 at 480 / 512 -2.0 / -1.8, at 540 / 600 8.1 / 5.7. So they need
-    RING_FILL of a round; tiles of 64 x 128 below a K of 4,096 eight tenths (1024 x 3072 at 1,288 / 1,516 / 1,592 rows -1.7 / -2.6 / -0.4, at 1,668 / 1,744 / 2,048 0.5 /
-    1.4 / 0.2), and three quarters suffice up to 256 rows, of which the library's kernels do worse (6144 x 2560 at 250 / 256 rows -2.6 / 7.4). Tiles
-    of 128 x 128 over a K of 2,048 are ahead at every fill (2048 x 2048 at 1,100 / 1,300 / 1,500 rows 0.2 / 1.9 / 0.8). Over a K beyond 8,192 the
-    library keeps rows in whole tiles of 128 (2560 x 9728 at 1,280 / 1,408 / 1,536 -3.6 / -0.7 / 0.4, at 1,344 / 1,450 9.9 / 12.8), and everything over a K beyond
-    16,384, where it takes kernels that do not add up K in one piece, whose bits are others."""
+    where the rows and features fill seven tenths of a round (128 rows of 6144 x 4096 3.4 us a layer); beyond, 256 rows of 4096 x 12288 54.5 / 60.5. Tiles of 128 x
+    128 over a K of 2,048 are ahead or level at every fill (2048 x 2048 at 1,100 / 1,300 / 1,500 rows 0.2 / 1.9 / 0.8 us a layer of a prompt).
+
+    The larger tiles take the same time however empty their round is. The library is ahead while its own tiles of 256 x 256 or of 192 x 256 are few,
+    up to 48 and 64 against tiles of 128 x 128, half as many against half of that tile; beyond, its time grows by a step. What a product gains in whole prompts (us a layer;
+    minus: loses): 1024 x 2048 at 1,060 / 1,136 / 1,288 / 1,516 rows -0.7 / -1.2 / -0.3 / -0.3, at 1,592 / 1,744 / 1,896 / 2,048 1.3 / 1.1 / 2.1 / 1.6; 2048 x 2048 at 560 / 700 / 760
+    -0.7 / -1.1 / -0.6, at 820 / 900 / 1,000 1.1 / 2.0 / 1.5; 1024 x 3072 at 2,800 / 3,050 -6.2 / -4.8, at 3,100 / 3,123 / 3,500 5.1 / 3.8 / 3.9; 2048 x 6144 at 1,500 / 1,536 -8.1 / -10.9, at
+    1,550 / 1,600 / 1,700 9.0 / 7.2 / 9.8; 2560 x 9728 at 1,150 -17.0, at 1,216 / 1,344 / 1,450 7.3 / 9.9 / 12.8; 6144 x 4096 at 480 / 512 -2.0 / -1.8, at 540 / 600 8.1 / 5.7. Beside that:
+    three quarters of a round at least; tiles of 64 x 128 over a K of 2,049 to 4,095 eight tenths of it up to 1,024 features, else all but a twentieth (1024 x 3072 at 1,288 / 1,516 /
+    1,592 rows -1.7 / -2.6 / -0.4, at 1,668 / 1,744 / 2,048 0.5 / 1.4 / 0.2; 2048 x 3072 at 826 / 936 rows in a chain 0.93 / 0.97 times as fast, at 992 and more level); over a K beyond 4,096
+    not rows in whole tiles of 128, which suit the library's tiles too (2560 x 9728 at 1,280 / 1,408 / 1,536 -3.6 / -0.7 / 0.4); up to 256 rows those in whole 64s, of which the library takes
+    slow kernels (6144 x 2560 at 250 / 256 rows -2.6 / 7.4). Of 1,830 products of 1,024 to 6,144 features and a K of 2,048 to 9,728, in chains, the rule is more than 2 % behind at 36, 6 % at most. Over a K
+    beyond 16,384 the library takes kernels that do not add up K in one piece, whose bits are others, and keeps everything."""
     if M <= 64 or K < 1024 or K > 16384:
         return None
     order = RING_TILES if K < 4096 else (RING_TILES[0], RING_TILES[2], RING_TILES[1], RING_TILES[3])
@@ -1839,10 +1839,15 @@ def ring_tile(M: int, N: int, K: int) -> tuple | None:
         return tile if K == 2048 else None
     if K <= 1536:
         return tile
-    if K > 8192 and M % 128 == 0:
+    if M <= 256:
+        return tile if M % 64 == 0 and fill >= 0.55 else None
+    if K > 4096 and M % 128 == 0:
         return None
-    need = 0.75 if M <= 256 else 0.8 if tile == (64, 128) and 2048 < K < 4096 else RING_FILL
-    return tile if fill >= need else None
+    if tile == (64, 128) and 2048 < K < 4096:
+        return tile if fill >= (0.8 if N <= 1024 else 0.95) else None
+    of_128 = tile[0] * tile[1] / (128 * 128)
+    few = -(-M // 256) * -(-N // 256) <= 48 * of_128 or -(-M // 192) * -(-N // 256) <= 64 * of_128
+    return tile if fill >= 0.75 and not few else None
 
 
 def tile_fits(x: torch.Tensor, w: torch.Tensor, slices: int = 1) -> bool:

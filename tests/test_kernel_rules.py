@@ -323,12 +323,12 @@ def test_short_requests_pass_the_recurrence_token_by_token():
 
 
 def test_the_ring_takes_rounds_that_are_full_enough():
-    """What was timed in whole prompts: tiles of 64 x 128 and more only where rows and features fill most of their round."""
+    """What was timed in whole prompts: tiles of 64 x 128 and more only where their round is full and the library's tiles are not few."""
     takes = lambda N, K, rows: [ops.ring_tile(M, N, K) is not None for M in rows]
-    assert takes(1024, 2048, (300, 1024, 1060, 1288, 1516, 1592, 2048)) == [True, True, False, False, False, False, True]
-    assert takes(1024, 2048, (1600, 1744)) == takes(2048, 2048, (820, 1300)) == [True, True]
+    assert takes(1024, 2048, (300, 1024, 1060, 1288, 1516, 1536, 1592, 2048)) == [True] * 2 + [False] * 4 + [True] * 2
     assert takes(1024, 3072, (620, 1024, 1288, 1516, 1592, 1668, 2048)) == [True, True, False, False, False, True, True]
+    assert takes(1024, 3072, (2800, 3050, 3100, 3123, 3500)) == [False, False, True, True, True] and takes(2048, 3072, (826, 1000)) == [False, True]
     assert takes(2048, 2048, (560, 760)) == takes(2048, 6144, (1500, 1536)) == takes(6144, 4096, (480, 512)) == [False, False]
-    assert takes(2048, 6144, (1600, 1850)) == takes(6144, 4096, (540, 600)) == takes(2560, 9728, (1344, 1450)) == [True, True]
-    assert takes(6144, 2560, (250, 256)) == [False, True] and takes(2560, 9728, (1280, 1408)) == [False, False]
+    assert takes(2048, 2048, (820, 1300)) == takes(2048, 6144, (1550, 1850)) == takes(6144, 4096, (540, 600)) == takes(2560, 9728, (1344, 1450)) == [True, True]
+    assert takes(6144, 2560, (250, 256)) == [False, True] and takes(2560, 9728, (1150, 1280, 1408)) == [False] * 3
     assert takes(1024, 1024, (100, 1100, 2048)) == takes(1536, 1536, (100, 700, 1300)) == [True] * 3
